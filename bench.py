@@ -281,14 +281,7 @@ def main():
             lib.libgint_amd_set_mixed_precision(h, 0.0)
         tu = (C.c_double * 5)()
         lib.libgint_amd_tune_info(h, tu)
-        tms = (C.c_double * 256)()
-        tpk = (C.c_int * 256)()
-        lib.libgint_amd_tune_detail(h, tms, tpk)
-        top = sorted(((tms[i], i) for i in range(256) if tms[i] > 0), reverse=True)[:12]
-        log("autotune: classes by sampled time: " + ", ".join(
-            f"({i // 64}{(i // 16) % 4}|{(i // 4) % 4}{i % 4}) {ms:.1f}ms/{'tweko'[tpk[i]]}" for ms, i in top))
-        tune = {"classes_templated": int(tu[1]), "classes_workgroup": int(tu[2]), "classes_matrix_core": int(tu[3]),
-                "seconds": round(tu[4], 2)}
+        tune = {"classes_own_contraction": int(tu[2]), "classes_contraction_kernel": int(tu[3])}
         lib.libgint_amd_destroy_handle(h)
         return slots, tot, info, t_ing, mixed, tune
 
@@ -329,24 +322,18 @@ def main():
     lib.libgint_amd_timing_eco(hr, te)
     nsr = len(range(0, st.n_sets, a.stride * rs))
     log(f"roofline sample (every {a.stride * rs}th set quartet, {nsr}): serialised instrumented step {t_ser:.3f}s; "
-        f"kernel ms fm_r {tm[0]:.0f} tq {tm[1]:.0f} gqs {tm[2]:.0f} fixup {tm[3]:.0f} eco {te[0]:.0f}")
-    tms = (C.c_double * 256)()
-    tpk = (C.c_int * 256)()
-    lib.libgint_amd_tune_detail(hr, tms, tpk)
-    top = sorted(((tms[i], i) for i in range(256) if tms[i] > 0), reverse=True)[:16]
-    log("roofline sample autotune: classes by sampled time: " + ", ".join(
-        f"({i // 64}{(i // 16) % 4}|{(i // 4) % 4}{i % 4}) {ms:.1f}ms/{'tweko'[tpk[i]]}" for ms, i in top))
-    for cat, nm in ((0, "fm_r by type L"), (1, "tq by type L"), (2, "gqs by type L"), (4, "eco by type L")):
+        f"kernel ms fm_r {tm[0]:.0f} sq {tm[2]:.0f} fixup {tm[3]:.0f} eco {te[0]:.0f}")
+    for cat, nm in ((0, "fm_r by type L"), (2, "sq by type L"), (4, "eco by type L")):
         det = (C.c_double * 256)()
         lib.libgint_amd_timing_detail(hr, cat, det)
         top = sorted(((det[i], i) for i in range(256) if det[i] > 0), reverse=True)[:12]
         log(f"{nm}: " + ", ".join(f"L{i} {ms:.0f}ms" for ms, i in top))
     lib.libgint_amd_destroy_handle(hr)
     value = slots / (tot / a.steps) if a.steps else None
-    names = ["fm_r", "tq", "gqs", "fixup", "eco"]
-    kms = [tm[i] for i in range(4)] + [te[0]]
-    kfl = [float(rstats[6]), tm[9], tm[10], 0.0, te[2]]
-    nl = [tm[4 + i] for i in range(4)] + [te[1]]
+    names = ["fm_r", "sq", "fixup", "eco"]
+    kms = [tm[0], tm[2], tm[3], te[0]]
+    kfl = [float(rstats[6]), tm[10], 0.0, te[2]]
+    nl = [tm[4], tm[6], tm[7], te[1]]
     dom = int(np.argmax(kms))
     achieved = kfl[dom] / (kms[dom] * 1e-3) / 1e12 if kms[dom] > 0 else 0.0
     traffic, traffic_src = measured_traffic(names[dom], s.describe())
@@ -358,10 +345,9 @@ def main():
             "timing": "HIP events around each launch on its stream, every launch serialised on one stream",
             "kernel_ms_serialised": {n: round(m, 2) for n, m in zip(names, kms)},
             "kernel_tflops": {n: round(f / (m * 1e-3) / 1e12, 4) if m > 0 else 0 for n, f, m in zip(names, kfl, kms)},
-            "flops": "fm_r: the reference chain's Fm + VRR FLOPs of the kept (slot, class) pairs; tq: "
-                     "contraction 2 n_prm ncp + HRR + SPH + 9 Ns per contracted quartet; eco (matrix cores): the "
-                     "contraction 2 n_prm ncp of the classes with many contractions; gqs: the rest of those "
-                     "classes and the contraction of the others"}
+            "flops": "fm_r: the reference chain's Fm + VRR FLOPs of the kept (slot, class) pairs; eco (matrix cores): "
+                     "the contraction 2 n_prm ncp of the classes it takes; sq: contraction 2 n_prm ncp of the others, "
+                     "HRR + SPH + 9 Ns per contracted quartet"}
 
     # max|dK| and the CPU baseline: a strided sample of the same stream,
     # through the product (stream mode) and the FP64 oracle on all cores
@@ -427,7 +413,7 @@ def main():
                    "abi_ingestion": abi, "set_level_ingestion_s": round(t_ing, 2),
                    "resident_plan_GiB": round(info[0] / 2**30, 3),
                    "path": "FP64, resident plan, fused Hermite cell sum per quartet type"},
-        "max_dK": check, "mixed_precision": mixed, "autotune": tune, "roofline": roof, "cpu_baseline": cpu,
+        "max_dK": check, "mixed_precision": mixed, "contraction": tune, "roofline": roof, "cpu_baseline": cpu,
     }
     print(json.dumps(out), flush=True)
 

@@ -118,18 +118,17 @@ void libgint_amd_enable_stats(void *handle, int on);
 void libgint_amd_stats(void *handle, uint64_t out[8]);
 /* per-kernel device time with HIP events on the handle's stream */
 void libgint_amd_enable_timing(void *handle, int on);
-/* out[0..3] ms in fm_r / the wavefront-per-set-quartet kernels tq /
-   the per-set-quartet quartet kernel gqs / fix-up, out[4..7] launches,
-   out[9], out[10] algorithmic FLOPs of tq and gqs (out[8] and out[11] = 0:
-   the fm_r FLOPs are libgint_amd_stats out[6]) */
+/* out[0..3] ms in fm_r / nothing / the quartet kernel sq / fix-up,
+   out[4..7] launches, out[10] algorithmic FLOPs of sq (the others 0: the
+   fm_r FLOPs are libgint_amd_stats out[6]) */
 void libgint_amd_timing(void *handle, double out[12]);
 /* the matrix-core contraction of the classes with many contractions (done
-   before the per-class kernel, which then reads its result): out[0] ms,
+   before the quartet kernel, which then reads its result): out[0] ms,
    [1] launches, [2] algorithmic FLOPs (2 n_prm ncp per contraction) */
 void libgint_amd_timing_eco(void *handle, double out[3]);
 void libgint_amd_reset_counters(void *handle);
-/* ms per launch key of one category of libgint_amd_timing (0 fm_r, 1 tq,
-   2 gqs, 3 fix-up, 4 matrix-core contraction) by the quartet type's total
+/* ms per launch key of one category of libgint_amd_timing (0 fm_r, 1 none,
+   2 sq, 3 fix-up, 4 matrix-core contraction) by the quartet type's total
    angular momentum */
 void libgint_amd_timing_detail(void *handle, int cat, double out[256]);
 /* bit 0: route every surviving slot through the class-dependent screening
@@ -137,14 +136,13 @@ void libgint_amd_timing_detail(void *handle, int cat, double out[256]);
    kernel of a chunk on the handle's stream, one after the other (per-kernel
    durations without overlap, for profiling; results are unchanged); bit 2:
    wait for the work of each quartet type and report its completion on
-   stderr (progress of long K-builds; results are unchanged); bit 3: every
-   class that can take it goes to the Kronecker HRR, whatever the autotuner
-   chose (resident plans) or the default rule (call streams), with the matrix-core contraction where the class
-   has one (else its own); bit 4: the same with the class's own contraction
-   where it fits (tests of that path; results are unchanged) */
+   stderr (progress of long K-builds; results are unchanged); bit 3: the
+   contraction of every type whose classes have one runs in the kernel of
+   its own (k_eco), whatever the rule on primitive quartets per row says;
+   bit 4: of no type (tests of both paths; results are unchanged) */
 void libgint_amd_set_debug(void *handle, int flags);
 /* libgint_amd_plan_execute replays the plan's launches (every chunk's
-   kernels on the handle's stream and its side streams) as one HIP graph:
+   kernels on the handle's stream and its side stream) as one HIP graph:
    captured at the first execution, replayed at the next ones while the
    buffers, P / K arrays, potential and debug flags it was captured with are
    unchanged (else captured again).  Executions with timing, statistics or
@@ -154,13 +152,8 @@ void libgint_amd_set_debug(void *handle, int flags);
 void libgint_amd_set_graph(void *handle, int on);
 /* out[0] graphs on, [1] captures, [2] replays, [3] a graph is held */
 void libgint_amd_graph_info(void *handle, uint64_t out[4]);
-/* Autotuner (default on): at the first libgint_amd_plan_execute of a plan,
-   each class of each quartet type gets the fastest of its schedules, timed
-   on the type's first set quartets (into a scratch K): the templated
-   one-wavefront kernel, the workgroup kernel with its own contraction, or
-   the matrix-core contraction followed by the workgroup kernel.  Decisions
-   are kept per (class, contractions, primitive quartets per row in powers
-   of two) for the process and reused.  on = 0 keeps the built-in choice. */
+/* No effect: the kernels of a quartet type are chosen by a rule on its
+   primitive quartets per row, not by timing.  Kept for callers that set it. */
 void libgint_amd_set_autotune(void *handle, int on);
 /* Mixed precision for resident plans (tau = 0, the default: FP64 only).
    The first execution after plan_end (or after tau is first set) runs in
@@ -176,15 +169,10 @@ void libgint_amd_set_mixed_precision(void *handle, double tau);
 /* out[0] tau, [1] calibrated, [2] set quartets routed to single precision
    by the last execution, [3] set quartets of the plan */
 void libgint_amd_mixed_info(void *handle, double out[4]);
-/* out[0] the plan is tuned, [1..3] classes given the templated kernel /
-   the workgroup kernel with its own contraction / the matrix-core
-   contraction (each with either HRR), [4] seconds spent */
+/* out[0] the plan's kernels are chosen, [1] 0, [2], [3] classes contracted
+   by k_sq itself / by k_eco, [4] 0 (seconds spent) */
 void libgint_amd_tune_info(void *handle, double out[5]);
-/* per class code ((la*4+lb)*4+lc)*4+ld: ms[] the chosen schedule's time on
-   the timing samples (summed over quartet types), pick[] that schedule
-   (0 templated, 1 workgroup, 2 matrix-core contraction + layered HRR,
-   3 matrix-core contraction + Kronecker HRR, 4 workgroup kernel's own
-   contraction + Kronecker HRR; last type timed) */
+/* nothing is timed: zeros */
 void libgint_amd_tune_detail(void *handle, double ms[256], int pick[256]);
 /* resident plans: the calls between plan_begin and plan_end are kept on the
    device; plan_execute adds their exchange terms to K for the density of the

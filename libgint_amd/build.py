@@ -24,9 +24,9 @@ TCG_SHA256 = None
 REF_SRC = "/root/reference/src"
 
 HOST_SRC = ["engine.cpp", "abi.cpp", "plan.cpp", "boys_table.cpp", "c0_file.cpp", "server.cpp"]
-DEV_SRC = ["kernels.hip", "kernels_tq.hip", "kernels_eco.hip"]
-# kernels_tq_part.hip is built once per part of the templated class kernels
-TQ_PARTS = 8
+DEV_SRC = ["kernels.hip", "kernels_sq.hip", "kernels_eco.hip"]
+# kernels_sq_part.hip is built once per highest angular momentum
+SQ_LM = (1, 2, 3)
 HIPFLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-munsafe-fp-atomics",
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall", "-Wno-unused-function"]
 HOSTFLAGS = ["-O2", "-std=c++17", "-fPIC", "-fopenmp", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__",
@@ -70,9 +70,9 @@ def build_lib(verbose=False, jobs=None):
     for src in DEV_SRC:
         o = os.path.join(BUILD, src + ".o")
         steps.append(([HIPCC] + HIPFLAGS + ["-c", os.path.join(CSRC, src), "-o", o], o))
-    for part in range(TQ_PARTS):
-        o = os.path.join(BUILD, "kernels_tq_part%d.o" % part)
-        steps.append(([HIPCC] + HIPFLAGS + ["-DGINT_TQ_PART=%d" % part, "-c", os.path.join(CSRC, "kernels_tq_part.hip"),
+    for lm in SQ_LM:
+        o = os.path.join(BUILD, "kernels_sq_lm%d.o" % lm)
+        steps.append(([HIPCC] + HIPFLAGS + ["-DGINT_SQ_LM=%d" % lm, "-c", os.path.join(CSRC, "kernels_sq_part.hip"),
                        "-o", o], o))
     # the compiles are independent: run them side by side (at most 16 jobs)
     jobs = jobs or min(16, os.cpu_count() or 1)

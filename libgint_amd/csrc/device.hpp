@@ -39,7 +39,7 @@ inline constexpr int class_code(int la, int lb, int lc, int ld) { return ((la * 
 
 // One row: a set quartet at bra/ket images (n1,n2) with its primitive
 // quartets (one libgint_add_shell call).  Its contracted blocks sit at
-// (row - first row of the chunk) * TypePlan::ebytes in the contraction buffer.
+// (row - first row of the chunk) * eco_row in the contraction buffer.
 struct RowRec {
    uint32_t prm_off;   // first primitive quartet of the row
    uint32_t n_prm;
@@ -128,10 +128,10 @@ struct ClassPlan {
    int sph_flops;            // 2 m n k over the four stages
 };
 
-// Plan of one quartet type.  Blocks (e0|f0) with e in [LA0,LA], f in
-// [LC0,LC] (e outer, layout [ie][jf] inside a block) are produced per
-// primitive quartet, summed over lattice cells; each class reads its own
-// sub-range of them.
+// Plan of one quartet type.  The blocks (e0|f0) with e in [LA0,LA], f in
+// [LC0,LC] are produced per primitive quartet, summed over lattice cells, as
+// one matrix: bra components (shell e outer) x ket components (shell f
+// outer); each class reads a rectangle of it.
 struct TypePlan {
    int nsh[4];
    int l[4][MAXSH];
@@ -139,7 +139,7 @@ struct TypePlan {
    int nclass;               // nsh0*nsh1*nsh2*nsh3, sa outer
    int LA0, LA, LC0, LC, L;
    int ncp;
-   int cpoff[7][7];
+   int bcoff[7];             // first bra component of shell e
    int nkc;                  // ket cartesian components, f in [LC0,LC]
    int kcoff[7];             // first of shell f among them
    int nbh;                  // bra Hermite triples t+u+v <= LA
@@ -147,15 +147,11 @@ struct TypePlan {
    int has00;                // LA0 == 0 && LC0 == 0
    int nL;                   // distinct class L values
    int Ls[16];
-   int ebytes;               // contracted doubles per row: sum over classes nlabcd ncp
    int cls_code[MAXTC];      // class_code(la,lb,lc,ld) of class k
    int cls_sh[MAXTC];        // sa | sb<<4 | sc<<8 | sd<<12
    int cls_gate[MAXTC];      // index into Ls
    int cls_nl[MAXTC];        // nla*nlb*nlc*nld
    int cls_ncp[MAXTC];
-   int cls_eoff[MAXTC];      // offset of class k inside a row's contracted doubles
-   int co_off[4][MAXSH];     // quartet kernel: coefficients of shell s of centre t in LDS, nl x 16
-   int nco_tot;
    int fun0[4][MAXSH];       // first spherical function of shell s within set t (sets list shells in order)
    int nfun[4];              // spherical functions of set t
    unsigned long long cls_mult[MAXTC];   // checksum multiplier of class k (odd)
@@ -258,6 +254,62 @@ struct EcoArgs {
    size_t row_doubles;        // contraction buffer doubles per row
 };
 
+// Work of k_sq (kernels_sq.hpp).  A side (bra or ket) of a type is cut into
+// tiles: runs of (shell pair, contraction pair) units.  A unit has the
+// Hermite-expanded components of shells l1 .. l1 + l2 as its rows (ket:
+// columns) before and (2 l1 + 1)(2 l2 + 1) functions after the transform.
+struct SqSp {             // the units of one shell pair in a tile
+   uint8_t l1, l2;
+   uint8_t s1, s2;        // its shells on the two centres
+   uint8_t c0, nc;        // its contraction pairs c0 .. c0 + nc - 1 (i1 n2 + i2)
+   uint8_t n2;            // contractions of the second shell
+   uint8_t pad;
+   uint16_t row0, fn0;    // first row and function in the tile
+   int16_t f1, f2;        // first function of the shells, from the start of the tile's function ranges
+};
+struct SqTile {
+   uint16_t nrow, nfn, nrc, nsp;
+   uint16_t comp0, ncomp;           // its components among the type's
+   uint16_t r1, n1, r2, n2;         // its function ranges on the two centres (start, count)
+   uint32_t sp, row, rc, fn;        // first entries in the tables
+};
+struct SqItem {           // one (bra tile, ket tile)
+   uint16_t bt, kt;
+   uint16_t lds_k, lm;    // its P and K blocks fit in LDS
+   int32_t eco_off;       // its class's place in a row of the contraction buffer, or -1: own contraction
+   int32_t o_wc, o_pk, o_c;   // LDS offsets, doubles
+};
+constexpr int SQ_NW = 16;      // primitive quartets per window (four matrix-core steps)
+constexpr int SQ_MAXROW = 80, SQ_MAXRC = 16, SQ_MAXFN = 56;   // of a tile
+// LDS tables of an item, bytes: ket columns, coefficient offsets of the
+// units, ket functions, window of primitive quartets
+constexpr int SQ_TAB_URB = 2 * SQ_MAXROW, SQ_TAB_URK = SQ_TAB_URB + 4 * SQ_MAXRC,
+              SQ_TAB_FN = SQ_TAB_URK + 4 * SQ_MAXRC, SQ_TAB_IP = SQ_TAB_FN + 4 * SQ_MAXFN,
+              SQ_TAB_BYTES = (SQ_TAB_IP + 4 * SQ_NW + 15) & ~15;
+struct SqArgs {
+   const SqItem *items;
+   const SqTile *tiles;
+   const SqSp *sps;
+   const uint16_t *rows;   // component (from comp0) | unit << 8
+   const uint32_t *rcs;    // unit, two words: contraction of the two sets, 8 bits each;
+                           // first row | first component << 8 | last + 1 << 16
+   const uint32_t *fns;    // function: c | d << 8 (from the tile's ranges) | shell pair << 16
+   int nitem;
+   int ncon[4];            // contractions of the four sets
+   int o_co;               // LDS offset, doubles, of the coefficients
+};
+struct SqPlan {
+   std::vector<SqItem> items;
+   std::vector<SqTile> tiles;
+   std::vector<SqSp> sps;
+   std::vector<uint16_t> rows;
+   std::vector<uint32_t> rcs, fns;
+   int lm = 0;
+   int lds_bytes = 0;
+   void *dev = nullptr;    // all tables on the device, one after the other
+   size_t off[6] = {};
+};
+
 // the K layout of class k of group g
 GINT_HDI KsGroup group_ks(const BatchDev &b, const TypePlan &tp, const GroupRec &g, int k)
 {
@@ -283,60 +335,21 @@ GINT_HDI size_t tra_index(int ia, int isa, int ib, int isb, int ic, int isc, int
           (size_t)id * nsd + isd;
 }
 
-struct Scratch {
-   double *ptr;
-   size_t doubles;
-   unsigned grid;   // workgroups of a k_gqs part that uses it (each its own slice)
-};
-
-constexpr unsigned SCRATCH_GRID = 2048;
-
 // The no-allocation executor (libgint_amd_plan_execute_noalloc) takes all
 // its device scratch from one static array of NOALLOC_BYTES per GPU:
 //   [0, 256)                      chunk counters (fix-up entries, overflow)
 //   fix-up list                   NOALLOC_FIX entries of 2 words
 //   fix-up workspace              NOALLOC_FIX x (MAX_NCP + 16) doubles
-//   gqs workspace                 NOALLOC_GWS_BYTES
 //   primitive blocks (ac0)        the rest, NOALLOC_AC0_BYTES
 constexpr size_t NOALLOC_BYTES = 176ull << 20;
 constexpr int MAX_NCP = 84 * 84;              // (e0|f0) doubles of an (f f|f f) type
 constexpr size_t NOALLOC_FIX = 256;
 constexpr size_t NOALLOC_OFF_FIX = 256;
 constexpr size_t NOALLOC_OFF_FIXWS = NOALLOC_OFF_FIX + ((2 * 4 * NOALLOC_FIX + 255) & ~(size_t)255);
-constexpr size_t NOALLOC_OFF_GWS = NOALLOC_OFF_FIXWS + ((NOALLOC_FIX * (MAX_NCP + 16) * 8 + 255) & ~(size_t)255);
-constexpr size_t NOALLOC_GWS_BYTES = 32ull << 20;
-constexpr size_t NOALLOC_OFF_AC0 = NOALLOC_OFF_GWS + NOALLOC_GWS_BYTES;
+constexpr size_t NOALLOC_OFF_AC0 = NOALLOC_OFF_FIXWS + ((NOALLOC_FIX * (MAX_NCP + 16) * 8 + 255) & ~(size_t)255);
 constexpr size_t NOALLOC_AC0_BYTES = NOALLOC_BYTES - NOALLOC_OFF_AC0;
 static_assert(NOALLOC_AC0_BYTES >= (120ull << 20), "no-allocation scratch layout");
 constexpr unsigned STATS_SLOTS = 4096;   // counter triples the kernels spread their statistics over
-
-// LDS plan of one class in the quartet kernel
-struct CqLayout {
-   int lb;          // contractions per pass
-   int lws;         // workspace doubles per contraction: 3 ycap + Nc
-   int o_ws;        // workspace in LDS (lb x lws), unless ws_global
-   int o_kp;        // coefficient products [lb][CQ_PCH]
-   int o_I;         // spherical integrals of every contraction [nq][Ns] (reduce)
-   int o_src;       // first entry of the class's block map (class element -> type element) in the type's maps
-   int reduce;
-   int ws_global;   // workspace in HBM (gws + blockIdx * lb * lws)
-   int skip;        // the class runs in its own templated kernel instead
-   int part;        // which of the GQS_PARTS concurrent launches takes the class
-   int bytes;
-   int eco;         // contracted on the matrix cores (k_eco): k_gqs reads the contraction buffer
-   int eco_off;     // the class's offset in a row of the contraction buffer
-   int o_kron;      // LDS of the Kronecker path: bra components x ket spherical pairs (whole 16x16 tiles), T tables
-   int kron_ws;     // doubles of the Kronecker path's row maps (up to 8 rows); 0: the class cannot take the path
-   int o_kmap;      // LDS offset of those maps, or -1: in the workgroup's HBM slice
-   int kron;        // the class takes the Kronecker path (a schedule of the autotuner)
-   int kron_kb;     // its contractions per pass
-   int o_kc;        // LDS of one contraction's blocks and CQ_PCH coefficient products for the Kronecker path
-                    // with the class's own contraction (no eco), or -1: that schedule does not fit
-   int o_kacc;      // LDS of the K accumulators (the four K blocks of a set quartet, summed over its
-                    // contractions before the atomics), or -1
-   int kacc;        // doubles of the accumulators per spin
-   int kacc_cap;    // doubles reserved for them (kacc or 2 kacc: one or two spins)
-};
 
 // address of the no-allocation scratch array on the current device, looked
 // up (hipGetSymbolAddress) once per device; null if the lookup failed
@@ -348,32 +361,23 @@ void *noalloc_scratch();
 int launch_zero_u32(uint32_t *p, int n, void *stream);
 int launch_fm_r(const TypePlan &tp, const DevTables &t, const BatchDev &b, void *stream);
 int launch_fixup(const TypePlan &tp, const DevTables &t, const BatchDev &b, uint32_t n_fix, void *stream);
-// one-wavefront-per-set-quartet kernels of the classes with at most 128
-// block columns (kernels_tq.hip)
-bool tq_has(int code);
-int launch_tq(int cls_k, const TypePlan &tp, const DevTables &t, const BatchDev &b, const KTargets &kt,
-              const int *srcmap, void *stream);
-// per-class LDS plans and block maps of a type for the quartet kernel
-void make_cq_plan(const TypePlan &tp, const std::vector<ClassPlan> &cps, std::vector<CqLayout> &lays,
-                  std::vector<int> &srcmaps, int *lds_bytes, int *gws_stride);
-// the k_gqs classes of a type over its GQS_PARTS launches, balanced by cost
-void assign_parts(const TypePlan &tp, const std::vector<ClassPlan> &cps, std::vector<CqLayout> &lays);
-// the classes of a type that k_gqs takes are split into this many launches,
-// balanced by their estimated cost, which run concurrently on separate streams
-constexpr int GQS_PARTS = 4;
-// npc: the classes of the type that this part takes (work items are
-// (set quartet, class) pairs)
-constexpr unsigned GQS_MAX_GRID = 8192;
-int launch_gqs(const TypePlan &tp, const ClassPlan *d_cps, const CqLayout *d_lays, const int *d_srcmaps, int lds_bytes,
-               int gws_stride, int part, int npc, const DevTables &t, const BatchDev &b, const KTargets &kt, Scratch s,
-               void *stream, bool wide = false);
-// contraction of primitive blocks on the matrix cores for the classes with
-// CqLayout::eco (kernels_eco.hip): k_gqs classes with at least this many
-// contractions
+// from the chunk's blocks to K (kernels_sq.hpp): the classes of one plan
+// (max_np: the most primitives of a set in the chunk's type)
+int launch_sq(const TypePlan &tp, int max_np, const BatchDev &b, const DevTables &t, const KTargets &kt,
+              const SqPlan &sp, void *stream);
+// contraction of primitive blocks on the matrix cores (kernels_eco.hip) for
+// classes with at least this many contractions
 constexpr int ECO_MIN_NQ = 8;
-// classes with at least this many contractions have a place in the
-// contraction buffer (the autotuner may move them to the matrix cores)
-constexpr int ECO_CAND_NQ = 4;
+struct EcoPlan {
+   std::vector<EcoItem> items;
+   std::vector<int> off;       // per class: its place in a row of the contraction buffer, or -1
+   std::vector<int> info;      // [MAXTC] first entry of the class's column map, [MAXTC] off
+   std::vector<int> srcmaps;   // class column -> type column
+   size_t row = 0;             // doubles per row of the buffer
+};
+void make_eco_plan(const TypePlan &tp, const std::vector<ClassPlan> &cps, EcoPlan &ep);
+void make_sq_plan(const TypePlan &tp, const std::vector<ClassPlan> &cps, const EcoPlan &ep, bool wf, int nspin, bool eco,
+                  SqPlan &sp);
 int launch_eco(const TypePlan &tp, const BatchDev &b, const EcoArgs &e, void *stream);
 // mixed precision: max |P| (*out, zeroed first) and the route of each set
 // quartet of a chunk from its calibrated magnitude

@@ -146,21 +146,21 @@ Engine::~Engine()
       if (ti.d_plan) (void)hipFree(ti.d_plan);
       if (ti.d_e1) (void)hipFree(ti.d_e1);
       if (ti.d_e2) (void)hipFree(ti.d_e2);
-      if (ti.d_cps) (void)hipFree(ti.d_cps);
-      if (ti.d_lays) (void)hipFree(ti.d_lays);
+      for (SqPlan *sp = &ti.sq[0][0][0]; sp != &ti.sq[0][0][0] + 8; sp++) {
+         if (sp->dev) (void)hipFree(sp->dev);
+      }
       if (ti.d_srcmaps) (void)hipFree(ti.d_srcmaps);
       if (ti.d_eco_info) (void)hipFree(ti.d_eco_info);
       if (ti.d_eco_items) (void)hipFree(ti.d_eco_items);
    }
    void *bufs[] = {d_data_, d_C0_, d_grid_, d_bw_, d_ftab_, d_cell_, d_neighs_, d_work_,
-                   d_fix_, d_fix_ws_, d_scratch_, d_stats_, d_fixcnt_, d_out_, d_mix_};
+                   d_fix_, d_fix_ws_, d_stats_, d_fixcnt_, d_out_, d_mix_};
    for (void *b : bufs)
       if (b) (void)hipFree(b);
    for (void *e : ev_pool_) (void)hipEventDestroy((hipEvent_t)e);
    for (void *e : ev_join_)
       if (e) (void)hipEventDestroy((hipEvent_t)e);
-   for (void *q : side_)
-      if (q) (void)hipStreamDestroy((hipStream_t)q);
+   if (side_) (void)hipStreamDestroy((hipStream_t)side_);
 }
 
 void Engine::init()
@@ -181,9 +181,8 @@ void Engine::init()
 
 void Engine::ensure_side()
 {
-   for (int i = 0; i < NSIDE; i++)
-      if (!side_[i]) HIPCHECK(hipStreamCreateWithFlags((hipStream_t *)&side_[i], hipStreamNonBlocking));
-   for (int i = 0; i <= NSIDE; i++)
+   if (!side_) HIPCHECK(hipStreamCreateWithFlags((hipStream_t *)&side_, hipStreamNonBlocking));
+   for (int i = 0; i < 2; i++)
       if (!ev_join_[i]) HIPCHECK(hipEventCreateWithFlags((hipEvent_t *)&ev_join_[i], hipEventDisableTiming));
 }
 
@@ -267,36 +266,6 @@ int Engine::set_sig(int i)
    return s.sig;
 }
 
-// The matrix-core contraction of a type: its classes with CqLayout::eco,
-// one work item per 64 columns x 64 contractions of each, and the row
-// length of the contraction buffer.
-static void make_eco_items(TypeInfo &ti)
-{
-   const TypePlan &tp = ti.plan;
-   ti.eco_items.clear();
-   ti.eco_row = 0;
-   ti.eco_info.assign(2 * MAXTC, 0);
-   for (int k = 0; k < tp.nclass; k++) {
-      const CqLayout &y = ti.lays[k];
-      ti.eco_info[k] = y.o_src;
-      ti.eco_info[MAXTC + k] = y.eco_off;
-      const int cols = tp.cls_ncp[k], nq = tp.cls_nl[k];
-      if (y.eco_off >= 0) ti.eco_row = std::max(ti.eco_row, (size_t)y.eco_off + (size_t)nq * cols);
-      if (!y.eco) continue;
-      for (int jt0 = 0; jt0 * 16 < cols; jt0 += 4)
-         for (int qb = 0; qb * 64 < nq; qb++) ti.eco_items.push_back(EcoItem{(uint16_t)k, (uint16_t)jt0, (uint16_t)qb, 0});
-   }
-   // items in the order of the first type column they read: the classes
-   // share the row's blocks (a block (e,f) serves every class with
-   // la <= e <= la+lb, lc <= f <= lc+ld), so items that run together read
-   // the same columns of a row that is larger than the caches
-   auto first_col = [&](const EcoItem &it) { return ti.srcmaps[ti.lays[it.k].o_src + it.jt0 * 16]; };
-   std::stable_sort(ti.eco_items.begin(), ti.eco_items.end(), [&](const EcoItem &a, const EcoItem &b) {
-      const int ca = first_col(a), cb = first_col(b);
-      return ca < cb || (ca == cb && (a.k < b.k || (a.k == b.k && a.qb < b.qb)));
-   });
-}
-
 int Engine::type_of(int i, int j, int k, int l)
 {
    const std::array<int, 4> sets = {i, j, k, l};
@@ -326,9 +295,11 @@ int Engine::type_of(int i, int j, int k, int l)
          const int code = ti.plan.cls_code[c];
          ti.cplans.push_back(make_plan(code / 64, (code / 16) % 4, (code / 4) % 4, code % 4));
       }
-      make_cq_plan(ti.plan, ti.cplans, ti.lays, ti.srcmaps, &ti.cq_lds, &ti.cq_gws);
-      for (const CqLayout &y : ti.lays) ti.cq_wide = ti.cq_wide || (y.kron && !y.skip);
-      make_eco_items(ti);
+      make_eco_plan(ti.plan, ti.cplans, ti.eco);
+      for (int sp = 0; sp < 2; sp++)
+         for (int e = 0; e < 2; e++)
+            for (int f = 0; f < 2; f++)
+               make_sq_plan(ti.plan, ti.cplans, ti.eco, f == 1, sp + 1, e == 1, ti.sq[sp][e][f]);
       types_.push_back(ti);
       q_.emplace_back();
       it = type_ids_.emplace(sig, (int)types_.size() - 1).first;
@@ -798,7 +769,6 @@ void Engine::plan_end()
    for (auto &d : plan_dev_) d.release();
    plan_dev_.clear();
    upload(q_, plan_dev_, true);
-   plan_tuned_ = false;
    mixed_calibrated_ = false;
    // tables and basis data resident now, so that an execution needs no
    // allocation (plan_execute_noalloc)
@@ -817,9 +787,6 @@ void Engine::plan_execute()
    RunBufs w{};
    KTargets kt{};
    if (!prepare_exec(plan_dev_, plan_max_index_, w, kt, FP_size_)) return;
-   // (not while an integral-output array is set: its classes write there)
-   if (autotune_on_ && !plan_tuned_ && !d_out_) autotune(w, kt);
-   if (debug_ & 24) force_kron(plan_dev_, (debug_ & 16) != 0);
    mixed_mode_ = 0;
    if (mixed_tau_ > 0.0 && !d_out_) {
       ensure_mixed();
@@ -1027,18 +994,32 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
          HIPCHECK(hipMemcpy(ti.d_e1, ti.e1.data(), sizeof(uint32_t) * ti.e1.size(), hipMemcpyHostToDevice));
          HIPCHECK(hipMalloc((void **)&ti.d_e2, sizeof(uint32_t) * ti.e2.size()));
          HIPCHECK(hipMemcpy(ti.d_e2, ti.e2.data(), sizeof(uint32_t) * ti.e2.size(), hipMemcpyHostToDevice));
-         HIPCHECK(hipMalloc((void **)&ti.d_cps, sizeof(ClassPlan) * ti.cplans.size()));
-         HIPCHECK(hipMemcpy(ti.d_cps, ti.cplans.data(), sizeof(ClassPlan) * ti.cplans.size(), hipMemcpyHostToDevice));
-         HIPCHECK(hipMalloc((void **)&ti.d_lays, sizeof(CqLayout) * ti.lays.size()));
-         HIPCHECK(hipMemcpy(ti.d_lays, ti.lays.data(), sizeof(CqLayout) * ti.lays.size(), hipMemcpyHostToDevice));
-         HIPCHECK(hipMalloc((void **)&ti.d_srcmaps, sizeof(int) * ti.srcmaps.size()));
-         HIPCHECK(hipMemcpy(ti.d_srcmaps, ti.srcmaps.data(), sizeof(int) * ti.srcmaps.size(), hipMemcpyHostToDevice));
-         HIPCHECK(hipMalloc((void **)&ti.d_eco_info, sizeof(int) * ti.eco_info.size()));
-         HIPCHECK(hipMemcpy(ti.d_eco_info, ti.eco_info.data(), sizeof(int) * ti.eco_info.size(), hipMemcpyHostToDevice));
-         if (!ti.eco_items.empty()) {
-            HIPCHECK(hipMalloc((void **)&ti.d_eco_items, sizeof(EcoItem) * ti.eco_items.size()));
-            HIPCHECK(hipMemcpy(ti.d_eco_items, ti.eco_items.data(), sizeof(EcoItem) * ti.eco_items.size(),
-                               hipMemcpyHostToDevice));
+         auto put = [](auto *&dst, const auto &v) {
+            if (v.empty()) return;
+            HIPCHECK(hipMalloc((void **)&dst, sizeof(v[0]) * v.size()));
+            HIPCHECK(hipMemcpy(dst, v.data(), sizeof(v[0]) * v.size(), hipMemcpyHostToDevice));
+         };
+         put(ti.d_srcmaps, ti.eco.srcmaps);
+         put(ti.d_eco_info, ti.eco.info);
+         put(ti.d_eco_items, ti.eco.items);
+         for (SqPlan *sp = &ti.sq[0][0][0]; sp != &ti.sq[0][0][0] + 8; sp++) {
+            if (sp->items.empty()) continue;
+            std::vector<char> all;
+            int n = 0;
+            auto add = [&](const auto &v) {
+               all.resize((all.size() + 15) & ~(size_t)15);
+               sp->off[n++] = all.size();
+               const char *p = (const char *)v.data();
+               all.insert(all.end(), p, p + sizeof(v[0]) * v.size());
+            };
+            add(sp->items);
+            add(sp->tiles);
+            add(sp->sps);
+            add(sp->rows);
+            add(sp->rcs);
+            add(sp->fns);
+            HIPCHECK(hipMalloc(&sp->dev, all.size()));
+            HIPCHECK(hipMemcpy(sp->dev, all.data(), all.size(), hipMemcpyHostToDevice));
          }
       }
       dev_put(D.rows, D.cap[0], Q.rows);
@@ -1060,15 +1041,18 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
          const GroupRec &g = Q.groups[gi];
          return (g.ksmode & KS_SETLEVEL) ? ks_from_set(Q.kss[g.ks], tp, k) : Q.ksg[(size_t)g.ks + k];
       };
-      D.class_used.assign(tp.nclass, 0);
-      for (size_t gi = 0; gi < D.n_groups; gi++) {
-         if (Q.groups[gi].ksmode & KS_SETLEVEL) {
-            for (int k = 0; k < tp.nclass; k++) D.class_used[k] = 1;
-            continue;
-         }
-         for (int k = 0; k < tp.nclass; k++)
-            if (ks_count(gks(gi, k).flags)) D.class_used[k] = 1;
+      D.used = false;
+      D.max_np = 1;
+      for (const GroupRec &g : Q.groups)
+         for (int x = 0; x < 4; x++) D.max_np = std::max(D.max_np, (int)((g.np4 >> (4 * x)) & 15) + 1);
+      for (size_t gi = 0; gi < D.n_groups && !D.used; gi++) {
+         D.used = (Q.groups[gi].ksmode & KS_SETLEVEL) != 0;
+         for (int k = 0; k < tp.nclass && !D.used; k++) D.used = ks_count(gks(gi, k).flags) != 0;
       }
+      // long rows: the contraction of the classes with many contractions on
+      // the matrix cores
+      D.eco = !ti.eco.items.empty() && (double)D.n_prm >= ECO_MIN_PRM * (double)D.n_rows;
+      const size_t eco_row = D.eco ? ti.eco.row : 0;
       // chunks of whole groups whose primitive blocks fit `wbytes`; a set
       // quartet larger than the allocating path's buffer gets a chunk of its
       // own, for which that buffer grows (ensure_work)
@@ -1079,7 +1063,7 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
          for (uint32_t r = g.row0; r < g.row1; r++) gp += Q.rows[r].n_prm;
          // its primitive blocks and, for the matrix-core classes, its rows of
          // the contraction buffer (behind the chunk's blocks in the work buffer)
-         gbytes[gi] = gp * sizeof(double) * (size_t)tp.ncp + (size_t)(g.row1 - g.row0) * ti.eco_row * sizeof(double);
+         gbytes[gi] = gp * sizeof(double) * (size_t)tp.ncp + (size_t)(g.row1 - g.row0) * eco_row * sizeof(double);
          D.max_group_bytes = std::max(D.max_group_bytes, gbytes[gi]);
       }
       auto make_chunks = [&](size_t wbytes, std::vector<Chunk> &out, bool flops) {
@@ -1088,7 +1072,7 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
          for (size_t gi = 0; gi < D.n_groups; gi++) {
             const GroupRec &g = Q.groups[gi];
             const size_t gb = gbytes[gi];
-            const size_t gp = (gb - (size_t)(g.row1 - g.row0) * ti.eco_row * sizeof(double)) /
+            const size_t gp = (gb - (size_t)(g.row1 - g.row0) * eco_row * sizeof(double)) /
                               (sizeof(double) * (size_t)tp.ncp);
             if (bytes + gb > wbytes && c.g1 > c.g0) {
                if (flops) D.max_chunk_bytes = std::max(D.max_chunk_bytes, bytes);
@@ -1115,9 +1099,7 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
                const ClassPlan &cp = ti.cplans[k];
                const double contr = nq * 2.0 * (double)gp * cp.ncp;
                const double f = nq * ((double)(g.row1 - g.row0) * cp.hrr_flops + cp.sph_flops + 9.0 * cp.Ns);
-               if (ti.lays[k].skip) {
-                  c.tq_flops += contr + f;
-               } else if (ti.lays[k].eco) {
+               if (D.eco && ti.eco.off[k] >= 0) {
                   c.eco_flops += contr;
                   c.k3_flops += f;
                } else {
@@ -1229,6 +1211,15 @@ DevTables Engine::dev_tables() const
    return t;
 }
 
+// whether a type's contraction runs on the matrix cores kernel (k_eco); the
+// debug bits 3 and 4 force it on or off (not in the no-allocation scratch,
+// whose chunks are cut for the rule)
+bool Engine::use_eco(const TypeInfo &ti, const TypeDev &td, bool forced) const
+{
+   if (ti.eco.items.empty() || !forced || !(debug_ & 24)) return td.eco;
+   return (debug_ & 8) != 0;
+}
+
 void Engine::run_chunk(const TypeInfo &ti, const TypeDev &td, const Chunk &c, const RunBufs &w, const KTargets &kt)
 {
    const TypePlan &tp = ti.plan;
@@ -1260,7 +1251,8 @@ void Engine::run_chunk(const TypeInfo &ti, const TypeDev &td, const Chunk &c, co
    b.force_fix = debug_ & 1;
    b.fix_ws = w.fix_ws;
    b.eco = w.ac0 + (size_t)(c.p1 - c.p0) * tp.ncp;
-   b.eco_row = ti.eco_row;
+   const bool eco = use_eco(ti, td, w.count);
+   b.eco_row = eco ? ti.eco.row : 0;
    b.gmag = mixed_mode_ == 1 ? td.gmag : nullptr;
    b.gflag = mixed_mode_ == 2 ? td.gflag : nullptr;
    auto evb = [&](int cat, void *q) { if (w.count) ev_begin(cat, q); };
@@ -1278,59 +1270,45 @@ void Engine::run_chunk(const TypeInfo &ti, const TypeDev &td, const Chunk &c, co
    eve(3, st);
    if (mixed_mode_ == 2 && launch_mixed_flags(tp, b, td.gmag, d_mix_, mixed_tau_, td.gflag, d_mix_ + 1, st))
       fatal("mixed-precision route launch", 0);
-   if (!ti.eco_items.empty()) {
+   if (eco) {
       EcoArgs e{};
       e.items = ti.d_eco_items;
-      e.n_items = (int)ti.eco_items.size();
+      e.n_items = (int)ti.eco.items.size();
       e.srcmaps = ti.d_srcmaps;
       e.src_off = ti.d_eco_info;
       e.eco_off = ti.d_eco_info + MAXTC;
-      e.row_doubles = ti.eco_row;
+      e.row_doubles = ti.eco.row;
       evb(4, st);
       ev_key_ = tp.L;
       rc = launch_eco(tp, b, e, st);
       if (rc) fatal("matrix-core contraction launch", rc);
       eve(4, st);
    }
-   // debug bit 1: every consumer on the main stream, one after the other
-   // (kernel durations without overlap, for profiling)
-   const bool serial = (debug_ & 2) != 0;
-   ensure_side();
-   HIPCHECK(hipEventRecord((hipEvent_t)ev_join_[0], st));
-   for (int i = 0; i < NSIDE; i++) HIPCHECK(hipStreamWaitEvent((hipStream_t)side_[i], (hipEvent_t)ev_join_[0], 0));
-   for (int part = 0; part < GQS_PARTS; part++) {
-      bool any = false;
-      int npc = 0;
-      for (int k = 0; k < tp.nclass; k++) {
-         if (ti.lays[k].skip || ti.lays[k].part != part) continue;
-         npc++;
-         any = any || td.class_used[k];
+   if (td.used) {
+      const SqPlan *sp = ti.sq[kt.nspin - 1][eco ? 1 : 0];
+      // debug bit 1: both launches on the main stream, one after the other
+      // (kernel durations without overlap, for profiling)
+      const bool both = !sp[0].items.empty() && !sp[1].items.empty() && (debug_ & 2) == 0;
+      if (both) {
+         ensure_side();
+         HIPCHECK(hipEventRecord((hipEvent_t)ev_join_[0], st));
+         HIPCHECK(hipStreamWaitEvent((hipStream_t)side_, (hipEvent_t)ev_join_[0], 0));
       }
-      if (!any) continue;
-      void *q = (part == 0 || serial) ? (void *)st : side_[(part - 1) % NSIDE];
-      evb(2, q);
-      ev_key_ = tp.L;
-      rc = launch_gqs(tp, ti.d_cps, ti.d_lays, ti.d_srcmaps, ti.cq_lds, ti.cq_gws, part, npc, t, b, kt, w.gws, q,
-                      ti.cq_wide);
-      if (rc) fatal("gqs launch", rc);
-      eve(2, q);
-   }
-   int si = 0;
-   for (int k = 0; k < tp.nclass; k++) {
-      if (!td.class_used[k] || !ti.lays[k].skip) continue;
-      void *q = serial ? (void *)st : side_[si++ % NSIDE];
-      evb(1, q);
-      ev_key_ = tp.L;
-      rc = launch_tq(k, tp, t, b, kt, ti.d_srcmaps + ti.lays[k].o_src, q);
-      if (rc) fatal("tq launch", rc);
-      eve(1, q);
-   }
-   for (int i = 0; i < NSIDE; i++) {
-      HIPCHECK(hipEventRecord((hipEvent_t)ev_join_[1 + i], (hipStream_t)side_[i]));
-      HIPCHECK(hipStreamWaitEvent(st, (hipEvent_t)ev_join_[1 + i], 0));
+      for (int i = 0; i < 2; i++) {
+         if (sp[i].items.empty()) continue;
+         void *q = both && i == 1 ? side_ : (void *)st;
+         evb(2, q);
+         ev_key_ = tp.L;
+         rc = launch_sq(tp, td.max_np, b, t, kt, sp[i], q);
+         if (rc) fatal("sq launch", rc);
+         eve(2, q);
+      }
+      if (both) {
+         HIPCHECK(hipEventRecord((hipEvent_t)ev_join_[1], (hipStream_t)side_));
+         HIPCHECK(hipStreamWaitEvent(st, (hipEvent_t)ev_join_[1], 0));
+      }
    }
    if (!w.count) return;
-   timing_.flops[1] += c.tq_flops;
    timing_.flops[2] += c.k3_flops;
    timing_.flops[4] += c.eco_flops;
    n_prmc_ += (uint64_t)(c.p1 - c.p0) * tp.nclass;
@@ -1345,7 +1323,7 @@ bool Engine::prepare_exec(std::vector<TypeDev> &devs, uint64_t max_index, RunBuf
    if (max_index >= n) fatal("add_qrtt offsets reach beyond the P / K size of set_P", (long long)max_index);
    ensure_tables();
    upload_data();
-   size_t ncp_max = 0, max_prm = 0, scr = 0, max_gb = 0;
+   size_t ncp_max = 0, max_prm = 0, max_gb = 0;
    for (auto &D : devs) {
       if (D.chunks.empty()) continue;
       const TypeInfo &ti = types_[D.type];
@@ -1353,25 +1331,21 @@ bool Engine::prepare_exec(std::vector<TypeDev> &devs, uint64_t max_index, RunBuf
          fatal("the truncated-Coulomb table has fewer derivative orders than this quartet's total angular momentum",
                ti.plan.L);
       ncp_max = std::max(ncp_max, (size_t)ti.plan.ncp);
-      max_gb = std::max(max_gb, D.max_chunk_bytes);
-      for (auto &c : D.chunks) max_prm = std::max(max_prm, (size_t)(c.p1 - c.p0));
-      scr = std::max(scr, (size_t)ti.cq_gws * SCRATCH_GRID * GQS_PARTS);
+      const size_t eco_row = use_eco(ti, D, true) ? ti.eco.row : 0;
+      for (auto &c : D.chunks) {
+         max_prm = std::max(max_prm, (size_t)(c.p1 - c.p0));
+         max_gb = std::max(max_gb, sizeof(double) * ((size_t)(c.p1 - c.p0) * (size_t)ti.plan.ncp +
+                                                     (size_t)(c.r1 - c.r0) * eco_row));
+      }
    }
    if (ncp_max == 0) return false;
    ensure_work(ncp_max, max_prm, max_gb);
-   if (scr > scratch_cap_) {
-      synchronize();
-      if (d_scratch_) HIPCHECK(hipFree(d_scratch_));
-      HIPCHECK(hipMalloc((void **)&d_scratch_, scr * sizeof(double)));
-      scratch_cap_ = scr;
-   }
    w.ac0 = d_work_;
    w.fix = d_fix_;
    w.fixcnt = d_fixcnt_;
    w.fix_ws = d_fix_ws_;
    w.fix_cap = (uint32_t)fix_cap_;
    w.stats = stats_on_ ? d_stats_ : nullptr;
-   w.gws = Scratch{d_scratch_, scratch_cap_, SCRATCH_GRID};
    w.count = true;
    kt.nspin = nspin_;
    kt.hf_fac = hf_fac_;
@@ -1418,7 +1392,6 @@ void Engine::execute(std::vector<TypeDev> &devs, uint64_t max_index)
    RunBufs w{};
    KTargets kt{};
    if (!prepare_exec(devs, max_index, w, kt, FP_size_)) return;
-   if (debug_ & 24) force_kron(devs, (debug_ & 16) != 0);
    launch_all(devs, w, kt);
 }
 
@@ -1439,7 +1412,7 @@ void Engine::drop_graph()
 void Engine::replay_graph(const RunBufs &w, const KTargets &kt)
 {
    const uint64_t key[] = {(uint64_t)w.ac0, (uint64_t)w.fix, (uint64_t)w.fix_ws, (uint64_t)w.fixcnt,
-                           (uint64_t)w.gws.ptr, (uint64_t)w.gws.doubles, (uint64_t)w.fix_cap,
+                           (uint64_t)w.fix_cap,
                            (uint64_t)kt.P[0], (uint64_t)kt.P[1], (uint64_t)kt.K[0], (uint64_t)kt.K[1],
                            (uint64_t)kt.nspin, graph_bits(kt.hf_fac), (uint64_t)kt.out, (uint64_t)d_data_,
                            (uint64_t)d_C0_, (uint64_t)d_neighs_, (uint64_t)neighs_.size(), graph_bits(R_cut_),
@@ -1508,8 +1481,6 @@ int Engine::plan_execute_noalloc(const double *Pa, const double *Pb, double *Ka,
          return err(-4, "a set quartet's primitive blocks exceed the no-allocation scratch (bytes of the largest)",
                     (long long)D.max_group_bytes);
       if (truncated_ && ti.plan.L > nder_) return err(-7, "the C0 table has too few derivative orders", ti.plan.L);
-      if (ti.cq_gws && NOALLOC_GWS_BYTES / 8 / ((size_t)GQS_PARTS * ti.cq_gws) < 1)
-         return err(-5, "a class workspace exceeds the no-allocation scratch", ti.cq_gws);
       ncp_max = std::max(ncp_max, (size_t)ti.plan.ncp);
    }
    if (!any) return 0;
@@ -1540,269 +1511,20 @@ int Engine::plan_execute_noalloc(const double *Pa, const double *Pb, double *Ka,
    for (auto &D : plan_dev_) {
       if (D.chunks.empty()) continue;
       const TypeInfo &ti = types_[D.type];
-      const unsigned g = ti.cq_gws ? (unsigned)std::min<size_t>(SCRATCH_GRID, NOALLOC_GWS_BYTES / 8 /
-                                                                                ((size_t)GQS_PARTS * ti.cq_gws))
-                                   : SCRATCH_GRID;
-      w.gws = Scratch{(double *)(base + NOALLOC_OFF_GWS), NOALLOC_GWS_BYTES / 8, g};
       for (auto &c : D.chunks_na) run_chunk(ti, D, c, w, kt);
    }
    return 0;
 }
 
-// ---------------------------------------------------------------------------
-// autotuner: per class of a quartet type, the schedule of its contraction,
-// HRR, spherical transform and K update, chosen by timing on a sample of the
-// plan (first execution after plan_end):
-//   0  the templated one-wavefront-per-set-quartet kernel (k_tqw), where
-//      the class has one,
-//   1  the workgroup kernel (k_gqs) with its own contraction loop,
-//   2  k_gqs after the matrix-core contraction (k_eco), where the class has
-//      a place in the contraction buffer.
-// Decisions are kept per (class, contractions, primitive quartets per row
-// in powers of two) for the life of the process and reused by later plans.
-// ---------------------------------------------------------------------------
-static std::mutex g_tune_mu;
-static std::map<uint64_t, int> g_tune;   // key -> schedule
-
-static uint64_t tune_key(int code, int nq, size_t n_prm, size_t n_rows)
+void Engine::tune_info(double out[5]) const
 {
-   const double avg = n_rows ? (double)n_prm / (double)n_rows : 1.0;
-   const int bucket = std::min(15, std::max(0, (int)std::floor(std::log2(std::max(avg, 1.0)))));
-   return (uint64_t)code | (uint64_t)nq << 8 | (uint64_t)bucket << 20;
-}
-
-void Engine::apply_schedule(TypeInfo &ti, int k, int v)
-{
-   CqLayout &y = ti.lays[k];
-   y.skip = v == 0 ? 1 : 0;
-   y.eco = (v == 2 || v == 3) ? 1 : 0;
-   y.kron = v >= 3 ? 1 : 0;
-}
-
-// debug bits 3 and 4: every class (of a plan, or of the call stream's
-// types) that can take the Kronecker path takes it, whatever the schedule: bit 3 with the matrix-core
-// contraction where the class has a place in the contraction buffer (else
-// its own), bit 4 with its own contraction where that fits (else the matrix
-// cores)
-void Engine::force_kron(std::vector<TypeDev> &devs, bool own_first)
-{
-   for (auto &D : devs) {
+   for (int i = 0; i < 5; i++) out[i] = 0.0;
+   for (const auto &D : plan_dev_) {
       if (D.chunks.empty()) continue;
-      TypeInfo &ti = types_[D.type];
-      bool any = false;
-      for (CqLayout &y : ti.lays) {
-         if (!y.kron_ws) continue;
-         const bool can_eco = y.eco_off >= 0, can_own = y.o_kc >= 0;
-         if (!can_eco && !can_own) continue;
-         const int eco = (can_eco && (!own_first || !can_own)) ? 1 : 0;
-         if (y.kron && !y.skip && y.eco == eco) continue;
-         y.skip = 0;
-         y.eco = eco;
-         y.kron = 1;
-         any = true;
-      }
-      if (any) upload_layouts(ti);
+      const TypeInfo &ti = types_[D.type];
+      out[0] = 1.0;
+      for (int k = 0; k < ti.plan.nclass; k++) out[D.eco && ti.eco.off[k] >= 0 ? 3 : 2] += 1.0;
    }
-}
-
-void Engine::upload_layouts(TypeInfo &ti)
-{
-   ti.cq_wide = false;
-   for (const CqLayout &y : ti.lays) ti.cq_wide = ti.cq_wide || (y.kron && !y.skip);
-   assign_parts(ti.plan, ti.cplans, ti.lays);
-   make_eco_items(ti);
-   HIPCHECK(hipMemcpy(ti.d_lays, ti.lays.data(), sizeof(CqLayout) * ti.lays.size(), hipMemcpyHostToDevice));
-   if (ti.d_eco_items) HIPCHECK(hipFree(ti.d_eco_items));
-   ti.d_eco_items = nullptr;
-   if (!ti.eco_items.empty()) {
-      HIPCHECK(hipMalloc((void **)&ti.d_eco_items, sizeof(EcoItem) * ti.eco_items.size()));
-      HIPCHECK(hipMemcpy(ti.d_eco_items, ti.eco_items.data(), sizeof(EcoItem) * ti.eco_items.size(),
-                         hipMemcpyHostToDevice));
-   }
-}
-
-void Engine::autotune(const RunBufs &w, const KTargets &kt)
-{
-   synchronize();
-   const auto t0 = std::chrono::steady_clock::now();
-   // a scratch K: the timed launches must not touch the caller's
-   double *Ks = nullptr;
-   HIPCHECK(hipMalloc((void **)&Ks, sizeof(double) * std::max<size_t>(FP_size_, 1) * (size_t)kt.nspin));
-   KTargets ks = kt;
-   ks.K[0] = Ks;
-   ks.K[1] = kt.nspin > 1 ? Ks + FP_size_ : nullptr;
-   ks.out = nullptr;
-   hipStream_t st = (hipStream_t)stream_;
-   hipEvent_t e0, e1;
-   HIPCHECK(hipEventCreate(&e0));
-   HIPCHECK(hipEventCreate(&e1));
-   EcoItem *d_items = nullptr;
-   size_t items_cap = 0;
-   const DevTables t = dev_tables();
-   for (auto &D : plan_dev_) {
-      if (D.chunks.empty()) continue;
-      TypeInfo &ti = types_[D.type];
-      const TypePlan &tp = ti.plan;
-      // decisions already known for every class of the type
-      std::vector<int> dec(tp.nclass, -1);
-      bool all = true;
-      {
-         std::lock_guard<std::mutex> lk(g_tune_mu);
-         for (int k = 0; k < tp.nclass; k++) {
-            auto it = g_tune.find(tune_key(tp.cls_code[k], tp.cls_nl[k], D.n_prm, D.n_rows));
-            if (it != g_tune.end()) dec[k] = it->second;
-            else if (D.class_used[k]) all = false;
-         }
-      }
-      if (!all) {
-         // the sample: the first set quartets of the first chunk, about
-         // TUNE_PRM primitive quartets (launches long enough to time), at
-         // most TUNE_GROUPS set quartets
-         const Chunk &c0 = D.chunks[0];
-         Chunk c = c0;
-         const double ppg = (double)(c0.p1 - c0.p0) / (double)std::max<uint32_t>(c0.g1 - c0.g0, 1);
-         const uint32_t ng = (uint32_t)std::max(1.0, std::min<double>(TUNE_GROUPS, TUNE_PRM / std::max(ppg, 1.0)));
-         c.g1 = std::min<uint32_t>(c0.g1, c0.g0 + ng);
-         if (c.g1 < c0.g1) {
-            GroupRec gl;
-            HIPCHECK(hipMemcpy(&gl, D.groups + (c.g1 - 1), sizeof gl, hipMemcpyDeviceToHost));
-            RowRec rl;
-            HIPCHECK(hipMemcpy(&rl, D.rows + (gl.row1 - 1), sizeof rl, hipMemcpyDeviceToHost));
-            c.r1 = gl.row1;
-            c.p1 = rl.prm_off + rl.n_prm;
-         }
-         BatchDev b{};   // every field zero / null unless set below
-         b.tp = ti.d_plan;
-         b.e1 = ti.d_e1;
-         b.e2 = ti.d_e2;
-         b.rows = D.rows;
-         b.groups = D.groups;
-         b.prm_row = D.prm_row;
-         b.prm_ip = D.prm_ip;
-         b.ksg = D.ksg;
-         b.kss = D.kss;
-         b.ksx = D.ksx;
-         b.data = d_data_;
-         b.ac0 = w.ac0;
-         b.p0 = c.p0;
-         b.p1 = c.p1;
-         b.r0 = c.r0;
-         b.r1 = c.r1;
-         b.g0 = c.g0;
-         b.g1 = c.g1;
-         b.stats = nullptr;
-         b.fix = w.fix;
-         b.fix_count = w.fixcnt;
-         b.fix_cap = w.fix_cap;
-         b.force_fix = 0;
-         b.fix_ws = w.fix_ws;
-         b.eco = w.ac0 + (size_t)(c.p1 - c.p0) * tp.ncp;
-         b.eco_row = ti.eco_row;
-         b.gmag = nullptr;    // no calibration and no single-precision route while timing
-         b.gflag = nullptr;
-         if (launch_zero_u32(w.fixcnt, 1, st) || launch_fm_r(tp, t, b, st) ||
-             launch_fixup(tp, t, b, std::min<uint32_t>(64u, w.fix_cap), st))
-            fatal("autotune: sample launch", 0);
-         const std::vector<CqLayout> keep = ti.lays;
-         for (int k = 0; k < tp.nclass; k++) {
-            if (!D.class_used[k] || dec[k] >= 0) continue;
-            double best = 1e300;
-            int bv = keep[k].skip ? 0 : (keep[k].eco ? (keep[k].kron ? 3 : 2) : (keep[k].kron ? 4 : 1));
-            // the sample's contraction FLOPs of the class: above TUNE_VALU_FLOPS
-            // the VALU contraction loop (schedule 1) is not timed where the
-            // matrix cores can take the class (it is slower there by an order
-            // of magnitude or two, and timing it would cost seconds)
-            const double cflops = 2.0 * tp.cls_nl[k] * (double)tp.cls_ncp[k] * (double)(c.p1 - c.p0);
-            for (int v = 0; v < 5; v++) {
-               if (v == 0 && !tq_has(tp.cls_code[k])) continue;
-               if ((v == 2 || v == 3) && keep[k].eco_off < 0) continue;
-               if (v >= 3 && !keep[k].kron_ws) continue;
-               if (v == 4 && keep[k].o_kc < 0) continue;
-               // the own contraction is not timed where the VALU
-               // contraction would be too slow (as schedule 1)
-               if (v == 4 && keep[k].eco_off >= 0 && cflops > TUNE_VALU_FLOPS) continue;
-               if (v == 1 && keep[k].eco_off >= 0 && cflops > TUNE_VALU_FLOPS) continue;
-               // this class alone in part 0 with schedule v
-               std::vector<CqLayout> L = keep;
-               for (auto &y : L) y.part = -1;
-               L[k].skip = v == 0 ? 1 : 0;
-               L[k].eco = (v == 2 || v == 3) ? 1 : 0;
-               L[k].kron = v >= 3 ? 1 : 0;
-               L[k].part = 0;
-               HIPCHECK(hipMemcpy(ti.d_lays, L.data(), sizeof(CqLayout) * L.size(), hipMemcpyHostToDevice));
-               std::vector<EcoItem> items;
-               if (v == 2 || v == 3) {
-                  for (int jt0 = 0; jt0 * 16 < tp.cls_ncp[k]; jt0 += 4)
-                     for (int qb = 0; qb * 64 < tp.cls_nl[k]; qb++)
-                        items.push_back(EcoItem{(uint16_t)k, (uint16_t)jt0, (uint16_t)qb, 0});
-                  if (items.size() > items_cap) {
-                     if (d_items) HIPCHECK(hipFree(d_items));
-                     items_cap = items.size() * 2;
-                     HIPCHECK(hipMalloc((void **)&d_items, sizeof(EcoItem) * items_cap));
-                  }
-                  HIPCHECK(hipMemcpy(d_items, items.data(), sizeof(EcoItem) * items.size(), hipMemcpyHostToDevice));
-               }
-               // the faster of two runs: the first may load the kernel's code object
-               float ms = 1e30f;
-               for (int rep = 0; rep < 2; rep++) {
-                  float msr = 0.f;
-                  HIPCHECK(hipEventRecord(e0, st));
-                  int rc = 0;
-                  if (v == 0) {
-                     rc = launch_tq(k, tp, t, b, ks, ti.d_srcmaps + keep[k].o_src, st);
-                  } else {
-                     if (v == 2 || v == 3) {
-                        EcoArgs e{};
-                        e.items = d_items;
-                        e.n_items = (int)items.size();
-                        e.srcmaps = ti.d_srcmaps;
-                        e.src_off = ti.d_eco_info;
-                        e.eco_off = ti.d_eco_info + MAXTC;
-                        e.row_doubles = ti.eco_row;
-                        rc = launch_eco(tp, b, e, st);
-                     }
-                     if (!rc)
-                        rc = launch_gqs(tp, ti.d_cps, ti.d_lays, ti.d_srcmaps, ti.cq_lds, ti.cq_gws, 0, 1, t, b, ks,
-                                        w.gws, st, v >= 3 || ti.cq_wide);
-                  }
-                  if (rc) fatal("autotune: candidate launch", rc);
-                  HIPCHECK(hipEventRecord(e1, st));
-                  HIPCHECK(hipEventSynchronize(e1));
-                  HIPCHECK(hipEventElapsedTime(&msr, e0, e1));
-                  ms = std::min(ms, msr);
-               }
-               if (ms < best) {
-                  best = ms;
-                  bv = v;
-               }
-            }
-            dec[k] = bv;
-            tune_ms_[tp.cls_code[k]] += best;
-            tune_pick_[tp.cls_code[k]] = bv;
-            std::lock_guard<std::mutex> lk(g_tune_mu);
-            g_tune[tune_key(tp.cls_code[k], tp.cls_nl[k], D.n_prm, D.n_rows)] = bv;
-         }
-      }
-      for (int k = 0; k < tp.nclass; k++)
-         if (dec[k] >= 0) {
-            apply_schedule(ti, k, dec[k]);
-            tune_counts_[dec[k]]++;
-         }
-      upload_layouts(ti);
-      if (debug_ & 4) {
-         std::fprintf(stderr, "libgint: autotune: quartet type L %d (%zu set quartets) %s at %.1f s\n", tp.L, D.n_groups,
-                      all ? "from earlier decisions" : "timed",
-                      std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
-         std::fflush(stderr);
-      }
-   }
-   HIPCHECK(hipStreamSynchronize(st));
-   if (d_items) HIPCHECK(hipFree(d_items));
-   HIPCHECK(hipFree(Ks));
-   HIPCHECK(hipEventDestroy(e0));
-   HIPCHECK(hipEventDestroy(e1));
-   tune_seconds_ += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-   plan_tuned_ = true;
 }
 
 // ---------------------------------------------------------------------------
@@ -1827,23 +1549,22 @@ uint64_t Engine::device_bytes() const
    for (const auto &d : plan_dev_)
       b += d.cap[0] * sizeof(RowRec) + d.cap[1] * sizeof(GroupRec) + d.cap[2] * 4 + d.cap[3] * 4 +
            d.cap[4] * sizeof(KsGroup) + d.cap[5] * sizeof(KsRec) + d.cap[6] * sizeof(KsSet);
-   b += work_bytes_ + fix_cap_ * 8 + fix_ws_cap_ * 8 + scratch_cap_ * 8 + d_data_cap_ * 8 + C0_.size() * 8 +
+   b += work_bytes_ + fix_cap_ * 8 + fix_ws_cap_ * 8 + d_data_cap_ * 8 + C0_.size() * 8 +
         d_neighs_cap_ * 8;
    return b;
 }
 
 uint64_t Engine::work_estimate() const
 {
-   size_t ncp_max = 0, mcb = 0, scr = 0;
+   size_t ncp_max = 0, mcb = 0;
    for (const auto &D : plan_dev_) {
       if (D.chunks.empty()) continue;
       const TypeInfo &ti = types_[D.type];
       ncp_max = std::max(ncp_max, (size_t)ti.plan.ncp);
       mcb = std::max(mcb, D.max_chunk_bytes);
-      scr = std::max(scr, (size_t)ti.cq_gws * SCRATCH_GRID * GQS_PARTS);
    }
    if (!ncp_max) return 0;
-   return std::max<size_t>(mcb, 1 << 20) + 2 * 4 * 4096 + 4096 * (ncp_max + 16) * 8 + scr * 8;
+   return std::max<size_t>(mcb, 1 << 20) + 2 * 4 * 4096 + 4096 * (ncp_max + 16) * 8;
 }
 
 uint64_t Engine::plan_host_bytes() const
@@ -1884,14 +1605,13 @@ void Engine::plan_evict()
    }
    plan_dev_.clear();
    mixed_calibrated_ = false;
-   void *bufs[] = {d_work_, d_fix_, d_fix_ws_, d_scratch_};
+   void *bufs[] = {d_work_, d_fix_, d_fix_ws_};
    for (void *b : bufs)
       if (b) HIPCHECK(hipFree(b));
    d_work_ = nullptr;
    d_fix_ = nullptr;
    d_fix_ws_ = nullptr;
-   d_scratch_ = nullptr;
-   work_bytes_ = fix_cap_ = fix_ws_cap_ = scratch_cap_ = 0;
+   work_bytes_ = fix_cap_ = fix_ws_cap_ = 0;
    evicted_ = true;
 }
 

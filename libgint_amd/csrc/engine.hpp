@@ -61,7 +61,7 @@ struct TypeQueue {
 
 struct Chunk {
    uint32_t g0, g1, r0, r1, p0, p1;
-   double tq_flops, k3_flops, eco_flops;
+   double k3_flops, eco_flops;
 };
 
 // one type's work on the device
@@ -80,7 +80,9 @@ struct TypeDev {
    std::vector<Chunk> chunks;
    std::vector<Chunk> chunks_na;          // the same work in chunks that fit the no-allocation scratch
    bool na_fit = true;                    // every set quartet fits it
-   std::vector<char> class_used;
+   int max_np = 1;                        // most primitives of a set
+   bool used = false;                     // some set quartet has calls
+   bool eco = false;                      // its contraction runs on the matrix cores
    double *gmag = nullptr;      // mixed precision: calibrated max |block element| per set quartet
    uint32_t *gflag = nullptr;   // mixed precision: route per set quartet (1 single precision)
    void release();
@@ -93,18 +95,13 @@ struct TypeInfo {
    std::vector<uint32_t> e1, e2;          // Hermite -> cartesian item descriptors
    uint32_t *d_e1 = nullptr, *d_e2 = nullptr;
    std::vector<ClassPlan> cplans;
-   std::vector<CqLayout> lays;            // quartet kernel: per-class LDS plans
-   std::vector<int> srcmaps;              // class block element -> type block element
-   int cq_lds = 0, cq_gws = 0;
-   bool cq_wide = false;   // a class takes the Kronecker path: k_gqs with four wavefronts
-   ClassPlan *d_cps = nullptr;
-   CqLayout *d_lays = nullptr;
+   // from the blocks to K: a launch for the classes without and one for those
+   // with f shells; [nspin - 1][0 own contraction, 1 matrix cores]
+   SqPlan sq[2][2][2];
+   // matrix-core contraction (k_eco), for types with many primitive
+   // quartets per row
+   EcoPlan eco;
    int *d_srcmaps = nullptr;
-   // matrix-core contraction (k_eco): work items of a row, [class map
-   // offsets, class buffer offsets], doubles per row of the buffer
-   std::vector<EcoItem> eco_items;
-   std::vector<int> eco_info;
-   size_t eco_row = 0;
    EcoItem *d_eco_items = nullptr;
    int *d_eco_info = nullptr;
 };
@@ -116,14 +113,13 @@ struct RunBufs {
    double *fix_ws;
    uint32_t fix_cap;
    unsigned long long *stats;
-   Scratch gws;
    bool count;   // host counters and timing events
 };
 
 struct Timing {
-   double ms[5] = {0, 0, 0, 0, 0};        // fm_r, tq, gqs, fixup, eco (matrix-core contraction)
+   double ms[5] = {0, 0, 0, 0, 0};        // fm_r, (unused), sq, fixup, eco (matrix-core contraction)
    uint64_t launches[5] = {0, 0, 0, 0, 0};
-   double flops[5] = {0, 0, 0, 0, 0};     // host-counted algorithmic FLOPs of tq [1], gqs [2] and eco [4]
+   double flops[5] = {0, 0, 0, 0, 0};     // host-counted algorithmic FLOPs of sq [2] and eco [4]
 };
 
 class Engine {
@@ -169,25 +165,18 @@ class Engine {
    void timing_detail(int cat, double out[256]);
    void reset_counters();
    void set_debug(int flags) { debug_ = flags; }
-   void force_kron(std::vector<TypeDev> &devs, bool own_first);
    void set_graph(bool on) { graph_on_ = on; }
-   void set_autotune(bool on) { autotune_on_ = on; }
+   void set_autotune(bool) {}
    void set_mixed_precision(double tau) { mixed_tau_ = tau > 0.0 ? tau : 0.0; }
    void mixed_info(double out[4]);
-   void tune_info(double out[5]) const
-   {
-      out[0] = plan_tuned_ ? 1.0 : 0.0;
-      for (int i = 0; i < 3; i++) out[1 + i] = (double)tune_counts_[i];
-      out[3] += (double)tune_counts_[3];
-      out[2] += (double)tune_counts_[4];
-      out[4] = tune_seconds_;
-   }
-   // per class code: ms of the chosen schedule on the timing samples, and the schedule
+   // no schedule is timed any more (the kernels are chosen by a rule): the
+   // classes of the plan on the workgroup kernel's own and on the matrix-core contraction
+   void tune_info(double out[5]) const;
    void tune_detail(double ms[256], int pick[256]) const
    {
       for (int i = 0; i < 256; i++) {
-         ms[i] = tune_ms_[i];
-         pick[i] = tune_pick_[i];
+         ms[i] = 0.0;
+         pick[i] = 0;
       }
    }
    void graph_info(uint64_t out[4]) const
@@ -231,9 +220,6 @@ class Engine {
    bool prepare_exec(std::vector<TypeDev> &devs, uint64_t max_index, RunBufs &w, KTargets &kt, uint64_t n);
    void launch_all(std::vector<TypeDev> &devs, const RunBufs &w, const KTargets &kt);
    void replay_graph(const RunBufs &w, const KTargets &kt);
-   void autotune(const RunBufs &w, const KTargets &kt);
-   void apply_schedule(TypeInfo &ti, int k, int v);
-   void upload_layouts(TypeInfo &ti);
    void drop_graph();
    static uint64_t graph_bits(double x)
    {
@@ -241,6 +227,7 @@ class Engine {
       std::memcpy(&u, &x, 8);
       return u;
    }
+   bool use_eco(const TypeInfo &ti, const TypeDev &td, bool forced) const;
    void run_chunk(const TypeInfo &ti, const TypeDev &td, const Chunk &c, const RunBufs &w, const KTargets &kt);
    DevTables dev_tables() const;
    void ensure_work(size_t ncp_max, size_t max_prm_chunk, size_t max_group_bytes);
@@ -252,12 +239,11 @@ class Engine {
    void ensure_side();
    int my_thr_ = 0, nomp_ = 1;
    void *stream_ = nullptr;
-   // the consumers of a chunk's blocks only add into K: the small-class
-   // kernels run on side streams beside gqs on stream_, and
-   // stream_ waits for them before the blocks are overwritten
-   static constexpr int NSIDE = 3;
-   void *side_[NSIDE] = {};
-   void *ev_join_[NSIDE + 1] = {};   // [0] blocks ready, [1 + i] side stream i done
+   // the kernels that take a chunk's blocks to K only add into it: the
+   // classes with f shells run on a side stream, and stream_ waits for it
+   // before the blocks are overwritten
+   void *side_ = nullptr;
+   void *ev_join_[2] = {};   // blocks ready, side stream done
 
    // geometry, potential
    double cell_[18];
@@ -313,8 +299,6 @@ class Engine {
    uint32_t *d_fix_ = nullptr;
    double *d_fix_ws_ = nullptr;
    size_t fix_cap_ = 0, fix_ws_cap_ = 0;
-   double *d_scratch_ = nullptr;
-   size_t scratch_cap_ = 0;
    void *noalloc_scratch_ = nullptr;   // this device's static scratch array (init)
    unsigned long long *d_stats_ = nullptr;   // [0..2] kernel statistics, [3] unused
    uint32_t *d_fixcnt_ = nullptr;             // [0] entries of the chunk, [1] slots beyond the list (sticky)
@@ -328,17 +312,8 @@ class Engine {
    double *d_P_[2] = {nullptr, nullptr};
    double *d_K_[2] = {nullptr, nullptr};
 
-   // autotuner: the schedule of each class, chosen at the plan's first execution
-   static constexpr uint32_t TUNE_GROUPS = 16384;  // at most this many set quartets in a type's timing sample
-   static constexpr double TUNE_PRM = 262144;       // primitive quartets aimed at in the sample
-   static constexpr double TUNE_VALU_FLOPS = 2e8;   // largest sample contraction timed on the VALU
-   bool autotune_on_ = true;
-   bool plan_tuned_ = false;
-   // classes given k_tqw / k_gqs / k_eco + k_gqs / k_eco + Kronecker k_gqs / Kronecker k_gqs with its own contraction
-   uint64_t tune_counts_[5] = {0, 0, 0, 0, 0};
-   double tune_seconds_ = 0.0;
-   double tune_ms_[256] = {};
-   int tune_pick_[256] = {};
+   // primitive quartets per row from which a type's contraction runs on the matrix cores
+   static constexpr double ECO_MIN_PRM = 96.0;
 
    // mixed precision (plans): set quartets whose calibrated bound times
    // max |P| is below tau take the single-precision contraction

@@ -10,7 +10,7 @@
 // Kc[ic][ipc] Kd[id][ipd] the coefficient product of contraction
 // q = (ia, ib, ic, id) (row-major, as the add_qrtt calls of the class).  C
 // goes to the contraction buffer, row (r - first row of the chunk), where
-// the per-class kernel (k_gqs) takes it in place of its own contraction loop.
+// k_sq takes it in place of its own contraction.
 //
 // A tile of v_mfma_f64_16x16x4f64 is 16 columns x 16 contractions over 4
 // primitive quartets.  A workgroup of 4 wavefronts takes 4 column tiles of

@@ -1,0 +1,690 @@
+// k_sq: from the primitive (e0|f0) blocks of a set quartet to its K updates,
+// one wavefront per (set quartet, bra tile, ket tile).  A tile is a run of
+// (shell pair, contraction pair) units of one side, so one item covers the
+// classes of several shell pairs at once.  For each (n1,n2) row:
+//
+//   contraction      C[unit, e][col] = sum over the primitive quartets n of
+//                    (K_a K_b)[n][unit] (K_c K_d)[n][col] A[n][e][f(col)]
+//                    (reference src/compute_ECO.cpp:12-214) in FP64
+//                    matrix-core tiles: 16 bra units x 16 (e, col) x 4
+//                    primitive quartets; or a copy of the blocks k_eco
+//                    contracted
+//   ket transform    HRR d -> c and cartesian -> spherical of the ket pair
+//                    (src/compute_HRR.cpp, src/compute_SPH.cpp:58-237), one
+//                    (row, unit) per lane, in registers, C in place
+//   bra transform    the same on the bra side, one (unit, ket function) per
+//                    lane
+//   K update         from the lane's integrals in registers (src/compute_KS.cpp:
+//                    8-117): its sums over a or b go to the item's four K
+//                    blocks in LDS, from there one atomic per element to K
+//
+// The transforms act on one side of the integral only, so the HRR is done
+// for (components + function) vectors instead of the full four-index block,
+// and every index and coefficient is a compile-time constant (the pair
+// (l1,l2) is a template parameter, chosen by a uniform branch).  One
+// wavefront per workgroup: the phases exchange data through LDS in program
+// order, with no barrier and no wait for loads in flight.
+//
+// One launch per type does what took one launch per class (a wavefront or a
+// workgroup per set quartet and class, the four-index HRR in LDS): 32 waters,
+// 27 cells, 262 k set quartets: 66 ms where those kernels took 250 (serialised,
+// with their matrix-core contraction); one molecule: 0.19 ms for 5.9.  Bound:
+// latency and instruction issue (waits in 55% of the wave cycles, VALU busy in
+// 35%; HBM below 1 TB/s), so tiles are cut small enough (38 rows x 38 columns,
+// 16 KB of LDS) for ten wavefronts per CU: an item's fixed cost is shared by
+// several shell pairs, and an item of every class alone had ten times the
+// instructions per integral.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <utility>
+
+#include "c2s_table.h"
+#include "device.hpp"
+#include "gint_math.h"
+
+namespace gint {
+namespace sq {
+
+__host__ __device__ constexpr int comp(int L, int i, int d)
+{
+   int n = 0;
+   for (int lx = L; lx >= 0; lx--)
+      for (int ly = L - lx; ly >= 0; ly--) {
+         if (n == i) return d == 0 ? lx : (d == 1 ? ly : L - lx - ly);
+         n++;
+      }
+   return 0;
+}
+__host__ __device__ constexpr int cidx(int L, int lx, int lz) { return (L - lx) * (L - lx + 1) / 2 + lz; }
+__host__ __device__ constexpr int n_co(int l) { return (l + 1) * (l + 2) / 2; }
+__host__ __device__ constexpr int co_below(int l) { return l * (l + 1) * (l + 2) / 6; }   // components of shells 0..l-1
+__host__ __device__ constexpr int n_side(int l1, int l2) { return co_below(l1 + l2 + 1) - co_below(l1); }
+__host__ __device__ constexpr double c2s(int l, int m, int k)
+{
+   constexpr double v[] = {GINT_C2S_VALUES};
+   constexpr int off[4] = {GINT_C2S_OFF_0, GINT_C2S_OFF_1, GINT_C2S_OFF_2, GINT_C2S_OFF_3};
+   return v[off[l] + m * n_co(l) + k];
+}
+__host__ __device__ constexpr int binom(int n, int k) { return (k == 0 || k == n) ? 1 : n; }   // n <= 3
+
+template <int... I, class F>
+__device__ __forceinline__ void for_seq(std::integer_sequence<int, I...>, F &&f)
+{
+   (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f)
+{
+   for_seq(std::make_integer_sequence<int, N>{}, static_cast<F &&>(f));
+}
+
+__device__ __forceinline__ double rpow(double r, int n) { return n == 0 ? 1.0 : (n == 1 ? r : (n == 2 ? r * r : r * r * r)); }
+
+// One side: from the components of shells l1 .. l1 + l2 on the first centre
+// to the spherical pairs (s1 s2).  The HRR (x, y + 1_d| = (x + 1_d, y| + R_d
+// (x, y|, R = AB or CD, unrolled:
+//    (x y| = sum_{0 <= i <= y} prod_d C(y_d, i_d) R_d^(y_d - i_d) (x + i, 0|
+// for one y at a time (few values live), then both c2s with their zeros
+// left out.
+template <int l1, int l2>
+__device__ __forceinline__ void side_transform(const double *in, const double R[3], double *out)
+{
+   constexpr int N1 = n_co(l1), S1 = 2 * l1 + 1, S2 = 2 * l2 + 1;
+#pragma unroll
+   for (int s = 0; s < S1 * S2; s++) out[s] = 0.0;
+   static_for<n_co(l2)>([&](auto Y) {
+      constexpr int y = decltype(Y)::value;
+      constexpr int y0 = comp(l2, y, 0), y1 = comp(l2, y, 1), y2 = comp(l2, y, 2);
+      double v[N1];
+#pragma unroll
+      for (int x = 0; x < N1; x++) v[x] = 0.0;
+      static_for<(y0 + 1) * (y1 + 1) * (y2 + 1)>([&](auto I) {
+         constexpr int i = decltype(I)::value;
+         constexpr int i2 = i % (y2 + 1), i1 = (i / (y2 + 1)) % (y1 + 1), i0 = i / ((y2 + 1) * (y1 + 1));
+         constexpr int e = l1 + i0 + i1 + i2;
+         constexpr double bin = (double)(binom(y0, i0) * binom(y1, i1) * binom(y2, i2));
+         const double m = bin * rpow(R[0], y0 - i0) * rpow(R[1], y1 - i1) * rpow(R[2], y2 - i2);
+         static_for<N1>([&](auto X) {
+            constexpr int x = decltype(X)::value;
+            constexpr int src = co_below(e) - co_below(l1) + cidx(e, comp(l1, x, 0) + i0, comp(l1, x, 2) + i2);
+            if constexpr (i0 == y0 && i1 == y1 && i2 == y2) v[x] += in[src];
+            else v[x] += m * in[src];
+         });
+      });
+      static_for<S1>([&](auto A) {
+         constexpr int s1 = decltype(A)::value;
+         double t = 0.0;
+         static_for<N1>([&](auto X) {
+            constexpr int x = decltype(X)::value;
+            constexpr double c = c2s(l1, s1, x);
+            if constexpr (c == 1.0) t += v[x];
+            else if constexpr (c != 0.0) t += c * v[x];
+         });
+         static_for<S2>([&](auto B) {
+            constexpr int s2 = decltype(B)::value;
+            constexpr double c = c2s(l2, s2, y);
+            if constexpr (c == 1.0) out[s1 * S2 + s2] += t;
+            else if constexpr (c != 0.0) out[s1 * S2 + s2] += c * t;
+         });
+      });
+   });
+}
+
+// Orders the LDS accesses of the workgroup's one wavefront: they execute in
+// program order, so the compiler's order is all it takes
+__device__ __forceinline__ void lds_order()
+{
+   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+   __builtin_amdgcn_wave_barrier();
+}
+
+// A record at a uniform address, through the scalar cache: nothing that a
+// kernel of the K-build reads this way is written by one (plans, records,
+// tables and basis data), which the compiler cannot see behind the stores
+template <class T>
+__device__ __forceinline__ T load_uniform(const T *p)
+{
+   static_assert(sizeof(T) % 4 == 0, "whole words");
+   typedef const __attribute__((address_space(4))) uint32_t *word_ptr;
+   const word_ptr q = (word_ptr)(uintptr_t)p;
+   union {
+      uint32_t w[sizeof(T) / 4];
+      T v;
+   } u;
+#pragma unroll
+   for (unsigned i = 0; i < sizeof(T) / 4; i++) u.w[i] = q[i];
+   return u.v;
+}
+struct GroupHead {   // the start of GroupRec
+   uint32_t row0, row1, R[4];
+};
+struct Vec3 {
+   double v[3];
+};
+struct Cell {
+   double v[18];
+};
+
+// x / d for 0 <= x < 2^22, d >= 1
+__device__ __forceinline__ int fdiv(int x, int d)
+{
+   int q = (int)((float)x * __builtin_amdgcn_rcpf((float)d));
+   const int rem = x - q * d;
+   if (rem < 0) q--;
+   else if (rem >= d) q++;
+   return q;
+}
+
+__device__ __forceinline__ unsigned blk_at(bool T, unsigned ld, unsigned r, unsigned c) { return T ? r * ld + c : c * ld + r; }
+__device__ __forceinline__ double symm_fac(uint32_t code)
+{
+   return code >= 4 ? 0.0 : (code == 0 ? 2.0 : (code == 1 ? 1.0 : (code == 2 ? 0.5 : 0.25)));
+}
+
+constexpr int SQ_EU = 4;   // components whose loads are in flight together in the contraction
+
+typedef double dbl4 __attribute__((ext_vector_type(4)));
+
+// What the K update of an item needs
+struct Upd {
+   const BatchDev &b;
+   const KTargets &kt;
+   const TypePlan &tp;
+   const GroupRec &g;
+   const SqSp *ksp;     // the ket tile's shell pairs
+   double *Pl, *Kl;     // LDS: the four P and K blocks of the item, per spin [ac | ad | bc | bd]
+   const uint32_t *fn;  // LDS: ket functions
+   bool lds;            // through them, else straight to K or the integral output
+   bool add;            // integral output: an earlier row wrote already
+   int NA, NB, NC, ND;
+};
+
+// the updates of bra contraction cb of shell pair q with ket function f, by
+// the K layout of the class: integral x (2 lb + 1) + y at I[(x (2 lb + 1) + y) is]
+__device__ __forceinline__ void k_update_class(const double *I, int is, const Upd &u, const SqSp &q, int cb, int f)
+{
+   const int SA = 2 * q.l1 + 1, SB = 2 * q.l2 + 1;
+   const uint32_t fe = u.fn[f];
+   const SqSp &kq = u.ksp[fe >> 16];
+   const TypePlan &tp = u.tp;
+   const int k = ((q.s1 * tp.nsh[1] + q.s2) * tp.nsh[2] + kq.s1) * tp.nsh[3] + kq.s2;
+   const KsGroup ks = group_ks(u.b, tp, u.g, k);
+   const int nlb = tp.nl[1][q.s2], nlc = tp.nl[2][kq.s1], nld = tp.nl[3][kq.s2];
+   const int nsc = 2 * kq.l1 + 1, nsd = 2 * kq.l2 + 1;
+   const int cf = (int)(fe & 255) - kq.f1, df = (int)((fe >> 8) & 255) - kq.f2;
+   const int ia = cb / nlb, ib = cb - ia * nlb, ic = cf / nsc, isc = cf - ic * nsc, id = df / nsd, isd = df - id * nsd;
+   const int l = (cb * nlc + ic) * nld + id;
+   if (l >= (int)ks_count(ks.flags)) return;
+   if (ks.flags & KS_OUTPUT) {
+      double *O = u.kt.out + ((size_t)ks.base[0] | (size_t)ks.base[1] << 32);
+      for (int x = 0; x < SA; x++)
+         for (int y = 0; y < SB; y++) {
+            double &o = O[tra_index(ia, x, ib, y, ic, isc, id, isd, nlb, nlc, nld, SA, SB, nsc, nsd)];
+            o = u.add ? o + I[(x * SB + y) * is] : I[(x * SB + y) * is];
+         }
+      return;
+   }
+   size_t off[4];
+   uint32_t ld01 = ks.ld01, ld23 = ks.ld23, flags = ks.flags;
+   if (flags & KS_EXPLICIT) {
+      const KsRec x = u.b.ksx[ks.expl + l];
+      for (int z = 0; z < 4; z++) off[z] = x.off[z];
+      ld01 = x.ld01;
+      ld23 = x.ld23;
+      flags = x.flags;
+   } else {
+      off[0] = (size_t)((long long)ks.base[0] + (long long)ia * ks.step[0] + (long long)ic * ks.step[1]);
+      off[1] = (size_t)((long long)ks.base[1] + (long long)ia * ks.step[2] + (long long)id * ks.step[3]);
+      off[2] = (size_t)((long long)ks.base[2] + (long long)ib * ks.step[4] + (long long)ic * ks.step[5]);
+      off[3] = (size_t)((long long)ks.base[3] + (long long)ib * ks.step[6] + (long long)id * ks.step[7]);
+   }
+   const double fac = -symm_fac((flags >> 4) & 7) * u.kt.hf_fac;
+   if (fac == 0.0) return;
+   const unsigned ldac = ld01 & 0xffff, ldad = ld01 >> 16, ldbc = ld23 & 0xffff, ldbd = ld23 >> 16;
+   const bool Tac = flags & 1, Tad = flags & 2, Tbc = flags & 4, Tbd = flags & 8;
+   for (int sp = 0; sp < u.kt.nspin; sp++) {
+      const double *P = sp ? u.kt.P[1] : u.kt.P[0];
+      double *K = sp ? u.kt.K[1] : u.kt.K[0];
+      for (int x = 0; x < SA; x++) {
+         double kc = 0.0, kd = 0.0;
+         for (int y = 0; y < SB; y++) {
+            kc += I[(x * SB + y) * is] * P[off[3] + blk_at(Tbd, ldbd, y, isd)];
+            kd += I[(x * SB + y) * is] * P[off[2] + blk_at(Tbc, ldbc, y, isc)];
+         }
+         unsafeAtomicAdd(&K[off[0] + blk_at(Tac, ldac, x, isc)], fac * kc);
+         unsafeAtomicAdd(&K[off[1] + blk_at(Tad, ldad, x, isd)], fac * kd);
+      }
+      for (int y = 0; y < SB; y++) {
+         double kc = 0.0, kd = 0.0;
+         for (int x = 0; x < SA; x++) {
+            kc += I[(x * SB + y) * is] * P[off[1] + blk_at(Tad, ldad, x, isd)];
+            kd += I[(x * SB + y) * is] * P[off[0] + blk_at(Tac, ldac, x, isc)];
+         }
+         unsafeAtomicAdd(&K[off[2] + blk_at(Tbc, ldbc, y, isc)], fac * kc);
+         unsafeAtomicAdd(&K[off[3] + blk_at(Tbd, ldbd, y, isd)], fac * kd);
+      }
+   }
+}
+
+// the same through the item's blocks in LDS (set-level K layout): the sums
+// over b go to K_ac and K_ad, those over a to K_bc and K_bd
+template <int la, int lb>
+__device__ __forceinline__ void k_update_lds(const double *I, const Upd &u, const SqSp &q, int cb, int f)
+{
+   constexpr int SA = 2 * la + 1, SB = 2 * lb + 1;
+   const uint32_t fe = u.fn[f];
+   const int c = fe & 255, d = (fe >> 8) & 255;
+   const int ia = cb / q.n2, ib = cb - ia * q.n2;
+   const int a0 = q.f1 + ia * SA, b0 = q.f2 + ib * SB;
+   const int oad = u.NA * u.NC, obc = oad + u.NA * u.ND, obd = obc + u.NB * u.NC;
+   const int nblk = obd + u.NB * u.ND;
+   for (int sp = 0; sp < u.kt.nspin; sp++) {
+      const double *P = u.Pl + sp * nblk;
+      double *K = u.Kl + sp * nblk;
+      {
+         double pc[SB], pd[SB];
+#pragma unroll
+         for (int y = 0; y < SB; y++) {
+            pc[y] = P[obc + (b0 + y) * u.NC + c];
+            pd[y] = P[obd + (b0 + y) * u.ND + d];
+         }
+#pragma unroll
+         for (int x = 0; x < SA; x++) {
+            double kc = 0.0, kd = 0.0;
+#pragma unroll
+            for (int y = 0; y < SB; y++) {
+               kc += I[x * SB + y] * pd[y];
+               kd += I[x * SB + y] * pc[y];
+            }
+            atomicAdd(&K[(a0 + x) * u.NC + c], kc);
+            atomicAdd(&K[oad + (a0 + x) * u.ND + d], kd);
+         }
+      }
+      double qc[SA], qd[SA];
+#pragma unroll
+      for (int x = 0; x < SA; x++) {
+         qc[x] = P[(a0 + x) * u.NC + c];
+         qd[x] = P[oad + (a0 + x) * u.ND + d];
+      }
+#pragma unroll
+      for (int y = 0; y < SB; y++) {
+         double kc = 0.0, kd = 0.0;
+#pragma unroll
+         for (int x = 0; x < SA; x++) {
+            kc += I[x * SB + y] * qd[x];
+            kd += I[x * SB + y] * qc[x];
+         }
+         atomicAdd(&K[obc + (b0 + y) * u.NC + c], kc);
+         atomicAdd(&K[obd + (b0 + y) * u.ND + d], kd);
+      }
+   }
+}
+
+// ket transform of the units of one shell pair in the rows of C (row stride
+// ts), in place: a unit's functions end where its columns ended at the
+// latest, and the lanes take (row, unit) in rising order, so nothing unread
+// is overwritten
+template <int l1, int l2>
+__device__ __forceinline__ void ket_units(double *T, int ts, int nrow, const SqSp &q, const double R[3], int lane)
+{
+   constexpr int NIN = n_side(l1, l2), NOUT = (2 * l1 + 1) * (2 * l2 + 1);
+   const int nc = q.nc, n = nrow * nc;
+   for (int i = lane; i < n; i += 64) {
+      const int r = fdiv(i, nc), u = i - r * nc;
+      const double *c = T + r * ts + q.row0 + u * NIN;
+      double in[NIN], out[NOUT];
+#pragma unroll
+      for (int x = 0; x < NIN; x++) in[x] = c[x];
+      side_transform<l1, l2>(in, R, out);
+      double *d = T + r * ts + q.fn0 + u * NOUT;
+#pragma unroll
+      for (int x = 0; x < NOUT; x++) d[x] = out[x];
+   }
+}
+
+// bra transform and K update of the units of one shell pair: lanes over
+// (unit, ket function)
+template <int l1, int l2>
+__device__ __forceinline__ void bra_units(double *D, int ds, int nfn, const SqSp &q, const double R[3], const Upd &u,
+                                          int lane)
+{
+   constexpr int NIN = n_side(l1, l2), NOUT = (2 * l1 + 1) * (2 * l2 + 1);
+   const int n = q.nc * nfn;
+   for (int i = lane; i < n; i += 64) {
+      const int c = fdiv(i, nfn), f = i - c * nfn;
+      double *d = D + (q.row0 + c * NIN) * ds + f;
+      double in[NIN], out[NOUT];
+#pragma unroll
+      for (int x = 0; x < NIN; x++) in[x] = d[x * ds];
+      side_transform<l1, l2>(in, R, out);
+      if (u.lds) {
+         k_update_lds<l1, l2>(out, u, q, q.c0 + c, f);
+      } else {
+         // back in place: k_update_class takes them from there
+#pragma unroll
+         for (int x = 0; x < NOUT; x++) d[x * ds] = out[x];
+      }
+   }
+}
+
+template <int LM>
+__device__ __forceinline__ void ket_transform(double *T, int ts, int nrow, const SqSp &q, const double R[3], int lane)
+{
+   switch (q.l1 * 4 + q.l2) {
+#define GINT_SQ_KET(a_, b_)                                                                              \
+   case a_ * 4 + b_:                                                                                     \
+      if constexpr (a_ <= LM && b_ <= LM) ket_units<a_, b_>(T, ts, nrow, q, R, lane);                    \
+      break;
+      GINT_SQ_KET(0, 0) GINT_SQ_KET(0, 1) GINT_SQ_KET(0, 2) GINT_SQ_KET(0, 3)
+      GINT_SQ_KET(1, 0) GINT_SQ_KET(1, 1) GINT_SQ_KET(1, 2) GINT_SQ_KET(1, 3)
+      GINT_SQ_KET(2, 0) GINT_SQ_KET(2, 1) GINT_SQ_KET(2, 2) GINT_SQ_KET(2, 3)
+      GINT_SQ_KET(3, 0) GINT_SQ_KET(3, 1) GINT_SQ_KET(3, 2) GINT_SQ_KET(3, 3)
+#undef GINT_SQ_KET
+   }
+}
+
+template <int LM>
+__device__ __forceinline__ void bra_transform(double *D, int ds, int nfn, const SqSp &q, const double R[3],
+                                              const Upd &u, int lane)
+{
+   switch (q.l1 * 4 + q.l2) {
+#define GINT_SQ_BRA(a_, b_)                                                                              \
+   case a_ * 4 + b_:                                                                                     \
+      if constexpr (a_ <= LM && b_ <= LM) bra_units<a_, b_>(D, ds, nfn, q, R, u, lane);                  \
+      break;
+      GINT_SQ_BRA(0, 0) GINT_SQ_BRA(0, 1) GINT_SQ_BRA(0, 2) GINT_SQ_BRA(0, 3)
+      GINT_SQ_BRA(1, 0) GINT_SQ_BRA(1, 1) GINT_SQ_BRA(1, 2) GINT_SQ_BRA(1, 3)
+      GINT_SQ_BRA(2, 0) GINT_SQ_BRA(2, 1) GINT_SQ_BRA(2, 2) GINT_SQ_BRA(2, 3)
+      GINT_SQ_BRA(3, 0) GINT_SQ_BRA(3, 1) GINT_SQ_BRA(3, 2) GINT_SQ_BRA(3, 3)
+#undef GINT_SQ_BRA
+   }
+}
+
+template <int LM>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LM == 3 ? 1 : (LM == 2 ? 3 : 4))))
+void k_sq(const TypePlan *__restrict__ tpp, DevTables t, BatchDev b, KTargets kt, SqArgs y)
+{
+   extern __shared__ __align__(16) double lds[];
+   const TypePlan &tp = *tpp;
+   const int lane = threadIdx.x;
+   const int ncpt = tp.ncp, nkc = tp.nkc;
+   const uint32_t nfix = min(b.fix_count[0], b.fix_cap);
+   char *tab = (char *)lds;
+   uint16_t *tcol = (uint16_t *)tab;
+   uint32_t *urb = (uint32_t *)(tab + SQ_TAB_URB), *urk = (uint32_t *)(tab + SQ_TAB_URK);
+   uint32_t *tfn = (uint32_t *)(tab + SQ_TAB_FN), *tip = (uint32_t *)(tab + SQ_TAB_IP);
+   double *co = lds + y.o_co;   // the set quartet's coefficients, contraction by contraction
+   const int m16 = lane & 15, k4 = lane >> 4;
+   {
+      const uint32_t item = blockIdx.x;
+      const uint32_t gi = b.g0 + item / (uint32_t)y.nitem;
+      const SqItem it = load_uniform(y.items + item % (uint32_t)y.nitem);
+      const SqTile bt = load_uniform(y.tiles + it.bt), ktl = load_uniform(y.tiles + it.kt);
+      const SqSp *bsp = y.sps + bt.sp, *ksp = y.sps + ktl.sp;
+      const GroupRec &g = b.groups[gi];
+      const int nfn = ktl.nfn, ncol = ktl.nrow, cs = ncol | 1, ncc = ktl.nrc;
+      double *WC = lds + it.o_wc, *C = lds + it.o_c;
+      lds_order();
+      const GroupHead gh = load_uniform((const GroupHead *)&g);
+      const uint32_t np4 = load_uniform(&g.np4);
+      // tables of the ket tile; the coefficients of its and the bra tile's units
+      for (int i = lane; i < ncol; i += 64) tcol[i] = y.rows[ktl.row + i];
+      for (int i = lane; i < nfn; i += 64) tfn[i] = y.fns[ktl.fn + i];
+      {
+         int off = 0;
+         for (int tc = 0; tc < 4; tc++) {
+            const int np = ((np4 >> (4 * tc)) & 15) + 1;
+            for (int s = 0; s < tp.nsh[tc]; s++) {
+               const int n = tp.nl[tc][s] * np;
+               const double *src = b.data + load_uniform(&g.Kof[tc][s]);
+               for (int i = lane; i < n; i += 64) co[off + i] = src[i];
+               off += n;
+            }
+         }
+      }
+      {
+         // first coefficient of the sets: their contractions follow each other
+         const int npa = (np4 & 15) + 1, npb = ((np4 >> 4) & 15) + 1, npc = ((np4 >> 8) & 15) + 1,
+                   npd = ((np4 >> 12) & 15) + 1;
+         const int ob = y.ncon[0] * npa, oc = ob + y.ncon[1] * npb, od = oc + y.ncon[2] * npc;
+         if (lane < 2 * SQ_MAXRC) {
+            const bool ket = lane >= SQ_MAXRC;
+            const int un = ket ? lane - SQ_MAXRC : lane;
+            if (un < (ket ? (int)ktl.nrc : (int)bt.nrc)) {
+               const uint32_t rc = y.rcs[2 * ((ket ? ktl.rc : bt.rc) + un)];
+               uint32_t *ur = ket ? urk : urb;
+               ur[un] = (uint32_t)((ket ? oc : 0) + (int)(rc & 255) * (ket ? npc : npa)) |
+                        (uint32_t)((ket ? od : ob) + (int)(rc >> 8) * (ket ? npd : npb)) << 16;
+            }
+         }
+      }
+      // the units of the lane's matrix-core results (4 r + lane / 16): first
+      // row less first component, and the components they have
+      int urow[4];
+      unsigned ulo[4], un_[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+         const int un = 4 * r + k4;
+         const uint32_t v = un < bt.nrc ? y.rcs[2 * (bt.rc + un) + 1] : 0u;
+         ulo[r] = (v >> 8) & 255;
+         un_[r] = (v >> 16) - ulo[r];
+         urow[r] = (int)(v & 255) - (int)ulo[r];
+      }
+      const bool setlevel = (load_uniform(&g.ksmode) & KS_SETLEVEL) != 0;
+      Upd u{b, kt, tp, g, ksp, lds + it.o_pk, nullptr, tfn, it.lds_k && setlevel, false, bt.n1, bt.n2, ktl.n1, ktl.n2};
+      const int nblk = (u.NA + u.NB) * (u.NC + u.ND);
+      u.Kl = u.Pl + kt.nspin * nblk;
+      double fac = 0.0;
+      // element e of the item's four blocks in P and K
+      KsSet kss{};
+      if (setlevel) {
+         kss = load_uniform(b.kss + load_uniform(&g.ks));
+         fac = -symm_fac((kss.flags >> 4) & 7) * kt.hf_fac;
+         if (fac == 0.0) return;
+      }
+      auto blocks = [&](auto &&f) {
+         auto one = [&](int qb, int e0, int nr, int nc, int r0, int c0) {
+            const unsigned ld = ((qb < 2 ? kss.ld01 : kss.ld23) >> (16 * (qb & 1))) & 0xffff;
+            const bool tr = (kss.flags >> qb) & 1;
+            const unsigned rs = tr ? ld : 1, cst = tr ? 1 : ld;
+            const size_t base = kss.base[qb];
+            for (int e = lane; e < nr * nc; e += 64) {
+               const int r = fdiv(e, nc), c = e - r * nc;
+               f(e0 + e, base + (size_t)(r0 + r) * rs + (size_t)(c0 + c) * cst);
+            }
+         };
+         const int oad = u.NA * u.NC, obc = oad + u.NA * u.ND, obd = obc + u.NB * u.NC;
+         one(0, 0, u.NA, u.NC, bt.r1, ktl.r1);
+         one(1, oad, u.NA, u.ND, bt.r1, ktl.r2);
+         one(2, obc, u.NB, u.NC, bt.r2, ktl.r1);
+         one(3, obd, u.NB, u.ND, bt.r2, ktl.r2);
+      };
+      if (u.lds)
+         blocks([&](int e, size_t o) {
+            for (int sp = 0; sp < kt.nspin; sp++) {
+               u.Pl[sp * nblk + e] = (sp ? kt.P[1] : kt.P[0])[o];
+               u.Kl[sp * nblk + e] = 0.0;
+            }
+         });
+      lds_order();
+      auto wbra = [&](int un, uint32_t ip) { return co[(urb[un] & 0xffff) + (ip & 15)] * co[(urb[un] >> 16) + ((ip >> 4) & 15)]; };
+      auto wket = [&](int un, uint32_t ip) {
+         return co[(urk[un] & 0xffff) + ((ip >> 8) & 15)] * co[(urk[un] >> 16) + ((ip >> 12) & 15)];
+      };
+      // minimum images of B and D
+      const Vec3 Ra = load_uniform((const Vec3 *)(b.data + gh.R[0])), Rb = load_uniform((const Vec3 *)(b.data + gh.R[1])),
+                 Rc = load_uniform((const Vec3 *)(b.data + gh.R[2])), Rd = load_uniform((const Vec3 *)(b.data + gh.R[3]));
+      double ABs[3], CDs[3];
+      {
+         const Cell cell = load_uniform((const Cell *)t.cell);
+         gint_pbc(Ra.v, Rb.v, cell.v, ABs);
+         gint_pbc(Rc.v, Rd.v, cell.v, CDs);
+      }
+      for (uint32_t r = gh.row0; r < gh.row1; r++) {
+         const RowRec row = load_uniform(b.rows + r);
+         double AB[3], CD[3];
+         {
+            const Vec3 g1 = load_uniform((const Vec3 *)(t.neighs + 3 * (row.n12 & 0xffff))),
+                       g2 = load_uniform((const Vec3 *)(t.neighs + 3 * (row.n12 >> 16)));
+#pragma unroll
+            for (int x = 0; x < 3; x++) {
+               const double Bx = Ra.v[x] + ABs[x] + g1.v[x];
+               const double Dx = Rc.v[x] + CDs[x] + g2.v[x];
+               AB[x] = Ra.v[x] - Bx;
+               CD[x] = Rc.v[x] - Dx;
+            }
+         }
+         lds_order();
+         if (it.eco_off >= 0) {
+            // contracted on the matrix cores by k_eco: the units of the tile
+            // are part of one class's contractions
+            const SqSp qb = load_uniform(bsp), qk = load_uniform(ksp);
+            const int nbra = bt.ncomp, nket = fdiv(ncol, qk.nc), ncp = nbra * nket;
+            const int nck = tp.nl[2][qk.s1] * tp.nl[3][qk.s2];
+            const double *E0 = b.eco + (size_t)(r - b.r0) * b.eco_row + it.eco_off;
+            for (int cu = 0; cu < qb.nc; cu++) {
+               const double *E = E0 + ((size_t)(qb.c0 + cu) * nck + qk.c0) * ncp;
+               for (int i = lane; i < qk.nc * ncp; i += 64) {
+                  const int c = fdiv(i, ncp), j = i - c * ncp, e = fdiv(j, nket);
+                  C[(cu * nbra + e) * cs + c * nket + (j - e * nket)] = E[i];
+               }
+            }
+         } else {
+            const uint32_t *IP = b.prm_ip + row.prm_off;
+            const double *A0 = b.ac0 + (size_t)(row.prm_off - b.p0) * ncpt + (size_t)bt.comp0 * nkc + ktl.comp0;
+            for (int w0 = 0; w0 < (int)row.n_prm; w0 += SQ_NW) {
+               const int nw = min(SQ_NW, (int)row.n_prm - w0);
+               lds_order();
+               if (lane < SQ_NW) tip[lane] = lane < nw ? IP[w0 + lane] : 0u;
+               lds_order();
+               for (int i = lane; i < nw * ncc; i += 64) {
+                  const int n = fdiv(i, ncc);
+                  WC[i] = wket(i - n * ncc, tip[n]);
+               }
+               double wb[4];
+               int no[4];   // the lane's primitive quartet of each step (past the window: its last, with weight 0)
+#pragma unroll
+               for (int z = 0; z < 4; z++) {
+                  const int n = 4 * z + k4;
+                  wb[z] = (n < nw && m16 < bt.nrc) ? wbra(m16, tip[n]) : 0.0;
+                  no[z] = min(n, nw - 1);
+               }
+               lds_order();
+               const double *Aw = A0 + (size_t)w0 * ncpt;
+               for (int c0 = 0; c0 < ncol; c0 += 16) {
+                  const bool okc = c0 + m16 < ncol;
+                  const uint32_t tc = tcol[okc ? c0 + m16 : 0];
+                  double wc[4];
+                  int ao[4];
+#pragma unroll
+                  for (int z = 0; z < 4; z++) {
+                     wc[z] = WC[no[z] * ncc + (int)(tc >> 8)];
+                     ao[z] = no[z] * ncpt + (int)(tc & 255);
+                  }
+                  double *cq[4];
+                  unsigned nq[4];
+#pragma unroll
+                  for (int q = 0; q < 4; q++) {
+                     cq[q] = C + urow[q] * cs + c0 + m16;
+                     nq[q] = okc ? un_[q] : 0u;
+                  }
+                  // 16 columns of component e after component, SQ_EU at a time
+                  auto tiles = [&](auto NZ) {
+                     constexpr int nz = decltype(NZ)::value;
+                     for (int e0 = 0; e0 < bt.ncomp; e0 += SQ_EU) {
+                        double a[SQ_EU][nz];
+#pragma unroll
+                        for (int v = 0; v < SQ_EU; v++) {
+                           const double *p = Aw + min(e0 + v, (int)bt.ncomp - 1) * nkc;
+#pragma unroll
+                           for (int z = 0; z < nz; z++) a[v][z] = p[ao[z]];
+                        }
+#pragma unroll
+                        for (int v = 0; v < SQ_EU; v++) {
+                           const int e = e0 + v;
+                           if (e >= bt.ncomp) break;
+                           dbl4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                           for (int z = 0; z < nz; z++)
+                              acc = __builtin_amdgcn_mfma_f64_16x16x4f64(wb[z], a[v][z] * wc[z], acc, 0, 0, 0);
+#pragma unroll
+                           for (int q = 0; q < 4; q++)
+                              if (4 * q < bt.nrc && (unsigned)e - ulo[q] < nq[q]) {
+                                 double *c = cq[q] + e * cs;
+                                 *c = w0 ? *c + acc[q] : acc[q];
+                              }
+                        }
+                     }
+                  };
+                  if (nw > 12) tiles(std::integral_constant<int, 4>{});
+                  else if (nw > 8) tiles(std::integral_constant<int, 3>{});
+                  else if (nw > 4) tiles(std::integral_constant<int, 2>{});
+                  else tiles(std::integral_constant<int, 1>{});
+               }
+            }
+         }
+         // slots of this row whose screening depends on the class
+         for (uint32_t e = 0; e < nfix; e++) {
+            const uint32_t p = b.fix[2 * e];
+            if (b.prm_row[p] != r) continue;
+            lds_order();
+            const uint32_t mask = b.fix[2 * e + 1] >> 8, ip = b.prm_ip[p];
+            const double *src = b.fix_ws + (size_t)e * (ncpt + 16);
+            const double *A = src + (size_t)bt.comp0 * nkc + ktl.comp0;
+            for (int qb = 0; qb < bt.nsp; qb++)
+               for (int qk = 0; qk < ktl.nsp; qk++) {
+                  const SqSp sb = load_uniform(bsp + qb), sk = load_uniform(ksp + qk);
+                  const int k = ((sb.s1 * tp.nsh[1] + sb.s2) * tp.nsh[2] + sk.s1) * tp.nsh[3] + sk.s2;
+                  const int gate = tp.cls_gate[k];
+                  const bool keep = (mask >> gate) & 1u;
+                  if (!keep && (sb.l1 || sk.l1)) continue;
+                  const int nr = sb.nc * (co_below(sb.l1 + sb.l2 + 1) - co_below(sb.l1));
+                  const int nc = sk.nc * (co_below(sk.l1 + sk.l2 + 1) - co_below(sk.l1));
+                  for (int i = lane; i < nr * nc; i += 64) {
+                     const int rr = fdiv(i, nc), cl = sk.row0 + i - rr * nc;
+                     const uint32_t tr = y.rows[bt.row + sb.row0 + rr], tc = tcol[cl];
+                     // a screened slot keeps its Fm[0] in (00|00) (reference src/compute_VRR.cpp:384-385)
+                     const double v = keep ? A[(tr & 255) * nkc + (tc & 255)]
+                                           : ((tr & 255) + (tc & 255) + bt.comp0 + ktl.comp0 == 0 ? src[ncpt + gate] : 0.0);
+                     C[(sb.row0 + rr) * cs + cl] += v * wbra(tr >> 8, ip) * wket(tc >> 8, ip);
+                  }
+               }
+         }
+         lds_order();
+         for (int q = 0; q < ktl.nsp; q++) {
+            const SqSp qk = load_uniform(ksp + q);
+            if (qk.l1 + qk.l2 > 0 || qk.row0 != qk.fn0) ket_transform<LM>(C, cs, bt.nrow, qk, CD, lane);
+         }
+         lds_order();
+         for (int q = 0; q < bt.nsp; q++) {
+            const SqSp qb = load_uniform(bsp + q);
+            bra_transform<LM>(C, cs, nfn, qb, AB, u, lane);
+            if (u.lds) continue;
+            lds_order();
+            const int nbra = co_below(qb.l1 + qb.l2 + 1) - co_below(qb.l1);
+            for (int i = lane; i < qb.nc * nfn; i += 64) {
+               const int c = fdiv(i, nfn), f = i - c * nfn;
+               k_update_class(C + (qb.row0 + c * nbra) * cs + f, cs, u, qb, qb.c0 + c, f);
+            }
+         }
+         u.add = true;
+      }
+      lds_order();
+      if (u.lds)
+         blocks([&](int e, size_t o) {
+            for (int sp = 0; sp < kt.nspin; sp++) {
+               const double v = u.Kl[sp * nblk + e];
+               if (v != 0.0) unsafeAtomicAdd(&(sp ? kt.K[1] : kt.K[0])[o], fac * v);
+            }
+         });
+   }
+}
+
+}  // namespace sq
+
+template <int LM>
+int launch_sq_lm(const BatchDev &b, const DevTables &t, const KTargets &kt, const SqArgs &y, unsigned grid, size_t lds,
+                 void *stream);
+
+}  // namespace gint

@@ -190,24 +190,23 @@ void make_type_plan(TypePlan &tp)
    p.LC = lmax[2] + lmax[3];
    p.L = p.LA + p.LC;
    int off = 0;
-   for (int e = p.LA0; e <= p.LA; e++)
-      for (int f = p.LC0; f <= p.LC; f++) {
-         p.cpoff[e][f] = off;
-         off += nco(e) * nco(f);
-      }
-   p.ncp = off;
-   off = 0;
    for (int f = p.LC0; f <= p.LC; f++) {
       p.kcoff[f] = off;
       off += nco(f);
    }
    p.nkc = off;
+   off = 0;
+   for (int e = p.LA0; e <= p.LA; e++) {
+      p.bcoff[e] = off;
+      off += nco(e);
+   }
+   p.ncp = off * p.nkc;
    p.nbh = nherm(p.LA);
    p.nh = nherm(p.L);
    p.has00 = (p.LA0 == 0 && p.LC0 == 0) ? 1 : 0;
 
    std::set<int> Lset;
-   int k = 0, eoff = 0;
+   int k = 0;
    long long ref = 0;
    for (int sa = 0; sa < p.nsh[0]; sa++)
       for (int sb = 0; sb < p.nsh[1]; sb++)
@@ -219,22 +218,12 @@ void make_type_plan(TypePlan &tp)
                p.cls_sh[k] = sa | sb << 4 | sc << 8 | sd << 12;
                p.cls_nl[k] = p.nl[0][sa] * p.nl[1][sb] * p.nl[2][sc] * p.nl[3][sd];
                p.cls_ncp[k] = cp.ncp;
-               p.cls_eoff[k] = eoff;
-               eoff += p.cls_nl[k] * cp.ncp;
                p.cls_mult[k] = class_mult(p.cls_code[k]);
                p.mult_all += p.cls_mult[k];
                Lset.insert(cp.L);
                ref += cp.fm_flops + cp.vrr_flops;
             }
    p.nclass = k;
-   p.ebytes = eoff;
-   int co = 0;
-   for (int t = 0; t < 4; t++)
-      for (int s2 = 0; s2 < p.nsh[t]; s2++) {
-         p.co_off[t][s2] = co;
-         co += p.nl[t][s2] * MAXNP;
-      }
-   p.nco_tot = co;
    for (int t = 0; t < 4; t++) {
       int f = 0;
       for (int s2 = 0; s2 < p.nsh[t]; s2++) {
@@ -303,11 +292,202 @@ void make_type_items(const TypePlan &tp, std::vector<uint32_t> &e1, std::vector<
       for (int ie = 0; ie < nco(e); ie++)
          for (int f = tp.LC0; f <= tp.LC; f++)
             for (int jl = 0; jl < nco(f); jl++) {
-               const int j = tp.cpoff[e][f] + ie * nco(f) + jl;
+               const int j = (tp.bcoff[e] + ie) * nkc + tp.kcoff[f] + jl;
                e2.push_back((uint32_t)ce[ie][0] | (uint32_t)ce[ie][1] << 3 | (uint32_t)ce[ie][2] << 6 |
                             (uint32_t)(tp.kcoff[f] + jl) << 9 | (uint32_t)j << 16);
             }
    }
+}
+
+// The matrix-core contraction of a type (k_eco): its classes of at least
+// ECO_MIN_NQ contractions, one work item per 64 columns x 64 contractions of
+// each, their places in a row of the contraction buffer and their columns
+// among the type's.
+void make_eco_plan(const TypePlan &tp, const std::vector<ClassPlan> &cps, EcoPlan &ep)
+{
+   ep = EcoPlan();
+   ep.off.assign(tp.nclass, -1);
+   ep.info.assign(2 * MAXTC, 0);
+   for (int k = 0; k < tp.nclass; k++) {
+      const int nq = tp.cls_nl[k], cols = tp.cls_ncp[k];
+      if (nq < ECO_MIN_NQ) continue;
+      ep.off[k] = (int)ep.row;
+      ep.info[k] = (int)ep.srcmaps.size();
+      ep.info[MAXTC + k] = (int)ep.row;
+      ep.row += (size_t)nq * cols;
+      const ClassPlan &cp = cps[k];
+      for (int e = cp.la; e <= cp.LA; e++)
+         for (int ie = 0; ie < nco(e); ie++)
+            for (int f = cp.lc; f <= cp.LC; f++)
+               for (int jf = 0; jf < nco(f); jf++)
+                  ep.srcmaps.push_back((tp.bcoff[e] + ie) * tp.nkc + tp.kcoff[f] + jf);
+      for (int jt0 = 0; jt0 * 16 < cols; jt0 += 4)
+         for (int qb = 0; qb * 64 < nq; qb++) ep.items.push_back(EcoItem{(uint16_t)k, (uint16_t)jt0, (uint16_t)qb, 0});
+   }
+   // items in the order of the first type column they read: the classes
+   // share the row's blocks (a block (e,f) serves every class with
+   // la <= e <= la+lb, lc <= f <= lc+ld), so items that run together read
+   // the same columns of a row that is larger than the caches
+   auto first_col = [&](const EcoItem &it) { return ep.srcmaps[ep.info[it.k] + it.jt0 * 16]; };
+   std::stable_sort(ep.items.begin(), ep.items.end(), [&](const EcoItem &a, const EcoItem &b) {
+      const int ca = first_col(a), cb = first_col(b);
+      return ca < cb || (ca == cb && (a.k < b.k || (a.k == b.k && a.qb < b.qb)));
+   });
+}
+
+// One side of a type (bra: sets 0, 1; ket: sets 2, 3) in tiles of at most
+// `max_row` rows and `max_fn` functions; units with an f shell (wf) or
+// without one; single: one shell pair per tile.
+static void make_sq_tiles(const TypePlan &tp, int side, bool wf, int max_row, int max_fn, bool single, SqPlan &sp,
+                          std::vector<int> &out)
+{
+   const int x = 2 * side, y = 2 * side + 1, low = side ? tp.LC0 : tp.LA0;
+   auto below = [](int l) { return l * (l + 1) * (l + 2) / 6; };
+   auto con0 = [&](int set, int s) {   // contractions of the set's shells before s
+      int n = 0;
+      for (int i = 0; i < s; i++) n += tp.nl[set][i];
+      return n;
+   };
+   SqTile t{};
+   int lo1 = 0, hi1 = 0, lo2 = 0, hi2 = 0, e0 = 0, e1 = 0;
+   auto close = [&]() {
+      if (!t.nrow) return;
+      t.comp0 = (uint16_t)(below(e0) - below(low));
+      t.ncomp = (uint16_t)(below(e1 + 1) - below(e0));
+      t.r1 = (uint16_t)lo1;
+      t.n1 = (uint16_t)(hi1 - lo1);
+      t.r2 = (uint16_t)lo2;
+      t.n2 = (uint16_t)(hi2 - lo2);
+      t.row = (uint32_t)sp.rows.size();
+      t.rc = (uint32_t)sp.rcs.size() / 2;
+      t.fn = (uint32_t)sp.fns.size();
+      int rc = 0;
+      for (int i = 0; i < t.nsp; i++) {
+         SqSp &q = sp.sps[t.sp + i];
+         q.f1 = (int16_t)(tp.fun0[x][q.s1] - lo1);
+         q.f2 = (int16_t)(tp.fun0[y][q.s2] - lo2);
+         for (int c = q.c0; c < q.c0 + q.nc; c++, rc++) {
+            const int i1 = c / q.n2, i2 = c % q.n2;
+            const int c0 = below(q.l1) - below(e0), nr = below(q.l1 + q.l2 + 1) - below(q.l1);
+            sp.rcs.push_back((uint32_t)(con0(x, q.s1) + i1) | (uint32_t)(con0(y, q.s2) + i2) << 8);
+            sp.rcs.push_back((uint32_t)(q.row0 + (c - q.c0) * nr) | (uint32_t)c0 << 8 | (uint32_t)(c0 + nr) << 16);
+            for (int r = 0; r < nr; r++) sp.rows.push_back((uint16_t)((c0 + r) | rc << 8));
+            for (int s1 = 0; s1 < nsph(q.l1); s1++)
+               for (int s2 = 0; s2 < nsph(q.l2); s2++)
+                  sp.fns.push_back((uint32_t)(q.f1 + i1 * nsph(q.l1) + s1) | (uint32_t)(q.f2 + i2 * nsph(q.l2) + s2) << 8 |
+                                   (uint32_t)i << 16);
+         }
+      }
+      out.push_back((int)sp.tiles.size());
+      sp.tiles.push_back(t);
+      t = SqTile{};
+   };
+   // the first shells apart (their function ranges stay short) unless the
+   // whole side is one tile
+   int all = 0, all_fn = 0;
+   for (int s1 = 0; s1 < tp.nsh[x]; s1++)
+      for (int s2 = 0; s2 < tp.nsh[y]; s2++) {
+         const int l1 = tp.l[x][s1], l2 = tp.l[y][s2], nc = tp.nl[x][s1] * tp.nl[y][s2];
+         all += nc * (below(l1 + l2 + 1) - below(l1));
+         all_fn += nc * nsph(l1) * nsph(l2);
+      }
+   const bool whole = all <= max_row && all_fn <= max_fn;
+   for (int s1 = 0; s1 < tp.nsh[x]; s1++)
+      for (int s2 = 0; s2 < tp.nsh[y]; s2++) {
+         const int l1 = tp.l[x][s1], l2 = tp.l[y][s2];
+         if (!whole && s2 == 0) close();
+         if ((l1 > 2 || l2 > 2) != wf) continue;
+         const int nr = below(l1 + l2 + 1) - below(l1), nf = nsph(l1) * nsph(l2);
+         const int nc = tp.nl[x][s1] * tp.nl[y][s2];
+         if (single) close();
+         for (int c = 0; c < nc; c++) {
+            if (t.nrow && (t.nrow + nr > max_row || t.nfn + nf > max_fn || t.nrc + 1 > SQ_MAXRC)) close();
+            if (!t.nrow) {
+               t.sp = (uint32_t)sp.sps.size();
+               lo1 = lo2 = 1 << 20;
+               hi1 = hi2 = 0;
+               e0 = 99;
+               e1 = 0;
+            }
+            if (!t.nsp || sp.sps.back().s1 != s1 || sp.sps.back().s2 != s2) {
+               SqSp q{};
+               q.l1 = (uint8_t)l1;
+               q.l2 = (uint8_t)l2;
+               q.s1 = (uint8_t)s1;
+               q.s2 = (uint8_t)s2;
+               q.c0 = (uint8_t)c;
+               q.n2 = (uint8_t)tp.nl[y][s2];
+               q.row0 = t.nrow;
+               q.fn0 = t.nfn;
+               sp.sps.push_back(q);
+               t.nsp++;
+               e0 = std::min(e0, l1);
+               e1 = std::max(e1, l1 + l2);
+            }
+            sp.sps.back().nc++;
+            const int i1 = tp.fun0[x][s1] + c / tp.nl[y][s2] * nsph(l1), i2 = tp.fun0[y][s2] + c % tp.nl[y][s2] * nsph(l2);
+            lo1 = std::min(lo1, i1);
+            hi1 = std::max(hi1, i1 + nsph(l1));
+            lo2 = std::min(lo2, i2);
+            hi2 = std::max(hi2, i2 + nsph(l2));
+            t.nrow += nr;
+            t.nfn += nf;
+            t.nrc++;
+         }
+      }
+   close();
+}
+
+// The k_sq launch of the classes of a type with f shells (wf) or without,
+// for nspin density matrices; eco: classes of at least ECO_MIN_NQ
+// contractions take their contracted blocks from the contraction buffer (a
+// tile is then part of one shell pair).
+void make_sq_plan(const TypePlan &tp, const std::vector<ClassPlan> &cps, const EcoPlan &ep, bool wf, int nspin, bool eco,
+                  SqPlan &sp)
+{
+   (void)cps;
+   sp = SqPlan();
+   int lx = 0;
+   for (int t = 0; t < 4; t++)
+      for (int s = 0; s < tp.nsh[t]; s++) lx = std::max(lx, tp.l[t][s]);
+   if (wf && lx < 3) return;
+   sp.lm = wf ? 3 : std::min(lx, 2);
+   if (sp.lm == 0) sp.lm = 1;
+   std::vector<int> bra[2], ket[2];
+   for (int f = 0; f < 2; f++) {
+      make_sq_tiles(tp, 0, f == 1, 38, SQ_MAXFN, eco, sp, bra[f]);
+      make_sq_tiles(tp, 1, f == 1, 38, 30, eco, sp, ket[f]);
+   }
+   int top = 0;
+   for (int fb = 0; fb < 2; fb++)
+      for (int fk = 0; fk < 2; fk++) {
+         if ((fb || fk) != wf) continue;
+         for (int bi : bra[fb])
+            for (int ki : ket[fk]) {
+               const SqTile &b = sp.tiles[bi], &k = sp.tiles[ki];
+               SqItem it{};
+               it.bt = (uint16_t)bi;
+               it.kt = (uint16_t)ki;
+               it.eco_off = -1;
+               if (eco) {
+                  const SqSp &qb = sp.sps[b.sp], &qk = sp.sps[k.sp];
+                  const int c = ((qb.s1 * tp.nsh[1] + qb.s2) * tp.nsh[2] + qk.s1) * tp.nsh[3] + qk.s2;
+                  it.eco_off = ep.off[c];
+               }
+               const int pk = 2 * nspin * (b.n1 + b.n2) * (k.n1 + k.n2);
+               it.lds_k = pk <= 512 * nspin ? 1 : 0;
+               int off = SQ_TAB_BYTES / 8;
+               it.o_wc = off;
+               off += SQ_NW * k.nrc;
+               it.o_pk = off;
+               off += it.lds_k ? pk : 0;
+               it.o_c = off;
+               off += b.nrow * (k.nrow | 1);
+               top = std::max(top, off);
+               sp.items.push_back(it);
+            }
+      }
+   sp.lds_bytes = 8 * top;
 }
 
 }  // namespace gint

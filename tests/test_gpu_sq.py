@@ -1,0 +1,47 @@
+"""The quartet kernel (blocks -> contraction, HRR, spherical transform, K) at
+the edges of its tiles and windows, against the oracle: rows of 1 to 81
+primitive quartets (its windows hold 16, in steps of 4), every kind of K
+layout record, one and two spins, shell structures whose sides are one tile,
+several tiles and, with f shells, tiles of a single contraction; the
+contraction in the kernel itself and in its own kernel (debug bits 4 and 3).
+Bar: 1e-10 Ha + 1e-11 max|K|, the K-build's conditioning (test_conditioning)."""
+import numpy as np
+import pytest
+
+from helpers import oracle
+
+pytestmark = pytest.mark.gpu
+KTOL_ABS, KTOL_REL = 1e-10, 1e-11
+
+CASES = {
+    "np1": dict(n_water=2, box_A=7.0, image_shells=1, np_max=1, seed=4),
+    "np2_one_cell": dict(n_water=2, box_A=5.0, np_min=2, np_max=2, seed=3),
+    "np3_calls_reordered": dict(n_water=2, box_A=5.0, np_min=3, np_max=3, seed=6, ks_mix=1),
+    "small_basis": dict(n_water=3, box_A=6.0, basis=1, np_min=2, np_max=3, seed=8),
+    "f_basis": dict(n_water=1, box_A=5.0, basis=4, np_min=2, np_max=3, seed=2),
+    "spdf_centre": dict(n_water=1, n_tm=1, box_A=6.0, np_max=2, np_tm=3, seed=9),
+}
+
+
+@pytest.mark.parametrize("spins", [1, 2])
+@pytest.mark.parametrize("debug", [8, 16])
+@pytest.mark.parametrize("name", list(CASES))
+def test_tiles_and_windows(name, debug, spins):
+    from libgint_amd import driver as D, load
+
+    lib, o = load(), oracle()
+    s = D.System(**CASES[name])
+    st = s.record()
+    P = s.P()
+    kw = dict(P=P)
+    if spins == 2:
+        kw["Pb"] = P[::-1].copy()
+    Ko, ho = D.kbuild(o, "oracle_", s, st, **kw)
+    o.oracle_destroy_handle(ho)
+    for plan in (False, True):
+        K, h = D.kbuild(lib, "libgint_", s, st, plan=plan, debug=debug, **kw)
+        lib.libgint_amd_destroy_handle(h)
+        for a, b in zip(np.atleast_2d(K), np.atleast_2d(Ko)):
+            err, kmax = np.max(np.abs(a - b)), np.max(np.abs(b))
+            print(name, "debug", debug, "plan", plan, "sets", st.n_sets, "prm", st.n_prm, "max|K|", kmax, "max|dK|", err)
+            assert kmax > 0 and err <= KTOL_ABS + KTOL_REL * kmax
