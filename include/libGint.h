@@ -128,15 +128,16 @@ void libgint_amd_timing(void *handle, double out[12]);
 void libgint_amd_timing_eco(void *handle, double out[3]);
 void libgint_amd_reset_counters(void *handle);
 /* ms per launch key of one category of libgint_amd_timing (0 fm_r, 1 none,
-   2 sq, 3 fix-up, 4 matrix-core contraction) by the quartet type's total
-   angular momentum */
+   2 sq, 3 fix-up, 4 matrix-core contraction): eco by the quartet type's total
+   angular momentum, sq by its kernel (1 to 4), the others under 0 (their
+   launches serve many types) */
 void libgint_amd_timing_detail(void *handle, int cat, double out[256]);
 /* bit 0: route every surviving slot through the class-dependent screening
    path (a test of that path; results are unchanged); bit 1: run every
-   kernel of a chunk on the handle's stream, one after the other (per-kernel
-   durations without overlap, for profiling; results are unchanged); bit 2:
-   wait for the work of each quartet type and report its completion on
-   stderr (progress of long K-builds; results are unchanged); bit 3: the
+   kernel on the handle's stream, one after the other (per-kernel durations
+   without overlap, for profiling; results are unchanged); bit 2: wait for
+   the work of each launch set (up to 64 chunks of quartet types) and report
+   its completion on stderr (progress of long K-builds; results are unchanged); bit 3: the
    contraction of every type whose classes have one runs in the kernel of
    its own (k_eco), whatever the rule on primitive quartets per row says;
    bit 4: of no type (tests of both paths; results are unchanged) */

@@ -25,8 +25,8 @@ REF_SRC = "/root/reference/src"
 
 HOST_SRC = ["engine.cpp", "abi.cpp", "plan.cpp", "boys_table.cpp", "c0_file.cpp", "server.cpp"]
 DEV_SRC = ["kernels.hip", "kernels_sq.hip", "kernels_eco.hip"]
-# kernels_sq_part.hip is built once per highest angular momentum
-SQ_LM = (1, 2, 3)
+# kernels_sq_part.hip is built once per register group of k_sq
+SQ_LM = (1, 2, 3, 4)
 HIPFLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-munsafe-fp-atomics",
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall", "-Wno-unused-function"]
 HOSTFLAGS = ["-O2", "-std=c++17", "-fPIC", "-fopenmp", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__",

@@ -208,9 +208,21 @@ struct DevTables {
    double R_cut;
 };
 
-// One chunk of one type's work, resident in HBM.  Primitive, row and group
-// indices are absolute within the type's arrays; ac0 and eco are indexed
-// from the chunk's first primitive and first row.
+// LDS layout of k_fm_r for one type
+struct FmLayout {
+   int SB;      // survivors per Hermite batch
+   int o_fmv;   // per lane: G_m, then D_m = (-2 rho)^m G_m
+   int o_sv;    // per lane: X Y Z of P-Q-g, TG1 (or T), TG2
+   int o_R;     // Hermite layers, 2 x SB x nh
+   int o_int;   // byte offset of 64 lane infos (branch | patch << 2) and 64 survivor lanes
+   int bytes;
+};
+
+// One chunk of one type's work.  Primitive, row and group indices are
+// absolute within the type's arrays; ac0 and eco are indexed from the
+// chunk's first primitive and first row.  The records of a launch sequence's
+// chunks lie in device memory; a kernel takes a list of them (so that one
+// launch covers many types) and adds the execution's buffers (RunDev).
 struct BatchDev {
    const TypePlan *tp;        // device copy
    const uint32_t *e1;        // Hermite -> cartesian stage 1 items: t u v fx fy fz (3 bits each), W slot << 18
@@ -222,21 +234,45 @@ struct BatchDev {
    const KsGroup *ksg;        // per class of the groups that are not KS_SETLEVEL (GroupRec::ks)
    const KsSet *kss;          // KS_SETLEVEL groups
    const KsRec *ksx;
-   const double *data;
-   double *ac0;               // [primitive - p0][ncp]
+   uint64_t ac_off, eco_off;  // the chunk's blocks and contraction buffer rows in the work buffer, doubles
+   size_t eco_row;            // doubles per row of the contraction buffer (k_eco); 0: none
+   double *gmag;              // calibration: max |block element| per set quartet (nullable; absolute group index)
+   uint32_t *gflag;           // mixed precision: 1 = single-precision contraction for the set quartet (nullable)
    uint32_t p0, p1;           // primitives of the chunk
    uint32_t r0, r1;           // rows
    uint32_t g0, g1;           // groups
+   FmLayout fm, fix_fm;       // k_fm_r: the chunk's own pass, the fix-up
+   // set from RunDev by the kernels
+   const double *data;
+   double *ac0;               // [primitive - p0][ncp]
+   double *eco;
    unsigned long long *stats; // STATS_SLOTS x {surviving (slot, class) pairs, checksum, K1 FLOPs} (nullable)
-   uint32_t *fix;             // mixed-gate slots: (primitive, n3 | mask << 8)
+   uint32_t *fix;             // mixed-gate slots: (primitive, n3 | mask << 8 | chunk of the launch << 24)
    uint32_t *fix_count;       // [0] entries, [1] slots beyond fix_cap (kept by every class instead)
-   uint32_t fix_cap;
+   double *fix_ws;            // fix-up workspace, fix_stride doubles per entry
+   uint32_t fix_cap, fix_stride;
    int force_fix;             // route every surviving slot through the fix-up path (test hook)
-   double *fix_ws;            // fix-up workspace, ncp doubles per entry
-   double *eco;               // contraction buffer: eco_row doubles per row of the chunk (k_eco)
-   size_t eco_row;
-   double *gmag;              // calibration: max |block element| per set quartet (nullable; absolute group index)
-   const uint32_t *gflag;     // mixed precision: 1 = single-precision contraction for the set quartet (nullable)
+   uint32_t id;               // the chunk's number in the launch
+};
+
+// Buffers of an execution.
+struct RunDev {
+   double *work;
+   const double *data;
+   unsigned long long *stats;
+   uint32_t *fix, *fix_count;
+   double *fix_ws;
+   uint32_t fix_cap, fix_stride;
+   int force_fix;
+   int mixed;   // 0 off, 1 calibrate (gmag), 2 route (gflag)
+};
+
+constexpr int MAX_LAUNCH_CHUNKS = 64;   // of one launch
+
+// A chunk's part of a launch: its units of work end at `end` of the launch's
+// numbering, where the next one's begin.
+struct WorkRef {
+   uint32_t batch, end;
 };
 
 // One work item of the matrix-core contraction (k_eco) of a row: class k,
@@ -297,6 +333,10 @@ struct SqArgs {
    int nitem;
    int ncon[4];            // contractions of the four sets
    int o_co;               // LDS offset, doubles, of the coefficients
+};
+struct SqRef {            // a chunk's part of a k_sq launch
+   uint32_t batch, end;    // items
+   SqArgs y;
 };
 struct SqPlan {
    std::vector<SqItem> items;
@@ -359,12 +399,16 @@ void *noalloc_scratch();
 // zeroes n words (a kernel, not a memset node, so that the launch sequence
 // can be captured in a graph)
 int launch_zero_u32(uint32_t *p, int n, void *stream);
-int launch_fm_r(const TypePlan &tp, const DevTables &t, const BatchDev &b, void *stream);
-int launch_fixup(const TypePlan &tp, const DevTables &t, const BatchDev &b, uint32_t n_fix, void *stream);
-// from the chunk's blocks to K (kernels_sq.hpp): the classes of one plan
-// (max_np: the most primitives of a set in the chunk's type)
-int launch_sq(const TypePlan &tp, int max_np, const BatchDev &b, const DevTables &t, const KTargets &kt,
-              const SqPlan &sp, void *stream);
+// k_fm_r over the chunks of a list (pair: two primitive quartets per
+// wavefront, units are pairs), and the fix-up of the listed slots
+int launch_fm_r(const BatchDev *batches, const WorkRef *refs, int nref, uint32_t units, bool pair, size_t lds,
+                const DevTables &t, const RunDev &run, void *stream);
+int launch_fixup(const BatchDev *batches, size_t lds, const DevTables &t, const RunDev &run, uint32_t n_fix, void *stream);
+// the layouts of a type and whether k_fm_r takes its primitive quartets in pairs
+void fm_layouts(const TypePlan &tp, int Ng, FmLayout &main, FmLayout &fix, bool *pair);
+// from the chunks' blocks to K (kernels_sq.hpp)
+int launch_sq(const BatchDev *batches, const SqRef *refs, int nref, uint32_t items, int lm, size_t lds,
+              const DevTables &t, const RunDev &run, const KTargets &kt, void *stream);
 // contraction of primitive blocks on the matrix cores (kernels_eco.hip) for
 // classes with at least this many contractions
 constexpr int ECO_MIN_NQ = 8;
@@ -376,14 +420,15 @@ struct EcoPlan {
    size_t row = 0;             // doubles per row of the buffer
 };
 void make_eco_plan(const TypePlan &tp, const std::vector<ClassPlan> &cps, EcoPlan &ep);
-void make_sq_plan(const TypePlan &tp, const std::vector<ClassPlan> &cps, const EcoPlan &ep, bool wf, int nspin, bool eco,
-                  SqPlan &sp);
-int launch_eco(const TypePlan &tp, const BatchDev &b, const EcoArgs &e, void *stream);
+void make_sq_plan(const TypePlan &tp, const EcoPlan &ep, int grp, int nspin, bool eco, SqPlan &sp);
+constexpr int SQ_GROUPS = 3;   // register groups of k_sq's items
+constexpr int SQ_KERNELS = 4;  // k_sq<1..4>: s and p shells; and d; and f with a transform no larger than (dd|'s; any
+int launch_eco(const BatchDev *batch, const RunDev &run, uint32_t nrow, const EcoArgs &e, void *stream);
 // mixed precision: max |P| (*out, zeroed first) and the route of each set
 // quartet of a chunk from its calibrated magnitude
 int launch_absmax(const double *P, size_t n, unsigned long long *out, bool zero, void *stream);
-int launch_mixed_flags(const TypePlan &tp, const BatchDev &b, const double *gmag, const unsigned long long *pmax,
-                       double tau, uint32_t *gflag, unsigned long long *count, void *stream);
+int launch_mixed_flags(const BatchDev *batch, const RunDev &run, uint32_t ng, const unsigned long long *pmax, double tau,
+                       unsigned long long *count, void *stream);
 // D (16 x 16, row-major) = A (16 x 4) B (4 x 16) through the matrix-core
 // tile the contraction uses, with its lane layout; 0 or -1
 int mfma_selftest(const double *A, const double *B, double *D, int prec);

@@ -99,6 +99,12 @@ void TypeDev::release()
    chunks.clear();
 }
 
+void LaunchPlan::release()
+{
+   if (dev) (void)hipFree(dev);
+   *this = LaunchPlan();
+}
+
 // ---------------------------------------------------------------------------
 // team-shared objects: streams per OpenMP thread (reference
 // src/libGint.cpp:26,37-60) and the device P / K of the current step
@@ -142,11 +148,12 @@ Engine::~Engine()
    if (own_stream_ && stream_) (void)hipStreamDestroy((hipStream_t)stream_);
    for (auto &d : stream_dev_) d.release();
    for (auto &d : plan_dev_) d.release();
+   for (LaunchPlan *lp : {&stream_lp_, &plan_lp_, &plan_na_lp_}) lp->release();
    for (auto &ti : types_) {
       if (ti.d_plan) (void)hipFree(ti.d_plan);
       if (ti.d_e1) (void)hipFree(ti.d_e1);
       if (ti.d_e2) (void)hipFree(ti.d_e2);
-      for (SqPlan *sp = &ti.sq[0][0][0]; sp != &ti.sq[0][0][0] + 8; sp++) {
+      for (SqPlan *sp = &ti.sq[0][0][0]; sp != &ti.sq[0][0][0] + 4 * SQ_GROUPS; sp++) {
          if (sp->dev) (void)hipFree(sp->dev);
       }
       if (ti.d_srcmaps) (void)hipFree(ti.d_srcmaps);
@@ -298,8 +305,7 @@ int Engine::type_of(int i, int j, int k, int l)
       make_eco_plan(ti.plan, ti.cplans, ti.eco);
       for (int sp = 0; sp < 2; sp++)
          for (int e = 0; e < 2; e++)
-            for (int f = 0; f < 2; f++)
-               make_sq_plan(ti.plan, ti.cplans, ti.eco, f == 1, sp + 1, e == 1, ti.sq[sp][e][f]);
+            for (int f = 0; f < SQ_GROUPS; f++) make_sq_plan(ti.plan, ti.eco, f, sp + 1, e == 1, ti.sq[sp][e][f]);
       types_.push_back(ti);
       q_.emplace_back();
       it = type_ids_.emplace(sig, (int)types_.size() - 1).first;
@@ -735,6 +741,7 @@ void Engine::dispatch_all()
    if (!d_P_[0]) fatal("integrals dispatched before set_P", 0);
    synchronize();   // the previous batch no longer reads the device arrays
    upload(q_, stream_dev_, false);
+   stream_lp_.valid = false;
    for (auto &Q : q_) {
       Q.rows.clear();
       Q.prm_ip.clear();
@@ -774,6 +781,8 @@ void Engine::plan_end()
    // allocation (plan_execute_noalloc)
    ensure_tables();
    upload_data();
+   plan_lp_.valid = false;
+   build_launches(plan_dev_, true, plan_na_lp_);
    pend_bytes_ = 0;
    plan_max_index_ = max_index_;
    max_index_ = 0;
@@ -786,12 +795,10 @@ void Engine::plan_execute()
    dispatch_all();
    RunBufs w{};
    KTargets kt{};
-   if (!prepare_exec(plan_dev_, plan_max_index_, w, kt, FP_size_)) return;
-   mixed_mode_ = 0;
-   if (mixed_tau_ > 0.0 && !d_out_) {
-      ensure_mixed();
-      mixed_mode_ = mixed_calibrated_ ? 2 : 1;
-   }
+   const bool mixed = mixed_tau_ > 0.0 && !d_out_;
+   if (mixed) ensure_mixed();
+   if (!prepare_exec(plan_dev_, plan_lp_, plan_max_index_, w, kt, FP_size_)) return;
+   if (mixed) w.run.mixed = mixed_calibrated_ ? 2 : 1;
    // per-launch events, device counters and host waits stay eager; so does
    // a handle of a team of several threads: while one thread captured its
    // stream, the others make allocating and synchronous calls of the
@@ -799,9 +806,8 @@ void Engine::plan_execute()
    if (graph_on_ && nomp_ == 1 && !timing_on_ && !stats_on_ && (debug_ & 6) == 0)
       replay_graph(w, kt);
    else
-      launch_all(plan_dev_, w, kt);
-   if (mixed_mode_ == 1) mixed_calibrated_ = true;
-   mixed_mode_ = 0;
+      launch_all(plan_dev_, plan_lp_, w, kt);
+   if (w.run.mixed == 1) mixed_calibrated_ = true;
 }
 
 // device arrays of the mixed-precision route (plans)
@@ -816,6 +822,7 @@ void Engine::ensure_mixed()
       HIPCHECK(hipMalloc((void **)&D.gmag, sizeof(double) * D.n_groups));
       HIPCHECK(hipMalloc((void **)&D.gflag, sizeof(uint32_t) * D.n_groups));
       mixed_calibrated_ = false;
+      plan_lp_.valid = false;   // its tables name the arrays
    }
 }
 
@@ -838,6 +845,8 @@ void Engine::plan_clear()
    drop_graph();
    for (auto &d : plan_dev_) d.release();
    plan_dev_.clear();
+   plan_lp_.release();
+   plan_na_lp_.release();
 }
 
 void Engine::queue_info(uint64_t out[8])
@@ -1002,7 +1011,7 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
          put(ti.d_srcmaps, ti.eco.srcmaps);
          put(ti.d_eco_info, ti.eco.info);
          put(ti.d_eco_items, ti.eco.items);
-         for (SqPlan *sp = &ti.sq[0][0][0]; sp != &ti.sq[0][0][0] + 8; sp++) {
+         for (SqPlan *sp = &ti.sq[0][0][0]; sp != &ti.sq[0][0][0] + 4 * SQ_GROUPS; sp++) {
             if (sp->items.empty()) continue;
             std::vector<char> all;
             int n = 0;
@@ -1075,7 +1084,6 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
             const size_t gp = (gb - (size_t)(g.row1 - g.row0) * eco_row * sizeof(double)) /
                               (sizeof(double) * (size_t)tp.ncp);
             if (bytes + gb > wbytes && c.g1 > c.g0) {
-               if (flops) D.max_chunk_bytes = std::max(D.max_chunk_bytes, bytes);
                out.push_back(c);
                c = Chunk{};
                c.g0 = c.g1 = (uint32_t)gi;
@@ -1107,12 +1115,8 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
                }
             }
          }
-         if (c.g1 > c.g0) {
-            if (flops) D.max_chunk_bytes = std::max(D.max_chunk_bytes, bytes);
-            out.push_back(c);
-         }
+         if (c.g1 > c.g0) out.push_back(c);
       };
-      D.max_chunk_bytes = 0;
       make_chunks(work, D.chunks, true);
       D.chunks_na.clear();
       D.na_fit = D.max_group_bytes <= NOALLOC_AC0_BYTES;
@@ -1122,11 +1126,11 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
    }
 }
 
-void Engine::ensure_work(size_t ncp_max, size_t max_prm_chunk, size_t max_chunk_bytes)
+void Engine::ensure_work(size_t ncp_max, size_t max_prm, size_t bytes)
 {
-   // as large as the largest chunk (at most half the budget, or one set
+   // as large as the largest launch set (at most half the budget, or one set
    // quartet that is larger); grows, never shrinks (plan_evict frees it)
-   const size_t want = std::max<size_t>(max_chunk_bytes, 1 << 20);
+   const size_t want = std::max<size_t>(bytes, 1 << 20);
    if (!d_work_ || want > work_bytes_) {
       synchronize();
       if (d_work_) HIPCHECK(hipFree(d_work_));
@@ -1140,7 +1144,7 @@ void Engine::ensure_work(size_t ncp_max, size_t max_prm_chunk, size_t max_chunk_
       HIPCHECK(hipMemset(d_fixcnt_, 0, 2 * sizeof(uint32_t)));
    }
    const size_t Ng = neighs_.size() / 3;
-   const size_t cap = (debug_ & 1) ? std::max<size_t>(4096, max_prm_chunk * Ng) : 4096;
+   const size_t cap = (debug_ & 1) ? std::max<size_t>(4096, max_prm * Ng) : 4096;
    if (cap > fix_cap_) {
       synchronize();
       if (d_fix_) HIPCHECK(hipFree(d_fix_));
@@ -1220,57 +1224,212 @@ bool Engine::use_eco(const TypeInfo &ti, const TypeDev &td, bool forced) const
    return (debug_ & 8) != 0;
 }
 
-void Engine::run_chunk(const TypeInfo &ti, const TypeDev &td, const Chunk &c, const RunBufs &w, const KTargets &kt)
+// The launch sequence of the uploaded work: chunks of all types, in the order
+// of the types, as many per launch set as fit the work buffer (na: the
+// static scratch), and the tables of its kernels, in one copy.
+void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
 {
-   const TypePlan &tp = ti.plan;
+   lp.sets.clear();
+   lp.ncp_max = lp.doubles = lp.n_prm = 0;
+   const size_t cap = (na ? NOALLOC_AC0_BYTES : budget_bytes_ / 2) / sizeof(double);
+   const int Ng = (int)neighs_.size() / 3;
+   std::vector<BatchDev> batches;
+   std::vector<char> lists;   // behind the BatchDevs
+   for (size_t d = 0; d < devs.size(); d++) {
+      const TypeDev &D = devs[d];
+      const auto &chunks = na ? D.chunks_na : D.chunks;
+      if (chunks.empty()) continue;
+      const TypeInfo &ti = types_[D.type];
+      const size_t eco_row = use_eco(ti, D, !na) ? ti.eco.row : 0;
+      lp.ncp_max = std::max(lp.ncp_max, (size_t)ti.plan.ncp);
+      for (size_t i = 0; i < chunks.size(); i++) {
+         const Chunk &c = chunks[i];
+         const size_t blocks = (size_t)(c.p1 - c.p0) * (size_t)ti.plan.ncp;
+         const size_t need = blocks + (size_t)(c.r1 - c.r0) * eco_row;
+         if (lp.sets.empty() || lp.sets.back().doubles + need > cap || lp.sets.back().chunks.size() == MAX_LAUNCH_CHUNKS) {
+            lp.sets.emplace_back();
+            lp.sets.back().b0 = (uint32_t)batches.size();
+         }
+         LaunchSet &ls = lp.sets.back();
+         BatchDev b{};   // every field zero / null unless set below
+         b.tp = ti.d_plan;
+         b.e1 = ti.d_e1;
+         b.e2 = ti.d_e2;
+         b.rows = D.rows;
+         b.groups = D.groups;
+         b.prm_row = D.prm_row;
+         b.prm_ip = D.prm_ip;
+         b.ksg = D.ksg;
+         b.kss = D.kss;
+         b.ksx = D.ksx;
+         b.ac_off = ls.doubles;
+         b.eco_off = ls.doubles + blocks;
+         b.eco_row = eco_row;
+         b.gmag = D.gmag;
+         b.gflag = D.gflag;
+         b.p0 = c.p0;
+         b.p1 = c.p1;
+         b.r0 = c.r0;
+         b.r1 = c.r1;
+         b.g0 = c.g0;
+         b.g1 = c.g1;
+         bool pair;
+         fm_layouts(ti.plan, Ng, b.fm, b.fix_fm, &pair);
+         ls.fix_lds = std::max(ls.fix_lds, (size_t)b.fix_fm.bytes);
+         batches.push_back(b);
+         ls.chunks.push_back({(int)d, (int)i});
+         ls.doubles += need;
+         ls.n_prm += c.p1 - c.p0;
+         lp.doubles = std::max(lp.doubles, ls.doubles);
+         lp.n_prm = std::max(lp.n_prm, ls.n_prm);
+      }
+   }
+   // the lists of each set: the kernels' units of its chunks, in falling
+   // order of the work of one unit (the last to start are short)
+   auto put = [&](ListRef &l, const auto &v) {
+      if (v.empty()) return;
+      lists.resize((lists.size() + 15) & ~(size_t)15);
+      l.off = lists.size();
+      l.n = (int)v.size();
+      l.units = v.back().end;
+      const char *p = (const char *)v.data();
+      lists.insert(lists.end(), p, p + sizeof(v[0]) * v.size());
+   };
+   for (LaunchSet &ls : lp.sets) {
+      std::vector<uint32_t> order(ls.chunks.size());
+      for (uint32_t i = 0; i < order.size(); i++) order[i] = i;
+      auto chunk = [&](uint32_t i) -> const Chunk & {
+         const TypeDev &D = devs[ls.chunks[i].first];
+         return (na ? D.chunks_na : D.chunks)[ls.chunks[i].second];
+      };
+      auto info = [&](uint32_t i) -> const TypeInfo & { return types_[devs[ls.chunks[i].first].type]; };
+      std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return info(a).plan.L > info(b).plan.L; });
+      // a set of little work in one launch, a larger one by the LDS that the
+      // types need, so that a large type does not cost the others occupancy
+      uint64_t prm = 0;
+      for (uint32_t i : order) prm += chunk(i).p1 - chunk(i).p0;
+      std::vector<WorkRef> fm[2][FM_BUCKETS];
+      for (uint32_t i : order) {
+         const TypeInfo &ti = info(i);
+         FmLayout main, fix;
+         bool pair;
+         fm_layouts(ti.plan, Ng, main, fix, &pair);
+         int k = FM_BUCKETS - 1;
+         if (prm > FM_ONE_LAUNCH) {
+            k = 0;
+            while ((size_t)main.bytes > FM_BUCKET_LDS[k]) k++;
+         }
+         auto &v = fm[pair ? 1 : 0][k];
+         const uint32_t n = chunk(i).p1 - chunk(i).p0;
+         const uint64_t end = (v.empty() ? 0ull : v.back().end) + (pair ? (n + 1) / 2 : n);
+         if (end > 0xffffffffull) fatal("launch set of more than 2^32 primitive quartets", (long long)end);
+         v.push_back(WorkRef{i, (uint32_t)end});
+         ListRef &l = ls.fm[pair ? 1 : 0][k];
+         l.lds = std::max(l.lds, (size_t)main.bytes);
+      }
+      for (int k = 0; k < 2; k++)
+         for (int x = 0; x < FM_BUCKETS; x++) put(ls.fm[k][x], fm[k][x]);
+      auto per_group = [&](uint32_t i) { return (double)(chunk(i).p1 - chunk(i).p0) / (double)(chunk(i).g1 - chunk(i).g0); };
+      std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return per_group(a) > per_group(b); });
+      for (int sp = 0; sp < 2; sp++) {
+         std::vector<SqRef> sq[SQ_KERNELS];
+         for (uint32_t i : order) {
+            const TypeDev &D = devs[ls.chunks[i].first];
+            const TypeInfo &ti = info(i);
+            if (!D.used) continue;
+            for (int f = 0; f < SQ_GROUPS; f++) {
+               const SqPlan &q = ti.sq[sp][batches[ls.b0 + i].eco_row ? 1 : 0][f];
+               if (q.items.empty()) continue;
+               SqRef r;
+               r.batch = i;
+               r.y = SqArgs{};
+               r.y.items = (const SqItem *)((const char *)q.dev + q.off[0]);
+               r.y.tiles = (const SqTile *)((const char *)q.dev + q.off[1]);
+               r.y.sps = (const SqSp *)((const char *)q.dev + q.off[2]);
+               r.y.rows = (const uint16_t *)((const char *)q.dev + q.off[3]);
+               r.y.rcs = (const uint32_t *)((const char *)q.dev + q.off[4]);
+               r.y.fns = (const uint32_t *)((const char *)q.dev + q.off[5]);
+               r.y.nitem = (int)q.items.size();
+               int ncon = 0;
+               for (int x = 0; x < 4; x++) {
+                  for (int s = 0; s < ti.plan.nsh[x]; s++) r.y.ncon[x] += ti.plan.nl[x][s];
+                  ncon += r.y.ncon[x];
+               }
+               r.y.o_co = q.lds_bytes / 8;
+               auto &v = sq[q.lm - 1];
+               ListRef &l = ls.sq[sp][q.lm - 1];
+               l.lds = std::max(l.lds, (size_t)q.lds_bytes + 8 * (size_t)(ncon * D.max_np));
+               const uint64_t end = (v.empty() ? 0ull : v.back().end) + (uint64_t)(chunk(i).g1 - chunk(i).g0) * q.items.size();
+               if (end > 0xffffffffull) fatal("launch set of more than 2^32 quartet items", (long long)end);
+               r.end = (uint32_t)end;
+               v.push_back(r);
+            }
+         }
+         for (int k = 0; k < SQ_KERNELS; k++) put(ls.sq[sp][k], sq[k]);
+      }
+   }
+   const size_t head = (sizeof(BatchDev) * batches.size() + 15) & ~(size_t)15;
+   const size_t total = head + lists.size();
+   for (LaunchSet &ls : lp.sets) {
+      for (auto &x : ls.fm)
+         for (ListRef &l : x) l.off += head;
+      for (auto &x : ls.sq)
+         for (ListRef &l : x) l.off += head;
+   }
+   if (total) {
+      std::vector<char> all(total, 0);
+      std::memcpy(all.data(), batches.data(), sizeof(BatchDev) * batches.size());
+      if (!lists.empty()) std::memcpy(all.data() + head, lists.data(), lists.size());
+      if (total > lp.cap) {
+         if (lp.dev) HIPCHECK(hipFree(lp.dev));
+         lp.cap = total + total / 2;
+         HIPCHECK(hipMalloc((void **)&lp.dev, lp.cap));
+      }
+      HIPCHECK(hipMemcpy(lp.dev, all.data(), total, hipMemcpyHostToDevice));
+   }
+   lp.key = launch_key(na);
+   lp.valid = true;
+}
+
+void Engine::run_set(std::vector<TypeDev> &devs, const LaunchPlan &lp, const LaunchSet &ls, const RunBufs &w,
+                     const KTargets &kt, bool na)
+{
    hipStream_t st = (hipStream_t)stream_;
    const DevTables t = dev_tables();
-   BatchDev b{};   // every field zero / null unless set below
-   b.tp = ti.d_plan;
-   b.e1 = ti.d_e1;
-   b.e2 = ti.d_e2;
-   b.rows = td.rows;
-   b.groups = td.groups;
-   b.prm_row = td.prm_row;
-   b.prm_ip = td.prm_ip;
-   b.ksg = td.ksg;
-   b.kss = td.kss;
-   b.ksx = td.ksx;
-   b.data = d_data_;
-   b.ac0 = w.ac0;
-   b.p0 = c.p0;
-   b.p1 = c.p1;
-   b.r0 = c.r0;
-   b.r1 = c.r1;
-   b.g0 = c.g0;
-   b.g1 = c.g1;
-   b.stats = w.stats;
-   b.fix = w.fix;
-   b.fix_count = w.fixcnt;
-   b.fix_cap = w.fix_cap;
-   b.force_fix = debug_ & 1;
-   b.fix_ws = w.fix_ws;
-   b.eco = w.ac0 + (size_t)(c.p1 - c.p0) * tp.ncp;
-   const bool eco = use_eco(ti, td, w.count);
-   b.eco_row = eco ? ti.eco.row : 0;
-   b.gmag = mixed_mode_ == 1 ? td.gmag : nullptr;
-   b.gflag = mixed_mode_ == 2 ? td.gflag : nullptr;
+   const BatchDev *batches = (const BatchDev *)lp.dev + ls.b0;
    auto evb = [&](int cat, void *q) { if (w.count) ev_begin(cat, q); };
    auto eve = [&](int cat, void *q) { if (w.count) ev_end(cat, q); };
 
-   if (launch_zero_u32(w.fixcnt, 1, st)) fatal("counter reset launch", 0);
-   evb(0, st);
-   ev_key_ = tp.L;
-   int rc = launch_fm_r(tp, t, b, st);
-   if (rc) fatal("fm_r launch", rc);
-   eve(0, st);
+   if (launch_zero_u32(w.run.fix_count, 1, st)) fatal("counter reset launch", 0);
+   int rc = 0;
+   for (int k = 0; k < 2; k++)
+      for (int x = FM_BUCKETS - 1; x >= 0; x--) {
+         const ListRef &l = ls.fm[k][x];
+         if (!l.n) continue;
+         evb(0, st);
+         rc = launch_fm_r(batches, (const WorkRef *)(lp.dev + l.off), l.n, l.units, k == 1, l.lds, t, w.run, st);
+         if (rc) fatal("fm_r launch", rc);
+         eve(0, st);
+      }
    evb(3, st);
-   rc = launch_fixup(tp, t, b, (debug_ & 1) ? w.fix_cap : std::min<uint32_t>(64u, w.fix_cap), st);
+   rc = launch_fixup(batches, ls.fix_lds, t, w.run, w.run.force_fix ? w.run.fix_cap : std::min<uint32_t>(64u, w.run.fix_cap),
+                     st);
    if (rc) fatal("fix-up launch", rc);
    eve(3, st);
-   if (mixed_mode_ == 2 && launch_mixed_flags(tp, b, td.gmag, d_mix_, mixed_tau_, td.gflag, d_mix_ + 1, st))
-      fatal("mixed-precision route launch", 0);
-   if (eco) {
+   for (size_t i = 0; i < ls.chunks.size(); i++) {
+      const TypeDev &D = devs[ls.chunks[i].first];
+      const TypeInfo &ti = types_[D.type];
+      const Chunk &c = (na ? D.chunks_na : D.chunks)[ls.chunks[i].second];
+      if (w.run.mixed == 2 &&
+          launch_mixed_flags(batches + i, w.run, c.g1 - c.g0, d_mix_, mixed_tau_, d_mix_ + 1, st))
+         fatal("mixed-precision route launch", 0);
+      if (w.count) {
+         timing_.flops[2] += c.k3_flops;
+         timing_.flops[4] += c.eco_flops;
+         n_prmc_ += (uint64_t)(c.p1 - c.p0) * ti.plan.nclass;
+         n_slots_ += (uint64_t)(c.p1 - c.p0) * (uint64_t)t.Ng * ti.plan.nclass;
+      }
+      if (!use_eco(ti, D, !na)) continue;
       EcoArgs e{};
       e.items = ti.d_eco_items;
       e.n_items = (int)ti.eco.items.size();
@@ -1279,73 +1438,70 @@ void Engine::run_chunk(const TypeInfo &ti, const TypeDev &td, const Chunk &c, co
       e.eco_off = ti.d_eco_info + MAXTC;
       e.row_doubles = ti.eco.row;
       evb(4, st);
-      ev_key_ = tp.L;
-      rc = launch_eco(tp, b, e, st);
+      ev_key_ = ti.plan.L;
+      rc = launch_eco(batches + i, w.run, c.r1 - c.r0, e, st);
       if (rc) fatal("matrix-core contraction launch", rc);
       eve(4, st);
    }
-   if (td.used) {
-      const SqPlan *sp = ti.sq[kt.nspin - 1][eco ? 1 : 0];
-      // debug bit 1: both launches on the main stream, one after the other
-      // (kernel durations without overlap, for profiling)
-      const bool both = !sp[0].items.empty() && !sp[1].items.empty() && (debug_ & 2) == 0;
-      if (both) {
-         ensure_side();
-         HIPCHECK(hipEventRecord((hipEvent_t)ev_join_[0], st));
-         HIPCHECK(hipStreamWaitEvent((hipStream_t)side_, (hipEvent_t)ev_join_[0], 0));
-      }
-      for (int i = 0; i < 2; i++) {
-         if (sp[i].items.empty()) continue;
-         void *q = both && i == 1 ? side_ : (void *)st;
-         evb(2, q);
-         ev_key_ = tp.L;
-         rc = launch_sq(tp, td.max_np, b, t, kt, sp[i], q);
-         if (rc) fatal("sq launch", rc);
-         eve(2, q);
-      }
-      if (both) {
-         HIPCHECK(hipEventRecord((hipEvent_t)ev_join_[1], (hipStream_t)side_));
-         HIPCHECK(hipStreamWaitEvent(st, (hipEvent_t)ev_join_[1], 0));
-      }
+   // debug bit 1: every launch on the main stream, one after the other
+   // (kernel durations without overlap, for profiling)
+   const ListRef *sq = ls.sq[kt.nspin - 1];
+   int nk = 0;
+   for (int k = 0; k < SQ_KERNELS; k++) nk += sq[k].n ? 1 : 0;
+   const bool side = nk > 1 && (debug_ & 2) == 0;
+   if (side) {
+      ensure_side();
+      HIPCHECK(hipEventRecord((hipEvent_t)ev_join_[0], st));
+      HIPCHECK(hipStreamWaitEvent((hipStream_t)side_, (hipEvent_t)ev_join_[0], 0));
    }
-   if (!w.count) return;
-   timing_.flops[2] += c.k3_flops;
-   timing_.flops[4] += c.eco_flops;
-   n_prmc_ += (uint64_t)(c.p1 - c.p0) * tp.nclass;
-   n_slots_ += (uint64_t)(c.p1 - c.p0) * (uint64_t)t.Ng * tp.nclass;
+   for (int k = SQ_KERNELS - 1; k >= 0; k--) {
+      if (!sq[k].n) continue;
+      void *q = side && k != 1 ? side_ : (void *)st;
+      evb(2, q);
+      ev_key_ = k + 1;
+      rc = launch_sq(batches, (const SqRef *)(lp.dev + sq[k].off), sq[k].n, sq[k].units, k + 1, sq[k].lds, t, w.run, kt, q);
+      if (rc) fatal("sq launch", rc);
+      eve(2, q);
+   }
+   if (side) {
+      HIPCHECK(hipEventRecord((hipEvent_t)ev_join_[1], (hipStream_t)side_));
+      HIPCHECK(hipStreamWaitEvent(st, (hipEvent_t)ev_join_[1], 0));
+   }
 }
 
 // Device buffers and targets of an execution (allocating or growing what
 // the work needs; nothing of this is captured in a graph); false when there
 // is no work.
-bool Engine::prepare_exec(std::vector<TypeDev> &devs, uint64_t max_index, RunBufs &w, KTargets &kt, uint64_t n)
+bool Engine::prepare_exec(std::vector<TypeDev> &devs, LaunchPlan &lp, uint64_t max_index, RunBufs &w, KTargets &kt,
+                          uint64_t n)
 {
    if (max_index >= n) fatal("add_qrtt offsets reach beyond the P / K size of set_P", (long long)max_index);
    ensure_tables();
    upload_data();
-   size_t ncp_max = 0, max_prm = 0, max_gb = 0;
    for (auto &D : devs) {
       if (D.chunks.empty()) continue;
       const TypeInfo &ti = types_[D.type];
       if (truncated_ && ti.plan.L > nder_)
          fatal("the truncated-Coulomb table has fewer derivative orders than this quartet's total angular momentum",
                ti.plan.L);
-      ncp_max = std::max(ncp_max, (size_t)ti.plan.ncp);
-      const size_t eco_row = use_eco(ti, D, true) ? ti.eco.row : 0;
-      for (auto &c : D.chunks) {
-         max_prm = std::max(max_prm, (size_t)(c.p1 - c.p0));
-         max_gb = std::max(max_gb, sizeof(double) * ((size_t)(c.p1 - c.p0) * (size_t)ti.plan.ncp +
-                                                     (size_t)(c.r1 - c.r0) * eco_row));
-      }
    }
-   if (ncp_max == 0) return false;
-   ensure_work(ncp_max, max_prm, max_gb);
-   w.ac0 = d_work_;
-   w.fix = d_fix_;
-   w.fixcnt = d_fixcnt_;
-   w.fix_ws = d_fix_ws_;
-   w.fix_cap = (uint32_t)fix_cap_;
-   w.stats = stats_on_ ? d_stats_ : nullptr;
+   if (!lp.valid || lp.key != launch_key(false)) {
+      HIPCHECK(hipStreamSynchronize((hipStream_t)stream_));   // the tables are no longer read
+      drop_graph();
+      build_launches(devs, false, lp);
+   }
+   if (lp.ncp_max == 0) return false;
+   ensure_work(lp.ncp_max, lp.n_prm, sizeof(double) * lp.doubles);
+   w.run.work = d_work_;
+   w.run.data = d_data_;
+   w.run.fix = d_fix_;
+   w.run.fix_count = d_fixcnt_;
+   w.run.fix_ws = d_fix_ws_;
+   w.run.fix_cap = (uint32_t)fix_cap_;
+   w.run.fix_stride = (uint32_t)lp.ncp_max + 16;
+   w.run.stats = stats_on_ ? d_stats_ : nullptr;
+   w.run.force_fix = debug_ & 1;
+   w.run.mixed = 0;
    w.count = true;
    kt.nspin = nspin_;
    kt.hf_fac = hf_fac_;
@@ -1357,32 +1513,30 @@ bool Engine::prepare_exec(std::vector<TypeDev> &devs, uint64_t max_index, RunBuf
    return true;
 }
 
-void Engine::launch_all(std::vector<TypeDev> &devs, const RunBufs &w, const KTargets &kt)
+void Engine::launch_all(std::vector<TypeDev> &devs, const LaunchPlan &lp, const RunBufs &w, const KTargets &kt)
 {
-   if (mixed_mode_ == 1) {
+   if (w.run.mixed == 1) {
       // calibration: every set quartet's magnitude from 0
       for (auto &D : devs)
          if (D.gmag && launch_zero_u32((uint32_t *)D.gmag, (int)(2 * D.n_groups), stream_))
             fatal("calibration reset launch", 0);
-   } else if (mixed_mode_ == 2) {
+   } else if (w.run.mixed == 2) {
       // max |P| of this density (both spins), and the routed count from 0
       if (launch_zero_u32((uint32_t *)(d_mix_ + 1), 2, stream_)) fatal("route counter reset", 0);
       for (int sp = 0; sp < kt.nspin; sp++)
          if (launch_absmax(kt.P[sp], FP_size_, d_mix_, sp == 0, stream_)) fatal("max |P| launch", 0);
    }
-   // debug bit 2: wait for each quartet type and report it on stderr
+   // debug bit 2: wait for each launch set and report it on stderr
    const bool progress = (debug_ & 4) != 0;
    const auto t0 = std::chrono::steady_clock::now();
-   size_t nty = 0, done = 0;
-   for (auto &D : devs) nty += D.chunks.empty() ? 0 : 1;
-   for (auto &D : devs) {
-      if (D.chunks.empty()) continue;
-      for (auto &c : D.chunks) run_chunk(types_[D.type], D, c, w, kt);
+   size_t done = 0;
+   for (const LaunchSet &ls : lp.sets) {
+      run_set(devs, lp, ls, w, kt, false);
       if (!progress) continue;
       synchronize();
       const double sec = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-      std::fprintf(stderr, "libgint: quartet type %zu of %zu done (L %d, %zu set quartets, %zu chunks) at %.1f s\n",
-                   ++done, nty, types_[D.type].plan.L, D.n_groups, D.chunks.size(), sec);
+      std::fprintf(stderr, "libgint: launch set %zu of %zu done (%zu chunks, %zu primitive quartets) at %.1f s\n", ++done,
+                   lp.sets.size(), ls.chunks.size(), ls.n_prm, sec);
       std::fflush(stderr);
    }
 }
@@ -1391,8 +1545,8 @@ void Engine::execute(std::vector<TypeDev> &devs, uint64_t max_index)
 {
    RunBufs w{};
    KTargets kt{};
-   if (!prepare_exec(devs, max_index, w, kt, FP_size_)) return;
-   launch_all(devs, w, kt);
+   if (!prepare_exec(devs, stream_lp_, max_index, w, kt, FP_size_)) return;
+   launch_all(devs, stream_lp_, w, kt);
 }
 
 // ---------------------------------------------------------------------------
@@ -1411,12 +1565,12 @@ void Engine::drop_graph()
 
 void Engine::replay_graph(const RunBufs &w, const KTargets &kt)
 {
-   const uint64_t key[] = {(uint64_t)w.ac0, (uint64_t)w.fix, (uint64_t)w.fix_ws, (uint64_t)w.fixcnt,
-                           (uint64_t)w.fix_cap,
+   const uint64_t key[] = {(uint64_t)w.run.work, (uint64_t)w.run.fix, (uint64_t)w.run.fix_ws, (uint64_t)w.run.fix_count,
+                           (uint64_t)w.run.fix_cap, (uint64_t)w.run.fix_stride, (uint64_t)plan_lp_.dev,
                            (uint64_t)kt.P[0], (uint64_t)kt.P[1], (uint64_t)kt.K[0], (uint64_t)kt.K[1],
                            (uint64_t)kt.nspin, graph_bits(kt.hf_fac), (uint64_t)kt.out, (uint64_t)d_data_,
                            (uint64_t)d_C0_, (uint64_t)d_neighs_, (uint64_t)neighs_.size(), graph_bits(R_cut_),
-                           (uint64_t)truncated_, (uint64_t)debug_, (uint64_t)ld_C0_, (uint64_t)mixed_mode_,
+                           (uint64_t)truncated_, (uint64_t)debug_, (uint64_t)ld_C0_, (uint64_t)w.run.mixed,
                            graph_bits(mixed_tau_), (uint64_t)d_mix_};
    constexpr size_t NK = sizeof key / sizeof key[0];
    static_assert(NK <= sizeof graph_key_ / sizeof graph_key_[0], "graph key");
@@ -1428,7 +1582,7 @@ void Engine::replay_graph(const RunBufs &w, const KTargets &kt)
       const double f1 = timing_.flops[1], f2 = timing_.flops[2], f4 = timing_.flops[4];
       hipGraph_t g = nullptr;
       HIPCHECK(hipStreamBeginCapture((hipStream_t)stream_, hipStreamCaptureModeThreadLocal));
-      launch_all(plan_dev_, w, kt);
+      launch_all(plan_dev_, plan_lp_, w, kt);
       HIPCHECK(hipStreamEndCapture((hipStream_t)stream_, &g));
       hipGraphExec_t ex = nullptr;
       HIPCHECK(hipGraphInstantiate(&ex, g, nullptr, nullptr, 0));
@@ -1490,13 +1644,17 @@ int Engine::plan_execute_noalloc(const double *Pa, const double *Pb, double *Ka,
    if (ncp_max > (size_t)MAX_NCP) return err(-4, "block size beyond the fix-up workspace", (long long)ncp_max);
    char *base = (char *)noalloc_scratch_;
    if (!base) return err(-8, "the no-allocation scratch array has no device address", 0);
+   if (!plan_na_lp_.valid || plan_na_lp_.key != launch_key(true))
+      return err(-6, "lattice vectors changed since libgint_amd_plan_end: record the plan again", 0);
    RunBufs w{};
-   w.ac0 = (double *)(base + NOALLOC_OFF_AC0);
-   w.fix = (uint32_t *)(base + NOALLOC_OFF_FIX);
-   w.fixcnt = (uint32_t *)base;
-   w.fix_ws = (double *)(base + NOALLOC_OFF_FIXWS);
-   w.fix_cap = (uint32_t)NOALLOC_FIX;
-   w.stats = nullptr;
+   w.run.work = (double *)(base + NOALLOC_OFF_AC0);
+   w.run.data = d_data_;
+   w.run.fix = (uint32_t *)(base + NOALLOC_OFF_FIX);
+   w.run.fix_count = (uint32_t *)base;
+   w.run.fix_ws = (double *)(base + NOALLOC_OFF_FIXWS);
+   w.run.fix_cap = (uint32_t)NOALLOC_FIX;
+   w.run.fix_stride = MAX_NCP + 16;
+   w.run.force_fix = debug_ & 1;
    w.count = false;
    KTargets kt{};
    kt.nspin = Pb ? 2 : 1;
@@ -1507,12 +1665,8 @@ int Engine::plan_execute_noalloc(const double *Pa, const double *Pb, double *Ka,
    kt.K[0] = Ka;
    kt.K[1] = Kb;
    // the overflow word (it is only read back by the allocating path)
-   if (launch_zero_u32(w.fixcnt, 2, stream_)) fatal("counter reset launch", 0);
-   for (auto &D : plan_dev_) {
-      if (D.chunks.empty()) continue;
-      const TypeInfo &ti = types_[D.type];
-      for (auto &c : D.chunks_na) run_chunk(ti, D, c, w, kt);
-   }
+   if (launch_zero_u32(w.run.fix_count, 2, stream_)) fatal("counter reset launch", 0);
+   for (const LaunchSet &ls : plan_na_lp_.sets) run_set(plan_dev_, plan_na_lp_, ls, w, kt, true);
    return 0;
 }
 
@@ -1549,6 +1703,7 @@ uint64_t Engine::device_bytes() const
    for (const auto &d : plan_dev_)
       b += d.cap[0] * sizeof(RowRec) + d.cap[1] * sizeof(GroupRec) + d.cap[2] * 4 + d.cap[3] * 4 +
            d.cap[4] * sizeof(KsGroup) + d.cap[5] * sizeof(KsRec) + d.cap[6] * sizeof(KsSet);
+   b += plan_lp_.cap + plan_na_lp_.cap;
    b += work_bytes_ + fix_cap_ * 8 + fix_ws_cap_ * 8 + d_data_cap_ * 8 + C0_.size() * 8 +
         d_neighs_cap_ * 8;
    return b;
@@ -1556,15 +1711,21 @@ uint64_t Engine::device_bytes() const
 
 uint64_t Engine::work_estimate() const
 {
-   size_t ncp_max = 0, mcb = 0;
+   // the launch sets of the resident plan: all of its blocks or half the budget
+   size_t ncp_max = 0, all = 0, largest = 0;
    for (const auto &D : plan_dev_) {
       if (D.chunks.empty()) continue;
       const TypeInfo &ti = types_[D.type];
       ncp_max = std::max(ncp_max, (size_t)ti.plan.ncp);
-      mcb = std::max(mcb, D.max_chunk_bytes);
+      for (const Chunk &c : D.chunks) {
+         const size_t b = sizeof(double) * ((size_t)(c.p1 - c.p0) * (size_t)ti.plan.ncp +
+                                            (size_t)(c.r1 - c.r0) * (D.eco ? ti.eco.row : 0));
+         all += b;
+         largest = std::max(largest, b);
+      }
    }
    if (!ncp_max) return 0;
-   return std::max<size_t>(mcb, 1 << 20) + 2 * 4 * 4096 + 4096 * (ncp_max + 16) * 8;
+   return std::max({std::min(all, budget_bytes_ / 2), largest, (size_t)1 << 20}) + 2 * 4 * 4096 + 4096 * (ncp_max + 16) * 8;
 }
 
 uint64_t Engine::plan_host_bytes() const
@@ -1605,6 +1766,8 @@ void Engine::plan_evict()
    }
    plan_dev_.clear();
    mixed_calibrated_ = false;
+   plan_lp_.release();
+   plan_na_lp_.release();
    void *bufs[] = {d_work_, d_fix_, d_fix_ws_};
    for (void *b : bufs)
       if (b) HIPCHECK(hipFree(b));
@@ -1619,6 +1782,8 @@ void Engine::plan_restore()
 {
    if (!evicted_) return;
    upload(plan_host_, plan_dev_, true);
+   plan_lp_.valid = false;
+   build_launches(plan_dev_, true, plan_na_lp_);
    plan_host_.clear();
    evicted_ = false;
 }
@@ -1629,7 +1794,7 @@ void Engine::plan_execute_into(const double *P0, const double *P1, double *K0, d
    if (evicted_) fatal("plan_execute_into with the plan off the device", 0);
    RunBufs w{};
    KTargets kt{};
-   if (!prepare_exec(plan_dev_, plan_max_index_, w, kt, n)) return;
+   if (!prepare_exec(plan_dev_, plan_lp_, plan_max_index_, w, kt, n)) return;
    kt.nspin = nspin;
    kt.P[0] = P0;
    kt.P[1] = P1;
@@ -1638,7 +1803,7 @@ void Engine::plan_execute_into(const double *P0, const double *P1, double *K0, d
    if (graph_on_ && nomp_ == 1 && !timing_on_ && !stats_on_ && (debug_ & 6) == 0)
       replay_graph(w, kt);
    else
-      launch_all(plan_dev_, w, kt);
+      launch_all(plan_dev_, plan_lp_, w, kt);
 }
 
 // ---------------------------------------------------------------------------

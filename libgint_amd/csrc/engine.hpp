@@ -76,7 +76,6 @@ struct TypeDev {
    size_t cap[7] = {0, 0, 0, 0, 0, 0, 0};   // allocated elements of each array
    size_t n_rows = 0, n_groups = 0, n_prm = 0, n_ksx = 0, n_ksg = 0, n_kss = 0;
    size_t max_group_bytes = 0;            // largest set quartet's primitive blocks
-   size_t max_chunk_bytes = 0;            // largest chunk's blocks and contraction buffer rows
    std::vector<Chunk> chunks;
    std::vector<Chunk> chunks_na;          // the same work in chunks that fit the no-allocation scratch
    bool na_fit = true;                    // every set quartet fits it
@@ -95,9 +94,8 @@ struct TypeInfo {
    std::vector<uint32_t> e1, e2;          // Hermite -> cartesian item descriptors
    uint32_t *d_e1 = nullptr, *d_e2 = nullptr;
    std::vector<ClassPlan> cplans;
-   // from the blocks to K: a launch for the classes without and one for those
-   // with f shells; [nspin - 1][0 own contraction, 1 matrix cores]
-   SqPlan sq[2][2][2];
+   // from the blocks to K: [nspin - 1][0 own contraction, 1 k_eco][register group]
+   SqPlan sq[2][2][SQ_GROUPS];
    // matrix-core contraction (k_eco), for types with many primitive
    // quartets per row
    EcoPlan eco;
@@ -106,13 +104,46 @@ struct TypeInfo {
    int *d_eco_info = nullptr;
 };
 
-// device buffers of one chunk's kernels
+// k_fm_r launches of a set by the LDS of the types (bytes, at most): a launch
+// takes the LDS of its largest type, and wavefronts per CU follow from it.
+// Measured with all types in one launch / in four: (pp|pp) to (ff|ff) in 256
+// cells 27.9 / 15.2 ms, s to f in 125 cells 28.6 / 15.2 ms.  A set of few
+// primitive quartets does not fill the chip and pays for the launches
+// instead: 5783 in 27 cells 0.69 ms in one launch, 0.9 in four.
+constexpr uint64_t FM_ONE_LAUNCH = 16384;   // a set of at most this many primitive quartets: one launch
+constexpr int FM_BUCKETS = 4;
+constexpr size_t FM_BUCKET_LDS[FM_BUCKETS] = {10 * 1024 + 512, 13 * 1024 + 512, 32 * 1024, 64 * 1024};
+
+// One launch of a launch set: its list of chunks among the set's tables
+struct ListRef {
+   size_t off = 0;       // bytes from the start of the tables
+   int n = 0;
+   uint32_t units = 0;   // units of work of all of them
+   size_t lds = 0;       // the most LDS one needs
+};
+// Chunks of any types that share the work buffer and are launched together
+struct LaunchSet {
+   std::vector<std::pair<int, int>> chunks;   // (index among the types' devs, chunk)
+   uint32_t b0 = 0;                           // first BatchDev of the set in the tables
+   size_t doubles = 0;                        // of the work buffer
+   size_t n_prm = 0;
+   ListRef fm[2][FM_BUCKETS];                 // k_fm_r: single, pairs; by LDS
+   ListRef sq[2][SQ_KERNELS];                 // k_sq: [nspin - 1][kernel - 1]
+   size_t fix_lds = 0;
+};
+// The launch sequence of an execution and its tables on the device
+struct LaunchPlan {
+   std::vector<LaunchSet> sets;
+   char *dev = nullptr;
+   size_t cap = 0, ncp_max = 0, doubles = 0, n_prm = 0;
+   bool valid = false;
+   uint64_t key = 0;   // cells and debug bits it was built for
+   void release();
+};
+
+// device buffers of an execution's kernels
 struct RunBufs {
-   double *ac0;
-   uint32_t *fix, *fixcnt;
-   double *fix_ws;
-   uint32_t fix_cap;
-   unsigned long long *stats;
+   RunDev run;
    bool count;   // host counters and timing events
 };
 
@@ -217,8 +248,11 @@ class Engine {
    bool set_level(const KsGroup *g, const TypePlan &tp, KsSet &s) const;
    void upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool release_host);
    void execute(std::vector<TypeDev> &devs, uint64_t max_index);
-   bool prepare_exec(std::vector<TypeDev> &devs, uint64_t max_index, RunBufs &w, KTargets &kt, uint64_t n);
-   void launch_all(std::vector<TypeDev> &devs, const RunBufs &w, const KTargets &kt);
+   bool prepare_exec(std::vector<TypeDev> &devs, LaunchPlan &lp, uint64_t max_index, RunBufs &w, KTargets &kt, uint64_t n);
+   void build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp);
+   void launch_all(std::vector<TypeDev> &devs, const LaunchPlan &lp, const RunBufs &w, const KTargets &kt);
+   void run_set(std::vector<TypeDev> &devs, const LaunchPlan &lp, const LaunchSet &ls, const RunBufs &w, const KTargets &kt,
+                bool na);
    void replay_graph(const RunBufs &w, const KTargets &kt);
    void drop_graph();
    static uint64_t graph_bits(double x)
@@ -228,9 +262,9 @@ class Engine {
       return u;
    }
    bool use_eco(const TypeInfo &ti, const TypeDev &td, bool forced) const;
-   void run_chunk(const TypeInfo &ti, const TypeDev &td, const Chunk &c, const RunBufs &w, const KTargets &kt);
    DevTables dev_tables() const;
-   void ensure_work(size_t ncp_max, size_t max_prm_chunk, size_t max_group_bytes);
+   void ensure_work(size_t ncp_max, size_t max_prm, size_t bytes);
+   uint64_t launch_key(bool na) const { return (uint64_t)neighs_.size() | (uint64_t)(na ? 0 : debug_ & 24) << 32; }
    void ensure_tables();
    void upload_data();
    void harvest_events();
@@ -239,9 +273,9 @@ class Engine {
    void ensure_side();
    int my_thr_ = 0, nomp_ = 1;
    void *stream_ = nullptr;
-   // the kernels that take a chunk's blocks to K only add into it: the
-   // classes with f shells run on a side stream, and stream_ waits for it
-   // before the blocks are overwritten
+   // the kernels that take the blocks to K only add into it: those of the
+   // types without d shells and of the classes with f shells run on a side
+   // stream, and stream_ waits for it before the blocks are overwritten
    void *side_ = nullptr;
    void *ev_join_[2] = {};   // blocks ready, side stream done
 
@@ -288,6 +322,7 @@ class Engine {
 
    // device
    std::vector<TypeDev> stream_dev_, plan_dev_;
+   LaunchPlan stream_lp_, plan_lp_, plan_na_lp_;   // the plan's with allocated and with the static scratch
    double *d_data_ = nullptr;
    size_t d_data_cap_ = 0;
    double *d_C0_ = nullptr;
@@ -319,7 +354,6 @@ class Engine {
    // max |P| is below tau take the single-precision contraction
    double mixed_tau_ = 0.0;
    bool mixed_calibrated_ = false;
-   int mixed_mode_ = 0;                    // of the execution being launched: 0 off, 1 calibrate, 2 route
    unsigned long long *d_mix_ = nullptr;   // [0] max |P| bits, [1] set quartets routed to single precision
    void ensure_mixed();
 

@@ -26,6 +26,7 @@
 
 #include "device.hpp"
 #include "gint_math.h"
+#include "uniform.hpp"
 
 namespace gint {
 
@@ -261,15 +262,6 @@ __device__ __forceinline__ double d_cheb_sum(const double *__restrict__ c, const
 // quartet.  FIX: one wavefront per listed (primitive, cell) slot, no
 // screening, blocks and per-L Fm[0] into the fix-up workspace.
 // ---------------------------------------------------------------------------
-struct FmLayout {
-   int SB;      // survivors per Hermite batch
-   int o_fmv;   // per lane: G_m, then D_m = (-2 rho)^m G_m
-   int o_sv;    // per lane: X Y Z of P-Q-g, TG1 (or T), TG2
-   int o_R;     // Hermite layers, 2 x SB x nh
-   int o_int;   // byte offset of 64 lane infos (branch | patch << 2) and 64 survivor lanes
-   int bytes;
-};
-
 constexpr int GEO = 24;   // doubles of the primitive geometry at the start of LDS
 enum { G_P = 0, G_Q = 3, G_PA = 6, G_QC = 9, G_KFAC = 12, G_RHO = 13, G_RR = 14, G_I2AB = 15, G_I2CD = 16 };
 
@@ -302,17 +294,30 @@ static FmLayout fm_layout(const TypePlan &tp, bool fix, bool pair = false)
 // quartets per wavefront.  Lanes 0-31 take the cells of the first, lanes
 // 32-63 those of the second; their survivors share the G_m and Hermite
 // batches and each quartet keeps its own cell sum and transform.
+//
+// One launch takes the chunks of a list, one after the other in the
+// numbering of its units (primitive quartets or pairs of them): a launch per
+// type left the chip to the slowest wavefronts of each, and small systems to
+// launch after launch of a few workgroups.
 template <bool FIX, bool PAIR>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_fm_r(const TypePlan *__restrict__ tpp, DevTables t, BatchDev b, FmLayout lay)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
+void k_fm_r(const BatchDev *__restrict__ batches, const WorkRef *__restrict__ refs, int nref, DevTables t, RunDev run)
 {
    static_assert(!(FIX && PAIR), "the fix-up takes one slot per wavefront");
    constexpr int NPR = PAIR ? 2 : 1;      // primitive quartets per wavefront
    constexpr int NACC = PAIR ? 4 : 8;     // Hermite functions per lane and quartet, / 64
    extern __shared__ double lds[];
-   const TypePlan &tp = *tpp;
    const int lane = threadIdx.x;
    const int half = PAIR ? lane >> 5 : 0;   // the lane's quartet
-   const int L = tp.L, nh = tp.nh, Lp1 = L + 1;
+   uint32_t ubase = 0;
+   const uint32_t nfix = FIX ? min(run.fix_count[0], run.fix_cap) : 0;
+   // (the fix-up: one entry per turn, each with its own chunk)
+   for (uint32_t turn = FIX ? blockIdx.x : 0; turn < (FIX ? nfix : (uint32_t)nref); turn += FIX ? gridDim.x : 1) {
+   const BatchDev b = load_batch(batches, FIX ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(run.fix[2 * turn + 1] >> 24))
+                                              : load_uniform(&refs[turn].batch), run);
+   const TypePlan &tp = *b.tp;
+   const FmLayout lay = FIX ? b.fix_fm : b.fm;
+   const int L = load_uniform(&tp.L), nh = load_uniform(&tp.nh), Lp1 = L + 1;
    const int SB = lay.SB;
    double *G = lds + GEO * half;      // geometry of the lane's quartet
    double *fmv = lds + lay.o_fmv;     // [64][L+1]
@@ -320,10 +325,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
    double *Rb = lds + lay.o_R;        // [2][SB][nh]
    int *svi = (int *)((char *)lds + lay.o_int);
    int *svl = svi + 64;
-   const uint32_t nwork = FIX ? min(b.fix_count[0], b.fix_cap) : (b.p1 - b.p0);
+   const uint32_t nwork = FIX ? turn + 1 : b.p1 - b.p0;
    const uint32_t *__restrict__ e1 = b.e1, *__restrict__ e2 = b.e2;
+   // the first unit of the chunk that is this workgroup's
+   const uint32_t skip = ubase % gridDim.x;
+   const uint32_t u0 = FIX ? turn : (blockIdx.x >= skip ? blockIdx.x - skip : blockIdx.x + gridDim.x - skip);
+   if (!FIX) ubase = load_uniform(&refs[turn].end);
 
-   for (uint32_t w0 = blockIdx.x * NPR; w0 < nwork; w0 += gridDim.x * NPR) {
+   for (uint32_t w0 = u0 * NPR; w0 < nwork; w0 += gridDim.x * NPR) {
       const uint32_t w = w0 + half;
       const bool hvalid = w < nwork;                    // the lane's quartet exists
       const int nprim = (int)min((uint32_t)NPR, nwork - w0);
@@ -423,7 +432,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
             }
             if (FIX) {
                // per-L Fm[0] of the slot, for the classes that screen it
-               double *f0 = b.fix_ws + (size_t)w * (tp.ncp + 16) + tp.ncp;
+               double *f0 = b.fix_ws + (size_t)w * b.fix_stride + tp.ncp;
                for (int i = 0; i < tp.nL; i++) {
                   double v = Fm0;
                   if (lsens) {
@@ -460,7 +469,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
                      const uint32_t idx = atomicAdd(&b.fix_count[0], 1u);
                      if (idx < b.fix_cap) {
                         b.fix[2 * idx] = p;
-                        b.fix[2 * idx + 1] = (uint32_t)n3 | (mask << 8);
+                        b.fix[2 * idx + 1] = (uint32_t)n3 | (mask << 8) | (b.id << 24);
                      } else {
                         // list full: every class keeps the slot (its G_0 is
                         // within rounding of the 1e-12 threshold)
@@ -588,7 +597,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
       for (int q = 0; q < NPR; q++) {
          if (q >= nprim) break;
          const double *Gq = lds + GEO * q;
-         double *dst = FIX ? b.fix_ws + (size_t)w * (tp.ncp + 16) : b.ac0 + (size_t)(w0 + q) * tp.ncp;
+         double *dst = FIX ? b.fix_ws + (size_t)w * b.fix_stride : b.ac0 + (size_t)(w0 + q) * tp.ncp;
          // calibration of the mixed-precision routing: the largest block
          // element of each set quartet (a positive double orders as its bits)
          unsigned long long *gm = nullptr;
@@ -701,6 +710,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
          }
       }
    }
+   __syncthreads();   // the next chunk's layout of LDS
+   }
 }
 
 // ---------------------------------------------------------------------------
@@ -714,32 +725,36 @@ size_t fm_r_lds_bytes(const TypePlan &tp)
    return (size_t)y.bytes <= LDS_LIMIT ? (size_t)y.bytes : 0;
 }
 
-int launch_fm_r(const TypePlan &tp, const DevTables &t, const BatchDev &b, void *stream)
+void fm_layouts(const TypePlan &tp, int Ng, FmLayout &main, FmLayout &fix, bool *pair)
 {
-   if (b.p1 <= b.p0) return 0;
-   const uint32_t n = b.p1 - b.p0;
    // two primitive quartets per wavefront when each takes at most half of
    // the lanes' cells and its cell sum fits 4 values per lane
    const FmLayout yp = fm_layout(tp, false, true);
-   if (t.Ng <= 32 && tp.nh <= 256 && (size_t)yp.bytes <= LDS_LIMIT) {
-      // workgroups stay resident and stride over the pairs
-      const unsigned grid = std::min((n + 1) / 2, 16384u);
-      hipLaunchKernelGGL((k_fm_r<false, true>), dim3(grid), dim3(64), yp.bytes, (hipStream_t)stream, b.tp, t, b, yp);
-      return hipGetLastError() == hipSuccess ? 0 : -1;
-   }
-   const FmLayout y = fm_layout(tp, false);
-   if ((size_t)y.bytes > LDS_LIMIT) return -3;
-   const unsigned grid = std::min(n, 16384u);
-   hipLaunchKernelGGL((k_fm_r<false, false>), dim3(grid), dim3(64), y.bytes, (hipStream_t)stream, b.tp, t, b, y);
+   *pair = Ng <= 32 && tp.nh <= 256 && (size_t)yp.bytes <= LDS_LIMIT;
+   main = *pair ? yp : fm_layout(tp, false);
+   fix = fm_layout(tp, true);
+}
+
+int launch_fm_r(const BatchDev *batches, const WorkRef *refs, int nref, uint32_t units, bool pair, size_t lds,
+                const DevTables &t, const RunDev &run, void *stream)
+{
+   if (!units) return 0;
+   if (lds > LDS_LIMIT) return -3;
+   // workgroups stay resident and stride over the units
+   const unsigned grid = std::min(units, 16384u);
+   if (pair)
+      hipLaunchKernelGGL((k_fm_r<false, true>), dim3(grid), dim3(64), lds, (hipStream_t)stream, batches, refs, nref, t, run);
+   else
+      hipLaunchKernelGGL((k_fm_r<false, false>), dim3(grid), dim3(64), lds, (hipStream_t)stream, batches, refs, nref, t, run);
    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int launch_fixup(const TypePlan &tp, const DevTables &t, const BatchDev &b, uint32_t n_fix, void *stream)
+int launch_fixup(const BatchDev *batches, size_t lds, const DevTables &t, const RunDev &run, uint32_t n_fix, void *stream)
 {
-   const FmLayout y = fm_layout(tp, true);
-   if ((size_t)y.bytes > LDS_LIMIT) return -3;
+   if (lds > LDS_LIMIT) return -3;
    const unsigned grid = std::max(1u, std::min(n_fix, 4096u));
-   hipLaunchKernelGGL((k_fm_r<true, false>), dim3(grid), dim3(64), y.bytes, (hipStream_t)stream, b.tp, t, b, y);
+   hipLaunchKernelGGL((k_fm_r<true, false>), dim3(grid), dim3(64), lds, (hipStream_t)stream, batches,
+                      (const WorkRef *)nullptr, 0, t, run);
    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -787,11 +802,12 @@ __global__ void k_absmax(const double *__restrict__ P, size_t n, unsigned long l
 // The mixed-precision route of each set quartet of a chunk: single
 // precision when its bound  max|block element| x max|coefficient|^4 x
 // primitive quartets  times max|P| is below tau.  count[0] += flagged.
-__global__ void k_mixed_flags(const TypePlan *__restrict__ tpp, BatchDev b, const double *__restrict__ gmag,
-                              const unsigned long long *__restrict__ pmax, double tau, uint32_t *gflag,
-                              unsigned long long *count)
+__global__ void k_mixed_flags(const BatchDev *__restrict__ batch, RunDev run, const unsigned long long *__restrict__ pmax,
+                              double tau, unsigned long long *count)
 {
-   const TypePlan &tp = *tpp;
+   const double *gmag = load_uniform(&batch->gmag);
+   const BatchDev b = load_batch(batch, 0, run);
+   const TypePlan &tp = *b.tp;
    const double maxP = __longlong_as_double((long long)*pmax);
    for (uint32_t gi = b.g0 + blockIdx.x * blockDim.x + threadIdx.x; gi < b.g1; gi += gridDim.x * blockDim.x) {
       const GroupRec &g = b.groups[gi];
@@ -806,7 +822,7 @@ __global__ void k_mixed_flags(const TypePlan *__restrict__ tpp, BatchDev b, cons
       double npr = 0.0;
       for (uint32_t r = g.row0; r < g.row1; r++) npr += (double)b.rows[r].n_prm;
       const bool f32 = gmag[gi] * c4 * npr * maxP < tau;
-      gflag[gi] = f32 ? 1u : 0u;
+      b.gflag[gi] = f32 ? 1u : 0u;
       if (f32) atomicAdd(count, 1ull);
    }
 }
@@ -819,14 +835,12 @@ int launch_absmax(const double *P, size_t n, unsigned long long *out, bool zero,
    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int launch_mixed_flags(const TypePlan &tp, const BatchDev &b, const double *gmag, const unsigned long long *pmax,
-                       double tau, uint32_t *gflag, unsigned long long *count, void *stream)
+int launch_mixed_flags(const BatchDev *batch, const RunDev &run, uint32_t ng, const unsigned long long *pmax, double tau,
+                       unsigned long long *count, void *stream)
 {
-   (void)tp;
-   if (b.g1 <= b.g0) return 0;
-   const unsigned grid = std::min<unsigned>((b.g1 - b.g0 + 255) / 256, 4096);
-   hipLaunchKernelGGL(k_mixed_flags, dim3(grid), dim3(256), 0, (hipStream_t)stream, b.tp, b, gmag, pmax, tau, gflag,
-                      count);
+   if (!ng) return 0;
+   const unsigned grid = std::min<unsigned>((ng + 255) / 256, 4096);
+   hipLaunchKernelGGL(k_mixed_flags, dim3(grid), dim3(256), 0, (hipStream_t)stream, batch, run, pmax, tau, count);
    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -29,6 +29,7 @@
 #include <hip/hip_runtime.h>
 
 #include "device.hpp"
+#include "uniform.hpp"
 
 namespace gint {
 
@@ -128,9 +129,10 @@ __device__ __forceinline__ void eco_batch(const double *a, const double *Wl, dbl
 
 // three wavefronts per SIMD: the 4 x 16 double accumulators, two batches of
 // block elements and the tile operands fit in 168 registers without spills
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_eco(const TypePlan *__restrict__ tpp, BatchDev b, EcoArgs e)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_eco(const BatchDev *__restrict__ batch, RunDev run, EcoArgs e)
 {
-   const TypePlan &tp = *tpp;
+   const BatchDev b = load_batch(batch, 0, run);
+   const TypePlan &tp = *b.tp;
    __shared__ double co[4][MAXNL][MAXNP];   // the class's four shells' coefficients
    __shared__ double W[ECO_PB][ECO_QB];     // coefficient products of the batch
    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -245,14 +247,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
    }
 }
 
-int launch_eco(const TypePlan &tp, const BatchDev &b, const EcoArgs &e, void *stream)
+int launch_eco(const BatchDev *batch, const RunDev &run, uint32_t nrow, const EcoArgs &e, void *stream)
 {
-   if (e.n_items <= 0 || b.r1 <= b.r0) return 0;
-   (void)tp;
-   const uint64_t nitems = (uint64_t)(b.r1 - b.r0) * (uint64_t)e.n_items;
+   if (e.n_items <= 0 || !nrow) return 0;
+   const uint64_t nitems = (uint64_t)nrow * (uint64_t)e.n_items;
    unsigned grid = (unsigned)std::min<uint64_t>(nitems, 65536);
    if (grid >= 64) grid &= ~7u;   // a multiple of the 8 XCDs (the kernel's item order)
-   hipLaunchKernelGGL(k_eco, dim3(grid), dim3(256), 0, (hipStream_t)stream, b.tp, b, e);
+   hipLaunchKernelGGL(k_eco, dim3(grid), dim3(256), 0, (hipStream_t)stream, batch, run, e);
    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -42,6 +42,7 @@
 #include "c2s_table.h"
 #include "device.hpp"
 #include "gint_math.h"
+#include "uniform.hpp"
 
 namespace gint {
 namespace sq {
@@ -139,23 +140,6 @@ __device__ __forceinline__ void lds_order()
    __builtin_amdgcn_wave_barrier();
 }
 
-// A record at a uniform address, through the scalar cache: nothing that a
-// kernel of the K-build reads this way is written by one (plans, records,
-// tables and basis data), which the compiler cannot see behind the stores
-template <class T>
-__device__ __forceinline__ T load_uniform(const T *p)
-{
-   static_assert(sizeof(T) % 4 == 0, "whole words");
-   typedef const __attribute__((address_space(4))) uint32_t *word_ptr;
-   const word_ptr q = (word_ptr)(uintptr_t)p;
-   union {
-      uint32_t w[sizeof(T) / 4];
-      T v;
-   } u;
-#pragma unroll
-   for (unsigned i = 0; i < sizeof(T) / 4; i++) u.w[i] = q[i];
-   return u.v;
-}
 struct GroupHead {   // the start of GroupRec
    uint32_t row0, row1, R[4];
 };
@@ -368,13 +352,20 @@ __device__ __forceinline__ void bra_units(double *D, int ds, int nfn, const SqSp
    }
 }
 
+// the shell pairs of kernel LM
+template <int LM>
+__device__ constexpr bool has_pair(int l1, int l2)
+{
+   return LM == 4 || (LM == 3 ? l1 + l2 <= 4 : (l1 <= LM && l2 <= LM));
+}
+
 template <int LM>
 __device__ __forceinline__ void ket_transform(double *T, int ts, int nrow, const SqSp &q, const double R[3], int lane)
 {
    switch (q.l1 * 4 + q.l2) {
 #define GINT_SQ_KET(a_, b_)                                                                              \
    case a_ * 4 + b_:                                                                                     \
-      if constexpr (a_ <= LM && b_ <= LM) ket_units<a_, b_>(T, ts, nrow, q, R, lane);                    \
+      if constexpr (has_pair<LM>(a_, b_)) ket_units<a_, b_>(T, ts, nrow, q, R, lane);                    \
       break;
       GINT_SQ_KET(0, 0) GINT_SQ_KET(0, 1) GINT_SQ_KET(0, 2) GINT_SQ_KET(0, 3)
       GINT_SQ_KET(1, 0) GINT_SQ_KET(1, 1) GINT_SQ_KET(1, 2) GINT_SQ_KET(1, 3)
@@ -391,7 +382,7 @@ __device__ __forceinline__ void bra_transform(double *D, int ds, int nfn, const 
    switch (q.l1 * 4 + q.l2) {
 #define GINT_SQ_BRA(a_, b_)                                                                              \
    case a_ * 4 + b_:                                                                                     \
-      if constexpr (a_ <= LM && b_ <= LM) bra_units<a_, b_>(D, ds, nfn, q, R, u, lane);                  \
+      if constexpr (has_pair<LM>(a_, b_)) bra_units<a_, b_>(D, ds, nfn, q, R, u, lane);                  \
       break;
       GINT_SQ_BRA(0, 0) GINT_SQ_BRA(0, 1) GINT_SQ_BRA(0, 2) GINT_SQ_BRA(0, 3)
       GINT_SQ_BRA(1, 0) GINT_SQ_BRA(1, 1) GINT_SQ_BRA(1, 2) GINT_SQ_BRA(1, 3)
@@ -402,13 +393,21 @@ __device__ __forceinline__ void bra_transform(double *D, int ds, int nfn, const 
 }
 
 template <int LM>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LM == 3 ? 1 : (LM == 2 ? 3 : 4))))
-void k_sq(const TypePlan *__restrict__ tpp, DevTables t, BatchDev b, KTargets kt, SqArgs y)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LM == 4 ? 1 : (LM >= 2 ? 3 : 4))))
+void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, int nref, uint32_t item0, DevTables t,
+          RunDev run, KTargets kt)
 {
    extern __shared__ __align__(16) double lds[];
-   const TypePlan &tp = *tpp;
    const int lane = threadIdx.x;
-   const int ncpt = tp.ncp, nkc = tp.nkc;
+   // the item's chunk: the first whose items end beyond it
+   uint32_t item = item0 + blockIdx.x;
+   const uint32_t end = lane < nref ? refs[lane].end : 0xffffffffu;
+   const int ri = __builtin_amdgcn_readfirstlane(__popcll(__ballot(end <= item)));
+   if (ri > 0) item -= load_uniform(&refs[ri - 1].end);
+   const SqArgs y = load_uniform(&refs[ri].y);
+   const BatchDev b = load_batch(batches, load_uniform(&refs[ri].batch), run);
+   const TypePlan &tp = *b.tp;
+   const int ncpt = load_uniform(&tp.ncp), nkc = load_uniform(&tp.nkc);
    const uint32_t nfix = min(b.fix_count[0], b.fix_cap);
    char *tab = (char *)lds;
    uint16_t *tcol = (uint16_t *)tab;
@@ -417,7 +416,6 @@ void k_sq(const TypePlan *__restrict__ tpp, DevTables t, BatchDev b, KTargets kt
    double *co = lds + y.o_co;   // the set quartet's coefficients, contraction by contraction
    const int m16 = lane & 15, k4 = lane >> 4;
    {
-      const uint32_t item = blockIdx.x;
       const uint32_t gi = b.g0 + item / (uint32_t)y.nitem;
       const SqItem it = load_uniform(y.items + item % (uint32_t)y.nitem);
       const SqTile bt = load_uniform(y.tiles + it.bt), ktl = load_uniform(y.tiles + it.kt);
@@ -626,11 +624,11 @@ void k_sq(const TypePlan *__restrict__ tpp, DevTables t, BatchDev b, KTargets kt
          }
          // slots of this row whose screening depends on the class
          for (uint32_t e = 0; e < nfix; e++) {
-            const uint32_t p = b.fix[2 * e];
-            if (b.prm_row[p] != r) continue;
+            const uint32_t p = b.fix[2 * e], word = b.fix[2 * e + 1];
+            if (word >> 24 != b.id || b.prm_row[p] != r) continue;
             lds_order();
-            const uint32_t mask = b.fix[2 * e + 1] >> 8, ip = b.prm_ip[p];
-            const double *src = b.fix_ws + (size_t)e * (ncpt + 16);
+            const uint32_t mask = (word >> 8) & 0xffff, ip = b.prm_ip[p];
+            const double *src = b.fix_ws + (size_t)e * b.fix_stride;
             const double *A = src + (size_t)bt.comp0 * nkc + ktl.comp0;
             for (int qb = 0; qb < bt.nsp; qb++)
                for (int qk = 0; qk < ktl.nsp; qk++) {
@@ -684,7 +682,7 @@ void k_sq(const TypePlan *__restrict__ tpp, DevTables t, BatchDev b, KTargets kt
 }  // namespace sq
 
 template <int LM>
-int launch_sq_lm(const BatchDev &b, const DevTables &t, const KTargets &kt, const SqArgs &y, unsigned grid, size_t lds,
-                 void *stream);
+int launch_sq_lm(const BatchDev *batches, const SqRef *refs, int nref, uint32_t item0, unsigned grid, size_t lds,
+                 const DevTables &t, const RunDev &run, const KTargets &kt, void *stream);
 
 }  // namespace gint

@@ -335,10 +335,14 @@ void make_eco_plan(const TypePlan &tp, const std::vector<ClassPlan> &cps, EcoPla
    });
 }
 
+// Registers of a pair's transform: 0 without f shells, 1 with one whose
+// transform is no larger than (dd|'s, 2 the others ((df|, (fd|, (ff|).
+static int sq_group(int l1, int l2) { return l1 <= 2 && l2 <= 2 ? 0 : (l1 + l2 <= 4 ? 1 : 2); }
+
 // One side of a type (bra: sets 0, 1; ket: sets 2, 3) in tiles of at most
-// `max_row` rows and `max_fn` functions; units with an f shell (wf) or
-// without one; single: one shell pair per tile.
-static void make_sq_tiles(const TypePlan &tp, int side, bool wf, int max_row, int max_fn, bool single, SqPlan &sp,
+// `max_row` rows and `max_fn` functions, of the shell pairs of register group
+// `grp` (sq_group); single: one shell pair per tile.
+static void make_sq_tiles(const TypePlan &tp, int side, int grp, int max_row, int max_fn, bool single, SqPlan &sp,
                           std::vector<int> &out)
 {
    const int x = 2 * side, y = 2 * side + 1, low = side ? tp.LC0 : tp.LA0;
@@ -396,7 +400,7 @@ static void make_sq_tiles(const TypePlan &tp, int side, bool wf, int max_row, in
       for (int s2 = 0; s2 < tp.nsh[y]; s2++) {
          const int l1 = tp.l[x][s1], l2 = tp.l[y][s2];
          if (!whole && s2 == 0) close();
-         if ((l1 > 2 || l2 > 2) != wf) continue;
+         if (sq_group(l1, l2) != grp) continue;
          const int nr = below(l1 + l2 + 1) - below(l1), nf = nsph(l1) * nsph(l2);
          const int nc = tp.nl[x][s1] * tp.nl[y][s2];
          if (single) close();
@@ -438,30 +442,26 @@ static void make_sq_tiles(const TypePlan &tp, int side, bool wf, int max_row, in
    close();
 }
 
-// The k_sq launch of the classes of a type with f shells (wf) or without,
-// for nspin density matrices; eco: classes of at least ECO_MIN_NQ
-// contractions take their contracted blocks from the contraction buffer (a
-// tile is then part of one shell pair).
-void make_sq_plan(const TypePlan &tp, const std::vector<ClassPlan> &cps, const EcoPlan &ep, bool wf, int nspin, bool eco,
-                  SqPlan &sp)
+// The k_sq launch of the items of a type whose larger register group
+// (sq_group) is `grp`, for nspin density matrices; eco: classes of at least
+// ECO_MIN_NQ contractions take their contracted blocks from the contraction
+// buffer (a tile is then part of one shell pair).
+void make_sq_plan(const TypePlan &tp, const EcoPlan &ep, int grp, int nspin, bool eco, SqPlan &sp)
 {
-   (void)cps;
    sp = SqPlan();
    int lx = 0;
    for (int t = 0; t < 4; t++)
       for (int s = 0; s < tp.nsh[t]; s++) lx = std::max(lx, tp.l[t][s]);
-   if (wf && lx < 3) return;
-   sp.lm = wf ? 3 : std::min(lx, 2);
-   if (sp.lm == 0) sp.lm = 1;
-   std::vector<int> bra[2], ket[2];
-   for (int f = 0; f < 2; f++) {
-      make_sq_tiles(tp, 0, f == 1, 38, SQ_MAXFN, eco, sp, bra[f]);
-      make_sq_tiles(tp, 1, f == 1, 38, 30, eco, sp, ket[f]);
+   sp.lm = grp ? 2 + grp : (lx <= 1 ? 1 : 2);
+   std::vector<int> bra[3], ket[3];
+   for (int f = 0; f <= grp; f++) {
+      make_sq_tiles(tp, 0, f, 38, SQ_MAXFN, eco, sp, bra[f]);
+      make_sq_tiles(tp, 1, f, 38, 30, eco, sp, ket[f]);
    }
    int top = 0;
-   for (int fb = 0; fb < 2; fb++)
-      for (int fk = 0; fk < 2; fk++) {
-         if ((fb || fk) != wf) continue;
+   for (int fb = 0; fb <= grp; fb++)
+      for (int fk = 0; fk <= grp; fk++) {
+         if (std::max(fb, fk) != grp) continue;
          for (int bi : bra[fb])
             for (int ki : ket[fk]) {
                const SqTile &b = sp.tiles[bi], &k = sp.tiles[ki];

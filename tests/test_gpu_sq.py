@@ -45,3 +45,33 @@ def test_tiles_and_windows(name, debug, spins):
             err, kmax = np.max(np.abs(a - b)), np.max(np.abs(b))
             print(name, "debug", debug, "plan", plan, "sets", st.n_sets, "prm", st.n_prm, "max|K|", kmax, "max|dK|", err)
             assert kmax > 0 and err <= KTOL_ABS + KTOL_REL * kmax
+
+
+# launch sets: the chunks of many quartet types from one launch per kernel, at
+# most 64 chunks in a set and within half the memory budget
+LAUNCH_SETS = {
+    "many_types": (dict(n_water=4, n_tm=2, box_A=8.0, np_max=2, np_tm=2, seed=13), 4096),
+    "several_sets_by_memory": (dict(n_water=5, box_A=7.0, np_min=3, np_max=3, seed=14), 64),
+}
+
+
+@pytest.mark.parametrize("flags", [0, 1, 2])
+@pytest.mark.parametrize("name", list(LAUNCH_SETS))
+def test_launch_sets(name, flags):
+    """flags: every surviving slot through the fix-up (1), one stream (2)"""
+    from libgint_amd import driver as D, load
+
+    lib, o = load(), oracle()
+    cfg, mib = LAUNCH_SETS[name]
+    s = D.System(**cfg)
+    st = s.record()
+    P = s.P()
+    Ko, ho = D.kbuild(o, "oracle_", s, st, P=P)
+    o.oracle_destroy_handle(ho)
+    kmax = np.max(np.abs(Ko))
+    for plan in (False, True):
+        K, h = D.kbuild(lib, "libgint_", s, st, P=P, plan=plan, debug=flags, max_mem_mib=mib)
+        lib.libgint_amd_destroy_handle(h)
+        err = np.max(np.abs(K - Ko))
+        print(name, "flags", flags, "plan", plan, "sets", st.n_sets, "prm", st.n_prm, "max|K|", kmax, "max|dK|", err)
+        assert kmax > 0 and err <= KTOL_ABS + KTOL_REL * kmax
