@@ -144,6 +144,9 @@ struct TypePlan {
    int kcoff[7];             // first of shell f among them
    int nbh;                  // bra Hermite triples t+u+v <= LA
    int nh;                   // Hermite triples t+u+v <= L
+   // Hermite -> cartesian transform (make_type_items)
+   int FC;                   // ket components per pass, a multiple of 4
+   int nkt, nbt;             // terms of the ket and of the bra expansion
    int has00;                // LA0 == 0 && LC0 == 0
    int nL;                   // distinct class L values
    int Ls[16];
@@ -161,6 +164,12 @@ struct TypePlan {
    long long prim_flops;     // per primitive quartet: Hermite -> cartesian transform
    long long ref_slot_flops; // per slot, summed over classes: the reference's Fm + VRR
 };
+
+// Place of Hermite triple (t,u,v), t+u+v <= L, in the cell sum of a type:
+// additive, so that the place of a sum of two triples is the sum of theirs,
+// and different for different triples (found by search up to L = 12)
+GINT_HDI int herm_place(int L, int t, int u, int v) { return t + u * (L + 1) + v * (L * (L + 1) + 1); }
+GINT_HDI int herm_places(int L) { return L * (L * (L + 1) + 1) + 1; }
 
 // The KsGroup of class k of a set quartet stored as a KsSet: offsets of
 // contraction (ia,ib,ic,id) are base + ia step[0] + ic step[1] (ac), ...
@@ -196,8 +205,10 @@ GINT_HDI KsGroup ks_from_set(const KsSet &s, const TypePlan &tp, int k)
 
 // Device-resident constant tables.
 struct DevTables {
-   const double *C0;
+   const double *C0;          // [patch][ld_C0]: the caller's table
    int ld_C0;
+   const double *Cm;          // orders 1 .. ldm of it as [patch][coefficient pair][order][2] (launch_pack_c0)
+   int ldm;
    const int *grid_lo, *grid_hi;
    const double *bw;
    const double *ftable;
@@ -209,12 +220,19 @@ struct DevTables {
 };
 
 // LDS layout of k_fm_r for one type
+// LDS of k_fm_r for a type: offsets in doubles, of the tables in bytes.
 struct FmLayout {
-   int SB;      // survivors per Hermite batch
-   int o_fmv;   // per lane: G_m, then D_m = (-2 rho)^m G_m
-   int o_sv;    // per lane: X Y Z of P-Q-g, TG1 (or T), TG2
-   int o_R;     // Hermite layers, 2 x SB x nh
-   int o_int;   // byte offset of 64 lane infos (branch | patch << 2) and 64 survivor lanes
+   int NB;      // primitive quartets per wavefront
+   int SV;      // surviving slots kept at once
+   int SB;      // of them in one Hermite recursion
+   int o_quirk; // [NB] screened slots' Fm[0] (behind the geometry)
+   int o_sv;    // [SV] X Y Z of P-Q-g, TG1 (or T), TG2
+   int o_fm;    // [SV][L+1] (-2 rho)^m G_m
+   int o_R;     // Hermite layers [SB][nh]; then the cell sum at its additive places
+   int o_e;     // one-dimensional expansions E of both sides, [2][3][28]
+   int o_c;     // the transform's coefficients: ket terms, bra terms
+   int o_W;     // [nbh][FC + 2]
+   int o_int;   // byte offset of the slot lists and the type's tables
    int bytes;
 };
 
@@ -225,8 +243,7 @@ struct FmLayout {
 // launch covers many types) and adds the execution's buffers (RunDev).
 struct BatchDev {
    const TypePlan *tp;        // device copy
-   const uint32_t *e1;        // Hermite -> cartesian stage 1 items: t u v fx fy fz (3 bits each), W slot << 18
-   const uint32_t *e2;        // stage 2 items: ex ey ez (3 bits each), column << 9, block element << 16
+   const uint32_t *items;     // the type's Hermite -> cartesian tables (make_type_items)
    const RowRec *rows;
    const GroupRec *groups;
    const uint32_t *prm_row;   // row of each primitive quartet
@@ -401,11 +418,16 @@ void *noalloc_scratch();
 int launch_zero_u32(uint32_t *p, int n, void *stream);
 // k_fm_r over the chunks of a list (pair: two primitive quartets per
 // wavefront, units are pairs), and the fix-up of the listed slots
-int launch_fm_r(const BatchDev *batches, const WorkRef *refs, int nref, uint32_t units, bool pair, size_t lds,
+int launch_fm_r(const BatchDev *batches, const WorkRef *refs, int nref, uint32_t units, int nacc, size_t lds,
                 const DevTables &t, const RunDev &run, void *stream);
+// Hermite functions per lane that k_fm_r takes for a type of nh: 1, 3 or 8
+inline int fm_nacc(int nh) { return nh <= 64 ? 1 : (nh <= 192 ? 3 : 8); }
 int launch_fixup(const BatchDev *batches, size_t lds, const DevTables &t, const RunDev &run, uint32_t n_fix, void *stream);
 // the layouts of a type and whether k_fm_r takes its primitive quartets in pairs
-void fm_layouts(const TypePlan &tp, int Ng, FmLayout &main, FmLayout &fix, bool *pair);
+void fm_layouts(const TypePlan &tp, FmLayout &main, FmLayout &fix);
+// orders 1 .. ldm of the caller's table in the order that k_fm_r reads them
+constexpr int CM_PAIRS = 53;   // of the 105 coefficients, the last one with a 0
+int launch_pack_c0(const double *C0, int ld_C0, int ldm, double *Cm, void *stream);
 // from the chunks' blocks to K (kernels_sq.hpp)
 int launch_sq(const BatchDev *batches, const SqRef *refs, int nref, uint32_t items, int lm, size_t lds,
               const DevTables &t, const RunDev &run, const KTargets &kt, void *stream);
@@ -439,7 +461,7 @@ ClassPlan make_plan(int la, int lb, int lc, int ld);
 // fills everything from nsh, l and nl
 void make_type_plan(TypePlan &tp);
 // item descriptors of the Hermite -> cartesian transform of a type
-void make_type_items(const TypePlan &tp, std::vector<uint32_t> &e1, std::vector<uint32_t> &e2);
+void make_type_items(const TypePlan &tp, std::vector<uint32_t> &items);
 uint64_t class_mult(int code);
 void boys_table(double *ftable);
 int device_math_selftest(const double *x, const double *y, int n, double *out);

@@ -151,8 +151,7 @@ Engine::~Engine()
    for (LaunchPlan *lp : {&stream_lp_, &plan_lp_, &plan_na_lp_}) lp->release();
    for (auto &ti : types_) {
       if (ti.d_plan) (void)hipFree(ti.d_plan);
-      if (ti.d_e1) (void)hipFree(ti.d_e1);
-      if (ti.d_e2) (void)hipFree(ti.d_e2);
+      if (ti.d_items) (void)hipFree(ti.d_items);
       for (SqPlan *sp = &ti.sq[0][0][0]; sp != &ti.sq[0][0][0] + 4 * SQ_GROUPS; sp++) {
          if (sp->dev) (void)hipFree(sp->dev);
       }
@@ -160,7 +159,7 @@ Engine::~Engine()
       if (ti.d_eco_info) (void)hipFree(ti.d_eco_info);
       if (ti.d_eco_items) (void)hipFree(ti.d_eco_items);
    }
-   void *bufs[] = {d_data_, d_C0_, d_grid_, d_bw_, d_ftab_, d_cell_, d_neighs_, d_work_,
+   void *bufs[] = {d_data_, d_C0_, d_Cm_, d_grid_, d_bw_, d_ftab_, d_cell_, d_neighs_, d_work_,
                    d_fix_, d_fix_ws_, d_stats_, d_fixcnt_, d_out_, d_mix_};
    for (void *b : bufs)
       if (b) (void)hipFree(b);
@@ -296,7 +295,7 @@ int Engine::type_of(int i, int j, int k, int l)
       if (truncated_ && ti.plan.L > nder_)
          fatal("the truncated-Coulomb table has fewer derivative orders than this quartet's total angular momentum",
                ti.plan.L);
-      make_type_items(ti.plan, ti.e1, ti.e2);
+      make_type_items(ti.plan, ti.items);
       if (!fm_r_lds_bytes(ti.plan)) fatal("quartet type exceeds the on-chip budget", ti.plan.L);
       for (int c = 0; c < ti.plan.nclass; c++) {
          const int code = ti.plan.cls_code[c];
@@ -943,6 +942,12 @@ void Engine::ensure_tables()
       if (d_C0_) HIPCHECK(hipFree(d_C0_));
       HIPCHECK(hipMalloc((void **)&d_C0_, sizeof(double) * C0_.size()));
       HIPCHECK(hipMemcpy(d_C0_, C0_.data(), sizeof(double) * C0_.size(), hipMemcpyHostToDevice));
+      if (nder_ > 0) {
+         if (d_Cm_) HIPCHECK(hipFree(d_Cm_));
+         HIPCHECK(hipMalloc((void **)&d_Cm_, sizeof(double) * cm_size()));
+         if (launch_pack_c0(d_C0_, ld_C0_, cm_orders(), d_Cm_, stream_)) fatal("coefficient table launch", 0);
+         HIPCHECK(hipStreamSynchronize((hipStream_t)stream_));
+      }
    }
    HIPCHECK(hipMemcpy(d_cell_, cell_, sizeof(double) * 18, hipMemcpyHostToDevice));
    if (neighs_.size() > d_neighs_cap_) {
@@ -999,10 +1004,8 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
       if (!ti.d_plan) {
          HIPCHECK(hipMalloc((void **)&ti.d_plan, sizeof(TypePlan)));
          HIPCHECK(hipMemcpy(ti.d_plan, &tp, sizeof(TypePlan), hipMemcpyHostToDevice));
-         HIPCHECK(hipMalloc((void **)&ti.d_e1, sizeof(uint32_t) * ti.e1.size()));
-         HIPCHECK(hipMemcpy(ti.d_e1, ti.e1.data(), sizeof(uint32_t) * ti.e1.size(), hipMemcpyHostToDevice));
-         HIPCHECK(hipMalloc((void **)&ti.d_e2, sizeof(uint32_t) * ti.e2.size()));
-         HIPCHECK(hipMemcpy(ti.d_e2, ti.e2.data(), sizeof(uint32_t) * ti.e2.size(), hipMemcpyHostToDevice));
+         HIPCHECK(hipMalloc((void **)&ti.d_items, sizeof(uint32_t) * ti.items.size()));
+         HIPCHECK(hipMemcpy(ti.d_items, ti.items.data(), sizeof(uint32_t) * ti.items.size(), hipMemcpyHostToDevice));
          auto put = [](auto *&dst, const auto &v) {
             if (v.empty()) return;
             HIPCHECK(hipMalloc((void **)&dst, sizeof(v[0]) * v.size()));
@@ -1203,6 +1206,8 @@ DevTables Engine::dev_tables() const
    DevTables t;
    t.C0 = d_C0_;
    t.ld_C0 = ld_C0_;
+   t.Cm = d_Cm_;
+   t.ldm = cm_orders();
    t.grid_lo = d_grid_;
    t.grid_hi = d_grid_ + TCG_GRID * TCG_GRID;
    t.bw = d_bw_;
@@ -1232,7 +1237,6 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
    lp.sets.clear();
    lp.ncp_max = lp.doubles = lp.n_prm = 0;
    const size_t cap = (na ? NOALLOC_AC0_BYTES : budget_bytes_ / 2) / sizeof(double);
-   const int Ng = (int)neighs_.size() / 3;
    std::vector<BatchDev> batches;
    std::vector<char> lists;   // behind the BatchDevs
    for (size_t d = 0; d < devs.size(); d++) {
@@ -1253,8 +1257,7 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
          LaunchSet &ls = lp.sets.back();
          BatchDev b{};   // every field zero / null unless set below
          b.tp = ti.d_plan;
-         b.e1 = ti.d_e1;
-         b.e2 = ti.d_e2;
+         b.items = ti.d_items;
          b.rows = D.rows;
          b.groups = D.groups;
          b.prm_row = D.prm_row;
@@ -1273,8 +1276,7 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
          b.r1 = c.r1;
          b.g0 = c.g0;
          b.g1 = c.g1;
-         bool pair;
-         fm_layouts(ti.plan, Ng, b.fm, b.fix_fm, &pair);
+         fm_layouts(ti.plan, b.fm, b.fix_fm);
          ls.fix_lds = std::max(ls.fix_lds, (size_t)b.fix_fm.bytes);
          batches.push_back(b);
          ls.chunks.push_back({(int)d, (int)i});
@@ -1308,27 +1310,24 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
       // types need, so that a large type does not cost the others occupancy
       uint64_t prm = 0;
       for (uint32_t i : order) prm += chunk(i).p1 - chunk(i).p0;
-      std::vector<WorkRef> fm[2][FM_BUCKETS];
+      // primitive quartets per wavefront: as many as leave every wavefront
+      // slot of the chip a few units
+      const int nb = (int)std::min<uint64_t>(64, std::max<uint64_t>(1, prm / FM_UNITS));
+      std::vector<WorkRef> fm[FM_BUCKETS];
       for (uint32_t i : order) {
-         const TypeInfo &ti = info(i);
-         FmLayout main, fix;
-         bool pair;
-         fm_layouts(ti.plan, Ng, main, fix, &pair);
-         int k = FM_BUCKETS - 1;
-         if (prm > FM_ONE_LAUNCH) {
-            k = 0;
-            while ((size_t)main.bytes > FM_BUCKET_LDS[k]) k++;
-         }
-         auto &v = fm[pair ? 1 : 0][k];
+         FmLayout &lay = batches[ls.b0 + i].fm;
+         lay.NB = std::min(lay.NB, nb);
+         const int nacc = fm_nacc(info(i).plan.nh);
+         const int k = prm <= FM_ONE_LAUNCH || nacc == 1 ? 0 : (nacc == 3 ? 1 : (lay.bytes <= FM_LARGE_LDS ? 2 : 3));
+         ls.fm_nacc[k] = std::max(ls.fm_nacc[k], nacc);
+         auto &v = fm[k];
          const uint32_t n = chunk(i).p1 - chunk(i).p0;
-         const uint64_t end = (v.empty() ? 0ull : v.back().end) + (pair ? (n + 1) / 2 : n);
+         const uint64_t end = (v.empty() ? 0ull : v.back().end) + (n + lay.NB - 1) / lay.NB;
          if (end > 0xffffffffull) fatal("launch set of more than 2^32 primitive quartets", (long long)end);
          v.push_back(WorkRef{i, (uint32_t)end});
-         ListRef &l = ls.fm[pair ? 1 : 0][k];
-         l.lds = std::max(l.lds, (size_t)main.bytes);
+         ls.fm[k].lds = std::max(ls.fm[k].lds, (size_t)lay.bytes);
       }
-      for (int k = 0; k < 2; k++)
-         for (int x = 0; x < FM_BUCKETS; x++) put(ls.fm[k][x], fm[k][x]);
+      for (int x = 0; x < FM_BUCKETS; x++) put(ls.fm[x], fm[x]);
       auto per_group = [&](uint32_t i) { return (double)(chunk(i).p1 - chunk(i).p0) / (double)(chunk(i).g1 - chunk(i).g0); };
       std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return per_group(a) > per_group(b); });
       for (int sp = 0; sp < 2; sp++) {
@@ -1371,8 +1370,7 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
    const size_t head = (sizeof(BatchDev) * batches.size() + 15) & ~(size_t)15;
    const size_t total = head + lists.size();
    for (LaunchSet &ls : lp.sets) {
-      for (auto &x : ls.fm)
-         for (ListRef &l : x) l.off += head;
+      for (ListRef &l : ls.fm) l.off += head;
       for (auto &x : ls.sq)
          for (ListRef &l : x) l.off += head;
    }
@@ -1402,15 +1400,14 @@ void Engine::run_set(std::vector<TypeDev> &devs, const LaunchPlan &lp, const Lau
 
    if (launch_zero_u32(w.run.fix_count, 1, st)) fatal("counter reset launch", 0);
    int rc = 0;
-   for (int k = 0; k < 2; k++)
-      for (int x = FM_BUCKETS - 1; x >= 0; x--) {
-         const ListRef &l = ls.fm[k][x];
-         if (!l.n) continue;
-         evb(0, st);
-         rc = launch_fm_r(batches, (const WorkRef *)(lp.dev + l.off), l.n, l.units, k == 1, l.lds, t, w.run, st);
-         if (rc) fatal("fm_r launch", rc);
-         eve(0, st);
-      }
+   for (int x = FM_BUCKETS - 1; x >= 0; x--) {
+      const ListRef &l = ls.fm[x];
+      if (!l.n) continue;
+      evb(0, st);
+      rc = launch_fm_r(batches, (const WorkRef *)(lp.dev + l.off), l.n, l.units, ls.fm_nacc[x], l.lds, t, w.run, st);
+      if (rc) fatal("fm_r launch", rc);
+      eve(0, st);
+   }
    evb(3, st);
    rc = launch_fixup(batches, ls.fix_lds, t, w.run, w.run.force_fix ? w.run.fix_cap : std::min<uint32_t>(64u, w.run.fix_cap),
                      st);
@@ -1569,7 +1566,7 @@ void Engine::replay_graph(const RunBufs &w, const KTargets &kt)
                            (uint64_t)w.run.fix_cap, (uint64_t)w.run.fix_stride, (uint64_t)plan_lp_.dev,
                            (uint64_t)kt.P[0], (uint64_t)kt.P[1], (uint64_t)kt.K[0], (uint64_t)kt.K[1],
                            (uint64_t)kt.nspin, graph_bits(kt.hf_fac), (uint64_t)kt.out, (uint64_t)d_data_,
-                           (uint64_t)d_C0_, (uint64_t)d_neighs_, (uint64_t)neighs_.size(), graph_bits(R_cut_),
+                           (uint64_t)d_C0_, (uint64_t)d_Cm_, (uint64_t)d_neighs_, (uint64_t)neighs_.size(), graph_bits(R_cut_),
                            (uint64_t)truncated_, (uint64_t)debug_, (uint64_t)ld_C0_, (uint64_t)w.run.mixed,
                            graph_bits(mixed_tau_), (uint64_t)d_mix_};
    constexpr size_t NK = sizeof key / sizeof key[0];
@@ -1704,7 +1701,7 @@ uint64_t Engine::device_bytes() const
       b += d.cap[0] * sizeof(RowRec) + d.cap[1] * sizeof(GroupRec) + d.cap[2] * 4 + d.cap[3] * 4 +
            d.cap[4] * sizeof(KsGroup) + d.cap[5] * sizeof(KsRec) + d.cap[6] * sizeof(KsSet);
    b += plan_lp_.cap + plan_na_lp_.cap;
-   b += work_bytes_ + fix_cap_ * 8 + fix_ws_cap_ * 8 + d_data_cap_ * 8 + C0_.size() * 8 +
+   b += work_bytes_ + fix_cap_ * 8 + fix_ws_cap_ * 8 + d_data_cap_ * 8 + C0_.size() * 8 + (d_Cm_ ? cm_size() * 8 : 0) +
         d_neighs_cap_ * 8;
    return b;
 }

@@ -14,6 +14,7 @@
 #pragma once
 #include <stdint.h>
 
+#include <algorithm>
 #include <array>
 #include <cstring>
 #include <map>
@@ -21,6 +22,7 @@
 #include <vector>
 
 #include "device.hpp"
+#include "tcg_patches.h"
 
 namespace gint {
 
@@ -91,8 +93,8 @@ struct TypeInfo {
    std::array<int, 4> sig;
    TypePlan plan;
    TypePlan *d_plan = nullptr;
-   std::vector<uint32_t> e1, e2;          // Hermite -> cartesian item descriptors
-   uint32_t *d_e1 = nullptr, *d_e2 = nullptr;
+   std::vector<uint32_t> items;           // Hermite -> cartesian tables
+   uint32_t *d_items = nullptr;
    std::vector<ClassPlan> cplans;
    // from the blocks to K: [nspin - 1][0 own contraction, 1 k_eco][register group]
    SqPlan sq[2][2][SQ_GROUPS];
@@ -104,15 +106,18 @@ struct TypeInfo {
    int *d_eco_info = nullptr;
 };
 
-// k_fm_r launches of a set by the LDS of the types (bytes, at most): a launch
-// takes the LDS of its largest type, and wavefronts per CU follow from it.
-// Measured with all types in one launch / in four: (pp|pp) to (ff|ff) in 256
-// cells 27.9 / 15.2 ms, s to f in 125 cells 28.6 / 15.2 ms.  A set of few
-// primitive quartets does not fill the chip and pays for the launches
+// k_fm_r launches of a set: by the Hermite functions per lane of the types
+// (fm_nacc), the largest in two lists, since a launch takes the LDS of its
+// largest type and wavefronts per CU follow from it (13 to 44 KB).  A set of
+// few primitive quartets does not fill the chip and pays for the launches
 // instead: 5783 in 27 cells 0.69 ms in one launch, 0.9 in four.
 constexpr uint64_t FM_ONE_LAUNCH = 16384;   // a set of at most this many primitive quartets: one launch
+constexpr int FM_LARGE_LDS = 26 * 1024;
 constexpr int FM_BUCKETS = 4;
-constexpr size_t FM_BUCKET_LDS[FM_BUCKETS] = {10 * 1024 + 512, 13 * 1024 + 512, 32 * 1024, 64 * 1024};
+// wavefronts that a set should give k_fm_r before one takes more than one
+// primitive quartet: a K-build of 5783 takes 0.5 ms with one to a wavefront,
+// 0.7 with 16; 5 million are done in 19.5 ms by sixteens, in 53.7 by twos
+constexpr uint64_t FM_UNITS = 8192;
 
 // One launch of a launch set: its list of chunks among the set's tables
 struct ListRef {
@@ -127,7 +132,8 @@ struct LaunchSet {
    uint32_t b0 = 0;                           // first BatchDev of the set in the tables
    size_t doubles = 0;                        // of the work buffer
    size_t n_prm = 0;
-   ListRef fm[2][FM_BUCKETS];                 // k_fm_r: single, pairs; by LDS
+   ListRef fm[FM_BUCKETS];                    // k_fm_r
+   int fm_nacc[FM_BUCKETS] = {0, 0, 0, 0};
    ListRef sq[2][SQ_KERNELS];                 // k_sq: [nspin - 1][kernel - 1]
    size_t fix_lds = 0;
 };
@@ -325,7 +331,9 @@ class Engine {
    LaunchPlan stream_lp_, plan_lp_, plan_na_lp_;   // the plan's with allocated and with the static scratch
    double *d_data_ = nullptr;
    size_t d_data_cap_ = 0;
-   double *d_C0_ = nullptr;
+   double *d_C0_ = nullptr, *d_Cm_ = nullptr;
+   int cm_orders() const { return std::min(nder_, 12); }   // an (ff|ff) quartet needs order 12
+   size_t cm_size() const { return (size_t)TCG_NPATCH * CM_PAIRS * 2 * cm_orders(); }
    int *d_grid_ = nullptr;
    double *d_bw_ = nullptr, *d_ftab_ = nullptr, *d_cell_ = nullptr, *d_neighs_ = nullptr;
    size_t d_neighs_cap_ = 0;

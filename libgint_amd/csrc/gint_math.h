@@ -132,6 +132,40 @@ GINT_HD void gint_boys(int nmax, double T, double *f, const double *ftable, doub
    for (int n = 0; n <= nmax; n++) f[n] *= fac;
 }
 
+/* F_0 of gint_boys(nmax, ...) alone: the same operations, so the same value */
+GINT_HD double gint_boys_f0(int nmax, double T, const double *ftable, double fac)
+{
+   GINT_NO_CONTRACT
+   if (T < 1.e-13) return fac / (2. * 0 + 1.);
+   double f;
+   if (T < 12.) {
+      const double tdelta = 0.1;
+      const int ld = 28;
+      int itab = (int)round(T / tdelta);
+      double ttab = (double)itab * tdelta;
+      const double *row = ftable + itab * ld + nmax;
+      double dt = ttab - T;
+      double tmp = dt;
+      f = row[0];
+      f += row[1] * tmp * 1.0;
+      tmp *= dt; f += row[2] * tmp * 0.5;
+      tmp *= dt; f += row[3] * tmp * (1. / 6.);
+      tmp *= dt; f += row[4] * tmp * (1. / 24.);
+      tmp *= dt; f += row[5] * tmp * (1. / 120.);
+      tmp *= dt; f += row[6] * tmp * (1. / 720.);
+      double expt = gint_exp(-T);
+      for (int n = nmax - 1; n >= 0; n--) f = (2.0 * T * f + expt) / (2. * n + 1.);
+   } else {
+      double tmp = 1.0 / T;
+      double tmp2 = tmp * tmp;
+      double tmp3 = tmp * tmp2;
+      double g = 0.4999489092 - 0.2473631686 * tmp + 0.321180909 * tmp2 - 0.3811559346 * tmp3;
+      double expt = gint_exp(-T);
+      f = 0.5 * sqrt(GINT_PI * tmp) - g * expt * tmp;
+   }
+   return f * fac;
+}
+
 /* Where G_m(R,T) comes from for one slot. */
 #define GINT_G_ZERO  0   /* beyond truncation: all G_m = 0            */
 #define GINT_G_BOYS  1   /* cutoff irrelevant: plain Boys function     */

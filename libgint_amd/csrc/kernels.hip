@@ -1,9 +1,8 @@
 // gfx950 kernels of the K-build.  A launch covers one chunk of one quartet
 // type (the shell structure of the four sets of a set quartet).
 //
-//   k_fm_r         one wavefront per primitive quartet (two when the cells
-//                  fit half the lanes).  Lanes evaluate
-//                  G_m(R,T) (or F_m) of 64 lattice cells at once and decide
+//   k_fm_r         one wavefront per run of primitive quartets.  Lanes evaluate
+//                  G_m(R,T) (or F_m) of 64 (quartet, cell) slots at once and decide
 //                  Fm[0] > 1e-12 for every class L of the type; surviving
 //                  cells run the McMurchie-Davidson Hermite recursion
 //                  R^(n)_tuv in LDS and the n = 0 layer is summed over cells
@@ -13,7 +12,7 @@
 //                  classes at once, reference src/compute_Fm.cpp (prepare,
 //                  Fm, Vm), src/compute_VRR.cpp and the cell sum of
 //                  src/compute_ECO.cpp:216-272.
-//   k_fm_r<true,.> slots whose screening differs between the classes of the
+//   k_fm_r<true>   slots whose screening differs between the classes of the
 //                  type (Fm[0] within rounding of 1e-12 at different L): the
 //                  slot's blocks alone, added by the consumers to the classes
 //                  that keep it.
@@ -233,12 +232,12 @@ __device__ __forceinline__ unsigned long long slot_hash(uint32_t set_ij, uint32_
 // sum_j T2_j sum_{l<14-j} T1_l c[jl]: the operations of gint_cheb_sum in the
 // same order (so the value is bitwise the host's), with T2_j produced by
 // the recurrence of gint_cheb14 inside the loop to keep few values live
-__device__ __forceinline__ double d_cheb_sum(const double *__restrict__ c, const double *T1, double x2)
+__device__ __forceinline__ double d_cheb_sum(const double *c, const double *T1, double x2)
 {
    GINT_NO_CONTRACT
    double tmp = 0.0, tm1 = 0.0, tm2 = 0.0;
    int jl = 0;
-#pragma unroll 7
+#pragma unroll
    for (int j = 0; j < 14; j++) {
       double t2;
       if (j == 0) t2 = 1.0;
@@ -257,107 +256,224 @@ __device__ __forceinline__ double d_cheb_sum(const double *__restrict__ c, const
    return tmp;
 }
 
-// ---------------------------------------------------------------------------
-// K1: G_m -> Hermite R -> cell sum -> (e0|f0), one wavefront per primitive
-// quartet.  FIX: one wavefront per listed (primitive, cell) slot, no
-// screening, blocks and per-L Fm[0] into the fix-up workspace.
-// ---------------------------------------------------------------------------
-constexpr int GEO = 24;   // doubles of the primitive geometry at the start of LDS
-enum { G_P = 0, G_Q = 3, G_PA = 6, G_QC = 9, G_KFAC = 12, G_RHO = 13, G_RR = 14, G_I2AB = 15, G_I2CD = 16 };
+// the same sum, from the table in coefficient pairs (c: the order's first
+// pair, ld: doubles from one pair to the next).  Not fused either: where G_m
+// is small against its terms, a slot's orders carry the rounding of this
+// order of operations, which far images' integrals amplify
+__device__ __forceinline__ double d_cheb_pairs(const double *c, int ld, const double *T1, double x2)
+{
+   GINT_NO_CONTRACT
+   double tmp = 0.0, tm1 = 0.0, tm2 = 0.0, odd = 0.0;
+   int jl = 0;
+#pragma unroll
+   for (int j = 0; j < 14; j++) {
+      double t2;
+      if (j == 0) t2 = 1.0;
+      else if (j == 1) t2 = GINT_SQRT2 * x2;
+      else if (j == 2) t2 = 2. * x2 * tm1 - GINT_SQRT2;
+      else t2 = 2. * x2 * tm1 - tm2;
+      double dot = 0.0;
+#pragma unroll
+      for (int l = 0; l < 14; l++)
+         if (l < 14 - j) {
+            const int k = jl + l;
+            double ck = odd;
+            if (k % 2 == 0) {
+               const double2 v = *(const double2 *)(c + (size_t)(k / 2) * ld);
+               ck = v.x;
+               odd = v.y;
+            }
+            dot += T1[l] * ck;
+         }
+      tmp += dot * t2;
+      jl += 14 - j;
+      tm2 = tm1;
+      tm1 = t2;
+   }
+   return tmp;
+}
 
-static FmLayout fm_layout(const TypePlan &tp, bool fix, bool pair = false)
+// A value whose uses stay where they are: what is unpacked from it is not
+// kept in registers over the loops around
+__device__ __forceinline__ uint32_t here(uint32_t v)
+{
+   asm volatile("" : "+v"(v));
+   return v;
+}
+
+// ---------------------------------------------------------------------------
+// K1: G_m -> Hermite R -> cell sum -> (e0|f0).  FIX: one wavefront per listed
+// (primitive, cell) slot, no screening, blocks and per-L Fm[0] into the
+// fix-up workspace.
+// ---------------------------------------------------------------------------
+constexpr int GEO = 14;   // doubles of a primitive quartet's geometry, at the start of LDS
+enum { G_PQ = 0, G_PA = 3, G_QC = 6, G_KFAC = 9, G_RHO = 10, G_RR = 11, G_I2AB = 12, G_I2CD = 13 };
+constexpr int EXP1 = 28;  // doubles of one direction's expansion, E^e_t at e (e + 1) / 2 + t
+constexpr int FM_CAND = 128;   // slots listed for evaluation
+
+// two doubles, stored at once
+struct __attribute__((packed, aligned(8))) Pair {
+   double a, b;
+};
+
+static FmLayout fm_layout(const TypePlan &tp, bool fix)
 {
    FmLayout y;
-   const int L = tp.L, nh = tp.nh;
-   const int geo = pair ? 2 * GEO : GEO;   // one geometry record per primitive quartet of the wavefront
-   y.o_fmv = geo;
-   y.o_sv = geo + 64 * (L + 1);
-   y.o_R = y.o_sv + 320;
-   // the Hermite batch fills what is left of a 10 KB budget: small enough
-   // that 4 wavefronts per SIMD fit in LDS
-   int SB = fix ? 1 : (1280 - y.o_R) / (2 * nh);
-   SB = std::max(1, std::min(16, SB));
-   y.SB = SB;
-   const int cell_phase = y.o_R + 2 * SB * nh;
-   const int e_phase = geo + nh + 6 * 28 + tp.nbh * tp.nkc;
-   const int dbl = std::max(cell_phase, e_phase);
-   y.o_int = 8 * dbl;
-   y.bytes = y.o_int + 4 * 128;
+   const int L = tp.L, nbr = tp.ncp / tp.nkc;
+   // the geometries, survivors and blocks of about 8 KB (L = 5) to 16 KB
+   // ((dd|dd)-like) per wavefront; beyond that the transform's tables rule
+   y.NB = fix ? 1 : (L <= 6 ? 16 : 8);
+   y.SV = fix ? 1 : (L <= 6 ? 24 : 16);
+   const int places = herm_places(L);
+   y.SB = fix ? 1 : std::max(1, std::min(4, places / tp.nh));
+   y.o_quirk = GEO * y.NB;
+   y.o_sv = y.o_quirk + y.NB;
+   y.o_fm = y.o_sv + 5 * y.SV;
+   y.o_R = y.o_fm + (L + 1) * y.SV;
+   y.o_e = y.o_R + std::max(places, y.SB * tp.nh);
+   y.o_c = y.o_e + 6 * EXP1;
+   y.o_W = (y.o_c + tp.nkt + tp.nbt + 1) & ~1;   // read two doubles at a time
+   y.o_int = 8 * (y.o_W + tp.nbh * (tp.FC + 2));
+   const int words = 2 * y.SV + tp.nkc + nbr;
+   const int shorts = FM_CAND + 2 * (tp.nkt + tp.nbt) + tp.nbh;
+   y.bytes = (y.o_int + 4 * words + 2 * shorts + 15) & ~15;
    return y;
 }
 
-// at most 128 VGPRs (4 wavefronts per SIMD, with the LDS budget above): the
-// kernel waits on memory half of its time, so wavefronts in flight pay more
-// than the few values it then keeps in scratch
+// A wavefront takes NB consecutive primitive quartets of a type:
+//   - their geometries, one lane each;
+//   - all their (quartet, cell) slots, 64 at a time: those within the
+//     truncation radius are listed, and G_0 and the screening decision of 64
+//     listed ones are taken at once, one lane each;
+//   - G_1..G_L of the survivors, one lane per (survivor, order);
+//   - quartet by quartet, the Hermite recursion of its survivors in place in
+//     LDS (a shell's values before those of the shells below, so one buffer
+//     does), their sum in registers, and the transform to (e0|f0) in two
+//     passes over LDS, four results per lane.
+// About one slot per quartet survives (of 27 to 256 cells), so what it costs
+// is the work per quartet, and the serial parts of it: the geometry is 700
+// operations, the G sums are loads from a table, and both leave most lanes
+// idle when a wavefront has one quartet or two.  Taking 16 (8 of the largest
+// types, for LDS) and four results per lane in the transform brought 5.0
+// million quartets in 27 cells from 53.7 to 19.5 ms, 6.1 million with s to f
+// shells in 125 cells from 81 to 24.4, a cluster of 1.1 million from 9.8 to
+// 2.9.  What bounds it now is latency: a wavefront waits 70% of its time,
+// mostly for LDS in the recursion and the transform (two fifths and a third
+// of it), and the vector units are busy a quarter.
 //
-// PAIR (at most 32 cells, at most 256 Hermite functions): two primitive
-// quartets per wavefront.  Lanes 0-31 take the cells of the first, lanes
-// 32-63 those of the second; their survivors share the G_m and Hermite
-// batches and each quartet keeps its own cell sum and transform.
+// At most 168 VGPRs (3 wavefronts per SIMD): with 128 more values go to
+// scratch in the loops, 23.2 instead of 19.5 ms.
+//
+// NACC: Hermite functions per lane, for types of at most 64 NACC.  Their
+// table and sums stay in registers; with those of the largest type for all
+// they went to scratch, and each reload waited for the blocks' stores.
 //
 // One launch takes the chunks of a list, one after the other in the
-// numbering of its units (primitive quartets or pairs of them): a launch per
-// type left the chip to the slowest wavefronts of each, and small systems to
-// launch after launch of a few workgroups.
-template <bool FIX, bool PAIR>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
+// numbering of its units (NB primitive quartets): a launch per type left the
+// chip to the slowest wavefronts of each, and small systems to launch after
+// launch of a few workgroups.
+template <bool FIX, int NACC>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
 void k_fm_r(const BatchDev *__restrict__ batches, const WorkRef *__restrict__ refs, int nref, DevTables t, RunDev run)
 {
-   static_assert(!(FIX && PAIR), "the fix-up takes one slot per wavefront");
-   constexpr int NPR = PAIR ? 2 : 1;      // primitive quartets per wavefront
-   constexpr int NACC = PAIR ? 4 : 8;     // Hermite functions per lane and quartet, / 64
    extern __shared__ double lds[];
    const int lane = threadIdx.x;
-   const int half = PAIR ? lane >> 5 : 0;   // the lane's quartet
+   const unsigned long long below = (1ull << lane) - 1ull;
    uint32_t ubase = 0;
    const uint32_t nfix = FIX ? min(run.fix_count[0], run.fix_cap) : 0;
    // (the fix-up: one entry per turn, each with its own chunk)
    for (uint32_t turn = FIX ? blockIdx.x : 0; turn < (FIX ? nfix : (uint32_t)nref); turn += FIX ? gridDim.x : 1) {
-   const BatchDev b = load_batch(batches, FIX ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(run.fix[2 * turn + 1] >> 24))
-                                              : load_uniform(&refs[turn].batch), run);
+   uint32_t u0 = turn, nunit = turn + 1, id = 0;
+   if (FIX) {
+      id = (uint32_t)__builtin_amdgcn_readfirstlane((int)(run.fix[2 * turn + 1] >> 24));
+   } else {
+      // the first unit of the chunk that is this workgroup's
+      const WorkRef ref = load_uniform(refs + turn);
+      const uint32_t skip = ubase % gridDim.x;
+      u0 = blockIdx.x >= skip ? blockIdx.x - skip : blockIdx.x + gridDim.x - skip;
+      nunit = ref.end - ubase;
+      ubase = ref.end;
+      id = ref.batch;
+      if (u0 >= nunit) continue;
+   }
+   const BatchDev b = load_batch(batches, id, run);
    const TypePlan &tp = *b.tp;
    const FmLayout lay = FIX ? b.fix_fm : b.fm;
    const int L = load_uniform(&tp.L), nh = load_uniform(&tp.nh), Lp1 = L + 1;
-   const int SB = lay.SB;
-   double *G = lds + GEO * half;      // geometry of the lane's quartet
-   double *fmv = lds + lay.o_fmv;     // [64][L+1]
-   double *sv = lds + lay.o_sv;       // [64][5]
-   double *Rb = lds + lay.o_R;        // [2][SB][nh]
-   int *svi = (int *)((char *)lds + lay.o_int);
-   int *svl = svi + 64;
-   const uint32_t nwork = FIX ? turn + 1 : b.p1 - b.p0;
-   const uint32_t *__restrict__ e1 = b.e1, *__restrict__ e2 = b.e2;
-   // the first unit of the chunk that is this workgroup's
-   const uint32_t skip = ubase % gridDim.x;
-   const uint32_t u0 = FIX ? turn : (blockIdx.x >= skip ? blockIdx.x - skip : blockIdx.x + gridDim.x - skip);
-   if (!FIX) ubase = load_uniform(&refs[turn].end);
+   const int nkc = load_uniform(&tp.nkc), ncp = load_uniform(&tp.ncp), nbh = load_uniform(&tp.nbh);
+   const int FC = load_uniform(&tp.FC), FW = FC + 2, nkt = load_uniform(&tp.nkt), nterm = nkt + load_uniform(&tp.nbt);
+   const int has00 = load_uniform(&tp.has00), nL = load_uniform(&tp.nL), nbr = ncp / nkc;
+   const int LA = load_uniform(&tp.LA), LC = load_uniform(&tp.LC);
+   const int NB = lay.NB, SV = lay.SV, SB = lay.SB;
+   double *quirk = lds + lay.o_quirk;   // [NB]
+   double *sv = lds + lay.o_sv;         // [SV][5]
+   double *fm = lds + lay.o_fm;         // [SV][L+1]
+   double *R = lds + lay.o_R;
+   double *E1 = lds + lay.o_e;          // [2][3][EXP1]: x y z; bra, ket
+   double *cf = lds + lay.o_c;          // [nkt], [nbt]
+   double *W = lds + lay.o_W;
+   int *svi = (int *)((char *)lds + lay.o_int);           // [SV] branch | patch << 2
+   int *svq = svi + SV;                                   // [SV] quartet
+   uint32_t *rec = (uint32_t *)(svq + SV);                // [nkc] ket components, then bra
+   uint16_t *cand = (uint16_t *)(rec + nkc + nbr);        // [FM_CAND] quartet << 8 | cell
+   uint16_t *pos = cand + FM_CAND;                        // bytes of the terms' places, [nkt], [nbt]
+   uint16_t *ent = pos + nterm;                           // the terms' entries of E, 5 bits each; bit 15: none
+   uint16_t *hpos = ent + nterm;                          // [nbh]
+   const uint32_t *__restrict__ items = b.items;
+   const unsigned all = (1u << nL) - 1u;
+   const int Ng = FIX ? 1 : t.Ng;
+   // exact quotients of the small numbers that they divide
+   const uint32_t qNg = (1u << 24) / (uint32_t)Ng + 1u, qL = 65536u / (uint32_t)max(L, 1) + 1u;
+   const int nblk = (nbh + 3) >> 2;
+   const uint32_t qblk = 65536u / (uint32_t)nblk + 1u;
 
-   for (uint32_t w0 = u0 * NPR; w0 < nwork; w0 += gridDim.x * NPR) {
-      const uint32_t w = w0 + half;
-      const bool hvalid = w < nwork;                    // the lane's quartet exists
-      const int nprim = (int)min((uint32_t)NPR, nwork - w0);
-      uint32_t p;
+   // the type's tables
+   lds_order();
+   for (int i = lane; i < nterm; i += 64) {
+      const uint32_t it = items[i];
+      pos[i] = (uint16_t)(((it >> 15) & 1023) * (i < nkt ? 8 : 8 * FW));
+      ent[i] = (uint16_t)((it & 0x7fff) | (it >> 31) << 15);
+   }
+   for (int i = lane; i < nkc + nbr; i += 64) rec[i] = items[nterm + i];
+   for (int i = lane; i < nbh; i += 64) hpos[i] = (uint16_t)(items[nterm + nkc + nbr + i] * 8);
+   // the lane's Hermite functions h = lane + 64 i: R_h = X_dir R_m1 + coef R_m2
+   uint32_t hent[NACC], hplace[NACC];
+#pragma unroll
+   for (int i = 0; i < NACC; i++) {
+      const int h = lane + 64 * i;
+      hent[i] = hplace[i] = 0;
+      if (h < nh) {
+         const HermEntry e = c_herm.e[h];
+         if (h) hent[i] = (uint32_t)e.m1 | (uint32_t)(e.m2 >= 0 ? e.m2 : 0) << 9 | (uint32_t)e.dir << 18 | (uint32_t)e.coef << 20;
+         hplace[i] = (uint32_t)herm_place(L, c_herm.tuv[h][0], c_herm.tuv[h][1], c_herm.tuv[h][2]);
+      }
+   }
+
+   for (uint32_t u = u0; u < nunit; u += FIX ? 1u : gridDim.x) {
+      // ---- geometry, one lane per quartet ----
+      const uint32_t w0 = FIX ? u : u * (uint32_t)NB;
+      const int nq = FIX ? 1 : (int)min((uint32_t)NB, b.p1 - b.p0 - w0);
+      uint32_t pfirst = b.p0 + w0;
       int fix_n3 = 0;
       if (FIX) {
-         p = b.fix[2 * w];
-         fix_n3 = (int)(b.fix[2 * w + 1] & 0xff);
-      } else {
-         p = b.p0 + (hvalid ? w : w0);
+         pfirst = b.fix[2 * u];
+         fix_n3 = (int)(b.fix[2 * u + 1] & 0xff);
       }
-      const uint32_t r = b.prm_row[p];
-      const RowRec row = b.rows[r];
-      const GroupRec &g = b.groups[row.group];
-      const uint32_t ip = b.prm_ip[p];
-      const int n1 = row.n12 & 0xffff, n2 = row.n12 >> 16;
-      if ((lane & (64 / NPR - 1)) == 0 && hvalid) {
+      lds_order();
+      if (lane < nq) {
+         const uint32_t p = pfirst + lane;
+         const RowRec row = b.rows[b.prm_row[p]];
+         const GroupRec &g = b.groups[row.group];
+         const uint32_t ip = b.prm_ip[p];
          const double *data = b.data;
          PrimGeo geo;
          prim_prepare(data + g.R[0], data + g.R[1], data + g.R[2], data + g.R[3], data[g.Z[0] + (ip & 15)],
                       data[g.Z[1] + ((ip >> 4) & 15)], data[g.Z[2] + ((ip >> 8) & 15)],
-                      data[g.Z[3] + ((ip >> 12) & 15)], n1, n2, t, geo);
+                      data[g.Z[3] + ((ip >> 12) & 15)], row.n12 & 0xffff, row.n12 >> 16, t, geo);
+         double *G = lds + GEO * lane;
          for (int k = 0; k < 3; k++) {
-            G[G_P + k] = geo.P[k];
-            G[G_Q + k] = geo.Q[k];
+            GINT_NO_CONTRACT
+            G[G_PQ + k] = geo.P[k] - geo.Q[k];
             G[G_PA + k] = geo.PA[k];
             G[G_QC + k] = geo.QC[k];
          }
@@ -366,51 +482,69 @@ void k_fm_r(const BatchDev *__restrict__ batches, const WorkRef *__restrict__ re
          G[G_RR] = geo.Rr;
          G[G_I2AB] = geo.i2ab;
          G[G_I2CD] = geo.i2cd;
+         quirk[lane] = 0.0;
       }
-      __syncthreads();
-      double acc[NPR][NACC];
-#pragma unroll
-      for (int q = 0; q < NPR; q++)
-#pragma unroll
-         for (int i = 0; i < NACC; i++) acc[q][i] = 0.0;
-      double quirk = 0.0;
+      lds_order();
+      double acc[NACC];
       unsigned long long n_surv = 0, csum = 0, n_any = 0;
-      bool any_surv[NPR];
-#pragma unroll
-      for (int q = 0; q < NPR; q++) any_surv[q] = false;
-      const unsigned all = (1u << tp.nL) - 1u;
-      const int ncell = FIX ? 1 : t.Ng;
-
-      for (int base = 0; base < ncell; base += 64) {
-         const int n3 = FIX ? fix_n3 : base + (PAIR ? (lane & 31) : lane);
-         const bool valid = FIX ? (lane == 0) : (hvalid && n3 < t.Ng);
+      const int nslot = nq * Ng;
+      int ncand = 0, s0 = 0;        // listed slots; the next slot to look at
+      int cur = -1, next = 0;       // the quartet being summed; the first one without its blocks
+      for (bool last = false; !last;) {
+         // ---- list the slots that are not beyond truncation ----
+         while (ncand < 64 && s0 < nslot) {
+            const int slot = s0 + lane;
+            int q = 0, n3 = 0;
+            bool keep = slot < nslot;
+            if (keep) {
+               q = (int)(((uint32_t)slot * qNg) >> 24);
+               n3 = FIX ? fix_n3 : slot - q * Ng;
+               if (t.truncated && !FIX) {
+                  GINT_NO_CONTRACT
+                  const double *G = lds + GEO * q;
+                  const double x = G[G_PQ + 0] - t.neighs[n3 * 3 + 0];
+                  const double y = G[G_PQ + 1] - t.neighs[n3 * 3 + 1];
+                  const double z = G[G_PQ + 2] - t.neighs[n3 * 3 + 2];
+                  const double rpq2 = x * x + y * y + z * z;
+                  const double Rr = G[G_RR];
+                  keep = !(G[G_RHO] * rpq2 > Rr * Rr + 11.0 * Rr + 50.0);
+               }
+            }
+            const unsigned long long m = __ballot(keep);
+            if (keep) cand[ncand + __popcll(m & below)] = (uint16_t)(q << 8 | n3);
+            ncand += __popcll(m);
+            s0 += 64;
+         }
+         lds_order();
+         const int ncd = min(ncand, 64);
+         // ---- G_0 and the decision of up to 64 listed slots ----
          int status = 0;  // 1 kept by every class, 2 screened by every class, 3 class-dependent
-         unsigned mask = 0;
-         double *myf = fmv + lane * Lp1;
-         if (valid) {
-            const double Kfac = G[G_KFAC], rho = G[G_RHO];
-            double X[3], T, Fm0 = 0.0, tg1 = 0.0, tg2 = 0.0;
-            int br, patch = 0;
+         int q = 0, br = 0, patch = 0;
+         double X[3] = {0.0, 0.0, 0.0}, Fm0 = 0.0, tg1 = 0.0, tg2 = 0.0;
+         if (lane < ncd) {
+            const int c = cand[lane], n3 = c & 255;
+            q = c >> 8;
+            const double *G = lds + GEO * q;
+            const double Kfac = G[G_KFAC];
+            unsigned mask = 0;
+            double T;
             {
                GINT_NO_CONTRACT
-               X[0] = G[G_P + 0] - G[G_Q + 0] - t.neighs[n3 * 3 + 0];
-               X[1] = G[G_P + 1] - G[G_Q + 1] - t.neighs[n3 * 3 + 1];
-               X[2] = G[G_P + 2] - G[G_Q + 2] - t.neighs[n3 * 3 + 2];
+               X[0] = G[G_PQ + 0] - t.neighs[n3 * 3 + 0];
+               X[1] = G[G_PQ + 1] - t.neighs[n3 * 3 + 1];
+               X[2] = G[G_PQ + 2] - t.neighs[n3 * 3 + 2];
                const double rpq2 = X[0] * X[0] + X[1] * X[1] + X[2] * X[2];
-               T = rho * rpq2;
+               T = G[G_RHO] * rpq2;
             }
             br = t.truncated ? gint_tcg_locate(G[G_RR], T, t.grid_lo, t.grid_hi, t.bw, &patch, &tg1, &tg2) : GINT_G_BOYS;
             if (br == GINT_G_PATCH) {
+               GINT_NO_CONTRACT
                double T1[14];
                gint_cheb14(tg1, T1);
-               {
-                  GINT_NO_CONTRACT
-                  Fm0 = d_cheb_sum(t.C0 + (size_t)t.ld_C0 * patch, T1, tg2) * Kfac;
-               }
-               myf[0] = Fm0;
+               Fm0 = d_cheb_sum(t.C0 + (size_t)t.ld_C0 * patch, T1, tg2) * Kfac;
             } else if (br == GINT_G_BOYS) {
-               gint_boys(L, T, myf, t.ftable, Kfac);
-               Fm0 = myf[0];
+               Fm0 = gint_boys_f0(L, T, t.ftable, Kfac);
+               tg1 = T;
             }
             const bool lsens = br == GINT_G_BOYS && T >= 1.e-13 && T < 12.;   // F_0 depends on the start order
             if (br == GINT_G_ZERO) {
@@ -420,38 +554,30 @@ void k_fm_r(const BatchDev *__restrict__ batches, const WorkRef *__restrict__ re
                // F_0 of the downward recursion depends on the starting order
                // by rounding only; decide each class L exactly this close to
                // the threshold
-               if (lsens && tp.nL > 1 && fabs(Fm0 - 1.e-12) <= 1.e-20) {
+               if (lsens && nL > 1 && fabs(Fm0 - 1.e-12) <= 1.e-20) {
                   mask = 0u;
-                  for (int i = 0; i < tp.nL; i++) {
-                     gint_boys(tp.Ls[i], T, myf, t.ftable, Kfac);
-                     if (myf[0] > 1.e-12) mask |= 1u << i;
-                  }
-                  gint_boys(L, T, myf, t.ftable, Kfac);
+                  for (int i = 0; i < nL; i++)
+                     if (gint_boys_f0(tp.Ls[i], T, t.ftable, Kfac) > 1.e-12) mask |= 1u << i;
                }
                status = mask == all ? 1 : (mask == 0u ? 2 : 3);
             }
             if (FIX) {
                // per-L Fm[0] of the slot, for the classes that screen it
-               double *f0 = b.fix_ws + (size_t)w * b.fix_stride + tp.ncp;
-               for (int i = 0; i < tp.nL; i++) {
-                  double v = Fm0;
-                  if (lsens) {
-                     gint_boys(tp.Ls[i], T, myf, t.ftable, Kfac);
-                     v = myf[0];
-                  }
-                  f0[i] = v;
-               }
-               if (lsens) gint_boys(L, T, myf, t.ftable, Kfac);
+               double *f0 = b.fix_ws + (size_t)u * b.fix_stride + ncp;
+               for (int i = 0; i < nL; i++) f0[i] = lsens ? gint_boys_f0(tp.Ls[i], T, t.ftable, Kfac) : Fm0;
                status = br == GINT_G_ZERO ? 2 : 1;
             } else if (b.force_fix && status == 1) {
                status = 3;
             }
             if (!FIX) {
                if (status == 2) {
-                  if (tp.has00) quirk += Fm0;
+                  if (has00) atomicAdd(&quirk[q], Fm0);
                } else {
                   if (b.stats) {
-                     const unsigned long long h = slot_hash(g.set_ij, g.set_kl, n1, n2, ip, n3);
+                     const uint32_t p = pfirst + q;
+                     const RowRec row = b.rows[b.prm_row[p]];
+                     const GroupRec &g = b.groups[row.group];
+                     const unsigned long long h = slot_hash(g.set_ij, g.set_kl, row.n12 & 0xffff, row.n12 >> 16, b.prm_ip[p], n3);
                      if (mask == all) {
                         n_surv += (unsigned long long)tp.nclass;
                         csum += h * tp.mult_all;
@@ -468,7 +594,7 @@ void k_fm_r(const BatchDev *__restrict__ batches, const WorkRef *__restrict__ re
                   if (status == 3) {
                      const uint32_t idx = atomicAdd(&b.fix_count[0], 1u);
                      if (idx < b.fix_cap) {
-                        b.fix[2 * idx] = p;
+                        b.fix[2 * idx] = pfirst + q;
                         b.fix[2 * idx + 1] = (uint32_t)n3 | (mask << 8) | (b.id << 24);
                      } else {
                         // list full: every class keeps the slot (its G_0 is
@@ -482,211 +608,253 @@ void k_fm_r(const BatchDev *__restrict__ batches, const WorkRef *__restrict__ re
                   }
                }
             }
-            if (status == 1) {
-               sv[lane * 5 + 0] = X[0];
-               sv[lane * 5 + 1] = X[1];
-               sv[lane * 5 + 2] = X[2];
-               sv[lane * 5 + 3] = br == GINT_G_PATCH ? tg1 : T;
-               sv[lane * 5 + 4] = tg2;
-               svi[lane] = br | (patch << 2);
-            }
          }
-         // survivors of this pass, in lane order
+         // the listed slots that are left move to the front
+         ncand -= ncd;
+         if (lane < ncand) cand[lane] = cand[64 + lane];
+         last = ncand == 0 && s0 >= nslot;
+         // ---- the survivors, in the order of the quartets, SV at a time ----
          const unsigned long long smask = __ballot(status == 1);
-         const int nsv = __popcll(smask);
-         const int nsv0 = PAIR ? __popcll(smask & 0xffffffffull) : nsv;   // survivors of the first quartet
-         if (status == 1) svl[__popcll(smask & ((1ull << lane) - 1ull))] = lane;
-         __syncthreads();
-         if (nsv == 0) continue;
-         any_surv[0] = any_surv[0] || nsv0 > 0;
-         if (PAIR) any_surv[NPR - 1] = any_surv[NPR - 1] || nsv > nsv0;
-         // G_1..G_L of the patch survivors, one (survivor, order) per lane
-         {
-            for (int idx = lane; idx < nsv * L; idx += 64) {
-               const int s = idx / L, m = idx - s * L + 1;
-               const int ln = svl[s];
-               const double Kfac = lds[GEO * (PAIR ? ln >> 5 : 0) + G_KFAC];
-               const int info = svi[ln];
-               if ((info & 3) == GINT_G_PATCH) {
-                  double T1[14];
-                  gint_cheb14(sv[ln * 5 + 3], T1);
-                  const double *c = t.C0 + (size_t)t.ld_C0 * (info >> 2) + m * TCG_NCOEF;
-                  fmv[ln * Lp1 + m] = d_cheb_sum(c, T1, sv[ln * 5 + 4]) * Kfac;
-               }
+         const int nsv = __popcll(smask), rank = __popcll(smask & below);
+         int k0 = 0;
+         do {
+            const int np = min(SV, nsv - k0);
+            const int r = rank - k0;
+            lds_order();
+            if (status == 1 && r >= 0 && r < SV) {
+               sv[r * 5 + 0] = X[0];
+               sv[r * 5 + 1] = X[1];
+               sv[r * 5 + 2] = X[2];
+               sv[r * 5 + 3] = tg1;
+               sv[r * 5 + 4] = tg2;
+               fm[r * Lp1] = Fm0;
+               svi[r] = br | patch << 2;
+               svq[r] = q;
             }
-         }
-         __syncthreads();
-         {
-            for (int idx = lane; idx < nsv * Lp1; idx += 64) {
-               const int s = idx / Lp1, m = idx - s * Lp1;
-               const int ln = svl[s];
-               const double m2rho = -2.0 * lds[GEO * (PAIR ? ln >> 5 : 0) + G_RHO];
-               double pw = 1.0;
+            lds_order();
+            // (-2 rho)^m G_m, one (survivor, order) per lane
+            for (int idx = lane; idx < np * L; idx += 64) {
+               const int s = (int)(((uint32_t)idx * qL) >> 16), m = idx - s * L + 1;
+               const int info = svi[s];
+               if ((info & 3) != GINT_G_PATCH) continue;
+               const double *G = lds + GEO * svq[s];
+               const double m2rho = -2.0 * G[G_RHO];
+               double pw = G[G_KFAC];
                for (int k = 0; k < m; k++) pw *= m2rho;
-               fmv[ln * Lp1 + m] *= pw;
+               const double *c = t.Cm + ((size_t)(info >> 2) * CM_PAIRS * t.ldm + (m - 1)) * 2;
+               double T1[14];
+               gint_cheb14(sv[s * 5 + 3], T1);
+               fm[s * Lp1 + m] = d_cheb_pairs(c, 2 * t.ldm, T1, sv[s * 5 + 4]) * pw;
             }
-         }
-         __syncthreads();
-         // Hermite recursion R^(n)_tuv = coef R^(n+1)_{tuv-2d} + X_d R^(n+1)_{tuv-d}
-         for (int s0 = 0; s0 < nsv; s0 += SB) {
-            const int nb = min(SB, nsv - s0);
-            double *prv = Rb, *cur = Rb + SB * nh;
-            if (lane < nb) prv[lane * nh] = fmv[svl[s0 + lane] * Lp1 + L];
-            __syncthreads();
-            for (int n = L - 1; n >= 1; n--) {
-               const int mn = d_nherm(L - n);
-               for (int h = lane; h < mn; h += 64) {
-                  if (h == 0) {
-                     for (int s = 0; s < nb; s++) cur[s * nh] = fmv[svl[s0 + s] * Lp1 + n];
-                  } else {
-                     const HermEntry e = c_herm.e[h];
-                     const double cf = (double)e.coef;
-                     for (int s = 0; s < nb; s++) {
-                        double v = sv[svl[s0 + s] * 5 + e.dir] * prv[s * nh + e.m1];
-                        if (e.m2 >= 0) v += cf * prv[s * nh + e.m2];
-                        cur[s * nh + h] = v;
-                     }
-                  }
-               }
-               __syncthreads();
-               double *tmp = prv;
-               prv = cur;
-               cur = tmp;
-            }
-            // the n = 0 layer goes straight into the cell sum of its quartet
-#pragma unroll
-            for (int i = 0; i < NACC; i++) {
-               const int h = lane + 64 * i;
-               if (h < nh) {
-                  double a0 = acc[0][i], a1 = acc[NPR - 1][i];
-                  if (h == 0) {
-                     for (int s = 0; s < nb; s++) {
-                        const double v = fmv[svl[s0 + s] * Lp1];
-                        if (!PAIR || s0 + s < nsv0) a0 += v;
-                        else a1 += v;
-                     }
-                  } else {
-                     const HermEntry e = c_herm.e[h];
-                     const double cf = (double)e.coef;
-                     for (int s = 0; s < nb; s++) {
-                        double v = sv[svl[s0 + s] * 5 + e.dir] * prv[s * nh + e.m1];
-                        if (e.m2 >= 0) v += cf * prv[s * nh + e.m2];
-                        if (!PAIR || s0 + s < nsv0) a0 += v;
-                        else a1 += v;
-                     }
-                  }
-                  acc[0][i] = a0;
-                  if (PAIR) acc[NPR - 1][i] = a1;
+            if (lane < np && (svi[lane] & 3) == GINT_G_BOYS) {
+               const double *G = lds + GEO * svq[lane];
+               double *f = fm + lane * Lp1;
+               gint_boys(L, sv[lane * 5 + 3], f, t.ftable, G[G_KFAC]);
+               const double m2rho = -2.0 * G[G_RHO];
+               double pw = 1.0;
+               for (int m = 1; m <= L; m++) {
+                  pw *= m2rho;
+                  f[m] *= pw;
                }
             }
-            __syncthreads();
-         }
-      }
+            lds_order();
 
-      // ---- Hermite -> cartesian, once per primitive quartet ----
-      double *sR = lds + lay.o_fmv;      // [nh]
-      double *Ex = sR + nh;              // [3][28] bra E^{e0}_t
-      double *Fk = Ex + 84;              // [3][28] ket (-1)^tau E^{f0}_tau
-      double *W = Fk + 84;               // [nbh][nkc]
-      // screened slots' Fm[0], summed per quartet (lane 0, and lane 32 for the second)
-      for (int off = 32 / NPR; off > 0; off >>= 1) quirk += __shfl_down(quirk, off, 64 / NPR);
-      double qsum[NPR];
+            for (int s = 0;;) {
+               int qs;
+               if (s < np) qs = __builtin_amdgcn_readfirstlane(svq[s]);
+               else if (last && k0 + np >= nsv) qs = nq;   // the end: what is left to write
+               else break;
+               if (qs != cur) {
+                  if (cur >= 0) {
+                     // ---- Hermite -> cartesian of the quartet `cur` ----
+                     const double *G = lds + GEO * cur;
+                     const int ln = (int)here((uint32_t)lane);
+                     lds_order();
 #pragma unroll
-      for (int q = 0; q < NPR; q++) qsum[q] = __shfl(quirk, 32 * q, 64);
+                     for (int i = 0; i < NACC; i++)
+                        if (ln + 64 * i < nh) R[here(hplace[i])] = acc[i];
+                     // E^{e+1}_t = E^e_{t-1} / (2 zeta) + x E^e_t + (t + 1) E^e_{t+1}, one
+                     // direction per lane (ket: (-1)^t E).  The recursion as such: the
+                     // errors of its steps cancel in the horizontal recurrence, those
+                     // of a closed form do not
+                     if (ln < 6) {
+                        const bool ket = ln >= 3;
+                        const double x = G[(ket ? G_QC - 3 : G_PA) + ln], i2 = ket ? G[G_I2CD] : G[G_I2AB];
+                        const int lm = ket ? LC : LA;
+                        double *E = E1 + EXP1 * ln;
+                        double e0[8] = {1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+                        E[0] = 1.0;
 #pragma unroll
-      for (int q = 0; q < NPR; q++) {
-         if (q >= nprim) break;
-         const double *Gq = lds + GEO * q;
-         double *dst = FIX ? b.fix_ws + (size_t)w * b.fix_stride : b.ac0 + (size_t)(w0 + q) * tp.ncp;
-         // calibration of the mixed-precision routing: the largest block
-         // element of each set quartet (a positive double orders as its bits)
-         unsigned long long *gm = nullptr;
-         if (!FIX && b.gmag) gm = (unsigned long long *)(b.gmag + b.rows[b.prm_row[b.p0 + w0 + q]].group);
-         if (!FIX && !any_surv[q]) {
-            // no cell survives: the blocks are zero but for the screened
-            // slots' Fm[0] in (00|00)
-            for (int j = lane; j < tp.ncp; j += 64) dst[j] = (j == 0 && tp.has00) ? qsum[q] : 0.0;
-            if (gm && lane == 0 && tp.has00) atomicMax(gm, (unsigned long long)__double_as_longlong(fabs(qsum[q])));
-            __syncthreads();
-            continue;
-         }
-         __syncthreads();
+                        for (int e = 0; e < 6; e++) {
+                           if (e >= lm) break;
+                           double below_ = 0.0;   // E^e_{t-1}
 #pragma unroll
-         for (int i = 0; i < NACC; i++) {
-            const int h = lane + 64 * i;
-            if (h < nh) sR[h] = acc[q][i];
-         }
-         if (lane < 6) {
-            const int d = lane % 3;
-            const bool ket = lane >= 3;
-            const int Lm = ket ? tp.LC : tp.LA;
-            const double x = ket ? Gq[G_QC + d] : Gq[G_PA + d];
-            const double i2 = ket ? Gq[G_I2CD] : Gq[G_I2AB];
-            double *E = (ket ? Fk : Ex) + d * 28;
-            E[0] = 1.0;
-            for (int e = 0; e < Lm; e++) {
-               const double *Ee = E + e * (e + 1) / 2;
-               double *En = E + (e + 1) * (e + 2) / 2;
-               for (int tt = 0; tt <= e + 1; tt++) {
-                  double v = 0.0;
-                  if (tt > 0) v += i2 * Ee[tt - 1];
-                  if (tt <= e) v += x * Ee[tt];
-                  if (tt + 1 <= e) v += (double)(tt + 1) * Ee[tt + 1];
-                  En[tt] = v;
+                           for (int tt = 0; tt <= e + 1; tt++) {
+                              double v = 0.0;
+                              if (tt > 0) v += i2 * below_;
+                              if (tt <= e) v += x * e0[tt];
+                              if (tt + 1 <= e) v += (double)(tt + 1) * e0[tt + 1];
+                              below_ = e0[tt];
+                              e0[tt] = v;
+                              E[(e + 1) * (e + 2) / 2 + tt] = ket && (tt & 1) ? -v : v;
+                           }
+                        }
+                     }
+                     lds_order();
+                     for (int i = ln; i < nterm; i += 64) {
+                        const uint32_t it = ent[i];
+                        const double *e = E1 + (i < nkt ? 3 * EXP1 : 0);
+                        const double v = e[it & 31] * e[EXP1 + ((it >> 5) & 31)] * e[2 * EXP1 + ((it >> 10) & 31)];
+                        cf[i] = it >> 15 ? 0.0 : v;
+                     }
+                     double *dst = FIX ? b.fix_ws + (size_t)u * b.fix_stride : b.ac0 + (size_t)(w0 + cur) * ncp;
+                     const double qsum = !FIX && has00 ? quirk[cur] : 0.0;
+                     double vmax = 0.0;
+                     for (int f0 = 0; f0 < nkc; f0 += FC) {
+                        const int nf = min(FC, nkc - f0);
+                        lds_order();
+                        // W[tuv][f] = sum of the ket component's terms over R[tuv + term]
+                        for (int idx = ln; idx < nf * nblk; idx += 64) {
+                           const int fi = (int)(((uint32_t)idx * qblk) >> 16), hb = idx - fi * nblk;
+                           const uint32_t rc = rec[f0 + fi];
+                           const int n = (int)(rc >> 20);
+                           const double *ck = cf + ((rc >> 8) & 0xfff);
+                           const uint16_t *pk = pos + ((rc >> 8) & 0xfff);
+                           const char *r0 = (const char *)R + hpos[hb];
+                           const char *r1 = (const char *)R + hpos[min(hb + nblk, nbh - 1)];
+                           const char *r2 = (const char *)R + hpos[min(hb + 2 * nblk, nbh - 1)];
+                           const char *r3 = (const char *)R + hpos[min(hb + 3 * nblk, nbh - 1)];
+                           double s0_ = 0.0, s1_ = 0.0, s2_ = 0.0, s3_ = 0.0;
+                           for (int k = 0; k < n; k += 2) {
+                              const double ca = ck[k], cb = ck[k + 1];
+                              const int pa = pk[k], pb = pk[k + 1];
+                              s0_ += ca * *(const double *)(r0 + pa);
+                              s1_ += ca * *(const double *)(r1 + pa);
+                              s2_ += ca * *(const double *)(r2 + pa);
+                              s3_ += ca * *(const double *)(r3 + pa);
+                              s0_ += cb * *(const double *)(r0 + pb);
+                              s1_ += cb * *(const double *)(r1 + pb);
+                              s2_ += cb * *(const double *)(r2 + pb);
+                              s3_ += cb * *(const double *)(r3 + pb);
+                           }
+                           double *w = W + hb * FW + (int)(rc & 0xff) - f0;
+                           w[0] = s0_;
+                           if (hb + nblk < nbh) w[nblk * FW] = s1_;
+                           if (hb + 2 * nblk < nbh) w[2 * nblk * FW] = s2_;
+                           if (hb + 3 * nblk < nbh) w[3 * nblk * FW] = s3_;
+                        }
+                        lds_order();
+                        // (e0|f0) = sum of the bra component's terms over W[tuv][f]
+                        const int nfb = (nf + 3) >> 2;
+                        const uint32_t qfb = 65536u / (uint32_t)nfb + 1u;
+                        for (int idx = ln; idx < nbr * nfb; idx += 64) {
+                           const int ei = (int)(((uint32_t)idx * qfb) >> 16), fb = idx - ei * nfb;
+                           const uint32_t rc = rec[nkc + ei];
+                           const int n = (int)(rc >> 20), e = (int)(rc & 0xff);
+                           const double *ck = cf + nkt + ((rc >> 8) & 0xfff);
+                           const uint16_t *pk = pos + nkt + ((rc >> 8) & 0xfff);
+                           const char *w = (const char *)(W + 4 * fb);
+                           double s0_ = 0.0, s1_ = 0.0, s2_ = 0.0, s3_ = 0.0;
+                           for (int k = 0; k < n; k += 2) {
+                              const double ca = ck[k], cb = ck[k + 1];
+                              const double2 *wa = (const double2 *)(w + pk[k]), *wb = (const double2 *)(w + pk[k + 1]);
+                              const double2 a0 = wa[0], a1 = wa[1], b0 = wb[0], b1 = wb[1];
+                              s0_ += ca * a0.x;
+                              s1_ += ca * a0.y;
+                              s2_ += ca * a1.x;
+                              s3_ += ca * a1.y;
+                              s0_ += cb * b0.x;
+                              s1_ += cb * b0.y;
+                              s2_ += cb * b1.x;
+                              s3_ += cb * b1.y;
+                           }
+                           const int f = f0 + 4 * fb;
+                           double *o = dst + e * nkc + f;
+                           if (e == 0 && f == 0) s0_ += qsum;
+                           if (f + 3 < nkc) {
+                              *(Pair *)o = Pair{s0_, s1_};
+                              *(Pair *)(o + 2) = Pair{s2_, s3_};
+                           } else {
+                              o[0] = s0_;
+                              if (f + 1 < nkc) o[1] = s1_;
+                              else s1_ = 0.0;
+                              if (f + 2 < nkc) o[2] = s2_;
+                              else s2_ = 0.0;
+                              s3_ = 0.0;
+                           }
+                           vmax = fmax(vmax, fmax(fmax(fabs(s0_), fabs(s1_)), fmax(fabs(s2_), fabs(s3_))));
+                        }
+                     }
+                     // calibration of the mixed-precision routing: the largest block
+                     // element of each set quartet (a positive double orders as its bits)
+                     if (!FIX && b.gmag) {
+                        for (int off = 32; off > 0; off >>= 1) vmax = fmax(vmax, __shfl_xor(vmax, off, 64));
+                        if (lane == 0)
+                           atomicMax((unsigned long long *)(b.gmag + b.rows[b.prm_row[pfirst + cur]].group),
+                                     (unsigned long long)__double_as_longlong(vmax));
+                     }
+                     next = cur + 1;
+                  }
+                  // quartets without a surviving cell: zero but for the
+                  // screened slots' Fm[0] in (00|00)
+                  for (; !FIX && next < qs; next++) {
+                     double *dst = b.ac0 + (size_t)(w0 + next) * ncp;
+                     const double qsum = has00 ? quirk[next] : 0.0;
+                     for (int j = lane; j < ncp; j += 64) dst[j] = j == 0 ? qsum : 0.0;
+                     if (b.gmag && lane == 0 && has00)
+                        atomicMax((unsigned long long *)(b.gmag + b.rows[b.prm_row[pfirst + next]].group),
+                                  (unsigned long long)__double_as_longlong(fabs(qsum)));
+                  }
+                  cur = qs;
+                  if (qs == nq) break;
+#pragma unroll
+                  for (int i = 0; i < NACC; i++) acc[i] = 0.0;
                }
+               // ---- Hermite recursion of the quartet's survivors ----
+               //    R^(n)_tuv = coef R^(n+1)_{tuv-2d} + X_d R^(n+1)_{tuv-d}
+               const int nb = min(SB, (int)__popcll(__ballot(lane >= s && lane < np && svq[min(lane, SV - 1)] == qs)));
+               const double *xs = sv + 5 * s, *fs = fm + Lp1 * s;
+               lds_order();
+               const int ln = (int)here((uint32_t)lane);
+               if (ln < nb) R[ln * nh] = fs[ln * Lp1 + L];
+               for (int n = L - 1; n >= 1; n--) {
+                  const int mn = d_nherm(L - n);
+#pragma unroll
+                  for (int i = NACC - 1; i >= 0; i--) {
+                     if (64 * i >= mn) continue;
+                     lds_order();
+                     const int h = lane + 64 * i;
+                     if (h >= mn) continue;
+                     const uint32_t he = here(hent[i]);
+                     const int m1 = he & 511, m2 = (he >> 9) & 511, dir = (he >> 18) & 3;
+                     const double c = (double)(he >> 20);
+                     for (int k = 0; k < nb; k++) {
+                        double *Rk = R + k * nh;
+                        double v = xs[5 * k + dir] * Rk[m1] + c * Rk[m2];
+                        if (h == 0) v = fs[k * Lp1 + n];
+                        Rk[h] = v;
+                     }
+                  }
+               }
+               // the n = 0 layer goes straight into the cell sum
+               lds_order();
+#pragma unroll
+               for (int i = 0; i < NACC; i++) {
+                  if (64 * i >= nh) continue;
+                  const uint32_t he = here(hent[i]);
+                  const int m1 = he & 511, m2 = (he >> 9) & 511, dir = (he >> 18) & 3;
+                  const double c = (double)(he >> 20);
+                  for (int k = 0; k < nb; k++) {
+                     const double *Rk = R + k * nh;
+                     double v = xs[5 * k + dir] * Rk[m1] + c * Rk[m2];
+                     if (i == 0 && lane == 0) v = fs[k * Lp1];
+                     acc[i] += v;
+                  }
+               }
+               s += nb;
             }
-            if (ket)
-               for (int e = 0; e <= Lm; e++)
-                  for (int tt = 1; tt <= e; tt += 2) E[e * (e + 1) / 2 + tt] = -E[e * (e + 1) / 2 + tt];
-         }
-         __syncthreads();
-         const int nkc = tp.nkc;
-         // W[tuv][f] = sum E^f_tau E^f_nu E^f_phi R[t+tau, u+nu, v+phi]
-         for (int idx = lane; idx < tp.nbh * nkc; idx += 64) {
-            const uint32_t it = e1[idx];
-            const int tt = it & 7, uu = (it >> 3) & 7, vv = (it >> 6) & 7;
-            const int fx = (it >> 9) & 7, fy = (it >> 12) & 7, fz = (it >> 15) & 7;
-            const double *Fx = Fk + fx * (fx + 1) / 2, *Fy = Fk + 28 + fy * (fy + 1) / 2, *Fz = Fk + 56 + fz * (fz + 1) / 2;
-            double s = 0.0;
-            for (int a = 0; a <= fx; a++)
-               for (int c = 0; c <= fy; c++) {
-                  const double cxy = Fx[a] * Fy[c];
-                  const int t1 = tt + a, u1 = uu + c;
-                  for (int d = 0; d <= fz; d++) {
-                     const int v1 = vv + d, N = t1 + u1 + v1;
-                     const int H = N * (N + 1) * (N + 2) / 6 + (N - t1) * (N - t1 + 1) / 2 + v1;
-                     s += cxy * Fz[d] * sR[H];
-                  }
-               }
-            W[it >> 18] = s;
-         }
-         __syncthreads();
-         // (e0|f0) = sum E^e_t E^e_u E^e_v W[tuv][f]
-         double vmax = 0.0;
-         for (int j = lane; j < tp.ncp; j += 64) {
-            const uint32_t it = e2[j];
-            const int ex = it & 7, ey = (it >> 3) & 7, ez = (it >> 6) & 7, col = (int)((it >> 9) & 127);
-            const double *Ea = Ex + ex * (ex + 1) / 2, *Eb = Ex + 28 + ey * (ey + 1) / 2, *Ec = Ex + 56 + ez * (ez + 1) / 2;
-            double s = 0.0;
-            for (int a = 0; a <= ex; a++)
-               for (int c = 0; c <= ey; c++) {
-                  const double cxy = Ea[a] * Eb[c];
-                  for (int d = 0; d <= ez; d++) {
-                     const int N = a + c + d;
-                     const int H = N * (N + 1) * (N + 2) / 6 + (N - a) * (N - a + 1) / 2 + d;
-                     s += cxy * Ec[d] * W[H * nkc + col];
-                  }
-               }
-            const int jd = (int)(it >> 16);
-            if (!FIX && jd == 0 && tp.has00) s += qsum[q];
-            dst[jd] = s;
-            vmax = fmax(vmax, fabs(s));
-         }
-         if (gm) {
-            for (int off = 32; off > 0; off >>= 1) vmax = fmax(vmax, __shfl_xor(vmax, off, 64));
-            if (lane == 0) atomicMax(gm, (unsigned long long)__double_as_longlong(vmax));
-         }
-         __syncthreads();
+            k0 += SV;
+         } while (k0 < nsv);
       }
 
       if (!FIX && b.stats) {
@@ -710,8 +878,27 @@ void k_fm_r(const BatchDev *__restrict__ batches, const WorkRef *__restrict__ re
          }
       }
    }
-   __syncthreads();   // the next chunk's layout of LDS
    }
+}
+
+// orders 1 .. ldm of the caller's table, as d_cheb_pairs reads them: the
+// orders of one coefficient pair side by side, so that the lanes of a
+// survivor read one or two cache lines
+__global__ void k_pack_c0(const double *__restrict__ C0, int ld_C0, int ldm, double *__restrict__ Cm)
+{
+   const int n = TCG_NPATCH * CM_PAIRS * ldm;
+   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+      const int m = i % ldm, k = i / ldm % CM_PAIRS, p = i / ldm / CM_PAIRS;
+      const double *c = C0 + (size_t)ld_C0 * p + (m + 1) * TCG_NCOEF + 2 * k;
+      Cm[2 * i] = c[0];
+      Cm[2 * i + 1] = 2 * k + 1 < TCG_NCOEF ? c[1] : 0.0;
+   }
+}
+
+int launch_pack_c0(const double *C0, int ld_C0, int ldm, double *Cm, void *stream)
+{
+   hipLaunchKernelGGL(k_pack_c0, dim3(512), dim3(256), 0, (hipStream_t)stream, C0, ld_C0, ldm, Cm);
+   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 // ---------------------------------------------------------------------------
@@ -725,27 +912,26 @@ size_t fm_r_lds_bytes(const TypePlan &tp)
    return (size_t)y.bytes <= LDS_LIMIT ? (size_t)y.bytes : 0;
 }
 
-void fm_layouts(const TypePlan &tp, int Ng, FmLayout &main, FmLayout &fix, bool *pair)
+void fm_layouts(const TypePlan &tp, FmLayout &main, FmLayout &fix)
 {
-   // two primitive quartets per wavefront when each takes at most half of
-   // the lanes' cells and its cell sum fits 4 values per lane
-   const FmLayout yp = fm_layout(tp, false, true);
-   *pair = Ng <= 32 && tp.nh <= 256 && (size_t)yp.bytes <= LDS_LIMIT;
-   main = *pair ? yp : fm_layout(tp, false);
+   main = fm_layout(tp, false);
    fix = fm_layout(tp, true);
 }
 
-int launch_fm_r(const BatchDev *batches, const WorkRef *refs, int nref, uint32_t units, bool pair, size_t lds,
+int launch_fm_r(const BatchDev *batches, const WorkRef *refs, int nref, uint32_t units, int nacc, size_t lds,
                 const DevTables &t, const RunDev &run, void *stream)
 {
    if (!units) return 0;
    if (lds > LDS_LIMIT) return -3;
    // workgroups stay resident and stride over the units
-   const unsigned grid = std::min(units, 16384u);
-   if (pair)
-      hipLaunchKernelGGL((k_fm_r<false, true>), dim3(grid), dim3(64), lds, (hipStream_t)stream, batches, refs, nref, t, run);
-   else
-      hipLaunchKernelGGL((k_fm_r<false, false>), dim3(grid), dim3(64), lds, (hipStream_t)stream, batches, refs, nref, t, run);
+   const dim3 grid(std::min(units, 16384u)), block(64);
+   hipStream_t st = (hipStream_t)stream;
+   switch (nacc) {
+      case 1: hipLaunchKernelGGL((k_fm_r<false, 1>), grid, block, lds, st, batches, refs, nref, t, run); break;
+      case 3: hipLaunchKernelGGL((k_fm_r<false, 3>), grid, block, lds, st, batches, refs, nref, t, run); break;
+      case 8: hipLaunchKernelGGL((k_fm_r<false, 8>), grid, block, lds, st, batches, refs, nref, t, run); break;
+      default: return -3;
+   }
    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -753,7 +939,7 @@ int launch_fixup(const BatchDev *batches, size_t lds, const DevTables &t, const 
 {
    if (lds > LDS_LIMIT) return -3;
    const unsigned grid = std::max(1u, std::min(n_fix, 4096u));
-   hipLaunchKernelGGL((k_fm_r<true, false>), dim3(grid), dim3(64), lds, (hipStream_t)stream, batches,
+   hipLaunchKernelGGL((k_fm_r<true, 8>), dim3(grid), dim3(64), lds, (hipStream_t)stream, batches,
                       (const WorkRef *)nullptr, 0, t, run);
    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -805,7 +991,7 @@ __global__ void k_absmax(const double *__restrict__ P, size_t n, unsigned long l
 __global__ void k_mixed_flags(const BatchDev *__restrict__ batch, RunDev run, const unsigned long long *__restrict__ pmax,
                               double tau, unsigned long long *count)
 {
-   const double *gmag = load_uniform(&batch->gmag);
+   const double *gmag = in_global(load_uniform(&batch->gmag));
    const BatchDev b = load_batch(batch, 0, run);
    const TypePlan &tp = *b.tp;
    const double maxP = __longlong_as_double((long long)*pmax);

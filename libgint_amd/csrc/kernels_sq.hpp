@@ -132,14 +132,6 @@ __device__ __forceinline__ void side_transform(const double *in, const double R[
    });
 }
 
-// Orders the LDS accesses of the workgroup's one wavefront: they execute in
-// program order, so the compiler's order is all it takes
-__device__ __forceinline__ void lds_order()
-{
-   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-   __builtin_amdgcn_wave_barrier();
-}
-
 struct GroupHead {   // the start of GroupRec
    uint32_t row0, row1, R[4];
 };
@@ -404,7 +396,12 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
    const uint32_t end = lane < nref ? refs[lane].end : 0xffffffffu;
    const int ri = __builtin_amdgcn_readfirstlane(__popcll(__ballot(end <= item)));
    if (ri > 0) item -= load_uniform(&refs[ri - 1].end);
-   const SqArgs y = load_uniform(&refs[ri].y);
+   SqArgs y = load_uniform(&refs[ri].y);
+   y.tiles = in_global(y.tiles);
+   y.sps = in_global(y.sps);
+   y.rows = in_global(y.rows);
+   y.rcs = in_global(y.rcs);
+   y.fns = in_global(y.fns);
    const BatchDev b = load_batch(batches, load_uniform(&refs[ri].batch), run);
    const TypePlan &tp = *b.tp;
    const int ncpt = load_uniform(&tp.ncp), nkc = load_uniform(&tp.nkc);

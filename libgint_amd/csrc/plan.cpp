@@ -204,6 +204,17 @@ void make_type_plan(TypePlan &tp)
    p.nbh = nherm(p.LA);
    p.nh = nherm(p.L);
    p.has00 = (p.LA0 == 0 && p.LC0 == 0) ? 1 : 0;
+   // ket components per pass of the transform: about 4 KB of [nbh][FC + 2]
+   p.FC = std::max(4, std::min((p.nkc + 3) & ~3, (512 / p.nbh - 2) & ~3));
+   auto nterms = [](int l0, int l1) {
+      int n = 0;
+      for (int l = l0; l <= l1; l++)
+         for (int lx = l; lx >= 0; lx--)
+            for (int ly = l - lx; ly >= 0; ly--) n += ((lx + 1) * (ly + 1) * (l - lx - ly + 1) + 1) & ~1;
+      return n;
+   };
+   p.nkt = nterms(p.LC0, p.LC);
+   p.nbt = nterms(p.LA0, p.LA);
 
    std::set<int> Lset;
    int k = 0;
@@ -260,7 +271,18 @@ void make_type_plan(TypePlan &tp)
    tp = p;
 }
 
-void make_type_items(const TypePlan &tp, std::vector<uint32_t> &e1, std::vector<uint32_t> &e2)
+// Tables of a type's Hermite -> cartesian transform: a component (ex,ey,ez)
+// has the terms E^ex_a E^ey_b E^ez_d of its one-centre expansion.
+//   items[0 .. nkt)  ket terms: entries e (e + 1) / 2 + a of the three
+//                    directions' E (5 bits each), place << 15 (herm_place),
+//                    bit 31: none, its coefficient is 0
+//   then             nbt bra terms, the place a Hermite triple's index
+//   then             nkc ket components, passes of FC, within a pass by
+//                    falling number of terms: component | first term << 8 |
+//                    terms << 20 (an even number, the last may be 0)
+//   then             the bra components by falling number of terms, likewise
+//   then             the places of the nbh bra Hermite triples
+void make_type_items(const TypePlan &tp, std::vector<uint32_t> &items)
 {
    // cartesian components of shell L in order: lx descending, then ly descending
    auto comps = [](int L) {
@@ -269,34 +291,41 @@ void make_type_items(const TypePlan &tp, std::vector<uint32_t> &e1, std::vector<
          for (int ly = L - lx; ly >= 0; ly--) v.push_back({lx, ly, L - lx - ly});
       return v;
    };
-   std::vector<std::array<int, 3>> ket, bra;
+   auto entry = [](int e, int a) { return (uint32_t)(e * (e + 1) / 2 + a); };
+   std::vector<std::array<int, 3>> ket, bra, herm;
    for (int f = tp.LC0; f <= tp.LC; f++)
       for (auto &c : comps(f)) ket.push_back(c);
+   for (int e = tp.LA0; e <= tp.LA; e++)
+      for (auto &c : comps(e)) bra.push_back(c);
    for (int N = 0; N <= tp.LA; N++)
-      for (auto &h : comps(N)) bra.push_back(h);
-   // stage 1, W[h][kc] = sum over the ket E of R: ket component outer, so the
-   // lanes of a wavefront share their loop bounds (fx, fy, fz)
-   e1.clear();
-   const int nkc = (int)ket.size();
-   for (int kc = 0; kc < nkc; kc++)
-      for (int h = 0; h < (int)bra.size(); h++) {
-         const auto &t = bra[h], &c = ket[kc];
-         e1.push_back((uint32_t)t[0] | (uint32_t)t[1] << 3 | (uint32_t)t[2] << 6 | (uint32_t)c[0] << 9 |
-                      (uint32_t)c[1] << 12 | (uint32_t)c[2] << 15 | (uint32_t)(h * nkc + kc) << 18);
+      for (auto &h : comps(N)) herm.push_back(h);
+   items.clear();
+   std::vector<uint32_t> rec[2];
+   for (int side = 0; side < 2; side++) {
+      const size_t first = items.size();
+      auto &cs = side == 0 ? ket : bra;
+      for (size_t i = 0; i < cs.size(); i++) {
+         const auto &c = cs[i];
+         const size_t start = items.size() - first;
+         for (int a = 0; a <= c[0]; a++)
+            for (int b = 0; b <= c[1]; b++)
+               for (int d = 0; d <= c[2]; d++) {
+                  const int N = a + b + d;
+                  const int place = side == 0 ? herm_place(tp.L, a, b, d)
+                                              : N * (N + 1) * (N + 2) / 6 + (N - a) * (N - a + 1) / 2 + d;
+                  items.push_back(entry(c[0], a) | entry(c[1], b) << 5 | entry(c[2], d) << 10 | (uint32_t)place << 15);
+               }
+         if ((items.size() - first - start) & 1) items.push_back(1u << 31);
+         const size_t n = items.size() - first - start;
+         rec[side].push_back((uint32_t)i | (uint32_t)start << 8 | (uint32_t)n << 20);
       }
-   // stage 2, (e0|f0) = sum over the bra E of W: bra component outer for the
-   // same reason; each item names its destination j in the type's blocks
-   e2.clear();
-   for (int e = tp.LA0; e <= tp.LA; e++) {
-      const auto ce = comps(e);
-      for (int ie = 0; ie < nco(e); ie++)
-         for (int f = tp.LC0; f <= tp.LC; f++)
-            for (int jl = 0; jl < nco(f); jl++) {
-               const int j = (tp.bcoff[e] + ie) * nkc + tp.kcoff[f] + jl;
-               e2.push_back((uint32_t)ce[ie][0] | (uint32_t)ce[ie][1] << 3 | (uint32_t)ce[ie][2] << 6 |
-                            (uint32_t)(tp.kcoff[f] + jl) << 9 | (uint32_t)j << 16);
-            }
    }
+   auto more = [](uint32_t a, uint32_t b) { return a >> 20 > b >> 20; };
+   for (size_t f0 = 0; f0 < ket.size(); f0 += tp.FC)
+      std::stable_sort(rec[0].begin() + f0, rec[0].begin() + std::min(f0 + tp.FC, ket.size()), more);
+   std::stable_sort(rec[1].begin(), rec[1].end(), more);
+   for (auto &r : rec) items.insert(items.end(), r.begin(), r.end());
+   for (auto &h : herm) items.push_back((uint32_t)herm_place(tp.L, h[0], h[1], h[2]));
 }
 
 // The matrix-core contraction of a type (k_eco): its classes of at least

@@ -1,4 +1,5 @@
-// Loads at uniform addresses through the scalar cache, for the kernels.
+// What the kernels of one wavefront per workgroup share: loads at uniform
+// addresses through the scalar cache, the order of LDS accesses.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -24,17 +25,45 @@ __device__ __forceinline__ T load_uniform(const T *p)
    return u.v;
 }
 
+// Orders the LDS accesses of the workgroup's one wavefront: they execute in
+// program order, so the compiler's order is all it takes
+__device__ __forceinline__ void lds_order()
+{
+   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+   __builtin_amdgcn_wave_barrier();
+}
+
+// A pointer to device memory that was itself loaded from memory: without
+// this the compiler takes it for one that may point to LDS and emits flat
+// accesses, which every later wait for LDS waits for too
+template <class T>
+__device__ __forceinline__ T *in_global(T *p)
+{
+   return (T *)(__attribute__((address_space(1))) T *)(uintptr_t)p;
+}
+
 // chunk `id` of a launch, with the execution's buffers
 __device__ __forceinline__ BatchDev load_batch(const BatchDev *batches, uint32_t id, const RunDev &run)
 {
    BatchDev b = load_uniform(batches + id);
-   b.data = run.data;
-   b.ac0 = run.work + b.ac_off;
-   b.eco = run.work + b.eco_off;
-   b.stats = run.stats;
-   b.fix = run.fix;
-   b.fix_count = run.fix_count;
-   b.fix_ws = run.fix_ws;
+   b.tp = in_global(b.tp);
+   b.items = in_global(b.items);
+   b.rows = in_global(b.rows);
+   b.groups = in_global(b.groups);
+   b.prm_row = in_global(b.prm_row);
+   b.prm_ip = in_global(b.prm_ip);
+   b.ksg = in_global(b.ksg);
+   b.kss = in_global(b.kss);
+   b.ksx = in_global(b.ksx);
+   b.gmag = in_global(b.gmag);
+   b.gflag = in_global(b.gflag);
+   b.data = in_global(run.data);
+   b.ac0 = in_global(run.work + b.ac_off);
+   b.eco = in_global(run.work + b.eco_off);
+   b.stats = in_global(run.stats);
+   b.fix = in_global(run.fix);
+   b.fix_count = in_global(run.fix_count);
+   b.fix_ws = in_global(run.fix_ws);
    b.fix_cap = run.fix_cap;
    b.fix_stride = run.fix_stride;
    b.force_fix = run.force_fix;
