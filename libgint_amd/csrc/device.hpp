@@ -330,15 +330,14 @@ struct SqItem {           // one (bra tile, ket tile)
    uint16_t bt, kt;
    uint16_t lds_k, lm;    // its P and K blocks fit in LDS
    int32_t eco_off;       // its class's place in a row of the contraction buffer, or -1: own contraction
-   int32_t o_wc, o_pk, o_c;   // LDS offsets, doubles
+   int32_t o_pk, o_c;     // LDS offsets, doubles
 };
 constexpr int SQ_NW = 16;      // primitive quartets per window (four matrix-core steps)
 constexpr int SQ_MAXROW = 80, SQ_MAXRC = 16, SQ_MAXFN = 56;   // of a tile
 // LDS tables of an item, bytes: ket columns, coefficient offsets of the
-// units, ket functions, window of primitive quartets
+// units, ket functions
 constexpr int SQ_TAB_URB = 2 * SQ_MAXROW, SQ_TAB_URK = SQ_TAB_URB + 4 * SQ_MAXRC,
-              SQ_TAB_FN = SQ_TAB_URK + 4 * SQ_MAXRC, SQ_TAB_IP = SQ_TAB_FN + 4 * SQ_MAXFN,
-              SQ_TAB_BYTES = (SQ_TAB_IP + 4 * SQ_NW + 15) & ~15;
+              SQ_TAB_FN = SQ_TAB_URK + 4 * SQ_MAXRC, SQ_TAB_BYTES = (SQ_TAB_FN + 4 * SQ_MAXFN + 15) & ~15;
 struct SqArgs {
    const SqItem *items;
    const SqTile *tiles;
@@ -347,6 +346,7 @@ struct SqArgs {
    const uint32_t *rcs;    // unit, two words: contraction of the two sets, 8 bits each;
                            // first row | first component << 8 | last + 1 << 16
    const uint32_t *fns;    // function: c | d << 8 (from the tile's ranges) | shell pair << 16
+   const uint16_t *cons;   // contraction of a set (set after set): shell | contraction of it << 8
    int nitem;
    int ncon[4];            // contractions of the four sets
    int o_co;               // LDS offset, doubles, of the coefficients
@@ -359,12 +359,13 @@ struct SqPlan {
    std::vector<SqItem> items;
    std::vector<SqTile> tiles;
    std::vector<SqSp> sps;
-   std::vector<uint16_t> rows;
+   std::vector<uint16_t> rows, cons;
    std::vector<uint32_t> rcs, fns;
    int lm = 0;
-   int lds_bytes = 0;
+   int nsmall = 0;         // items that need at most SQ_SMALL_LDS, the first ones
+   int lds_small = 0, lds_bytes = 0;   // LDS of those and of all
    void *dev = nullptr;    // all tables on the device, one after the other
-   size_t off[6] = {};
+   size_t off[7] = {};
 };
 
 // the K layout of class k of group g
@@ -443,6 +444,12 @@ struct EcoPlan {
 };
 void make_eco_plan(const TypePlan &tp, const std::vector<ClassPlan> &cps, EcoPlan &ep);
 void make_sq_plan(const TypePlan &tp, const EcoPlan &ep, int grp, int nspin, bool eco, SqPlan &sp);
+// k_sq<4>'s items of at most this much LDS (bytes, without the coefficients)
+// are launched apart: a launch takes the LDS of its largest item (48 KB of an
+// (ff|ff) class), three times the mean.  64 molecules in f shells: 20.1 ->
+// 17.0 ms.  Not so the other kernels, whose items come to 17 KB at most: apart
+// they read a set quartet's blocks twice, 47.5 -> 53.2 ms with s to f shells.
+constexpr int SQ_SMALL_LDS = 18 * 1024;
 constexpr int SQ_GROUPS = 3;   // register groups of k_sq's items
 constexpr int SQ_KERNELS = 4;  // k_sq<1..4>: s and p shells; and d; and f with a transform no larger than (dd|'s; any
 int launch_eco(const BatchDev *batch, const RunDev &run, uint32_t nrow, const EcoArgs &e, void *stream);

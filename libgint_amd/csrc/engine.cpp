@@ -1030,6 +1030,7 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
             add(sp->rows);
             add(sp->rcs);
             add(sp->fns);
+            add(sp->cons);
             HIPCHECK(hipMalloc(&sp->dev, all.size()));
             HIPCHECK(hipMemcpy(sp->dev, all.data(), all.size(), hipMemcpyHostToDevice));
          }
@@ -1331,7 +1332,7 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
       auto per_group = [&](uint32_t i) { return (double)(chunk(i).p1 - chunk(i).p0) / (double)(chunk(i).g1 - chunk(i).g0); };
       std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return per_group(a) > per_group(b); });
       for (int sp = 0; sp < 2; sp++) {
-         std::vector<SqRef> sq[SQ_KERNELS];
+         std::vector<SqRef> sq[SQ_KERNELS][2];
          for (uint32_t i : order) {
             const TypeDev &D = devs[ls.chunks[i].first];
             const TypeInfo &ti = info(i);
@@ -1348,23 +1349,33 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
                r.y.rows = (const uint16_t *)((const char *)q.dev + q.off[3]);
                r.y.rcs = (const uint32_t *)((const char *)q.dev + q.off[4]);
                r.y.fns = (const uint32_t *)((const char *)q.dev + q.off[5]);
-               r.y.nitem = (int)q.items.size();
+               r.y.cons = (const uint16_t *)((const char *)q.dev + q.off[6]);
                int ncon = 0;
                for (int x = 0; x < 4; x++) {
                   for (int s = 0; s < ti.plan.nsh[x]; s++) r.y.ncon[x] += ti.plan.nl[x][s];
                   ncon += r.y.ncon[x];
                }
-               r.y.o_co = q.lds_bytes / 8;
-               auto &v = sq[q.lm - 1];
-               ListRef &l = ls.sq[sp][q.lm - 1];
-               l.lds = std::max(l.lds, (size_t)q.lds_bytes + 8 * (size_t)(ncon * D.max_np));
-               const uint64_t end = (v.empty() ? 0ull : v.back().end) + (uint64_t)(chunk(i).g1 - chunk(i).g0) * q.items.size();
-               if (end > 0xffffffffull) fatal("launch set of more than 2^32 quartet items", (long long)end);
-               r.end = (uint32_t)end;
-               v.push_back(r);
+               // a set of little work in one launch (see FM_ONE_LAUNCH)
+               const int nsmall = prm <= FM_ONE_LAUNCH ? 0 : q.nsmall;
+               const SqItem *items = r.y.items;
+               for (int z = 0; z < 2; z++) {
+                  r.y.nitem = z ? nsmall : (int)q.items.size() - nsmall;
+                  if (!r.y.nitem) continue;
+                  r.y.items = items + (z ? 0 : nsmall);
+                  const int bytes = z ? q.lds_small : q.lds_bytes;
+                  r.y.o_co = bytes / 8;
+                  auto &v = sq[q.lm - 1][z];
+                  ListRef &l = ls.sq[sp][q.lm - 1][z];
+                  l.lds = std::max(l.lds, (size_t)bytes + 8 * (size_t)(ncon * D.max_np));
+                  const uint64_t end = (v.empty() ? 0ull : v.back().end) + (uint64_t)(chunk(i).g1 - chunk(i).g0) * r.y.nitem;
+                  if (end > 0xffffffffull) fatal("launch set of more than 2^32 quartet items", (long long)end);
+                  r.end = (uint32_t)end;
+                  v.push_back(r);
+               }
             }
          }
-         for (int k = 0; k < SQ_KERNELS; k++) put(ls.sq[sp][k], sq[k]);
+         for (int k = 0; k < SQ_KERNELS; k++)
+            for (int z = 0; z < 2; z++) put(ls.sq[sp][k][z], sq[k][z]);
       }
    }
    const size_t head = (sizeof(BatchDev) * batches.size() + 15) & ~(size_t)15;
@@ -1372,7 +1383,8 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
    for (LaunchSet &ls : lp.sets) {
       for (ListRef &l : ls.fm) l.off += head;
       for (auto &x : ls.sq)
-         for (ListRef &l : x) l.off += head;
+         for (auto &k : x)
+            for (ListRef &l : k) l.off += head;
    }
    if (total) {
       std::vector<char> all(total, 0);
@@ -1442,24 +1454,25 @@ void Engine::run_set(std::vector<TypeDev> &devs, const LaunchPlan &lp, const Lau
    }
    // debug bit 1: every launch on the main stream, one after the other
    // (kernel durations without overlap, for profiling)
-   const ListRef *sq = ls.sq[kt.nspin - 1];
+   const auto &sq = ls.sq[kt.nspin - 1];
    int nk = 0;
-   for (int k = 0; k < SQ_KERNELS; k++) nk += sq[k].n ? 1 : 0;
+   for (int k = 0; k < SQ_KERNELS; k++) nk += sq[k][0].n || sq[k][1].n ? 1 : 0;
    const bool side = nk > 1 && (debug_ & 2) == 0;
    if (side) {
       ensure_side();
       HIPCHECK(hipEventRecord((hipEvent_t)ev_join_[0], st));
       HIPCHECK(hipStreamWaitEvent((hipStream_t)side_, (hipEvent_t)ev_join_[0], 0));
    }
-   for (int k = SQ_KERNELS - 1; k >= 0; k--) {
-      if (!sq[k].n) continue;
-      void *q = side && k != 1 ? side_ : (void *)st;
-      evb(2, q);
-      ev_key_ = k + 1;
-      rc = launch_sq(batches, (const SqRef *)(lp.dev + sq[k].off), sq[k].n, sq[k].units, k + 1, sq[k].lds, t, w.run, kt, q);
-      if (rc) fatal("sq launch", rc);
-      eve(2, q);
-   }
+   for (int k = SQ_KERNELS - 1; k >= 0; k--)
+      for (const ListRef &l : sq[k]) {
+         if (!l.n) continue;
+         void *q = side && k != 1 ? side_ : (void *)st;
+         evb(2, q);
+         ev_key_ = k + 1;
+         rc = launch_sq(batches, (const SqRef *)(lp.dev + l.off), l.n, l.units, k + 1, l.lds, t, w.run, kt, q);
+         if (rc) fatal("sq launch", rc);
+         eve(2, q);
+      }
    if (side) {
       HIPCHECK(hipEventRecord((hipEvent_t)ev_join_[1], (hipStream_t)side_));
       HIPCHECK(hipStreamWaitEvent(st, (hipEvent_t)ev_join_[1], 0));

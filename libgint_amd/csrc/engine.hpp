@@ -134,7 +134,7 @@ struct LaunchSet {
    size_t n_prm = 0;
    ListRef fm[FM_BUCKETS];                    // k_fm_r
    int fm_nacc[FM_BUCKETS] = {0, 0, 0, 0};
-   ListRef sq[2][SQ_KERNELS];                 // k_sq: [nspin - 1][kernel - 1]
+   ListRef sq[2][SQ_KERNELS][2];              // k_sq: [nspin - 1][kernel - 1][large items, small items]
    size_t fix_lds = 0;
 };
 // The launch sequence of an execution and its tables on the device

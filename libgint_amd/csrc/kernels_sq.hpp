@@ -25,15 +25,23 @@
 // wavefront per workgroup: the phases exchange data through LDS in program
 // order, with no barrier and no wait for loads in flight.
 //
-// One launch per type does what took one launch per class (a wavefront or a
-// workgroup per set quartet and class, the four-index HRR in LDS): 32 waters,
-// 27 cells, 262 k set quartets: 66 ms where those kernels took 250 (serialised,
-// with their matrix-core contraction); one molecule: 0.19 ms for 5.9.  Bound:
-// latency and instruction issue (waits in 55% of the wave cycles, VALU busy in
-// 35%; HBM below 1 TB/s), so tiles are cut small enough (38 rows x 38 columns,
-// 16 KB of LDS) for ten wavefronts per CU: an item's fixed cost is shared by
-// several shell pairs, and an item of every class alone had ten times the
-// instructions per integral.
+// A wavefront or a workgroup per set quartet and class, with the four-index
+// HRR in LDS, took 250 ms for 262 k set quartets (32 waters, 27 cells), items
+// of several shell pairs 66.  What brought that to 43 (MI355X):
+//   - the item's set-up: all of its loads that do not wait for each other at
+//     once, instead of a load after another per shell (28 k -> 12 k cycles)
+//   - the items of a set quartet on one XCD, so that its blocks come from one
+//     L2 (xcd_run: 72 -> 29 GB from memory, 58 -> 46 ms; runs of 16 items 50,
+//     of 512 49; of k_sq<4>'s large items 16 are better, 27.5 for 28.4 ms)
+//   - tiles of at most 42 rows x 32 columns: whole matrix-core tiles of 16
+//     columns, and LDS (17 KB at most) for eight wavefronts per CU or more
+//     (38 x 38: 45.7, 30 x 38: 44.0, 35 x 32: 42.1, but 34 for 29.6 ms in f
+//     shells)
+//   - in the contraction four independent matrix-core chains, with the next
+//     loads in flight (f shells: 58 -> 53 ms) and weights taken per column
+//     from the coefficients, not from a table of the window
+// Bound: latency, at two wavefronts per SIMD (VALU busy 31%, matrix cores
+// 22%; HBM 0.7 TB/s), and matrix-core tiles that few units fill.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -132,16 +140,6 @@ __device__ __forceinline__ void side_transform(const double *in, const double R[
    });
 }
 
-struct GroupHead {   // the start of GroupRec
-   uint32_t row0, row1, R[4];
-};
-struct Vec3 {
-   double v[3];
-};
-struct Cell {
-   double v[18];
-};
-
 // x / d for 0 <= x < 2^22, d >= 1
 __device__ __forceinline__ int fdiv(int x, int d)
 {
@@ -151,6 +149,64 @@ __device__ __forceinline__ int fdiv(int x, int d)
    else if (rem >= d) q++;
    return q;
 }
+
+// Where coefficient i of a set quartet lies in the basis data: the sets'
+// contractions follow each other, np coefficients each
+struct CoefMap {
+   const uint16_t *cons;
+   const uint32_t *Kof;   // [4][MAXSH]
+   int n0, n1, n2;        // first contraction of sets 1 to 3
+   int ob, oc, od;        // their first coefficient
+   int npa, npb, npc, npd;
+};
+__device__ __forceinline__ uint32_t coef_at(const CoefMap m, int i)
+{
+   const int tc = (i >= m.ob) + (i >= m.oc) + (i >= m.od);
+   const int np = tc == 0 ? m.npa : (tc == 1 ? m.npb : (tc == 2 ? m.npc : m.npd));
+   const int x = i - (tc == 0 ? 0 : (tc == 1 ? m.ob : (tc == 2 ? m.oc : m.od)));
+   const int con = fdiv(x, np);
+   const uint32_t c = m.cons[(tc == 0 ? 0 : (tc == 1 ? m.n0 : (tc == 2 ? m.n1 : m.n2))) + con];
+   return m.Kof[tc * MAXSH + (int)(c & 255)] + (c >> 8) * (uint32_t)np + (uint32_t)(x - con * np);
+}
+
+// Where element e of an item's four blocks (ac, ad, bc, bd) lies in P and K
+struct BlockMap {
+   KsSet s;
+   int NC, ND, oad, obc, obd;
+   unsigned ra, rb, rc, rd;   // first function of the tiles on the four centres
+};
+__device__ __forceinline__ size_t block_at(const BlockMap m, int e)
+{
+   const bool bc = e >= m.obc, d = e >= (bc ? m.obd : m.oad);   // rows of b; columns of d
+   const int nc = d ? m.ND : m.NC;
+   const int x = e - (bc ? (d ? m.obd : m.obc) : (d ? m.oad : 0));
+   const unsigned ld = ((bc ? m.s.ld23 : m.s.ld01) >> (d ? 16 : 0)) & 0xffff;
+   const bool tr = (m.s.flags >> ((bc ? 2 : 0) + (d ? 1 : 0))) & 1;
+   const int r = fdiv(x, nc), c = x - r * nc;
+   const size_t base = bc ? (d ? m.s.base[3] : m.s.base[2]) : (d ? m.s.base[1] : m.s.base[0]);
+   return base + (size_t)((bc ? m.rb : m.ra) + r) * (tr ? ld : 1) + (size_t)((d ? m.rd : m.rc) + c) * (tr ? 1 : ld);
+}
+
+// Workgroups go round the eight XCDs, each with its own L2, and the items of a
+// set quartet read the same blocks: runs of 64 items to one XCD
+template <uint32_t RUN>
+__device__ __forceinline__ uint32_t xcd_run(uint32_t w, uint32_t n)
+{
+   constexpr uint32_t XCDS = 8;
+   if (w >= n / (RUN * XCDS) * (RUN * XCDS)) return w;
+   const uint32_t x = w % XCDS, k = w / XCDS;
+   return (k / RUN * XCDS + x) * RUN + k % RUN;
+}
+
+struct GroupHead {   // the start of GroupRec
+   uint32_t row0, row1, R[4];
+};
+struct Vec3 {
+   double v[3];
+};
+struct Cell {
+   double v[18];
+};
 
 __device__ __forceinline__ unsigned blk_at(bool T, unsigned ld, unsigned r, unsigned c) { return T ? r * ld + c : c * ld + r; }
 __device__ __forceinline__ double symm_fac(uint32_t code)
@@ -385,14 +441,14 @@ __device__ __forceinline__ void bra_transform(double *D, int ds, int nfn, const 
 }
 
 template <int LM>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LM == 4 ? 1 : (LM >= 2 ? 3 : 4))))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LM == 4 ? 2 : 3)))
 void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, int nref, uint32_t item0, DevTables t,
           RunDev run, KTargets kt)
 {
    extern __shared__ __align__(16) double lds[];
    const int lane = threadIdx.x;
    // the item's chunk: the first whose items end beyond it
-   uint32_t item = item0 + blockIdx.x;
+   uint32_t item = item0 + xcd_run<LM == 4 ? 16 : 64>(blockIdx.x, gridDim.x);
    const uint32_t end = lane < nref ? refs[lane].end : 0xffffffffu;
    const int ri = __builtin_amdgcn_readfirstlane(__popcll(__ballot(end <= item)));
    if (ri > 0) item -= load_uniform(&refs[ri - 1].end);
@@ -402,6 +458,7 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
    y.rows = in_global(y.rows);
    y.rcs = in_global(y.rcs);
    y.fns = in_global(y.fns);
+   y.cons = in_global(y.cons);
    const BatchDev b = load_batch(batches, load_uniform(&refs[ri].batch), run);
    const TypePlan &tp = *b.tp;
    const int ncpt = load_uniform(&tp.ncp), nkc = load_uniform(&tp.nkc);
@@ -409,7 +466,7 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
    char *tab = (char *)lds;
    uint16_t *tcol = (uint16_t *)tab;
    uint32_t *urb = (uint32_t *)(tab + SQ_TAB_URB), *urk = (uint32_t *)(tab + SQ_TAB_URK);
-   uint32_t *tfn = (uint32_t *)(tab + SQ_TAB_FN), *tip = (uint32_t *)(tab + SQ_TAB_IP);
+   uint32_t *tfn = (uint32_t *)(tab + SQ_TAB_FN);
    double *co = lds + y.o_co;   // the set quartet's coefficients, contraction by contraction
    const int m16 = lane & 15, k4 = lane >> 4;
    {
@@ -418,90 +475,94 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
       const SqTile bt = load_uniform(y.tiles + it.bt), ktl = load_uniform(y.tiles + it.kt);
       const SqSp *bsp = y.sps + bt.sp, *ksp = y.sps + ktl.sp;
       const GroupRec &g = b.groups[gi];
-      const int nfn = ktl.nfn, ncol = ktl.nrow, cs = ncol | 1, ncc = ktl.nrc;
-      double *WC = lds + it.o_wc, *C = lds + it.o_c;
+      const int nfn = ktl.nfn, ncol = ktl.nrow, cs = ncol | 1;
+      double *C = lds + it.o_c;
       lds_order();
       const GroupHead gh = load_uniform((const GroupHead *)&g);
       const uint32_t np4 = load_uniform(&g.np4);
-      // tables of the ket tile; the coefficients of its and the bra tile's units
-      for (int i = lane; i < ncol; i += 64) tcol[i] = y.rows[ktl.row + i];
-      for (int i = lane; i < nfn; i += 64) tfn[i] = y.fns[ktl.fn + i];
-      {
-         int off = 0;
-         for (int tc = 0; tc < 4; tc++) {
-            const int np = ((np4 >> (4 * tc)) & 15) + 1;
-            for (int s = 0; s < tp.nsh[tc]; s++) {
-               const int n = tp.nl[tc][s] * np;
-               const double *src = b.data + load_uniform(&g.Kof[tc][s]);
-               for (int i = lane; i < n; i += 64) co[off + i] = src[i];
-               off += n;
-            }
-         }
-      }
-      {
-         // first coefficient of the sets: their contractions follow each other
-         const int npa = (np4 & 15) + 1, npb = ((np4 >> 4) & 15) + 1, npc = ((np4 >> 8) & 15) + 1,
-                   npd = ((np4 >> 12) & 15) + 1;
-         const int ob = y.ncon[0] * npa, oc = ob + y.ncon[1] * npb, od = oc + y.ncon[2] * npc;
-         if (lane < 2 * SQ_MAXRC) {
-            const bool ket = lane >= SQ_MAXRC;
-            const int un = ket ? lane - SQ_MAXRC : lane;
-            if (un < (ket ? (int)ktl.nrc : (int)bt.nrc)) {
-               const uint32_t rc = y.rcs[2 * ((ket ? ktl.rc : bt.rc) + un)];
-               uint32_t *ur = ket ? urk : urb;
-               ur[un] = (uint32_t)((ket ? oc : 0) + (int)(rc & 255) * (ket ? npc : npa)) |
-                        (uint32_t)((ket ? od : ob) + (int)(rc >> 8) * (ket ? npd : npb)) << 16;
-            }
-         }
-      }
+      // Tables of the ket tile, the units' coefficients, the set quartet's P
+      // blocks: what does not depend on another load first and together, since
+      // an item waited for its set-up longer than it took for most rows (28 k
+      // cycles; the coefficients alone were a load after another per shell).
+      const int npa = (np4 & 15) + 1, npb = ((np4 >> 4) & 15) + 1, npc = ((np4 >> 8) & 15) + 1, npd = ((np4 >> 12) & 15) + 1;
+      const int n0 = y.ncon[0], n1 = n0 + y.ncon[1], n2 = n1 + y.ncon[2];
+      // first coefficient of the sets: contraction after contraction
+      const int ob = y.ncon[0] * npa, oc = ob + y.ncon[1] * npb, od = oc + y.ncon[2] * npc, oe = od + y.ncon[3] * npd;
+      const bool uket = lane >= SQ_MAXRC;   // unit of the lane
+      const int un0 = uket ? lane - SQ_MAXRC : lane;
+      const bool uok = lane < 2 * SQ_MAXRC && un0 < (uket ? (int)ktl.nrc : (int)bt.nrc);
+      const uint16_t vcol = lane < ncol ? y.rows[ktl.row + lane] : (uint16_t)0;
+      const uint32_t vfn = lane < nfn ? y.fns[ktl.fn + lane] : 0u;
+      const uint32_t vrc = uok ? y.rcs[2 * ((uket ? +ktl.rc : +bt.rc) + un0)] : 0u;
       // the units of the lane's matrix-core results (4 r + lane / 16): first
       // row less first component, and the components they have
-      int urow[4];
-      unsigned ulo[4], un_[4];
+      uint32_t vunit[4];
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-         const int un = 4 * r + k4;
-         const uint32_t v = un < bt.nrc ? y.rcs[2 * (bt.rc + un) + 1] : 0u;
-         ulo[r] = (v >> 8) & 255;
-         un_[r] = (v >> 16) - ulo[r];
-         urow[r] = (int)(v & 255) - (int)ulo[r];
-      }
+      for (int r = 0; r < 4; r++) vunit[r] = 4 * r + k4 < bt.nrc ? y.rcs[2 * (bt.rc + 4 * r + k4) + 1] : 0u;
+      const CoefMap cm{y.cons, &g.Kof[0][0], n0, n1, n2, ob, oc, od, npa, npb, npc, npd};
+      uint32_t cat[2];
+#pragma unroll
+      for (int z = 0; z < 2; z++) cat[z] = lane + 64 * z < oe ? coef_at(cm, lane + 64 * z) : 0u;
+      double cv[2];
+#pragma unroll
+      for (int z = 0; z < 2; z++) cv[z] = lane + 64 * z < oe ? b.data[cat[z]] : 0.0;
       const bool setlevel = (load_uniform(&g.ksmode) & KS_SETLEVEL) != 0;
       Upd u{b, kt, tp, g, ksp, lds + it.o_pk, nullptr, tfn, it.lds_k && setlevel, false, bt.n1, bt.n2, ktl.n1, ktl.n2};
       const int nblk = (u.NA + u.NB) * (u.NC + u.ND);
       u.Kl = u.Pl + kt.nspin * nblk;
       double fac = 0.0;
-      // element e of the item's four blocks in P and K
+      // where element e of the item's four blocks lies in P and K
       KsSet kss{};
       if (setlevel) {
          kss = load_uniform(b.kss + load_uniform(&g.ks));
          fac = -symm_fac((kss.flags >> 4) & 7) * kt.hf_fac;
          if (fac == 0.0) return;
       }
-      auto blocks = [&](auto &&f) {
-         auto one = [&](int qb, int e0, int nr, int nc, int r0, int c0) {
-            const unsigned ld = ((qb < 2 ? kss.ld01 : kss.ld23) >> (16 * (qb & 1))) & 0xffff;
-            const bool tr = (kss.flags >> qb) & 1;
-            const unsigned rs = tr ? ld : 1, cst = tr ? 1 : ld;
-            const size_t base = kss.base[qb];
-            for (int e = lane; e < nr * nc; e += 64) {
-               const int r = fdiv(e, nc), c = e - r * nc;
-               f(e0 + e, base + (size_t)(r0 + r) * rs + (size_t)(c0 + c) * cst);
+      const int oad = u.NA * u.NC, obc = oad + u.NA * u.ND, obd = obc + u.NB * u.NC;
+      const BlockMap bm{kss, u.NC, u.ND, oad, obc, obd, bt.r1, bt.r2, ktl.r1, ktl.r2};
+      double pv[2][2];
+#pragma unroll
+      for (int z = 0; z < 2; z++) {
+         pv[z][0] = pv[z][1] = 0.0;
+         if (u.lds && lane + 64 * z < nblk) {
+            const size_t o = block_at(bm, lane + 64 * z);
+            pv[z][0] = kt.P[0][o];
+            if (kt.nspin > 1) pv[z][1] = kt.P[1][o];
+         }
+      }
+      if (lane < ncol) tcol[lane] = vcol;
+      for (int i = lane + 64; i < ncol; i += 64) tcol[i] = y.rows[ktl.row + i];
+      if (lane < nfn) tfn[lane] = vfn;
+      if (uok)
+         (uket ? urk : urb)[un0] = (uint32_t)((uket ? oc : 0) + (int)(vrc & 255) * (uket ? npc : npa)) |
+                                   (uint32_t)((uket ? od : ob) + (int)(vrc >> 8) * (uket ? npd : npb)) << 16;
+      int urow[4];
+      unsigned ulo[4], un_[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+         ulo[r] = (vunit[r] >> 8) & 255;
+         un_[r] = (vunit[r] >> 16) - ulo[r];
+         urow[r] = (int)(vunit[r] & 255) - (int)ulo[r];
+      }
+#pragma unroll
+      for (int z = 0; z < 2; z++)
+         if (lane + 64 * z < oe) co[lane + 64 * z] = cv[z];
+      for (int i = lane + 128; i < oe; i += 64) co[i] = b.data[coef_at(cm, i)];
+      if (u.lds) {
+         for (int sp = 0; sp < kt.nspin; sp++)
+            for (int e = lane; e < nblk; e += 64) u.Kl[sp * nblk + e] = 0.0;
+#pragma unroll
+         for (int z = 0; z < 2; z++)
+            if (lane + 64 * z < nblk) {
+               u.Pl[lane + 64 * z] = pv[z][0];
+               if (kt.nspin > 1) u.Pl[nblk + lane + 64 * z] = pv[z][1];
             }
-         };
-         const int oad = u.NA * u.NC, obc = oad + u.NA * u.ND, obd = obc + u.NB * u.NC;
-         one(0, 0, u.NA, u.NC, bt.r1, ktl.r1);
-         one(1, oad, u.NA, u.ND, bt.r1, ktl.r2);
-         one(2, obc, u.NB, u.NC, bt.r2, ktl.r1);
-         one(3, obd, u.NB, u.ND, bt.r2, ktl.r2);
-      };
-      if (u.lds)
-         blocks([&](int e, size_t o) {
-            for (int sp = 0; sp < kt.nspin; sp++) {
-               u.Pl[sp * nblk + e] = (sp ? kt.P[1] : kt.P[0])[o];
-               u.Kl[sp * nblk + e] = 0.0;
-            }
-         });
+         for (int e = lane + 128; e < nblk; e += 64) {
+            const size_t o = block_at(bm, e);
+            u.Pl[e] = kt.P[0][o];
+            if (kt.nspin > 1) u.Pl[nblk + e] = kt.P[1][o];
+         }
+      }
       lds_order();
       auto wbra = [&](int un, uint32_t ip) { return co[(urb[un] & 0xffff) + (ip & 15)] * co[(urb[un] >> 16) + ((ip >> 4) & 15)]; };
       auto wket = [&](int un, uint32_t ip) {
@@ -548,75 +609,85 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
          } else {
             const uint32_t *IP = b.prm_ip + row.prm_off;
             const double *A0 = b.ac0 + (size_t)(row.prm_off - b.p0) * ncpt + (size_t)bt.comp0 * nkc + ktl.comp0;
+            // the lane's primitive quartet of each step of a window (past its
+            // end: the last one, with weight 0)
+            uint32_t ipn[4];
+            auto exponents = [&](int w0) __attribute__((always_inline)) {
+#pragma unroll
+               for (int z = 0; z < 4; z++) ipn[z] = IP[min(w0 + 4 * z + k4, (int)row.n_prm - 1)];
+            };
+            exponents(0);
             for (int w0 = 0; w0 < (int)row.n_prm; w0 += SQ_NW) {
                const int nw = min(SQ_NW, (int)row.n_prm - w0);
-               lds_order();
-               if (lane < SQ_NW) tip[lane] = lane < nw ? IP[w0 + lane] : 0u;
-               lds_order();
-               for (int i = lane; i < nw * ncc; i += 64) {
-                  const int n = fdiv(i, ncc);
-                  WC[i] = wket(i - n * ncc, tip[n]);
-               }
                double wb[4];
-               int no[4];   // the lane's primitive quartet of each step (past the window: its last, with weight 0)
-#pragma unroll
-               for (int z = 0; z < 4; z++) {
-                  const int n = 4 * z + k4;
-                  wb[z] = (n < nw && m16 < bt.nrc) ? wbra(m16, tip[n]) : 0.0;
-                  no[z] = min(n, nw - 1);
-               }
-               lds_order();
-               const double *Aw = A0 + (size_t)w0 * ncpt;
-               for (int c0 = 0; c0 < ncol; c0 += 16) {
-                  const bool okc = c0 + m16 < ncol;
-                  const uint32_t tc = tcol[okc ? c0 + m16 : 0];
-                  double wc[4];
-                  int ao[4];
+               uint32_t ip[4];
+               int no[4];
+               {
+                  const uint32_t ub = urb[min(m16, bt.nrc - 1)];
 #pragma unroll
                   for (int z = 0; z < 4; z++) {
-                     wc[z] = WC[no[z] * ncc + (int)(tc >> 8)];
-                     ao[z] = no[z] * ncpt + (int)(tc & 255);
+                     ip[z] = ipn[z];
+                     const double v = co[(ub & 0xffff) + (ip[z] & 15)] * co[(ub >> 16) + ((ip[z] >> 4) & 15)];
+                     wb[z] = (4 * z + k4 < nw && m16 < bt.nrc) ? v : 0.0;
+                     no[z] = min(4 * z + k4, nw - 1);
                   }
-                  double *cq[4];
-                  unsigned nq[4];
+               }
+               if (w0 + SQ_NW < (int)row.n_prm) exponents(w0 + SQ_NW);
+               const double *Aw = A0 + (size_t)w0 * ncpt;
+               // 16 columns of a component at a time, SQ_EU components in a
+               // step; the loads of a step are in flight during the one before
+               auto tiles = [&](auto NZ) {
+                  constexpr int nz = decltype(NZ)::value;
+                  double a[SQ_EU][nz], an[SQ_EU][nz];
+                  auto load = [&](double (&x)[SQ_EU][nz], int c0, int e0) {
+                     const int f = (int)(tcol[min(c0 + m16, ncol - 1)] & 255);
 #pragma unroll
-                  for (int q = 0; q < 4; q++) {
-                     cq[q] = C + urow[q] * cs + c0 + m16;
-                     nq[q] = okc ? un_[q] : 0u;
-                  }
-                  // 16 columns of component e after component, SQ_EU at a time
-                  auto tiles = [&](auto NZ) {
-                     constexpr int nz = decltype(NZ)::value;
-                     for (int e0 = 0; e0 < bt.ncomp; e0 += SQ_EU) {
-                        double a[SQ_EU][nz];
+                     for (int v = 0; v < SQ_EU; v++) {
+                        const double *p = Aw + min(e0 + v, (int)bt.ncomp - 1) * nkc;
 #pragma unroll
-                        for (int v = 0; v < SQ_EU; v++) {
-                           const double *p = Aw + min(e0 + v, (int)bt.ncomp - 1) * nkc;
-#pragma unroll
-                           for (int z = 0; z < nz; z++) a[v][z] = p[ao[z]];
-                        }
-#pragma unroll
-                        for (int v = 0; v < SQ_EU; v++) {
-                           const int e = e0 + v;
-                           if (e >= bt.ncomp) break;
-                           dbl4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                           for (int z = 0; z < nz; z++)
-                              acc = __builtin_amdgcn_mfma_f64_16x16x4f64(wb[z], a[v][z] * wc[z], acc, 0, 0, 0);
-#pragma unroll
-                           for (int q = 0; q < 4; q++)
-                              if (4 * q < bt.nrc && (unsigned)e - ulo[q] < nq[q]) {
-                                 double *c = cq[q] + e * cs;
-                                 *c = w0 ? *c + acc[q] : acc[q];
-                              }
-                        }
+                        for (int z = 0; z < nz; z++) x[v][z] = p[no[z] * ncpt + f];
                      }
                   };
-                  if (nw > 12) tiles(std::integral_constant<int, 4>{});
-                  else if (nw > 8) tiles(std::integral_constant<int, 3>{});
-                  else if (nw > 4) tiles(std::integral_constant<int, 2>{});
-                  else tiles(std::integral_constant<int, 1>{});
-               }
+                  load(a, 0, 0);
+                  for (int c0 = 0; c0 < ncol; c0 += 16) {
+                     const bool okc = c0 + m16 < ncol;
+                     const uint32_t uk = urk[tcol[min(c0 + m16, ncol - 1)] >> 8];
+                     double wc[nz];
+#pragma unroll
+                     for (int z = 0; z < nz; z++)
+                        wc[z] = co[(uk & 0xffff) + ((ip[z] >> 8) & 15)] * co[(uk >> 16) + ((ip[z] >> 12) & 15)];
+                     for (int e0 = 0; e0 < bt.ncomp; e0 += SQ_EU) {
+                        const bool lastc = e0 + SQ_EU >= bt.ncomp;
+                        if (!lastc || c0 + 16 < ncol) load(an, lastc ? c0 + 16 : c0, lastc ? 0 : e0 + SQ_EU);
+                        // (past the last component: computed, not stored)
+                        dbl4 acc[SQ_EU];
+#pragma unroll
+                        for (int v = 0; v < SQ_EU; v++) acc[v] = dbl4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                        for (int z = 0; z < nz; z++)
+#pragma unroll
+                           for (int v = 0; v < SQ_EU; v++)
+                              acc[v] = __builtin_amdgcn_mfma_f64_16x16x4f64(wb[z], a[v][z] * wc[z], acc[v], 0, 0, 0);
+#pragma unroll
+                        for (int q = 0; q < 4; q++) {
+                           if (4 * q >= bt.nrc) break;
+                           double *c = C + (urow[q] + e0) * cs + c0 + m16;
+                           const unsigned n = okc ? un_[q] : 0u;
+#pragma unroll
+                           for (int v = 0; v < SQ_EU; v++)
+                              if ((unsigned)(e0 + v) - ulo[q] < n) c[v * cs] = w0 ? c[v * cs] + acc[v][q] : acc[v][q];
+                        }
+#pragma unroll
+                        for (int v = 0; v < SQ_EU; v++)
+#pragma unroll
+                           for (int z = 0; z < nz; z++) a[v][z] = an[v][z];
+                     }
+                  }
+               };
+               if (nw > 12) tiles(std::integral_constant<int, 4>{});
+               else if (nw > 8) tiles(std::integral_constant<int, 3>{});
+               else if (nw > 4) tiles(std::integral_constant<int, 2>{});
+               else tiles(std::integral_constant<int, 1>{});
             }
          }
          // slots of this row whose screening depends on the class
@@ -667,12 +738,13 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
       }
       lds_order();
       if (u.lds)
-         blocks([&](int e, size_t o) {
+         for (int e = lane; e < nblk; e += 64) {
+            const size_t o = block_at(bm, e);
             for (int sp = 0; sp < kt.nspin; sp++) {
                const double v = u.Kl[sp * nblk + e];
                if (v != 0.0) unsafeAtomicAdd(&(sp ? kt.K[1] : kt.K[0])[o], fac * v);
             }
-         });
+         }
    }
 }
 

@@ -482,12 +482,15 @@ void make_sq_plan(const TypePlan &tp, const EcoPlan &ep, int grp, int nspin, boo
    for (int t = 0; t < 4; t++)
       for (int s = 0; s < tp.nsh[t]; s++) lx = std::max(lx, tp.l[t][s]);
    sp.lm = grp ? 2 + grp : (lx <= 1 ? 1 : 2);
+   for (int t = 0; t < 4; t++)
+      for (int s = 0; s < tp.nsh[t]; s++)
+         for (int i = 0; i < tp.nl[t][s]; i++) sp.cons.push_back((uint16_t)(s | i << 8));
    std::vector<int> bra[3], ket[3];
    for (int f = 0; f <= grp; f++) {
-      make_sq_tiles(tp, 0, f, 38, SQ_MAXFN, eco, sp, bra[f]);
-      make_sq_tiles(tp, 1, f, 38, 30, eco, sp, ket[f]);
+      make_sq_tiles(tp, 0, f, 42, SQ_MAXFN, eco, sp, bra[f]);
+      make_sq_tiles(tp, 1, f, 32, 30, eco, sp, ket[f]);
    }
-   int top = 0;
+   std::vector<SqItem> large;
    for (int fb = 0; fb <= grp; fb++)
       for (int fk = 0; fk <= grp; fk++) {
          if (std::max(fb, fk) != grp) continue;
@@ -506,17 +509,18 @@ void make_sq_plan(const TypePlan &tp, const EcoPlan &ep, int grp, int nspin, boo
                const int pk = 2 * nspin * (b.n1 + b.n2) * (k.n1 + k.n2);
                it.lds_k = pk <= 512 * nspin ? 1 : 0;
                int off = SQ_TAB_BYTES / 8;
-               it.o_wc = off;
-               off += SQ_NW * k.nrc;
                it.o_pk = off;
                off += it.lds_k ? pk : 0;
                it.o_c = off;
                off += b.nrow * (k.nrow | 1);
-               top = std::max(top, off);
-               sp.items.push_back(it);
+               const bool small = sp.lm == SQ_KERNELS && 8 * off <= SQ_SMALL_LDS;
+               if (small) sp.lds_small = std::max(sp.lds_small, 8 * off);
+               sp.lds_bytes = std::max(sp.lds_bytes, 8 * off);
+               (small ? sp.items : large).push_back(it);
             }
       }
-   sp.lds_bytes = 8 * top;
+   sp.nsmall = (int)sp.items.size();
+   sp.items.insert(sp.items.end(), large.begin(), large.end());
 }
 
 }  // namespace gint
