@@ -236,6 +236,13 @@ struct FmLayout {
    int bytes;
 };
 
+// Part `part` of `parts` of a set quartet for k_sq: every parts-th window of
+// SQ_NW primitive quartets, counted through its rows
+struct SqSeg {
+   uint32_t group;
+   uint16_t part, parts;
+};
+
 // One chunk of one type's work.  Primitive, row and group indices are
 // absolute within the type's arrays; ac0 and eco are indexed from the
 // chunk's first primitive and first row.  The records of a launch sequence's
@@ -243,6 +250,8 @@ struct FmLayout {
 // launch covers many types) and adds the execution's buffers (RunDev).
 struct BatchDev {
    const TypePlan *tp;        // device copy
+   const SqSeg *segs;         // the chunk's set quartets for k_sq, in parts, by falling work (null: whole, as stored)
+   const uint32_t *rorder;    // its rows by falling work, absolute, for k_eco (null: as stored)
    const uint32_t *items;     // the type's Hermite -> cartesian tables (make_type_items)
    const RowRec *rows;
    const GroupRec *groups;

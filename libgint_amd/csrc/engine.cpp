@@ -82,11 +82,14 @@ void TypeQueue::release()
 
 void TypeDev::release()
 {
-   void *p[9] = {rows, groups, prm_ip, prm_row, ksg, ksx, kss, gmag, gflag};
+   void *p[11] = {rows, groups, prm_ip, prm_row, ksg, ksx, kss, gmag, gflag, segs, rorder};
    for (void *x : p)
       if (x) (void)hipFree(x);
    gmag = nullptr;
    gflag = nullptr;
+   segs = nullptr;
+   rorder = nullptr;
+   ordered = false;
    rows = nullptr;
    groups = nullptr;
    prm_ip = prm_row = nullptr;
@@ -1122,6 +1125,49 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
          if (c.g1 > c.g0) out.push_back(c);
       };
       make_chunks(work, D.chunks, true);
+      // The work of set quartets and rows spans three orders of magnitude (7
+      // primitive quartets in the middle, 4096 to 16384 at the top): in the
+      // order of the stream the largest start at any time and a launch ends
+      // on a few of them.  Parts of about SEG_PRM, by falling work within
+      // each chunk (to a factor 2):
+      D.ordered = D.n_prm > ORDER_MIN_PRM;
+      if (D.ordered) {
+         std::vector<SqSeg> segs, sorted;
+         std::vector<uint32_t> rorder;
+         // out[first[class]++] = x: classes of falling work
+         auto by_work = [](auto &out, const auto &in, auto &&work) {
+            size_t first[33] = {};
+            for (const auto &x : in) first[__builtin_clz(work(x) | 1)]++;
+            size_t at = out.size();
+            out.resize(at + in.size());
+            for (size_t &f : first) {
+               const size_t n = f;
+               f = at;
+               at += n;
+            }
+            for (const auto &x : in) out[first[__builtin_clz(work(x) | 1)]++] = x;
+         };
+         std::vector<uint32_t> gp(D.n_groups, 0), rows;
+         for (size_t g = 0; g < D.n_groups; g++)
+            for (uint32_t r = Q.groups[g].row0; r < Q.groups[g].row1; r++) gp[g] += Q.rows[r].n_prm;
+         for (Chunk &c : D.chunks) {
+            segs.clear();
+            for (uint32_t g = c.g0; g < c.g1; g++) {
+               const uint32_t parts = gp[g] <= 2 * SEG_PRM ? 1 : std::min(1024u, (gp[g] + SEG_PRM - 1) / SEG_PRM);
+               for (uint32_t k = 0; k < parts; k++) segs.push_back(SqSeg{g, (uint16_t)k, (uint16_t)parts});
+            }
+            c.s0 = (uint32_t)sorted.size();
+            by_work(sorted, segs, [&](const SqSeg &x) { return gp[x.group] / x.parts; });
+            c.s1 = (uint32_t)sorted.size();
+            if (D.eco) {
+               rows.clear();
+               for (uint32_t r = c.r0; r < c.r1; r++) rows.push_back(r);
+               by_work(rorder, rows, [&](uint32_t r) { return (uint32_t)Q.rows[r].n_prm; });
+            }
+         }
+         dev_put(D.segs, D.cap[7], sorted);
+         if (D.eco) dev_put(D.rorder, D.cap[8], rorder);
+      }
       D.chunks_na.clear();
       D.na_fit = D.max_group_bytes <= NOALLOC_AC0_BYTES;
       if (D.na_fit) make_chunks(NOALLOC_AC0_BYTES, D.chunks_na, false);
@@ -1265,6 +1311,8 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
          b.prm_ip = D.prm_ip;
          b.ksg = D.ksg;
          b.kss = D.kss;
+         b.segs = !na && D.ordered ? D.segs + c.s0 : nullptr;
+         b.rorder = !na && D.ordered && D.eco ? D.rorder : nullptr;
          b.ksx = D.ksx;
          b.ac_off = ls.doubles;
          b.eco_off = ls.doubles + blocks;
@@ -1329,8 +1377,8 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
          ls.fm[k].lds = std::max(ls.fm[k].lds, (size_t)lay.bytes);
       }
       for (int x = 0; x < FM_BUCKETS; x++) put(ls.fm[x], fm[x]);
-      auto per_group = [&](uint32_t i) { return (double)(chunk(i).p1 - chunk(i).p0) / (double)(chunk(i).g1 - chunk(i).g0); };
-      std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return per_group(a) > per_group(b); });
+      auto largest = [&](uint32_t i) { return devs[ls.chunks[i].first].max_group_bytes; };
+      std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return largest(a) > largest(b); });
       for (int sp = 0; sp < 2; sp++) {
          std::vector<SqRef> sq[SQ_KERNELS][2];
          for (uint32_t i : order) {
@@ -1355,6 +1403,7 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
                   for (int s = 0; s < ti.plan.nsh[x]; s++) r.y.ncon[x] += ti.plan.nl[x][s];
                   ncon += r.y.ncon[x];
                }
+               const uint32_t nseg = !na && D.ordered ? chunk(i).s1 - chunk(i).s0 : chunk(i).g1 - chunk(i).g0;
                // a set of little work in one launch (see FM_ONE_LAUNCH)
                const int nsmall = prm <= FM_ONE_LAUNCH ? 0 : q.nsmall;
                const SqItem *items = r.y.items;
@@ -1367,7 +1416,7 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
                   auto &v = sq[q.lm - 1][z];
                   ListRef &l = ls.sq[sp][q.lm - 1][z];
                   l.lds = std::max(l.lds, (size_t)bytes + 8 * (size_t)(ncon * D.max_np));
-                  const uint64_t end = (v.empty() ? 0ull : v.back().end) + (uint64_t)(chunk(i).g1 - chunk(i).g0) * r.y.nitem;
+                  const uint64_t end = (v.empty() ? 0ull : v.back().end) + (uint64_t)nseg * r.y.nitem;
                   if (end > 0xffffffffull) fatal("launch set of more than 2^32 quartet items", (long long)end);
                   r.end = (uint32_t)end;
                   v.push_back(r);
@@ -1712,7 +1761,7 @@ uint64_t Engine::device_bytes() const
    uint64_t b = 0;
    for (const auto &d : plan_dev_)
       b += d.cap[0] * sizeof(RowRec) + d.cap[1] * sizeof(GroupRec) + d.cap[2] * 4 + d.cap[3] * 4 +
-           d.cap[4] * sizeof(KsGroup) + d.cap[5] * sizeof(KsRec) + d.cap[6] * sizeof(KsSet);
+           d.cap[4] * sizeof(KsGroup) + d.cap[5] * sizeof(KsRec) + d.cap[6] * sizeof(KsSet) + d.cap[7] * sizeof(SqSeg) + d.cap[8] * sizeof(uint32_t);
    b += plan_lp_.cap + plan_na_lp_.cap;
    b += work_bytes_ + fix_cap_ * 8 + fix_ws_cap_ * 8 + d_data_cap_ * 8 + C0_.size() * 8 + (d_Cm_ ? cm_size() * 8 : 0) +
         d_neighs_cap_ * 8;

@@ -63,6 +63,7 @@ struct TypeQueue {
 
 struct Chunk {
    uint32_t g0, g1, r0, r1, p0, p1;
+   uint32_t s0, s1;   // its parts of set quartets in TypeDev::segs
    double k3_flops, eco_flops;
 };
 
@@ -75,7 +76,10 @@ struct TypeDev {
    KsGroup *ksg = nullptr;
    KsSet *kss = nullptr;
    KsRec *ksx = nullptr;
-   size_t cap[7] = {0, 0, 0, 0, 0, 0, 0};   // allocated elements of each array
+   SqSeg *segs = nullptr;                 // set quartets of each chunk in parts, by falling work
+   uint32_t *rorder = nullptr;            // rows of each chunk by falling work (eco)
+   size_t cap[9] = {};                    // allocated elements of each array
+   bool ordered = false;                  // segs (and rorder) are this work's
    size_t n_rows = 0, n_groups = 0, n_prm = 0, n_ksx = 0, n_ksg = 0, n_kss = 0;
    size_t max_group_bytes = 0;            // largest set quartet's primitive blocks
    std::vector<Chunk> chunks;
@@ -118,6 +122,16 @@ constexpr int FM_BUCKETS = 4;
 // primitive quartet: a K-build of 5783 takes 0.5 ms with one to a wavefront,
 // 0.7 with 16; 5 million are done in 19.5 ms by sixteens, in 53.7 by twos
 constexpr uint64_t FM_UNITS = 8192;
+
+// Types of at most this many primitive quartets are not put in order: their
+// kernels are over before an order shows, and it is one more copy per type.
+// 64 molecules and 8 centres with s to f shells, ordered: k_eco 54.5 -> 20.2
+// ms, k_sq 103 -> 93; 32 molecules 42.9 -> 40.4
+constexpr size_t ORDER_MIN_PRM = 2048;
+// primitive quartets of a set quartet's part, for those of more than two
+// parts: a part of 256 is 16 windows, ten times its set-up and K update; with
+// set quartets of up to 16384 whole, 76.5 ms for the same took 93
+constexpr uint32_t SEG_PRM = 256;
 
 // One launch of a launch set: its list of chunks among the set's tables
 struct ListRef {

@@ -40,6 +40,9 @@
 //   - in the contraction four independent matrix-core chains, with the next
 //     loads in flight (f shells: 58 -> 53 ms) and weights taken per column
 //     from the coefficients, not from a table of the window
+//   - large set quartets in parts and by falling work (SqSeg):
+//     no launch ends on a few wavefronts; 93 -> 76 ms where the largest have
+//     16384 primitive quartets
 // Bound: latency, at two wavefronts per SIMD (VALU busy 31%, matrix cores
 // 22%; HBM 0.7 TB/s), and matrix-core tiles that few units fill.
 #pragma once
@@ -185,17 +188,6 @@ __device__ __forceinline__ size_t block_at(const BlockMap m, int e)
    const int r = fdiv(x, nc), c = x - r * nc;
    const size_t base = bc ? (d ? m.s.base[3] : m.s.base[2]) : (d ? m.s.base[1] : m.s.base[0]);
    return base + (size_t)((bc ? m.rb : m.ra) + r) * (tr ? ld : 1) + (size_t)((d ? m.rd : m.rc) + c) * (tr ? 1 : ld);
-}
-
-// Workgroups go round the eight XCDs, each with its own L2, and the items of a
-// set quartet read the same blocks: runs of 64 items to one XCD
-template <uint32_t RUN>
-__device__ __forceinline__ uint32_t xcd_run(uint32_t w, uint32_t n)
-{
-   constexpr uint32_t XCDS = 8;
-   if (w >= n / (RUN * XCDS) * (RUN * XCDS)) return w;
-   const uint32_t x = w % XCDS, k = w / XCDS;
-   return (k / RUN * XCDS + x) * RUN + k % RUN;
 }
 
 struct GroupHead {   // the start of GroupRec
@@ -470,7 +462,13 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
    double *co = lds + y.o_co;   // the set quartet's coefficients, contraction by contraction
    const int m16 = lane & 15, k4 = lane >> 4;
    {
-      const uint32_t gi = b.g0 + item / (uint32_t)y.nitem;
+      SqSeg seg{b.g0 + item / (uint32_t)y.nitem, 0, 1};
+      if (b.segs) seg = load_uniform(b.segs + item / (uint32_t)y.nitem);
+      if (kt.out) {   // integrals of a row are written by one wavefront after the other's
+         if (seg.part) return;
+         seg.parts = 1;
+      }
+      const uint32_t gi = seg.group;
       const SqItem it = load_uniform(y.items + item % (uint32_t)y.nitem);
       const SqTile bt = load_uniform(y.tiles + it.bt), ktl = load_uniform(y.tiles + it.kt);
       const SqSp *bsp = y.sps + bt.sp, *ksp = y.sps + ktl.sp;
@@ -479,6 +477,8 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
       double *C = lds + it.o_c;
       lds_order();
       const GroupHead gh = load_uniform((const GroupHead *)&g);
+      const bool eco = it.eco_off >= 0;   // contracted by k_eco: the parts take whole rows in turn
+      if (eco && seg.part >= gh.row1 - gh.row0) return;
       const uint32_t np4 = load_uniform(&g.np4);
       // Tables of the ket tile, the units' coefficients, the set quartet's P
       // blocks: what does not depend on another load first and together, since
@@ -577,8 +577,20 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
          gint_pbc(Ra.v, Rb.v, cell.v, ABs);
          gint_pbc(Rc.v, Rd.v, cell.v, CDs);
       }
+      int ahead = seg.part;   // windows to the next one of the item's part
+      const int parts = seg.parts;
       for (uint32_t r = gh.row0; r < gh.row1; r++) {
          const RowRec row = load_uniform(b.rows + r);
+         const int nwin = ((int)row.n_prm + SQ_NW - 1) / SQ_NW, win = eco ? 0 : ahead;   // the first one in this row
+         if (eco) {
+            if (parts > 1 && (r - gh.row0) % (uint32_t)parts != seg.part) continue;
+         } else if (parts > 1) {
+            if (win >= nwin) {
+               ahead -= nwin;
+               continue;
+            }
+            ahead = win + fdiv(nwin - win + parts - 1, parts) * parts - nwin;
+         }
          double AB[3], CD[3];
          {
             const Vec3 g1 = load_uniform((const Vec3 *)(t.neighs + 3 * (row.n12 & 0xffff))),
@@ -592,7 +604,7 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
             }
          }
          lds_order();
-         if (it.eco_off >= 0) {
+         if (eco) {
             // contracted on the matrix cores by k_eco: the units of the tile
             // are part of one class's contractions
             const SqSp qb = load_uniform(bsp), qk = load_uniform(ksp);
@@ -616,8 +628,9 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
 #pragma unroll
                for (int z = 0; z < 4; z++) ipn[z] = IP[min(w0 + 4 * z + k4, (int)row.n_prm - 1)];
             };
-            exponents(0);
-            for (int w0 = 0; w0 < (int)row.n_prm; w0 += SQ_NW) {
+            const int wfirst = win * SQ_NW, wstep = parts * SQ_NW;
+            exponents(wfirst);
+            for (int w0 = wfirst; w0 < (int)row.n_prm; w0 += wstep) {
                const int nw = min(SQ_NW, (int)row.n_prm - w0);
                double wb[4];
                uint32_t ip[4];
@@ -632,7 +645,7 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
                      no[z] = min(4 * z + k4, nw - 1);
                   }
                }
-               if (w0 + SQ_NW < (int)row.n_prm) exponents(w0 + SQ_NW);
+               if (w0 + wstep < (int)row.n_prm) exponents(w0 + wstep);
                const double *Aw = A0 + (size_t)w0 * ncpt;
                // 16 columns of a component at a time, SQ_EU components in a
                // step; the loads of a step are in flight during the one before
@@ -675,7 +688,7 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
                            const unsigned n = okc ? un_[q] : 0u;
 #pragma unroll
                            for (int v = 0; v < SQ_EU; v++)
-                              if ((unsigned)(e0 + v) - ulo[q] < n) c[v * cs] = w0 ? c[v * cs] + acc[v][q] : acc[v][q];
+                              if ((unsigned)(e0 + v) - ulo[q] < n) c[v * cs] = w0 != wfirst ? c[v * cs] + acc[v][q] : acc[v][q];
                         }
 #pragma unroll
                         for (int v = 0; v < SQ_EU; v++)
@@ -691,7 +704,7 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
             }
          }
          // slots of this row whose screening depends on the class
-         for (uint32_t e = 0; e < nfix; e++) {
+         for (uint32_t e = 0; e < nfix && win == 0; e++) {
             const uint32_t p = b.fix[2 * e], word = b.fix[2 * e + 1];
             if (word >> 24 != b.id || b.prm_row[p] != r) continue;
             lds_order();

@@ -42,12 +42,25 @@ __device__ __forceinline__ T *in_global(T *p)
    return (T *)(__attribute__((address_space(1))) T *)(uintptr_t)p;
 }
 
+// Workgroups go round the eight XCDs, each with its own L2, and the items of a
+// set quartet read the same blocks: runs of RUN items to one XCD
+template <uint32_t RUN>
+__device__ __forceinline__ uint32_t xcd_run(uint32_t w, uint32_t n)
+{
+   constexpr uint32_t XCDS = 8;
+   if (w >= n / (RUN * XCDS) * (RUN * XCDS)) return w;
+   const uint32_t x = w % XCDS, k = w / XCDS;
+   return (k / RUN * XCDS + x) * RUN + k % RUN;
+}
+
 // chunk `id` of a launch, with the execution's buffers
 __device__ __forceinline__ BatchDev load_batch(const BatchDev *batches, uint32_t id, const RunDev &run)
 {
    BatchDev b = load_uniform(batches + id);
    b.tp = in_global(b.tp);
    b.items = in_global(b.items);
+   b.segs = in_global(b.segs);
+   b.rorder = in_global(b.rorder);
    b.rows = in_global(b.rows);
    b.groups = in_global(b.groups);
    b.prm_row = in_global(b.prm_row);

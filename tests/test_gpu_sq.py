@@ -5,6 +5,8 @@ layout record, one and two spins, shell structures whose sides are one tile,
 several tiles and, with f shells, tiles of a single contraction; the
 contraction in the kernel itself and in its own kernel (debug bits 4 and 3).
 Bar: 1e-10 Ha + 1e-11 max|K|, the K-build's conditioning (test_conditioning)."""
+import functools
+
 import numpy as np
 import pytest
 
@@ -51,8 +53,25 @@ def test_tiles_and_windows(name, debug, spins):
 # most 64 chunks in a set and within half the memory budget
 LAUNCH_SETS = {
     "many_types": (dict(n_water=4, n_tm=2, box_A=8.0, np_max=2, np_tm=2, seed=13), 4096),
+    # set quartets of 1296 primitive quartets, in parts; of one and many rows, with long rows contracted by k_eco
+    "parts_one_row": (dict(n_water=2, box_A=5.0, np_min=6, np_max=6, seed=15), 4096),
+    "parts_many_rows": (dict(n_water=2, box_A=6.0, image_shells=1, np_min=6, np_max=6, basis=1, zmin=0.3, seed=16), 4096),
+    "parts_spdf": (dict(n_water=1, n_tm=1, box_A=5.0, np_min=3, np_max=3, np_tm=7, seed=17), 4096),
     "several_sets_by_memory": (dict(n_water=5, box_A=7.0, np_min=3, np_max=3, seed=14), 64),
 }
+
+
+@functools.cache
+def launch_set_reference(name):
+    from libgint_amd import driver as D
+
+    o = oracle()
+    s = D.System(**LAUNCH_SETS[name][0])
+    st = s.record()
+    P = s.P()
+    Ko, ho = D.kbuild(o, "oracle_", s, st, P=P)
+    o.oracle_destroy_handle(ho)
+    return s, st, P, Ko
 
 
 @pytest.mark.parametrize("flags", [0, 1, 2])
@@ -61,13 +80,9 @@ def test_launch_sets(name, flags):
     """flags: every surviving slot through the fix-up (1), one stream (2)"""
     from libgint_amd import driver as D, load
 
-    lib, o = load(), oracle()
-    cfg, mib = LAUNCH_SETS[name]
-    s = D.System(**cfg)
-    st = s.record()
-    P = s.P()
-    Ko, ho = D.kbuild(o, "oracle_", s, st, P=P)
-    o.oracle_destroy_handle(ho)
+    lib = load()
+    mib = LAUNCH_SETS[name][1]
+    s, st, P, Ko = launch_set_reference(name)
     kmax = np.max(np.abs(Ko))
     for plan in (False, True):
         K, h = D.kbuild(lib, "libgint_", s, st, P=P, plan=plan, debug=flags, max_mem_mib=mib)
