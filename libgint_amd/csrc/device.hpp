@@ -373,7 +373,7 @@ struct SqPlan {
    int lm = 0;
    int nsmall = 0;         // items that need at most SQ_SMALL_LDS, the first ones
    int lds_small = 0, lds_bytes = 0;   // LDS of those and of all
-   void *dev = nullptr;    // all tables on the device, one after the other
+   char *dev = nullptr;    // all tables on the device, one after the other
    size_t off[7] = {};
 };
 

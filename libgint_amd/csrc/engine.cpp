@@ -83,8 +83,12 @@ void TypeQueue::release()
 void TypeDev::release()
 {
    void *p[11] = {rows, groups, prm_ip, prm_row, ksg, ksx, kss, gmag, gflag, segs, rorder};
+   if (in_arena)
+      for (int i = 0; i < 11; i++)
+         if (i != 7 && i != 8) p[i] = nullptr;
    for (void *x : p)
       if (x) (void)hipFree(x);
+   in_arena = false;
    gmag = nullptr;
    gflag = nullptr;
    segs = nullptr;
@@ -100,6 +104,27 @@ void TypeDev::release()
    n_rows = n_groups = n_prm = n_ksx = n_ksg = n_kss = 0;
    max_group_bytes = 0;
    chunks.clear();
+}
+
+void UploadArena::send()
+{
+   if (host.size() > cap) {
+      release();
+      const size_t want = host.size() + host.size() / 2;
+      HIPCHECK(hipMalloc((void **)&dev, want));
+      cap = want;
+   }
+   if (!host.empty()) HIPCHECK(hipMemcpy(dev, host.data(), host.size(), hipMemcpyHostToDevice));
+   for (auto &x : at) *x.first = dev + x.second;
+   host.clear();
+   at.clear();
+}
+
+void UploadArena::release()
+{
+   if (dev) (void)hipFree(dev);
+   dev = nullptr;
+   cap = 0;
 }
 
 void LaunchPlan::release()
@@ -150,17 +175,12 @@ Engine::~Engine()
    drop_graph();
    if (own_stream_ && stream_) (void)hipStreamDestroy((hipStream_t)stream_);
    for (auto &d : stream_dev_) d.release();
+   stream_arena_.release();
    for (auto &d : plan_dev_) d.release();
+   plan_arena_.release();
    for (LaunchPlan *lp : {&stream_lp_, &plan_lp_, &plan_na_lp_}) lp->release();
    for (auto &ti : types_) {
-      if (ti.d_plan) (void)hipFree(ti.d_plan);
-      if (ti.d_items) (void)hipFree(ti.d_items);
-      for (SqPlan *sp = &ti.sq[0][0][0]; sp != &ti.sq[0][0][0] + 4 * SQ_GROUPS; sp++) {
-         if (sp->dev) (void)hipFree(sp->dev);
-      }
-      if (ti.d_srcmaps) (void)hipFree(ti.d_srcmaps);
-      if (ti.d_eco_info) (void)hipFree(ti.d_eco_info);
-      if (ti.d_eco_items) (void)hipFree(ti.d_eco_items);
+      ti.tables.release();
    }
    void *bufs[] = {d_data_, d_C0_, d_Cm_, d_grid_, d_bw_, d_ftab_, d_cell_, d_neighs_, d_work_,
                    d_fix_, d_fix_ws_, d_stats_, d_fixcnt_, d_out_, d_mix_};
@@ -742,7 +762,7 @@ void Engine::dispatch_all()
    if (!any || recording_) return;
    if (!d_P_[0]) fatal("integrals dispatched before set_P", 0);
    synchronize();   // the previous batch no longer reads the device arrays
-   upload(q_, stream_dev_, false);
+   upload(q_, stream_dev_, false, stream_arena_);
    stream_lp_.valid = false;
    for (auto &Q : q_) {
       Q.rows.clear();
@@ -776,8 +796,9 @@ void Engine::plan_end()
    synchronize();
    drop_graph();
    for (auto &d : plan_dev_) d.release();
+   plan_arena_.release();
    plan_dev_.clear();
-   upload(q_, plan_dev_, true);
+   upload(q_, plan_dev_, true, plan_arena_);
    mixed_calibrated_ = false;
    // tables and basis data resident now, so that an execution needs no
    // allocation (plan_execute_noalloc)
@@ -846,6 +867,7 @@ void Engine::plan_clear()
    synchronize();
    drop_graph();
    for (auto &d : plan_dev_) d.release();
+   plan_arena_.release();
    plan_dev_.clear();
    plan_lp_.release();
    plan_na_lp_.release();
@@ -990,33 +1012,42 @@ static void dev_put(T *&ptr, size_t &cap, const std::vector<T> &v)
 
 // Copy the queues to the device and split each type's work into chunks
 // whose primitive blocks and contracted rows fit the work buffer.
-void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool release_host)
+void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool release_host, UploadArena &arena)
 {
+   size_t bytes = 0;
+   for (const TypeQueue &Q : qs)
+      bytes += Q.rows.size() * sizeof(RowRec) + Q.groups.size() * (sizeof(GroupRec) + sizeof(SqSeg)) + Q.prm_ip.size() * 8 +
+               Q.ksg.size() * sizeof(KsGroup) + Q.ksx.size() * sizeof(KsRec) + Q.kss.size() * sizeof(KsSet);
+   const bool gather = bytes <= UploadArena::MAX;
+   if (gather) arena.host.reserve(bytes + bytes / 4 + 16 * 16 * qs.size());
+   auto put = [&](TypeDev &D, auto *&ptr, int i, const auto &v) {
+      if (gather) arena.put(ptr, v);
+      else dev_put(ptr, D.cap[i], v);
+   };
    const size_t work = budget_bytes_ / 2;
    if (devs.size() < qs.size()) devs.resize(qs.size());
    for (size_t ty = 0; ty < qs.size(); ty++) {
       TypeQueue &Q = qs[ty];
       TypeDev &D = devs[ty];
       D.type = (int)ty;
+      if (D.in_arena != gather) {
+         D.release();   // the arrays of the other kind
+         D.in_arena = gather;
+      }
       D.chunks.clear();
       D.chunks_na.clear();
       D.n_groups = D.n_rows = D.n_prm = D.n_ksx = 0;
       if (Q.empty()) continue;
       TypeInfo &ti = types_[ty];
       const TypePlan &tp = ti.plan;
-      if (!ti.d_plan) {
-         HIPCHECK(hipMalloc((void **)&ti.d_plan, sizeof(TypePlan)));
-         HIPCHECK(hipMemcpy(ti.d_plan, &tp, sizeof(TypePlan), hipMemcpyHostToDevice));
-         HIPCHECK(hipMalloc((void **)&ti.d_items, sizeof(uint32_t) * ti.items.size()));
-         HIPCHECK(hipMemcpy(ti.d_items, ti.items.data(), sizeof(uint32_t) * ti.items.size(), hipMemcpyHostToDevice));
-         auto put = [](auto *&dst, const auto &v) {
-            if (v.empty()) return;
-            HIPCHECK(hipMalloc((void **)&dst, sizeof(v[0]) * v.size()));
-            HIPCHECK(hipMemcpy(dst, v.data(), sizeof(v[0]) * v.size(), hipMemcpyHostToDevice));
-         };
-         put(ti.d_srcmaps, ti.eco.srcmaps);
-         put(ti.d_eco_info, ti.eco.info);
-         put(ti.d_eco_items, ti.eco.items);
+      if (!ti.tables.dev) {
+         // all tables of the type in one allocation and one copy
+         UploadArena &a = ti.tables;
+         a.put(ti.d_plan, std::vector<TypePlan>(1, tp));
+         a.put(ti.d_items, ti.items);
+         a.put(ti.d_srcmaps, ti.eco.srcmaps);
+         a.put(ti.d_eco_info, ti.eco.info);
+         a.put(ti.d_eco_items, ti.eco.items);
          for (SqPlan *sp = &ti.sq[0][0][0]; sp != &ti.sq[0][0][0] + 4 * SQ_GROUPS; sp++) {
             if (sp->items.empty()) continue;
             std::vector<char> all;
@@ -1034,17 +1065,18 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
             add(sp->rcs);
             add(sp->fns);
             add(sp->cons);
-            HIPCHECK(hipMalloc(&sp->dev, all.size()));
-            HIPCHECK(hipMemcpy(sp->dev, all.data(), all.size(), hipMemcpyHostToDevice));
+            a.put(sp->dev, all);
          }
+         a.send();
+         std::vector<char>().swap(a.host);
       }
-      dev_put(D.rows, D.cap[0], Q.rows);
-      dev_put(D.groups, D.cap[1], Q.groups);
-      dev_put(D.prm_ip, D.cap[2], Q.prm_ip);
-      dev_put(D.prm_row, D.cap[3], Q.prm_row);
-      dev_put(D.ksg, D.cap[4], Q.ksg);
-      dev_put(D.ksx, D.cap[5], Q.ksx);
-      dev_put(D.kss, D.cap[6], Q.kss);
+      put(D, D.rows, 0, Q.rows);
+      put(D, D.groups, 1, Q.groups);
+      put(D, D.prm_ip, 2, Q.prm_ip);
+      put(D, D.prm_row, 3, Q.prm_row);
+      put(D, D.ksg, 4, Q.ksg);
+      put(D, D.ksx, 5, Q.ksx);
+      put(D, D.kss, 6, Q.kss);
       D.n_groups = Q.groups.size();
       D.n_rows = Q.rows.size();
       D.n_prm = Q.prm_ip.size();
@@ -1165,8 +1197,8 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
                by_work(rorder, rows, [&](uint32_t r) { return (uint32_t)Q.rows[r].n_prm; });
             }
          }
-         dev_put(D.segs, D.cap[7], sorted);
-         if (D.eco) dev_put(D.rorder, D.cap[8], rorder);
+         put(D, D.segs, 7, sorted);
+         if (D.eco) put(D, D.rorder, 8, rorder);
       }
       D.chunks_na.clear();
       D.na_fit = D.max_group_bytes <= NOALLOC_AC0_BYTES;
@@ -1174,6 +1206,7 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
       n_rows_ += D.n_rows;
       if (release_host) Q.release();
    }
+   if (gather) arena.send();
 }
 
 void Engine::ensure_work(size_t ncp_max, size_t max_prm, size_t bytes)
@@ -1758,7 +1791,7 @@ void Engine::use_private_stream()
 
 uint64_t Engine::device_bytes() const
 {
-   uint64_t b = 0;
+   uint64_t b = plan_arena_.cap;
    for (const auto &d : plan_dev_)
       b += d.cap[0] * sizeof(RowRec) + d.cap[1] * sizeof(GroupRec) + d.cap[2] * 4 + d.cap[3] * 4 +
            d.cap[4] * sizeof(KsGroup) + d.cap[5] * sizeof(KsRec) + d.cap[6] * sizeof(KsSet) + d.cap[7] * sizeof(SqSeg) + d.cap[8] * sizeof(uint32_t);
@@ -1823,6 +1856,7 @@ void Engine::plan_evict()
       }
       D.release();
    }
+   plan_arena_.release();
    plan_dev_.clear();
    mixed_calibrated_ = false;
    plan_lp_.release();
@@ -1840,7 +1874,7 @@ void Engine::plan_evict()
 void Engine::plan_restore()
 {
    if (!evicted_) return;
-   upload(plan_host_, plan_dev_, true);
+   upload(plan_host_, plan_dev_, true, plan_arena_);
    plan_lp_.valid = false;
    build_launches(plan_dev_, true, plan_na_lp_);
    plan_host_.clear();

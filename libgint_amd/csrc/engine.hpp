@@ -67,6 +67,29 @@ struct Chunk {
    double k3_flops, eco_flops;
 };
 
+// The arrays of all types of a dispatch in one device allocation and one
+// copy: seven to nine copies per type took most of a small dispatch (16 types
+// of two or three molecules: 2.7 of 3.7 ms).  Put them, then send.  Work of
+// more than MAX bytes goes array by array: there the copies are the time, and
+// gathering it first would be a second one.
+struct UploadArena {
+   static constexpr size_t MAX = 8 << 20;
+   char *dev = nullptr;
+   size_t cap = 0;
+   std::vector<char> host;
+   std::vector<std::pair<void **, size_t>> at;   // pointers to set, offsets
+   template <class T>
+   void put(T *&ptr, const std::vector<T> &v)
+   {
+      host.resize((host.size() + 15) & ~(size_t)15);
+      at.emplace_back((void **)&ptr, host.size());
+      const char *p = (const char *)v.data();
+      host.insert(host.end(), p, p + sizeof(T) * v.size());
+   }
+   void send();      // the arrays of the last send must no longer be in use
+   void release();
+};
+
 // one type's work on the device
 struct TypeDev {
    int type = -1;
@@ -80,6 +103,7 @@ struct TypeDev {
    uint32_t *rorder = nullptr;            // rows of each chunk by falling work (eco)
    size_t cap[9] = {};                    // allocated elements of each array
    bool ordered = false;                  // segs (and rorder) are this work's
+   bool in_arena = false;                 // the arrays lie in an UploadArena, which frees them
    size_t n_rows = 0, n_groups = 0, n_prm = 0, n_ksx = 0, n_ksg = 0, n_kss = 0;
    size_t max_group_bytes = 0;            // largest set quartet's primitive blocks
    std::vector<Chunk> chunks;
@@ -96,6 +120,7 @@ struct TypeDev {
 struct TypeInfo {
    std::array<int, 4> sig;
    TypePlan plan;
+   UploadArena tables;                    // what the pointers to device memory below lie in
    TypePlan *d_plan = nullptr;
    std::vector<uint32_t> items;           // Hermite -> cartesian tables
    uint32_t *d_items = nullptr;
@@ -266,7 +291,7 @@ class Engine {
    int set_sig(int i);
    KsGroup compress(std::vector<KsRec> &calls, const TypePlan &tp, int k, std::vector<KsRec> &ksx);
    bool set_level(const KsGroup *g, const TypePlan &tp, KsSet &s) const;
-   void upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool release_host);
+   void upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool release_host, UploadArena &arena);
    void execute(std::vector<TypeDev> &devs, uint64_t max_index);
    bool prepare_exec(std::vector<TypeDev> &devs, LaunchPlan &lp, uint64_t max_index, RunBufs &w, KTargets &kt, uint64_t n);
    void build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp);
@@ -342,6 +367,7 @@ class Engine {
 
    // device
    std::vector<TypeDev> stream_dev_, plan_dev_;
+   UploadArena stream_arena_, plan_arena_;
    LaunchPlan stream_lp_, plan_lp_, plan_na_lp_;   // the plan's with allocated and with the static scratch
    double *d_data_ = nullptr;
    size_t d_data_cap_ = 0;
