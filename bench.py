@@ -323,11 +323,11 @@ def main():
     nsr = len(range(0, st.n_sets, a.stride * rs))
     log(f"roofline sample (every {a.stride * rs}th set quartet, {nsr}): serialised instrumented step {t_ser:.3f}s; "
         f"kernel ms fm_r {tm[0]:.0f} sq {tm[2]:.0f} fixup {tm[3]:.0f} eco {te[0]:.0f}")
-    for cat, nm in ((0, "fm_r by type L"), (2, "sq by type L"), (4, "eco by type L")):
+    for cat, nm in ((2, "sq by kernel"), (4, "eco by type L")):
         det = (C.c_double * 256)()
         lib.libgint_amd_timing_detail(hr, cat, det)
         top = sorted(((det[i], i) for i in range(256) if det[i] > 0), reverse=True)[:12]
-        log(f"{nm}: " + ", ".join(f"L{i} {ms:.0f}ms" for ms, i in top))
+        log(f"{nm}: " + ", ".join(f"{i} {ms:.0f}ms" for ms, i in top))
     lib.libgint_amd_destroy_handle(hr)
     value = slots / (tot / a.steps) if a.steps else None
     names = ["fm_r", "sq", "fixup", "eco"]
