@@ -459,6 +459,7 @@ void make_sq_plan(const TypePlan &tp, const EcoPlan &ep, int grp, int nspin, boo
 // 17.0 ms.  Not so the other kernels, whose items come to 17 KB at most: apart
 // they read a set quartet's blocks twice, 47.5 -> 53.2 ms with s to f shells.
 constexpr int SQ_SMALL_LDS = 18 * 1024;
+constexpr size_t SQ_TYPE_LDS = 13 * 1024 + 256;   // twelve wavefronts per CU, what k_sq<1..3>'s registers allow
 constexpr int SQ_GROUPS = 3;   // register groups of k_sq's items
 constexpr int SQ_KERNELS = 4;  // k_sq<1..4>: s and p shells; and d; and f with a transform no larger than (dd|'s; any
 int launch_eco(const BatchDev *batch, const RunDev &run, uint32_t nrow, const EcoArgs &e, void *stream);

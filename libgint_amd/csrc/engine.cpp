@@ -1446,9 +1446,12 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
                   r.y.items = items + (z ? 0 : nsmall);
                   const int bytes = z ? q.lds_small : q.lds_bytes;
                   r.y.o_co = bytes / 8;
-                  auto &v = sq[q.lm - 1][z];
-                  ListRef &l = ls.sq[sp][q.lm - 1][z];
-                  l.lds = std::max(l.lds, (size_t)bytes + 8 * (size_t)(ncon * D.max_np));
+                  const size_t lds = (size_t)bytes + 8 * (size_t)(ncon * D.max_np);
+                  // a type of little LDS apart, like the small items of k_sq<4>
+                  const int zl = prm > FM_ONE_LAUNCH && q.lm < SQ_KERNELS && lds <= SQ_TYPE_LDS ? 1 : z;
+                  auto &v = sq[q.lm - 1][zl];
+                  ListRef &l = ls.sq[sp][q.lm - 1][zl];
+                  l.lds = std::max(l.lds, lds);
                   const uint64_t end = (v.empty() ? 0ull : v.back().end) + (uint64_t)nseg * r.y.nitem;
                   if (end > 0xffffffffull) fatal("launch set of more than 2^32 quartet items", (long long)end);
                   r.end = (uint32_t)end;
