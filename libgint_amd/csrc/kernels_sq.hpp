@@ -6,7 +6,7 @@
 //   contraction      C[unit, e][col] = sum over the primitive quartets n of
 //                    (K_a K_b)[n][unit] (K_c K_d)[n][col] A[n][e][f(col)]
 //                    (reference src/compute_ECO.cpp:12-214) in FP64
-//                    matrix-core tiles: 16 bra units x 16 (e, col) x 4
+//                    matrix-core tiles: 4 or 16 bra units x 16 (e, col) x 4
 //                    primitive quartets; or a copy of the blocks k_eco
 //                    contracted
 //   ket transform    HRR d -> c and cartesian -> spherical of the ket pair
@@ -27,7 +27,7 @@
 //
 // A wavefront or a workgroup per set quartet and class, with the four-index
 // HRR in LDS, took 250 ms for 262 k set quartets (32 waters, 27 cells), items
-// of several shell pairs 66.  What brought that to 43 (MI355X):
+// of several shell pairs 66.  What brought that to 34 (MI355X):
 //   - the item's set-up: all of its loads that do not wait for each other at
 //     once, instead of a load after another per shell (28 k -> 12 k cycles)
 //   - the items of a set quartet on one XCD, so that its blocks come from one
@@ -43,11 +43,13 @@
 //   - large set quartets in parts and by falling work (SqSeg):
 //     no launch ends on a few wavefronts; 93 -> 76 ms where the largest have
 //     16384 primitive quartets
-// Bound: latency, at two wavefronts per SIMD (VALU busy 31%, matrix cores
-// 22%; HBM 0.7 TB/s), and matrix-core tiles that few units fill.
+//   - matrix-core tiles of 4 rows for tiles of at most 8 units (39 -> 34 ms)
+// Bound: latency and instruction issue, at two wavefronts per SIMD (waits in
+// 41% of the wave cycles, VALU busy 34%; HBM 1 TB/s).
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
 #include <utility>
 
 #include "c2s_table.h"
@@ -432,8 +434,11 @@ __device__ __forceinline__ void bra_transform(double *D, int ds, int nfn, const 
    }
 }
 
+// Wavefronts per SIMD: three of the s, p, d kernels (two: 52 ms, four: 51.6
+// for 45.5, spills), two of the f kernels (k_sq<3> 25.3 -> 23.8 ms from three,
+// k_sq<4> 20.1 -> 16.5 from one)
 template <int LM>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LM == 4 ? 2 : 3)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LM >= 3 ? 2 : 3)))
 void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, int nref, uint32_t item0, DevTables t,
           RunDev run, KTargets kt)
 {
@@ -577,6 +582,11 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
          gint_pbc(Ra.v, Rb.v, cell.v, ABs);
          gint_pbc(Rc.v, Rd.v, cell.v, CDs);
       }
+      // at most 8 units: matrix-core tiles of 4 rows, 16 cycles each where one
+      // of 16 rows takes 64; the same lanes hold the same elements of theirs
+      // and of rows 0 to 3 of that.  39.4 -> 33.7 ms for 32 waters, 72.0 ->
+      // 56.9 with s to f shells; for at most 4 units only 34.2 and 57.5
+      const bool few = bt.nrc <= 8;
       int ahead = seg.part;   // windows to the next one of the item's part
       const int parts = seg.parts;
       for (uint32_t r = gh.row0; r < gh.row1; r++) {
@@ -632,24 +642,31 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
             exponents(wfirst);
             for (int w0 = wfirst; w0 < (int)row.n_prm; w0 += wstep) {
                const int nw = min(SQ_NW, (int)row.n_prm - w0);
-               double wb[4];
+               double wb[4], wb1[4];   // weights of the lane's bra unit; of its second one (few units)
                uint32_t ip[4];
                int no[4];
                {
-                  const uint32_t ub = urb[min(m16, bt.nrc - 1)];
+                  auto weights = [&](double (&w)[4], int un) {
+                     const uint32_t ub = urb[min(un, bt.nrc - 1)];
+#pragma unroll
+                     for (int z = 0; z < 4; z++) {
+                        const double v = co[(ub & 0xffff) + (ip[z] & 15)] * co[(ub >> 16) + ((ip[z] >> 4) & 15)];
+                        w[z] = (4 * z + k4 < nw && un < bt.nrc) ? v : 0.0;
+                     }
+                  };
 #pragma unroll
                   for (int z = 0; z < 4; z++) {
                      ip[z] = ipn[z];
-                     const double v = co[(ub & 0xffff) + (ip[z] & 15)] * co[(ub >> 16) + ((ip[z] >> 4) & 15)];
-                     wb[z] = (4 * z + k4 < nw && m16 < bt.nrc) ? v : 0.0;
                      no[z] = min(4 * z + k4, nw - 1);
                   }
+                  weights(wb, few ? lane & 3 : m16);
+                  if (few && bt.nrc > 4) weights(wb1, 4 + (lane & 3));
                }
                if (w0 + wstep < (int)row.n_prm) exponents(w0 + wstep);
                const double *Aw = A0 + (size_t)w0 * ncpt;
                // 16 columns of a component at a time, SQ_EU components in a
                // step; the loads of a step are in flight during the one before
-               auto tiles = [&](auto NZ) {
+               auto tiles = [&](auto NZ, auto FEW) {
                   constexpr int nz = decltype(NZ)::value;
                   double a[SQ_EU][nz], an[SQ_EU][nz];
                   auto load = [&](double (&x)[SQ_EU][nz], int c0, int e0) {
@@ -673,22 +690,51 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
                         const bool lastc = e0 + SQ_EU >= bt.ncomp;
                         if (!lastc || c0 + 16 < ncol) load(an, lastc ? c0 + 16 : c0, lastc ? 0 : e0 + SQ_EU);
                         // (past the last component: computed, not stored)
-                        dbl4 acc[SQ_EU];
-#pragma unroll
-                        for (int v = 0; v < SQ_EU; v++) acc[v] = dbl4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                        for (int z = 0; z < nz; z++)
-#pragma unroll
-                           for (int v = 0; v < SQ_EU; v++)
-                              acc[v] = __builtin_amdgcn_mfma_f64_16x16x4f64(wb[z], a[v][z] * wc[z], acc[v], 0, 0, 0);
-#pragma unroll
-                        for (int q = 0; q < 4; q++) {
-                           if (4 * q >= bt.nrc) break;
+                        auto store = [&](int q, auto &&value) {
                            double *c = C + (urow[q] + e0) * cs + c0 + m16;
                            const unsigned n = okc ? un_[q] : 0u;
 #pragma unroll
                            for (int v = 0; v < SQ_EU; v++)
-                              if ((unsigned)(e0 + v) - ulo[q] < n) c[v * cs] = w0 != wfirst ? c[v * cs] + acc[v][q] : acc[v][q];
+                              if ((unsigned)(e0 + v) - ulo[q] < n) c[v * cs] = w0 != wfirst ? c[v * cs] + value(v) : value(v);
+                        };
+#pragma unroll
+                        for (int v = 0; v < SQ_EU; v++)
+#pragma unroll
+                           for (int z = 0; z < nz; z++) a[v][z] *= wc[z];
+                        if constexpr (decltype(FEW)::value) {
+                           double acc[SQ_EU];
+#pragma unroll
+                           for (int v = 0; v < SQ_EU; v++) acc[v] = 0.0;
+#pragma unroll
+                           for (int z = 0; z < nz; z++)
+#pragma unroll
+                              for (int v = 0; v < SQ_EU; v++)
+                                 acc[v] = __builtin_amdgcn_mfma_f64_4x4x4f64(wb[z], a[v][z], acc[v], 0, 0, 0);
+                           store(0, [&](int v) { return acc[v]; });
+                           if (bt.nrc > 4) {
+#pragma unroll
+                              for (int v = 0; v < SQ_EU; v++) acc[v] = 0.0;
+#pragma unroll
+                              for (int z = 0; z < nz; z++)
+#pragma unroll
+                                 for (int v = 0; v < SQ_EU; v++)
+                                    acc[v] = __builtin_amdgcn_mfma_f64_4x4x4f64(wb1[z], a[v][z], acc[v], 0, 0, 0);
+                              store(1, [&](int v) { return acc[v]; });
+                           }
+                        } else {
+                           dbl4 acc[SQ_EU];
+#pragma unroll
+                           for (int v = 0; v < SQ_EU; v++) acc[v] = dbl4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                           for (int z = 0; z < nz; z++)
+#pragma unroll
+                              for (int v = 0; v < SQ_EU; v++)
+                                 acc[v] = __builtin_amdgcn_mfma_f64_16x16x4f64(wb[z], a[v][z], acc[v], 0, 0, 0);
+#pragma unroll
+                           for (int q = 0; q < 4; q++) {
+                              if (4 * q >= bt.nrc) break;
+                              store(q, [&](int v) { return acc[v][q]; });
+                           }
                         }
 #pragma unroll
                         for (int v = 0; v < SQ_EU; v++)
@@ -697,10 +743,14 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
                      }
                   }
                };
-               if (nw > 12) tiles(std::integral_constant<int, 4>{});
-               else if (nw > 8) tiles(std::integral_constant<int, 3>{});
-               else if (nw > 4) tiles(std::integral_constant<int, 2>{});
-               else tiles(std::integral_constant<int, 1>{});
+               auto windows = [&](auto FEW) {
+                  if (nw > 12) tiles(std::integral_constant<int, 4>{}, FEW);
+                  else if (nw > 8) tiles(std::integral_constant<int, 3>{}, FEW);
+                  else if (nw > 4) tiles(std::integral_constant<int, 2>{}, FEW);
+                  else tiles(std::integral_constant<int, 1>{}, FEW);
+               };
+               if (few) windows(std::true_type{});
+               else windows(std::false_type{});
             }
          }
          // slots of this row whose screening depends on the class
