@@ -44,6 +44,8 @@
 //     no launch ends on a few wavefronts; 93 -> 76 ms where the largest have
 //     16384 primitive quartets
 //   - matrix-core tiles of 4 rows for tiles of at most 8 units (39 -> 34 ms)
+//   - the contraction's loads at a uniform base plus 32 bits per lane instead
+//     of 64-bit addresses (K-build with s to f shells 96.5 -> 95.7 ms)
 // Bound: latency and instruction issue, at two wavefronts per SIMD (waits in
 // 41% of the wave cycles, VALU busy 34%; HBM 1 TB/s).
 #pragma once
@@ -670,12 +672,12 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
                   constexpr int nz = decltype(NZ)::value;
                   double a[SQ_EU][nz], an[SQ_EU][nz];
                   auto load = [&](double (&x)[SQ_EU][nz], int c0, int e0) {
-                     const int f = (int)(tcol[min(c0 + m16, ncol - 1)] & 255);
+                     const uint32_t f = (uint32_t)(tcol[min(c0 + m16, ncol - 1)] & 255);
 #pragma unroll
                      for (int v = 0; v < SQ_EU; v++) {
-                        const double *p = Aw + min(e0 + v, (int)bt.ncomp - 1) * nkc;
+                        const char *p = (const char *)(Aw + min(e0 + v, (int)bt.ncomp - 1) * nkc);
 #pragma unroll
-                        for (int z = 0; z < nz; z++) x[v][z] = p[no[z] * ncpt + f];
+                        for (int z = 0; z < nz; z++) x[v][z] = *(const double *)(p + 8 * ((uint32_t)(no[z] * ncpt) + f));
                      }
                   };
                   load(a, 0, 0);
