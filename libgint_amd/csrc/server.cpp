@@ -260,7 +260,7 @@ class Server {
    void work()
    {
       for (;;) {
-         int64_t id;
+         int64_t id = -1;   // the wait leaves it so when the server stops
          std::vector<int> evict;
          // a copy of the request and pointers to the clients, taken under
          // mu_: indexing a deque while submit / add_client push_back reads
@@ -277,8 +277,7 @@ class Server {
                id = pick(evict);
                return id >= 0;
             });
-            if (stop_ && id < 0) return;
-            if (id < 0) continue;
+            if (id < 0) return;
             reqs_[id].state = 1;
             reqs_[id].start = Clock::now();
             req = reqs_[id];

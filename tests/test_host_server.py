@@ -1,0 +1,19 @@
+"""The request loop without a GPU (tests/host): a server that is destroyed
+while its worker has not come back from the last request."""
+import subprocess
+
+import pytest
+
+import hostlib
+
+
+@pytest.fixture(scope="module")
+def build(tmp_path_factory):
+    return str(tmp_path_factory.mktemp("host"))
+
+
+@pytest.mark.parametrize("requests", [0, 1, 3])
+def test_destroyed_right_after_a_request(build, requests):
+    exe = hostlib.program(build, "server_stop.cpp")
+    r = subprocess.run([exe, str(requests)], capture_output=True, text=True, timeout=20)
+    assert r.returncode == 0 and r.stdout == "stopped\n", (r.returncode, r.stdout, r.stderr)
