@@ -138,10 +138,11 @@ class Server {
       r.K = K;
       r.arrival = Clock::now();
       reqs_.push_back(r);
-      queue_.push_back((int64_t)reqs_.size() - 1);
+      const int64_t id = (int64_t)reqs_.size() - 1;
+      queue_.push_back(id);
       lk.unlock();
       cv_.notify_all();
-      return (int64_t)reqs_.size() - 1;
+      return id;
    }
 
    int wait(int64_t id, double out[3])

@@ -1,26 +1,11 @@
 // A server destroyed as soon as its last request is done: the worker, held up
-// between finishing the request and waiting for the next one (by the wrapper
-// of pthread_cond_broadcast, which its notifications go through), must leave
-// its loop.  argv: requests before the end.
-#include <dlfcn.h>
-#include <pthread.h>
-#include <unistd.h>
-
+// between finishing the request and waiting for the next one, must leave its
+// loop.  argv: requests before the end.
 #include <cstdio>
 #include <cstdlib>
 
 #include "../../include/libGint.h"
-
-static pthread_t g_main;
-
-extern "C" int pthread_cond_broadcast(pthread_cond_t *c)
-{
-   using fn = int (*)(pthread_cond_t *);
-   static const fn real = (fn)dlvsym(RTLD_NEXT, "pthread_cond_broadcast", "GLIBC_2.3.2");
-   const int rc = real(c);
-   if (!pthread_equal(pthread_self(), g_main)) usleep(50000);
-   return rc;
-}
+#include "slow_notify.hpp"
 
 int main(int argc, char **argv)
 {
