@@ -1582,7 +1582,7 @@ bool Engine::prepare_exec(std::vector<TypeDev> &devs, LaunchPlan &lp, uint64_t m
    }
    if (!lp.valid || lp.key != launch_key(false)) {
       HIPCHECK(hipStreamSynchronize((hipStream_t)stream_));   // the tables are no longer read
-      drop_graph();
+      if (&lp == &plan_lp_) drop_graph();                     // it names them
       build_launches(devs, false, lp);
    }
    if (lp.ncp_max == 0) return false;

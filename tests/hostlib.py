@@ -34,3 +34,19 @@ def program(out, source):
     exe = os.path.join(out, source + ".exe")
     _run(["g++"] + FLAGS + [os.path.join(HERE, source)] + objects(out) + ["-o", exe, "-lpthread", "-ldl"])
     return exe
+
+
+def library(out):
+    """them as a library, with the product's entry points declared"""
+    import ctypes as C
+
+    from libgint_amd import ABI
+
+    so = os.path.join(out, "libgint_host.so")
+    if not os.path.exists(so):
+        _run(["g++", "-shared", "-fopenmp"] + objects(out) + ["-o", so])
+    lib = C.CDLL(so)
+    for name, (res, args) in ABI.items():
+        f = getattr(lib, name)
+        f.restype, f.argtypes = res, args
+    return lib

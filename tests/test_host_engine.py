@@ -1,0 +1,44 @@
+"""The host engine without a GPU (tests/host): what a plan keeps while other
+calls come in between."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import hostlib
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    return hostlib.library(str(tmp_path_factory.mktemp("host")))
+
+
+def _planned(lib, **kw):
+    from libgint_amd import driver as D
+
+    s = D.System(**kw)
+    st = s.record()
+    P = s.P()
+    h, table = D.setup_handle(lib, "libgint_", s, P=P)
+    lib.libgint_amd_plan_begin(h)
+    st.replay(table, h)
+    lib.libgint_amd_plan_end(h)
+    return s, st, P, h, table
+
+
+def test_graph_kept_over_streamed_work(lib):
+    """a plan's captured graph serves its next execution also when set
+    quartets were streamed through the handle in between"""
+    from libgint_amd import driver as D
+
+    s, st, P, h, table = _planned(lib, n_water=1, box_A=4.0, np_max=2, seed=2)
+    K = np.zeros(s.P_size)
+    info = (C.c_uint64 * 4)()
+    for _ in range(3):
+        lib.libgint_set_P(h, D._ptr(P), s.P_size)
+        lib.libgint_amd_plan_execute(h)
+        st.replay(table, h, 0, st.n_sets // 2)
+        lib.libgint_get_K(h, D._ptr(K))
+    lib.libgint_amd_graph_info(h, info)
+    lib.libgint_amd_destroy_handle(h)
+    assert list(info) == [1, 1, 3, 1]
