@@ -1739,8 +1739,6 @@ int Engine::plan_execute_noalloc(const double *Pa, const double *Pb, double *Ka,
    if (ncp_max > (size_t)MAX_NCP) return err(-4, "block size beyond the fix-up workspace", (long long)ncp_max);
    char *base = (char *)noalloc_scratch_;
    if (!base) return err(-8, "the no-allocation scratch array has no device address", 0);
-   if (!plan_na_lp_.valid || plan_na_lp_.key != launch_key(true))
-      return err(-6, "lattice vectors changed since libgint_amd_plan_end: record the plan again", 0);
    RunBufs w{};
    w.run.work = (double *)(base + NOALLOC_OFF_AC0);
    w.run.data = d_data_;

@@ -182,7 +182,7 @@ struct LaunchPlan {
    char *dev = nullptr;
    size_t cap = 0, ncp_max = 0, doubles = 0, n_prm = 0;
    bool valid = false;
-   uint64_t key = 0;   // cells and debug bits it was built for
+   uint64_t key = 0;   // launch_key it was built for
    void release();
 };
 
@@ -309,7 +309,9 @@ class Engine {
    bool use_eco(const TypeInfo &ti, const TypeDev &td, bool forced) const;
    DevTables dev_tables() const;
    void ensure_work(size_t ncp_max, size_t max_prm, size_t bytes);
-   uint64_t launch_key(bool na) const { return (uint64_t)neighs_.size() | (uint64_t)(na ? 0 : debug_ & 24) << 32; }
+   // what the launch lists depend on beside the work: forced contractions (the
+   // static scratch's chunks are cut for the rule, so not there)
+   uint64_t launch_key(bool na) const { return na ? 0 : (uint64_t)(debug_ & 24); }
    void ensure_tables();
    void upload_data();
    void harvest_events();

@@ -42,3 +42,26 @@ def test_graph_kept_over_streamed_work(lib):
     lib.libgint_amd_graph_info(h, info)
     lib.libgint_amd_destroy_handle(h)
     assert list(info) == [1, 1, 3, 1]
+
+
+def test_noalloc_after_new_lattice_vectors(lib):
+    """plan_execute_noalloc refuses while new lattice vectors are not on the
+    device, and takes the plan again once plan_execute has put them there"""
+    from libgint_amd import driver as D
+
+    s, st, P, h, table = _planned(lib, n_water=1, box_A=6.0, image_shells=1, np_max=2, seed=2)
+    n = s.P_size
+    dK = np.zeros(n)
+    ptr = lambda a: a.ctypes.data  # noqa: E731
+
+    def noalloc():
+        return lib.libgint_amd_plan_execute_noalloc(h, ptr(P), None, ptr(dK), None, n)
+
+    assert noalloc() == 0
+    g = np.concatenate([s.neighs(), s.neighs() + 1.0])
+    lib.libgint_set_neighs(h, D._ptr(g), 2 * s.Ng)
+    assert noalloc() == -6
+    lib.libgint_set_P(h, D._ptr(P), n)
+    lib.libgint_amd_plan_execute(h)
+    assert noalloc() == 0
+    lib.libgint_amd_destroy_handle(h)
