@@ -189,7 +189,7 @@ void libgint_amd_plan_clear(void *handle);
    (Pb: spin b, or NULL) and the exchange terms ADDED into the caller's
    device array K (Kb), n doubles each (K is not zeroed).  Every scratch
    buffer of the kernels (primitive blocks, fix-up list, class workspace,
-   counters) is carved from one static device array of 176 MiB per GPU,
+   counters) is carved from one static device array of 177 MiB per GPU,
    held until the process ends; the call allocates and frees nothing.  It
    is asynchronous on the handle's stream (libgint_amd_synchronize waits).
    Calls on one GPU share that array, which keeps the last call's contents:
@@ -198,7 +198,7 @@ void libgint_amd_plan_clear(void *handle);
    message on stderr and nothing launched: -1 protocol (recording, no
    libgint_init, an open set quartet), -2 missing arrays, -3 the plan's
    offsets reach beyond n, -4 one set quartet's primitive blocks exceed the
-   array's 130 MiB block region (libgint_amd_plan_execute takes those),
+   array's 162 MiB block region (libgint_amd_plan_execute takes those),
    -5 a class workspace beyond its 32 MiB region, -6 tables or basis data
    changed since libgint_amd_plan_end, -7 the C0 table has too few orders,
    -8 the array has no device address. */

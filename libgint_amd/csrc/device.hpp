@@ -267,16 +267,13 @@ struct BatchDev {
    uint32_t p0, p1;           // primitives of the chunk
    uint32_t r0, r1;           // rows
    uint32_t g0, g1;           // groups
+   uint32_t fix_at, fix_cap;  // its entries of the fix-up list: the first, how many there may be
    FmLayout fm, fix_fm;       // k_fm_r: the chunk's own pass, the fix-up
    // set from RunDev by the kernels
    const double *data;
    double *ac0;               // [primitive - p0][ncp]
    double *eco;
    unsigned long long *stats; // STATS_SLOTS x {surviving (slot, class) pairs, checksum, K1 FLOPs} (nullable)
-   uint32_t *fix;             // mixed-gate slots: (primitive, n3 | mask << 8 | chunk of the launch << 24)
-   uint32_t *fix_count;       // [0] entries, [1] slots beyond fix_cap (kept by every class instead)
-   double *fix_ws;            // fix-up workspace, fix_stride doubles per entry
-   uint32_t fix_cap, fix_stride;
    int force_fix;             // route every surviving slot through the fix-up path (test hook)
    uint32_t id;               // the chunk's number in the launch
 };
@@ -286,14 +283,27 @@ struct RunDev {
    double *work;
    const double *data;
    unsigned long long *stats;
-   uint32_t *fix, *fix_count;
-   double *fix_ws;
-   uint32_t fix_cap, fix_stride;
+   uint32_t *fix;         // fix-up list: FIX_HEAD words, then the entries
+   double *fix_ws;        // its workspace
+   uint32_t fix_doubles;  // doubles of it
    int force_fix;
    int mixed;   // 0 off, 1 calibrate (gmag), 2 route (gflag)
 };
 
 constexpr int MAX_LAUNCH_CHUNKS = 64;   // of one launch
+
+// The fix-up list of a launch set, of the slots that some classes keep and
+// others screen: each chunk has room for FIX_CAP entries of its own
+// (NOALLOC_FIX in the static scratch), and all of them share a workspace that
+// holds as many of the set's largest type.  A slot that finds no room is kept
+// by every class and counted.  An entry: primitive (FIX_VOID: none, the
+// workspace was full), n3 | mask of the classes' L << 8, its first double of
+// ncp + 16 in the workspace.
+constexpr uint32_t FIX_CAP = 4096, FIX_WORDS = 3, FIX_VOID = 0xffffffffu;
+// The words before the entries: [0..63] entries of the set's chunks (may
+// exceed their room), [64, 65] doubles taken, cleared for each set; [66]
+// slots without an entry, cleared when the host has read it
+constexpr int FIX_USED = MAX_LAUNCH_CHUNKS, FIX_CLEAR = FIX_USED + 2, FIX_LOST = FIX_CLEAR, FIX_HEAD = 128;
 
 // A chunk's part of a launch: its units of work end at `end` of the launch's
 // numbering, where the next one's begin.
@@ -404,18 +414,16 @@ GINT_HDI size_t tra_index(int ia, int isa, int ib, int isb, int ic, int isc, int
 
 // The no-allocation executor (libgint_amd_plan_execute_noalloc) takes all
 // its device scratch from one static array of NOALLOC_BYTES per GPU:
-//   [0, 256)                      chunk counters (fix-up entries, overflow)
-//   fix-up list                   NOALLOC_FIX entries of 2 words
-//   fix-up workspace              NOALLOC_FIX x (MAX_NCP + 16) doubles
+//   fix-up list                   its counters, NOALLOC_FIX entries for each chunk of a launch set
+//   fix-up workspace              NOALLOC_FIX x (MAX_NCP + 16) doubles, shared by them
 //   primitive blocks (ac0)        the rest, NOALLOC_AC0_BYTES
-constexpr size_t NOALLOC_BYTES = 176ull << 20;
+constexpr size_t NOALLOC_BYTES = 177ull << 20;
 constexpr int MAX_NCP = 84 * 84;              // (e0|f0) doubles of an (f f|f f) type
 constexpr size_t NOALLOC_FIX = 256;
-constexpr size_t NOALLOC_OFF_FIX = 256;
-constexpr size_t NOALLOC_OFF_FIXWS = NOALLOC_OFF_FIX + ((2 * 4 * NOALLOC_FIX + 255) & ~(size_t)255);
+constexpr size_t NOALLOC_OFF_FIXWS = (4 * (FIX_HEAD + FIX_WORDS * NOALLOC_FIX * MAX_LAUNCH_CHUNKS) + 255) & ~(size_t)255;
 constexpr size_t NOALLOC_OFF_AC0 = NOALLOC_OFF_FIXWS + ((NOALLOC_FIX * (MAX_NCP + 16) * 8 + 255) & ~(size_t)255);
 constexpr size_t NOALLOC_AC0_BYTES = NOALLOC_BYTES - NOALLOC_OFF_AC0;
-static_assert(NOALLOC_AC0_BYTES >= (120ull << 20), "no-allocation scratch layout");
+static_assert(NOALLOC_AC0_BYTES >= (162ull << 20), "no-allocation scratch layout");
 constexpr unsigned STATS_SLOTS = 4096;   // counter triples the kernels spread their statistics over
 
 // address of the no-allocation scratch array on the current device, looked
@@ -432,7 +440,8 @@ int launch_fm_r(const BatchDev *batches, const WorkRef *refs, int nref, uint32_t
                 const DevTables &t, const RunDev &run, void *stream);
 // Hermite functions per lane that k_fm_r takes for a type of nh: 1, 3 or 8
 inline int fm_nacc(int nh) { return nh <= 64 ? 1 : (nh <= 192 ? 3 : 8); }
-int launch_fixup(const BatchDev *batches, size_t lds, const DevTables &t, const RunDev &run, uint32_t n_fix, void *stream);
+int launch_fixup(const BatchDev *batches, int nbatch, size_t lds, const DevTables &t, const RunDev &run, uint32_t n_fix,
+                 void *stream);
 // the layouts of a type and whether k_fm_r takes its primitive quartets in pairs
 void fm_layouts(const TypePlan &tp, FmLayout &main, FmLayout &fix);
 // orders 1 .. ldm of the caller's table in the order that k_fm_r reads them

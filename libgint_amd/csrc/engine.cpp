@@ -183,7 +183,7 @@ Engine::~Engine()
       ti.tables.release();
    }
    void *bufs[] = {d_data_, d_C0_, d_Cm_, d_grid_, d_bw_, d_ftab_, d_cell_, d_neighs_, d_work_,
-                   d_fix_, d_fix_ws_, d_stats_, d_fixcnt_, d_out_, d_mix_};
+                   d_fix_, d_fix_ws_, d_stats_, d_out_, d_mix_};
    for (void *b : bufs)
       if (b) (void)hipFree(b);
    for (void *e : ev_pool_) (void)hipEventDestroy((hipEvent_t)e);
@@ -417,21 +417,25 @@ void Engine::synchronize()
    if (!stream_) return;
    HIPCHECK(hipStreamSynchronize((hipStream_t)stream_));
    harvest_events();
-   if (d_fixcnt_) {
-      // slots whose screening differs between the classes of a type but
-      // found the fix-up list full were kept by every class: an error of at
-      // most their G_0 ~ 1e-12 times the contraction coefficients in K
-      uint32_t c[2];
-      HIPCHECK(hipMemcpy(c, d_fixcnt_, sizeof c, hipMemcpyDeviceToHost));
-      if (c[1]) {
-         if (!fix_overflow_)
-            std::fprintf(stderr, "libgint: %u slots with class-dependent screening beyond the fix-up list of %zu "
-                         "were kept by every class\n", c[1], fix_cap_);
-         fix_overflow_ += c[1];
-         uint32_t z = 0;
-         HIPCHECK(hipMemcpy(d_fixcnt_ + 1, &z, sizeof z, hipMemcpyHostToDevice));
-      }
-   }
+   if (d_fix_) take_fix_lost(d_fix_ + FIX_LOST);
+   if (na_lost_read_) take_fix_lost((uint32_t *)noalloc_scratch_ + FIX_LOST);
+   na_lost_read_ = false;
+}
+
+// slots whose screening differs between the classes of a type but found no
+// room in the fix-up list were kept by every class: an error of at most their
+// G_0 ~ 1e-12 times the contraction coefficients in K
+void Engine::take_fix_lost(uint32_t *word)
+{
+   uint32_t n;
+   HIPCHECK(hipMemcpy(&n, word, sizeof n, hipMemcpyDeviceToHost));
+   if (!n) return;
+   if (!fix_overflow_)
+      std::fprintf(stderr, "libgint: %u slots with class-dependent screening beyond the fix-up list were kept by every "
+                   "class\n", n);
+   fix_overflow_ += n;
+   const uint32_t z = 0;
+   HIPCHECK(hipMemcpy(word, &z, sizeof z, hipMemcpyHostToDevice));
 }
 
 // ---------------------------------------------------------------------------
@@ -806,6 +810,7 @@ void Engine::plan_end()
    upload_data();
    plan_lp_.valid = false;
    build_launches(plan_dev_, true, plan_na_lp_);
+   na_lost_new_ = true;
    pend_bytes_ = 0;
    plan_max_index_ = max_index_;
    max_index_ = 0;
@@ -982,6 +987,7 @@ void Engine::ensure_tables()
    }
    HIPCHECK(hipMemcpy(d_neighs_, neighs_.data(), sizeof(double) * neighs_.size(), hipMemcpyHostToDevice));
    tables_dirty_ = false;
+   na_lost_new_ = true;
 }
 
 void Engine::upload_data()
@@ -1209,11 +1215,11 @@ void Engine::upload(std::vector<TypeQueue> &qs, std::vector<TypeDev> &devs, bool
    if (gather) arena.send();
 }
 
-void Engine::ensure_work(size_t ncp_max, size_t max_prm, size_t bytes)
+void Engine::ensure_work(const LaunchPlan &lp)
 {
    // as large as the largest launch set (at most half the budget, or one set
    // quartet that is larger); grows, never shrinks (plan_evict frees it)
-   const size_t want = std::max<size_t>(bytes, 1 << 20);
+   const size_t want = std::max<size_t>(sizeof(double) * lp.doubles, 1 << 20);
    if (!d_work_ || want > work_bytes_) {
       synchronize();
       if (d_work_) HIPCHECK(hipFree(d_work_));
@@ -1223,23 +1229,19 @@ void Engine::ensure_work(size_t ncp_max, size_t max_prm, size_t bytes)
    if (!d_stats_) {
       HIPCHECK(hipMalloc((void **)&d_stats_, 3 * STATS_SLOTS * sizeof(unsigned long long)));
       HIPCHECK(hipMemset(d_stats_, 0, 3 * STATS_SLOTS * sizeof(unsigned long long)));
-      HIPCHECK(hipMalloc((void **)&d_fixcnt_, 2 * sizeof(uint32_t)));
-      HIPCHECK(hipMemset(d_fixcnt_, 0, 2 * sizeof(uint32_t)));
    }
-   const size_t Ng = neighs_.size() / 3;
-   const size_t cap = (debug_ & 1) ? std::max<size_t>(4096, max_prm * Ng) : 4096;
-   if (cap > fix_cap_) {
+   if (lp.n_fix > fix_cap_) {
       synchronize();
       if (d_fix_) HIPCHECK(hipFree(d_fix_));
-      HIPCHECK(hipMalloc((void **)&d_fix_, 2 * sizeof(uint32_t) * cap));
-      fix_cap_ = cap;
+      HIPCHECK(hipMalloc((void **)&d_fix_, sizeof(uint32_t) * (FIX_HEAD + FIX_WORDS * lp.n_fix)));
+      HIPCHECK(hipMemset(d_fix_, 0, sizeof(uint32_t) * FIX_HEAD));
+      fix_cap_ = lp.n_fix;
    }
-   const size_t ws = fix_cap_ * (ncp_max + 16);
-   if (ws > fix_ws_cap_) {
+   if (lp.fix_doubles > fix_ws_cap_) {
       synchronize();
       if (d_fix_ws_) HIPCHECK(hipFree(d_fix_ws_));
-      HIPCHECK(hipMalloc((void **)&d_fix_ws_, sizeof(double) * ws));
-      fix_ws_cap_ = ws;
+      HIPCHECK(hipMalloc((void **)&d_fix_ws_, sizeof(double) * lp.fix_doubles));
+      fix_ws_cap_ = lp.fix_doubles;
    }
 }
 
@@ -1315,7 +1317,8 @@ bool Engine::use_eco(const TypeInfo &ti, const TypeDev &td, bool forced) const
 void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
 {
    lp.sets.clear();
-   lp.ncp_max = lp.doubles = lp.n_prm = 0;
+   lp.ncp_max = lp.doubles = lp.n_fix = lp.fix_doubles = 0;
+   const bool force_fix = !na && (debug_ & 1);
    const size_t cap = (na ? NOALLOC_AC0_BYTES : budget_bytes_ / 2) / sizeof(double);
    std::vector<BatchDev> batches;
    std::vector<char> lists;   // behind the BatchDevs
@@ -1358,6 +1361,13 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
          b.r1 = c.r1;
          b.g0 = c.g0;
          b.g1 = c.g1;
+         // entries for the fix-up: with every surviving slot through it, as
+         // many as there are slots
+         const size_t slots = (size_t)(c.p1 - c.p0) * (neighs_.size() / 3);
+         b.fix_at = (uint32_t)ls.n_fix;
+         b.fix_cap = na ? (uint32_t)NOALLOC_FIX : (force_fix ? (uint32_t)std::max<size_t>(FIX_CAP, slots) : FIX_CAP);
+         ls.n_fix += b.fix_cap;
+         ls.fix_doubles += (size_t)b.fix_cap * (size_t)(ti.plan.ncp + 16);
          fm_layouts(ti.plan, b.fm, b.fix_fm);
          ls.fix_lds = std::max(ls.fix_lds, (size_t)b.fix_fm.bytes);
          batches.push_back(b);
@@ -1365,9 +1375,12 @@ void Engine::build_launches(std::vector<TypeDev> &devs, bool na, LaunchPlan &lp)
          ls.doubles += need;
          ls.n_prm += c.p1 - c.p0;
          lp.doubles = std::max(lp.doubles, ls.doubles);
-         lp.n_prm = std::max(lp.n_prm, ls.n_prm);
+         lp.n_fix = std::max(lp.n_fix, ls.n_fix);
+         if (force_fix) lp.fix_doubles = std::max(lp.fix_doubles, ls.fix_doubles);
       }
    }
+   if (!force_fix) lp.fix_doubles = FIX_CAP * (lp.ncp_max + 16);
+   lp.fix_doubles = std::min<size_t>(lp.fix_doubles, 0xffffffffu);   // places are 32 bits
    // the lists of each set: the kernels' units of its chunks, in falling
    // order of the work of one unit (the last to start are short)
    auto put = [&](ListRef &l, const auto &v) {
@@ -1495,7 +1508,7 @@ void Engine::run_set(std::vector<TypeDev> &devs, const LaunchPlan &lp, const Lau
    auto evb = [&](int cat, void *q) { if (w.count) ev_begin(cat, q); };
    auto eve = [&](int cat, void *q) { if (w.count) ev_end(cat, q); };
 
-   if (launch_zero_u32(w.run.fix_count, 1, st)) fatal("counter reset launch", 0);
+   if (launch_zero_u32(w.run.fix, FIX_CLEAR, st)) fatal("counter reset launch", 0);
    int rc = 0;
    for (int x = FM_BUCKETS - 1; x >= 0; x--) {
       const ListRef &l = ls.fm[x];
@@ -1506,8 +1519,7 @@ void Engine::run_set(std::vector<TypeDev> &devs, const LaunchPlan &lp, const Lau
       eve(0, st);
    }
    evb(3, st);
-   rc = launch_fixup(batches, ls.fix_lds, t, w.run, w.run.force_fix ? w.run.fix_cap : std::min<uint32_t>(64u, w.run.fix_cap),
-                     st);
+   rc = launch_fixup(batches, (int)ls.chunks.size(), ls.fix_lds, t, w.run, w.run.force_fix ? (uint32_t)ls.n_fix : 64u, st);
    if (rc) fatal("fix-up launch", rc);
    eve(3, st);
    for (size_t i = 0; i < ls.chunks.size(); i++) {
@@ -1586,14 +1598,12 @@ bool Engine::prepare_exec(std::vector<TypeDev> &devs, LaunchPlan &lp, uint64_t m
       build_launches(devs, false, lp);
    }
    if (lp.ncp_max == 0) return false;
-   ensure_work(lp.ncp_max, lp.n_prm, sizeof(double) * lp.doubles);
+   ensure_work(lp);
    w.run.work = d_work_;
    w.run.data = d_data_;
    w.run.fix = d_fix_;
-   w.run.fix_count = d_fixcnt_;
    w.run.fix_ws = d_fix_ws_;
-   w.run.fix_cap = (uint32_t)fix_cap_;
-   w.run.fix_stride = (uint32_t)lp.ncp_max + 16;
+   w.run.fix_doubles = (uint32_t)lp.fix_doubles;
    w.run.stats = stats_on_ ? d_stats_ : nullptr;
    w.run.force_fix = debug_ & 1;
    w.run.mixed = 0;
@@ -1660,8 +1670,8 @@ void Engine::drop_graph()
 
 void Engine::replay_graph(const RunBufs &w, const KTargets &kt)
 {
-   const uint64_t key[] = {(uint64_t)w.run.work, (uint64_t)w.run.fix, (uint64_t)w.run.fix_ws, (uint64_t)w.run.fix_count,
-                           (uint64_t)w.run.fix_cap, (uint64_t)w.run.fix_stride, (uint64_t)plan_lp_.dev,
+   const uint64_t key[] = {(uint64_t)w.run.work, (uint64_t)w.run.fix, (uint64_t)w.run.fix_ws,
+                           (uint64_t)w.run.fix_doubles, (uint64_t)plan_lp_.dev,
                            (uint64_t)kt.P[0], (uint64_t)kt.P[1], (uint64_t)kt.K[0], (uint64_t)kt.K[1],
                            (uint64_t)kt.nspin, graph_bits(kt.hf_fac), (uint64_t)kt.out, (uint64_t)d_data_,
                            (uint64_t)d_C0_, (uint64_t)d_Cm_, (uint64_t)d_neighs_, (uint64_t)neighs_.size(), graph_bits(R_cut_),
@@ -1742,11 +1752,9 @@ int Engine::plan_execute_noalloc(const double *Pa, const double *Pb, double *Ka,
    RunBufs w{};
    w.run.work = (double *)(base + NOALLOC_OFF_AC0);
    w.run.data = d_data_;
-   w.run.fix = (uint32_t *)(base + NOALLOC_OFF_FIX);
-   w.run.fix_count = (uint32_t *)base;
+   w.run.fix = (uint32_t *)base;
    w.run.fix_ws = (double *)(base + NOALLOC_OFF_FIXWS);
-   w.run.fix_cap = (uint32_t)NOALLOC_FIX;
-   w.run.fix_stride = MAX_NCP + 16;
+   w.run.fix_doubles = (uint32_t)(NOALLOC_FIX * (MAX_NCP + 16));
    w.run.force_fix = debug_ & 1;
    w.count = false;
    KTargets kt{};
@@ -1757,8 +1765,8 @@ int Engine::plan_execute_noalloc(const double *Pa, const double *Pb, double *Ka,
    kt.P[1] = Pb;
    kt.K[0] = Ka;
    kt.K[1] = Kb;
-   // the overflow word (it is only read back by the allocating path)
-   if (launch_zero_u32(w.run.fix_count, 2, stream_)) fatal("counter reset launch", 0);
+   na_lost_read_ = na_lost_read_ || na_lost_new_;
+   na_lost_new_ = false;
    for (const LaunchSet &ls : plan_na_lp_.sets) run_set(plan_dev_, plan_na_lp_, ls, w, kt, true);
    return 0;
 }
@@ -1797,7 +1805,7 @@ uint64_t Engine::device_bytes() const
       b += d.cap[0] * sizeof(RowRec) + d.cap[1] * sizeof(GroupRec) + d.cap[2] * 4 + d.cap[3] * 4 +
            d.cap[4] * sizeof(KsGroup) + d.cap[5] * sizeof(KsRec) + d.cap[6] * sizeof(KsSet) + d.cap[7] * sizeof(SqSeg) + d.cap[8] * sizeof(uint32_t);
    b += plan_lp_.cap + plan_na_lp_.cap;
-   b += work_bytes_ + fix_cap_ * 8 + fix_ws_cap_ * 8 + d_data_cap_ * 8 + C0_.size() * 8 + (d_Cm_ ? cm_size() * 8 : 0) +
+   b += work_bytes_ + fix_cap_ * 4 * FIX_WORDS + fix_ws_cap_ * 8 + d_data_cap_ * 8 + C0_.size() * 8 + (d_Cm_ ? cm_size() * 8 : 0) +
         d_neighs_cap_ * 8;
    return b;
 }
@@ -1805,7 +1813,7 @@ uint64_t Engine::device_bytes() const
 uint64_t Engine::work_estimate() const
 {
    // the launch sets of the resident plan: all of its blocks or half the budget
-   size_t ncp_max = 0, all = 0, largest = 0;
+   size_t ncp_max = 0, all = 0, largest = 0, chunks = 0;
    for (const auto &D : plan_dev_) {
       if (D.chunks.empty()) continue;
       const TypeInfo &ti = types_[D.type];
@@ -1814,11 +1822,13 @@ uint64_t Engine::work_estimate() const
          const size_t b = sizeof(double) * ((size_t)(c.p1 - c.p0) * (size_t)ti.plan.ncp +
                                             (size_t)(c.r1 - c.r0) * (D.eco ? ti.eco.row : 0));
          all += b;
+         chunks++;
          largest = std::max(largest, b);
       }
    }
    if (!ncp_max) return 0;
-   return std::max({std::min(all, budget_bytes_ / 2), largest, (size_t)1 << 20}) + 2 * 4 * 4096 + 4096 * (ncp_max + 16) * 8;
+   return std::max({std::min(all, budget_bytes_ / 2), largest, (size_t)1 << 20}) +
+          4 * FIX_WORDS * FIX_CAP * std::min<size_t>(chunks, MAX_LAUNCH_CHUNKS) + FIX_CAP * (ncp_max + 16) * 8;
 }
 
 uint64_t Engine::plan_host_bytes() const

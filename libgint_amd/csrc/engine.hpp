@@ -175,12 +175,13 @@ struct LaunchSet {
    int fm_nacc[FM_BUCKETS] = {0, 0, 0, 0};
    ListRef sq[2][SQ_KERNELS][2];              // k_sq: [nspin - 1][kernel - 1][large items, small items]
    size_t fix_lds = 0;
+   size_t n_fix = 0, fix_doubles = 0;         // fix-up entries; workspace of all of them
 };
 // The launch sequence of an execution and its tables on the device
 struct LaunchPlan {
    std::vector<LaunchSet> sets;
    char *dev = nullptr;
-   size_t cap = 0, ncp_max = 0, doubles = 0, n_prm = 0;
+   size_t cap = 0, ncp_max = 0, doubles = 0, n_fix = 0, fix_doubles = 0;
    bool valid = false;
    uint64_t key = 0;   // launch_key it was built for
    void release();
@@ -240,7 +241,11 @@ class Engine {
    Timing timing();
    void timing_detail(int cat, double out[256]);
    void reset_counters();
-   void set_debug(int flags) { debug_ = flags; }
+   void set_debug(int flags)
+   {
+      debug_ = flags;
+      na_lost_new_ = true;
+   }
    void set_graph(bool on) { graph_on_ = on; }
    void set_autotune(bool) {}
    void set_mixed_precision(double tau) { mixed_tau_ = tau > 0.0 ? tau : 0.0; }
@@ -308,10 +313,15 @@ class Engine {
    }
    bool use_eco(const TypeInfo &ti, const TypeDev &td, bool forced) const;
    DevTables dev_tables() const;
-   void ensure_work(size_t ncp_max, size_t max_prm, size_t bytes);
+   void ensure_work(const LaunchPlan &lp);
+   void take_fix_lost(uint32_t *word);
    // what the launch lists depend on beside the work: forced contractions (the
-   // static scratch's chunks are cut for the rule, so not there)
-   uint64_t launch_key(bool na) const { return na ? 0 : (uint64_t)(debug_ & 24); }
+   // static scratch's chunks are cut for the rule, so not there) and every
+   // slot through the fix-up
+   uint64_t launch_key(bool na) const
+   {
+      return na ? 0 : (uint64_t)(debug_ & 25) | (debug_ & 1 ? (uint64_t)neighs_.size() << 32 : 0);
+   }
    void ensure_tables();
    void upload_data();
    void harvest_events();
@@ -386,8 +396,10 @@ class Engine {
    size_t fix_cap_ = 0, fix_ws_cap_ = 0;
    void *noalloc_scratch_ = nullptr;   // this device's static scratch array (init)
    unsigned long long *d_stats_ = nullptr;   // [0..2] kernel statistics, [3] unused
-   uint32_t *d_fixcnt_ = nullptr;             // [0] entries of the chunk, [1] slots beyond the list (sticky)
-   uint64_t fix_overflow_ = 0;                // such slots seen so far (kept by every class)
+   // the static scratch's lost entries to be read by the next synchronize: once
+   // for a plan and its tables, since its slots do not depend on the density
+   bool na_lost_new_ = true, na_lost_read_ = false;
+   uint64_t fix_overflow_ = 0;                // slots without a fix-up entry so far (kept by every class)
    bool stats_on_ = false;
    uint64_t n_slots_ = 0, n_prmc_ = 0, n_q_ = 0, n_rows_ = 0;
 

@@ -380,12 +380,25 @@ void k_fm_r(const BatchDev *__restrict__ batches, const WorkRef *__restrict__ re
    const int lane = threadIdx.x;
    const unsigned long long below = (1ull << lane) - 1ull;
    uint32_t ubase = 0;
-   const uint32_t nfix = FIX ? min(run.fix_count[0], run.fix_cap) : 0;
-   // (the fix-up: one entry per turn, each with its own chunk)
+   // the fix-up: one entry per turn, those of the set's chunks (nref) one
+   // after the other; lane c holds where chunk c's entries end
+   uint32_t nfix = 0, fix_end = 0;
+   if (FIX) {
+      fix_end = lane < nref ? run.fix[lane] : 0u;
+      if (!__ballot(fix_end != 0u)) return;
+      if (lane < nref) fix_end = min(fix_end, batches[lane].fix_cap);
+      for (int off = 1; off < 64; off <<= 1) {
+         const uint32_t v = __shfl_up(fix_end, off, 64);
+         if (lane >= off) fix_end += v;
+      }
+      nfix = __shfl(fix_end, 63, 64);
+   }
    for (uint32_t turn = FIX ? blockIdx.x : 0; turn < (FIX ? nfix : (uint32_t)nref); turn += FIX ? gridDim.x : 1) {
    uint32_t u0 = turn, nunit = turn + 1, id = 0;
    if (FIX) {
-      id = (uint32_t)__builtin_amdgcn_readfirstlane((int)(run.fix[2 * turn + 1] >> 24));
+      id = (uint32_t)__builtin_amdgcn_readfirstlane(__popcll(__ballot(fix_end <= turn)));
+      if (id) u0 -= (uint32_t)__builtin_amdgcn_readfirstlane((int)__shfl(fix_end, (int)id - 1, 64));
+      nunit = u0 + 1;
    } else {
       // the first unit of the chunk that is this workgroup's
       const WorkRef ref = load_uniform(refs + turn);
@@ -455,9 +468,13 @@ void k_fm_r(const BatchDev *__restrict__ batches, const WorkRef *__restrict__ re
       const int nq = FIX ? 1 : (int)min((uint32_t)NB, b.p1 - b.p0 - w0);
       uint32_t pfirst = b.p0 + w0;
       int fix_n3 = 0;
+      double *fix_out = nullptr;
       if (FIX) {
-         pfirst = b.fix[2 * u];
-         fix_n3 = (int)(b.fix[2 * u + 1] & 0xff);
+         const uint32_t *fe = in_global(run.fix) + FIX_HEAD + FIX_WORDS * (b.fix_at + u);
+         pfirst = fe[0];
+         if (pfirst == FIX_VOID) continue;
+         fix_n3 = (int)(fe[1] & 0xff);
+         fix_out = in_global(run.fix_ws) + fe[2];
       }
       lds_order();
       if (lane < nq) {
@@ -563,7 +580,7 @@ void k_fm_r(const BatchDev *__restrict__ batches, const WorkRef *__restrict__ re
             }
             if (FIX) {
                // per-L Fm[0] of the slot, for the classes that screen it
-               double *f0 = b.fix_ws + (size_t)u * b.fix_stride + ncp;
+               double *f0 = fix_out + ncp;
                for (int i = 0; i < nL; i++) f0[i] = lsens ? gint_boys_f0(tp.Ls[i], T, t.ftable, Kfac) : Fm0;
                status = br == GINT_G_ZERO ? 2 : 1;
             } else if (b.force_fix && status == 1) {
@@ -592,14 +609,23 @@ void k_fm_r(const BatchDev *__restrict__ batches, const WorkRef *__restrict__ re
                      }
                   }
                   if (status == 3) {
-                     const uint32_t idx = atomicAdd(&b.fix_count[0], 1u);
-                     if (idx < b.fix_cap) {
-                        b.fix[2 * idx] = pfirst + q;
-                        b.fix[2 * idx + 1] = (uint32_t)n3 | (mask << 8) | (b.id << 24);
-                     } else {
-                        // list full: every class keeps the slot (its G_0 is
-                        // within rounding of the 1e-12 threshold)
-                        atomicAdd(&b.fix_count[1], 1u);
+                     // (the list's place read here: kept, it costs registers)
+                     const BatchDev *bd = in_global(batches) + here(id);
+                     const uint32_t idx = atomicAdd(run.fix + id, 1u);
+                     bool room = idx < bd->fix_cap;
+                     if (room) {
+                        const unsigned long long at =
+                            atomicAdd((unsigned long long *)(run.fix + FIX_USED), (unsigned long long)(ncp + 16));
+                        room = at + (unsigned long long)(ncp + 16) <= run.fix_doubles;
+                        uint32_t *fe = in_global(run.fix) + FIX_HEAD + FIX_WORDS * (bd->fix_at + idx);
+                        fe[0] = room ? pfirst + q : FIX_VOID;
+                        fe[1] = (uint32_t)n3 | (mask << 8);
+                        fe[2] = (uint32_t)at;
+                     }
+                     if (!room) {
+                        // every class keeps the slot (its G_0 is within
+                        // rounding of the 1e-12 threshold)
+                        atomicAdd(run.fix + FIX_LOST, 1u);
                         status = 1;
                         n_any++;
                      }
@@ -707,7 +733,7 @@ void k_fm_r(const BatchDev *__restrict__ batches, const WorkRef *__restrict__ re
                         const double v = e[it & 31] * e[EXP1 + ((it >> 5) & 31)] * e[2 * EXP1 + ((it >> 10) & 31)];
                         cf[i] = it >> 15 ? 0.0 : v;
                      }
-                     double *dst = FIX ? b.fix_ws + (size_t)u * b.fix_stride : b.ac0 + (size_t)(w0 + cur) * ncp;
+                     double *dst = FIX ? fix_out : b.ac0 + (size_t)(w0 + cur) * ncp;
                      const double qsum = !FIX && has00 ? quirk[cur] : 0.0;
                      double vmax = 0.0;
                      for (int f0 = 0; f0 < nkc; f0 += FC) {
@@ -935,12 +961,14 @@ int launch_fm_r(const BatchDev *batches, const WorkRef *refs, int nref, uint32_t
    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int launch_fixup(const BatchDev *batches, size_t lds, const DevTables &t, const RunDev &run, uint32_t n_fix, void *stream)
+int launch_fixup(const BatchDev *batches, int nbatch, size_t lds, const DevTables &t, const RunDev &run, uint32_t n_fix,
+                 void *stream)
 {
+   if (nbatch > MAX_LAUNCH_CHUNKS) return -4;
    if (lds > LDS_LIMIT) return -3;
    const unsigned grid = std::max(1u, std::min(n_fix, 4096u));
    hipLaunchKernelGGL((k_fm_r<true, 8>), dim3(grid), dim3(64), lds, (hipStream_t)stream, batches,
-                      (const WorkRef *)nullptr, 0, t, run);
+                      (const WorkRef *)nullptr, nbatch, t, run);
    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -461,7 +461,7 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
    const BatchDev b = load_batch(batches, load_uniform(&refs[ri].batch), run);
    const TypePlan &tp = *b.tp;
    const int ncpt = load_uniform(&tp.ncp), nkc = load_uniform(&tp.nkc);
-   const uint32_t nfix = min(b.fix_count[0], b.fix_cap);
+   const uint32_t nfix = min(in_global(run.fix)[b.id], b.fix_cap);
    char *tab = (char *)lds;
    uint16_t *tcol = (uint16_t *)tab;
    uint32_t *urb = (uint32_t *)(tab + SQ_TAB_URB), *urk = (uint32_t *)(tab + SQ_TAB_URK);
@@ -757,11 +757,13 @@ void k_sq(const BatchDev *__restrict__ batches, const SqRef *__restrict__ refs, 
          }
          // slots of this row whose screening depends on the class
          for (uint32_t e = 0; e < nfix && win == 0; e++) {
-            const uint32_t p = b.fix[2 * e], word = b.fix[2 * e + 1];
-            if (word >> 24 != b.id || b.prm_row[p] != r) continue;
+            // (where its list begins is read again: kept, it costs registers that the rows need)
+            const uint32_t *fe = in_global(run.fix) + FIX_HEAD + FIX_WORDS * (load_uniform(&batches[b.id].fix_at) + e);
+            const uint32_t p = fe[0], word = fe[1];
+            if (p == FIX_VOID || b.prm_row[p] != r) continue;
             lds_order();
             const uint32_t mask = (word >> 8) & 0xffff, ip = b.prm_ip[p];
-            const double *src = b.fix_ws + (size_t)e * b.fix_stride;
+            const double *src = in_global(run.fix_ws) + fe[2];
             const double *A = src + (size_t)bt.comp0 * nkc + ktl.comp0;
             for (int qb = 0; qb < bt.nsp; qb++)
                for (int qk = 0; qk < ktl.nsp; qk++) {

@@ -74,11 +74,6 @@ __device__ __forceinline__ BatchDev load_batch(const BatchDev *batches, uint32_t
    b.ac0 = in_global(run.work + b.ac_off);
    b.eco = in_global(run.work + b.eco_off);
    b.stats = in_global(run.stats);
-   b.fix = in_global(run.fix);
-   b.fix_count = in_global(run.fix_count);
-   b.fix_ws = in_global(run.fix_ws);
-   b.fix_cap = run.fix_cap;
-   b.fix_stride = run.fix_stride;
    b.force_fix = run.force_fix;
    b.id = id;
    if (run.mixed != 1) b.gmag = nullptr;

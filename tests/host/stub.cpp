@@ -5,6 +5,8 @@
 
 #include <cstdlib>
 #include <cstring>
+#include <utility>
+#include <vector>
 
 #include "device.hpp"
 
@@ -75,7 +77,14 @@ int launch_zero_u32(uint32_t *p, int n, void *)
 }
 void launch_zero_f64(double *p, size_t n, void *) { std::memset(p, 0, 8 * n); }
 int launch_fm_r(const BatchDev *, const WorkRef *, int, uint32_t, int, size_t, const DevTables &, const RunDev &, void *) { return 0; }
-int launch_fixup(const BatchDev *, size_t, const DevTables &, const RunDev &, uint32_t, void *) { return 0; }
+// the fix-up entries of the last launch's chunks
+static std::vector<std::pair<uint32_t, uint32_t>> g_fix;
+int launch_fixup(const BatchDev *b, int n, size_t, const DevTables &, const RunDev &, uint32_t, void *)
+{
+   g_fix.clear();
+   for (int i = 0; i < n; i++) g_fix.emplace_back(b[i].fix_at, b[i].fix_cap);
+   return 0;
+}
 int launch_sq(const BatchDev *, const SqRef *, int, uint32_t, int, size_t, const DevTables &, const RunDev &, const KTargets &, void *)
 {
    return 0;
@@ -99,3 +108,9 @@ void fm_layouts(const TypePlan &, FmLayout &main, FmLayout &fix)
 }
 
 }  // namespace gint
+
+extern "C" {
+int stub_fix_chunks() { return (int)gint::g_fix.size(); }
+int stub_fix_at(int i) { return (int)gint::g_fix[i].first; }
+int stub_fix_cap(int i) { return (int)gint::g_fix[i].second; }
+}

@@ -1,5 +1,5 @@
 """The host engine without a GPU (tests/host): what a plan keeps while other
-calls come in between."""
+calls come in between, and the room that its launch sets have."""
 import ctypes as C
 
 import numpy as np
@@ -65,3 +65,22 @@ def test_noalloc_after_new_lattice_vectors(lib):
     lib.libgint_amd_plan_execute(h)
     assert noalloc() == 0
     lib.libgint_amd_destroy_handle(h)
+
+
+@pytest.mark.parametrize("noalloc,entries", [(False, 4096), (True, 256)])
+def test_fixup_entries_of_every_chunk(lib, noalloc, entries):
+    """every chunk of a launch set has its own entries of the fix-up list (a
+    slot beyond them is kept by every class)"""
+    from libgint_amd import driver as D
+
+    s, st, P, h, table = _planned(lib, n_water=2, n_tm=1, box_A=6.0, np_max=2, np_tm=2, seed=2)
+    if noalloc:
+        dK = np.zeros(s.P_size)
+        assert lib.libgint_amd_plan_execute_noalloc(h, P.ctypes.data, None, dK.ctypes.data, None, s.P_size) == 0
+    else:
+        lib.libgint_set_P(h, D._ptr(P), s.P_size)
+        lib.libgint_amd_plan_execute(h)
+    n = lib.stub_fix_chunks()
+    rooms = [(lib.stub_fix_at(i), lib.stub_fix_cap(i)) for i in range(n)]
+    lib.libgint_amd_destroy_handle(h)
+    assert n > 1 and rooms == [(entries * i, entries) for i in range(n)]
