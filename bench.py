@@ -273,11 +273,11 @@ def main():
             dk = float(np.max(np.abs(Km - K)))
             mixed = {"tau": a.mixed, "s_per_step": round(sum(mtimes) / len(mtimes), 4),
                      "speedup_vs_fp64": round((tot / a.steps) / (sum(mtimes) / len(mtimes)), 4),
-                     "max_abs_dK_vs_fp64": dk, "bar_Ha": 1e-8, "routed_set_quartets": int(mi[2]),
+                     "max_abs_dK_vs_fp64": dk, "bar_Ha": 1e-8, "set_quartets_below_tau": int(mi[2]),
                      "set_quartets": int(mi[3]),
-                     "path": "single-precision matrix-core contraction of the routed set quartets, the rest FP64"}
+                     "path": "single-precision contraction in k_eco for its classes of the set quartets below tau, the rest FP64"}
             log(f"mixed precision tau {a.mixed}: {mixed['s_per_step']}s per step (x{mixed['speedup_vs_fp64']}), "
-                f"routed {int(mi[2])} of {int(mi[3])} set quartets, max|dK| vs FP64 {dk:.3e}")
+                f"{int(mi[2])} of {int(mi[3])} set quartets below tau, max|dK| vs FP64 {dk:.3e}")
             lib.libgint_amd_set_mixed_precision(h, 0.0)
         tu = (C.c_double * 5)()
         lib.libgint_amd_tune_info(h, tu)

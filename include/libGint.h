@@ -159,16 +159,20 @@ void libgint_amd_set_autotune(void *handle, int on);
 /* Mixed precision for resident plans (tau = 0, the default: FP64 only).
    The first execution after plan_end (or after tau is first set) runs in
    FP64 and records each set quartet's largest primitive block element;
-   later executions send a set quartet whose bound -- that element times
+   later executions flag a set quartet whose bound -- that element times
    its largest contraction coefficients (one per centre) times its
-   primitive quartets times max |P| of the density -- is below tau to the
-   single-precision matrix-core contraction (each batch of 16 primitive
-   quartets summed in single precision, batches, HRR, spherical transform
-   and K in double precision).  The Boys function, the Hermite recursion
-   and the other classes stay FP64. */
+   primitive quartets times max |P| of the density -- is below tau.  Of a
+   flagged set quartet, the classes that the matrix-core contraction kernel
+   takes (libgint_amd_tune_info out[3]: classes of many contractions, in
+   types of many primitive quartets per row) are contracted in single
+   precision (each batch of 16 primitive quartets; batches, HRR, spherical
+   transform and K in double precision).  The other classes, and types that
+   the kernel does not take, stay FP64, as do the Boys function and the
+   Hermite recursion. */
 void libgint_amd_set_mixed_precision(void *handle, double tau);
-/* out[0] tau, [1] calibrated, [2] set quartets routed to single precision
-   by the last execution, [3] set quartets of the plan */
+/* out[0] tau, [1] calibrated, [2] set quartets flagged by the last
+   execution (below tau, also where no class of theirs has a single-precision
+   contraction), [3] set quartets of the plan */
 void libgint_amd_mixed_info(void *handle, double out[4]);
 /* out[0] the plan's kernels are chosen, [1] 0, [2], [3] classes contracted
    by k_sq itself / by k_eco, [4] 0 (seconds spent) */

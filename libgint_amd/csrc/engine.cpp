@@ -1626,7 +1626,7 @@ void Engine::launch_all(std::vector<TypeDev> &devs, const LaunchPlan &lp, const 
          if (D.gmag && launch_zero_u32((uint32_t *)D.gmag, (int)(2 * D.n_groups), stream_))
             fatal("calibration reset launch", 0);
    } else if (w.run.mixed == 2) {
-      // max |P| of this density (both spins), and the routed count from 0
+      // max |P| of this density (both spins), and the count of flagged set quartets from 0
       if (launch_zero_u32((uint32_t *)(d_mix_ + 1), 2, stream_)) fatal("route counter reset", 0);
       for (int sp = 0; sp < kt.nspin; sp++)
          if (launch_absmax(kt.P[sp], FP_size_, d_mix_, sp == 0, stream_)) fatal("max |P| launch", 0);

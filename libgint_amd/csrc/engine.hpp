@@ -416,7 +416,7 @@ class Engine {
    // max |P| is below tau take the single-precision contraction
    double mixed_tau_ = 0.0;
    bool mixed_calibrated_ = false;
-   unsigned long long *d_mix_ = nullptr;   // [0] max |P| bits, [1] set quartets routed to single precision
+   unsigned long long *d_mix_ = nullptr;   // [0] max |P| bits, [1] set quartets below tau
    void ensure_mixed();
 
    bool own_stream_ = false;

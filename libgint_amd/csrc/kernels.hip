@@ -1013,9 +1013,10 @@ __global__ void k_absmax(const double *__restrict__ P, size_t n, unsigned long l
    if ((threadIdx.x & 63) == 0) atomicMax(out, (unsigned long long)__double_as_longlong(m));
 }
 
-// The mixed-precision route of each set quartet of a chunk: single
-// precision when its bound  max|block element| x max|coefficient|^4 x
-// primitive quartets  times max|P| is below tau.  count[0] += flagged.
+// The mixed-precision flag of each set quartet of a chunk, for k_eco (where
+// k_sq contracts it, it is counted and no more): its bound  max|block
+// element| x max|coefficient|^4 x primitive quartets  times max|P| is below
+// tau.  count[0] += flagged.
 __global__ void k_mixed_flags(const BatchDev *__restrict__ batch, RunDev run, const unsigned long long *__restrict__ pmax,
                               double tau, unsigned long long *count)
 {
