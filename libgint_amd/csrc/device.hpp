@@ -108,19 +108,12 @@ struct KsRec {
 };
 static_assert(sizeof(KsRec) == 32, "KsRec layout");
 
-// Plan of one angular-momentum class: HRR layers, cart->sph, sizes.
+// One angular-momentum class: its blocks and what its recurrences cost.
 struct ClassPlan {
    int la, lb, lc, ld;
    int L, LA, LC;
    int ncp;                  // its (e0|f0) block set, e in [la,LA], f in [lc,LC], e outer
-   int cpoff[7][7];
-   int Nc, Ns;
-   int koff[4][7][7];        // ket HRR layer dd: block (e,c), e in [la,LA], c in [lc,LC-dd]
-   int ksize[4];
-   int boff[4][7];           // bra HRR layer bb: block a in [la, LA-bb]
-   int bsize[4];
-   int ycap;                 // capacity of one layer buffer (>= ncp, Nc, every layer)
-   int hrr_ws;               // HRR workspace doubles per workgroup: 3 ycap + Nc
+   int Ns;                   // spherical integrals
    // algorithmic FLOPs of the reference chain for this class
    int fm_flops;             // 52 + 211 (L+1) per surviving slot
    int vrr_flops;            // reference plan VRR (weights 3/8/3/8/11/6 per element)
@@ -219,7 +212,6 @@ struct DevTables {
    double R_cut;
 };
 
-// LDS layout of k_fm_r for one type
 // LDS of k_fm_r for a type: offsets in doubles, of the tables in bytes.
 struct FmLayout {
    int NB;      // primitive quartets per wavefront
@@ -320,7 +312,7 @@ struct EcoItem {
 struct EcoArgs {
    const EcoItem *items;      // the items of one row (the same for every row of the type)
    int n_items;
-   const int *srcmaps;        // the type's class column maps (make_cq_plan)
+   const int *srcmaps;        // the type's class column maps (make_eco_plan)
    const int *src_off;        // [MAXTC] first entry of class k's map
    const int *eco_off;        // [MAXTC] class k's offset in a row of the contraction buffer
    size_t row_doubles;        // contraction buffer doubles per row
@@ -347,7 +339,7 @@ struct SqTile {
 };
 struct SqItem {           // one (bra tile, ket tile)
    uint16_t bt, kt;
-   uint16_t lds_k, lm;    // its P and K blocks fit in LDS
+   uint16_t lds_k, pad;   // its P and K blocks fit in LDS
    int32_t eco_off;       // its class's place in a row of the contraction buffer, or -1: own contraction
    int32_t o_pk, o_c;     // LDS offsets, doubles
 };
@@ -434,15 +426,15 @@ void *noalloc_scratch();
 // zeroes n words (a kernel, not a memset node, so that the launch sequence
 // can be captured in a graph)
 int launch_zero_u32(uint32_t *p, int n, void *stream);
-// k_fm_r over the chunks of a list (pair: two primitive quartets per
-// wavefront, units are pairs), and the fix-up of the listed slots
+// k_fm_r over the chunks of a list (a unit: FmLayout::NB primitive quartets),
+// and the fix-up of the listed slots of the set's nbatch chunks
 int launch_fm_r(const BatchDev *batches, const WorkRef *refs, int nref, uint32_t units, int nacc, size_t lds,
                 const DevTables &t, const RunDev &run, void *stream);
 // Hermite functions per lane that k_fm_r takes for a type of nh: 1, 3 or 8
 inline int fm_nacc(int nh) { return nh <= 64 ? 1 : (nh <= 192 ? 3 : 8); }
 int launch_fixup(const BatchDev *batches, int nbatch, size_t lds, const DevTables &t, const RunDev &run, uint32_t n_fix,
                  void *stream);
-// the layouts of a type and whether k_fm_r takes its primitive quartets in pairs
+// the LDS layouts of a type for k_fm_r and for the fix-up
 void fm_layouts(const TypePlan &tp, FmLayout &main, FmLayout &fix);
 // orders 1 .. ldm of the caller's table in the order that k_fm_r reads them
 constexpr int CM_PAIRS = 53;   // of the 105 coefficients, the last one with a 0

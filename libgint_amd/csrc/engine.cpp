@@ -1684,7 +1684,7 @@ void Engine::replay_graph(const RunBufs &w, const KTargets &kt)
    if (!same) {
       drop_graph();
       const uint64_t s0 = n_slots_, p0 = n_prmc_;
-      const double f1 = timing_.flops[1], f2 = timing_.flops[2], f4 = timing_.flops[4];
+      const double f2 = timing_.flops[2], f4 = timing_.flops[4];
       hipGraph_t g = nullptr;
       HIPCHECK(hipStreamBeginCapture((hipStream_t)stream_, hipStreamCaptureModeThreadLocal));
       launch_all(plan_dev_, plan_lp_, w, kt);
@@ -1697,12 +1697,10 @@ void Engine::replay_graph(const RunBufs &w, const KTargets &kt)
       // host-side counts of one execution, added at every replay
       graph_counts_[0] = n_slots_ - s0;
       graph_counts_[1] = n_prmc_ - p0;
-      graph_flops_[0] = timing_.flops[1] - f1;
-      graph_flops_[1] = timing_.flops[2] - f2;
-      graph_flops_[2] = timing_.flops[4] - f4;
+      graph_flops_[0] = timing_.flops[2] - f2;
+      graph_flops_[1] = timing_.flops[4] - f4;
       n_slots_ = s0;
       n_prmc_ = p0;
-      timing_.flops[1] = f1;
       timing_.flops[2] = f2;
       timing_.flops[4] = f4;
       graph_captures_++;
@@ -1710,9 +1708,8 @@ void Engine::replay_graph(const RunBufs &w, const KTargets &kt)
    HIPCHECK(hipGraphLaunch((hipGraphExec_t)graph_exec_, (hipStream_t)stream_));
    n_slots_ += graph_counts_[0];
    n_prmc_ += graph_counts_[1];
-   timing_.flops[1] += graph_flops_[0];
-   timing_.flops[2] += graph_flops_[1];
-   timing_.flops[4] += graph_flops_[2];
+   timing_.flops[2] += graph_flops_[0];
+   timing_.flops[4] += graph_flops_[1];
    graph_replays_++;
 }
 

@@ -194,7 +194,7 @@ struct RunBufs {
 };
 
 struct Timing {
-   double ms[5] = {0, 0, 0, 0, 0};        // fm_r, (unused), sq, fixup, eco (matrix-core contraction)
+   double ms[5] = {0, 0, 0, 0, 0};        // fm_r, none, sq, fixup, eco (matrix-core contraction)
    uint64_t launches[5] = {0, 0, 0, 0, 0};
    double flops[5] = {0, 0, 0, 0, 0};     // host-counted algorithmic FLOPs of sq [2] and eco [4]
 };
@@ -428,7 +428,7 @@ class Engine {
    void *graph_exec_ = nullptr;
    uint64_t graph_key_[32] = {};
    uint64_t graph_counts_[2] = {0, 0};
-   double graph_flops_[3] = {0, 0, 0};
+   double graph_flops_[2] = {0, 0};
    uint64_t graph_captures_ = 0, graph_replays_ = 0;
 
    bool timing_on_ = false;

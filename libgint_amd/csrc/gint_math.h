@@ -224,24 +224,6 @@ GINT_HD void gint_cheb14(double x, double *t)
    for (int i = 3; i < 14; i++) t[i] = 2. * x * t[i - 1] - t[i - 2];
 }
 
-/* one derivative order of a patch expansion, in the fixed order of
-   reference src/t_c_g0_n.cpp:163-178 */
-GINT_HD double gint_cheb_sum(const double *c105, const double *T1, const double *T2)
-{
-   GINT_NO_CONTRACT
-   double tmp = 0.0;
-   int jl = 0;
-   for (int j = 0; j < 14; j++) {
-      double dot = 0.0;
-      for (int l = 0; l < 14 - j; l++) {
-         dot += T1[l] * c105[jl];
-         jl++;
-      }
-      tmp += dot * T2[j];
-   }
-   return tmp;
-}
-
 /*
  * Host-side set-up of the patch lookup: the 128 x 128 grids (cell (i1,i2)
  * belongs to the box that contains it; boxes are unions of whole cells;

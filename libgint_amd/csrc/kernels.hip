@@ -1,5 +1,6 @@
-// gfx950 kernels of the K-build.  A launch covers one chunk of one quartet
-// type (the shell structure of the four sets of a set quartet).
+// gfx950 kernels of the K-build.  A launch covers the chunks of a launch set,
+// each of one quartet type (the shell structure of the four sets of a set
+// quartet).
 //
 //   k_fm_r         one wavefront per run of primitive quartets.  Lanes evaluate
 //                  G_m(R,T) (or F_m) of 64 (quartet, cell) slots at once and decide
@@ -30,49 +31,9 @@
 namespace gint {
 
 // ---------------------------------------------------------------------------
-// cartesian and Hermite index tables, built at compile time
+// Hermite index tables, built at compile time
 // ---------------------------------------------------------------------------
 constexpr int NSHELL = 13;  // shells 0..12
-
-struct CartTables {
-   unsigned char comp[NSHELL][91][3];  // lx ly lz of component i of shell L
-   unsigned char first[NSHELL][91];    // first non-zero direction
-   signed char minus[NSHELL][91][3];   // index of i - 1_d in shell L-1, -1 if none
-   signed char plus[7][28][3];         // index of i + 1_d in shell L+1
-};
-
-constexpr int cart_index(int L, int lx, int lz) { return (L - lx) * (L - lx + 1) / 2 + lz; }
-
-constexpr CartTables make_cart_tables()
-{
-   CartTables t{};
-   for (int L = 0; L < NSHELL; L++) {
-      int i = 0;
-      for (int lx = L; lx >= 0; lx--)
-         for (int ly = L - lx; ly >= 0; ly--) {
-            int lz = L - lx - ly;
-            int v[3] = {lx, ly, lz};
-            for (int d = 0; d < 3; d++) t.comp[L][i][d] = (unsigned char)v[d];
-            t.first[L][i] = (unsigned char)(lx > 0 ? 0 : (ly > 0 ? 1 : 2));
-            for (int d = 0; d < 3; d++) {
-               if (v[d] > 0) {
-                  int w[3] = {v[0], v[1], v[2]};
-                  w[d]--;
-                  t.minus[L][i][d] = (signed char)cart_index(L - 1, w[0], w[2]);
-               } else {
-                  t.minus[L][i][d] = -1;
-               }
-               if (L < 7) {
-                  int u[3] = {v[0], v[1], v[2]};
-                  u[d]++;
-                  t.plus[L][i][d] = (signed char)cart_index(L + 1, u[0], u[2]);
-               }
-            }
-            i++;
-         }
-   }
-   return t;
-}
 
 // Hermite triples (t,u,v), ordered by N = t+u+v, then like the cartesian
 // components of shell N; the first nherm(K) entries are those with N <= K.
@@ -125,9 +86,7 @@ constexpr HermTables make_herm_tables()
    return h;
 }
 
-__constant__ CartTables c_cart = make_cart_tables();
 __constant__ HermTables c_herm = make_herm_tables();
-__device__ __forceinline__ int d_nco(int l) { return (l + 1) * (l + 2) / 2; }
 __device__ __forceinline__ int d_nherm(int L) { return (L + 1) * (L + 2) * (L + 3) / 6; }
 
 // ---------------------------------------------------------------------------
@@ -229,9 +188,10 @@ __device__ __forceinline__ unsigned long long slot_hash(uint32_t set_ij, uint32_
    return z;
 }
 
-// sum_j T2_j sum_{l<14-j} T1_l c[jl]: the operations of gint_cheb_sum in the
-// same order (so the value is bitwise the host's), with T2_j produced by
-// the recurrence of gint_cheb14 inside the loop to keep few values live
+// sum_j T2_j sum_{l<14-j} T1_l c[jl]: the operations of reference
+// src/t_c_g0_n.cpp:163-178 in the same order (so the value is bitwise the
+// oracle's), with T2_j produced by the recurrence of gint_cheb14 inside the
+// loop to keep few values live
 __device__ __forceinline__ double d_cheb_sum(const double *c, const double *T1, double x2)
 {
    GINT_NO_CONTRACT

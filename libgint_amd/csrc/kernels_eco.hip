@@ -97,7 +97,6 @@ int mfma_selftest(const double *A, const double *B, double *D, int prec)
 
 constexpr int ECO_PB = 16;   // primitive quartets per LDS batch of coefficient products
 constexpr int ECO_QB = 64;   // contractions per work item
-constexpr int ECO_JB = 64;   // columns per work item (4 wavefronts x 16)
 
 // one batch of ECO_PB primitive quartets into the wavefront's NQT tiles of
 // 16 contractions: a[kk] the lane's block element of primitive quartet
@@ -105,31 +104,25 @@ constexpr int ECO_JB = 64;   // columns per work item (4 wavefronts x 16)
 // sums the batch in a single-precision tile and adds it to the double
 // accumulators.
 template <int NQT>
-__device__ __forceinline__ void eco_batch(const double *a, const double *Wl, dbl4 *acc, bool f32, int left)
+__device__ __forceinline__ void eco_batch(const double *a, const double *Wl, dbl4 *acc, bool f32)
 {
    if (f32) {
+      flt4 s32[NQT];
 #pragma unroll
-      for (int k0 = 0; k0 < ECO_PB / 4; k0 += 4) {
-         if (4 * k0 >= left) break;
-         flt4 s32[NQT];
+      for (int t = 0; t < NQT; t++) s32[t] = flt4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-         for (int t = 0; t < NQT; t++) s32[t] = flt4{0.f, 0.f, 0.f, 0.f};
+      for (int kk = 0; kk < ECO_PB / 4; kk++)
 #pragma unroll
-         for (int kk = k0; kk < k0 + 4; kk++)
+         for (int t = 0; t < NQT; t++) s32[t] = mfma_f32_16x16x4((float)a[kk], (float)Wl[4 * kk * ECO_QB + 16 * t], s32[t]);
 #pragma unroll
-            for (int t = 0; t < NQT; t++) s32[t] = mfma_f32_16x16x4((float)a[kk], (float)Wl[4 * kk * ECO_QB + 16 * t], s32[t]);
+      for (int t = 0; t < NQT; t++)
 #pragma unroll
-         for (int t = 0; t < NQT; t++)
-#pragma unroll
-            for (int rr = 0; rr < 4; rr++) acc[t][rr] += (double)s32[t][rr];
-      }
+         for (int rr = 0; rr < 4; rr++) acc[t][rr] += (double)s32[t][rr];
    } else {
 #pragma unroll
-      for (int kk = 0; kk < ECO_PB / 4; kk++) {
-         if (kk % 4 == 0 && 4 * kk >= left) break;
+      for (int kk = 0; kk < ECO_PB / 4; kk++)
 #pragma unroll
          for (int t = 0; t < NQT; t++) acc[t] = mfma_f64_16x16x4(a[kk], Wl[4 * kk * ECO_QB + 16 * t], acc[t]);
-      }
    }
 }
 
@@ -230,10 +223,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
          if (tv) {
             const double *Wl = &W[lane >> 4][lane & 15];
             switch (nqt) {
-               case 1: eco_batch<1>(a, Wl, acc, f32, n - pb); break;
-               case 2: eco_batch<2>(a, Wl, acc, f32, n - pb); break;
-               case 3: eco_batch<3>(a, Wl, acc, f32, n - pb); break;
-               default: eco_batch<4>(a, Wl, acc, f32, n - pb); break;
+               case 1: eco_batch<1>(a, Wl, acc, f32); break;
+               case 2: eco_batch<2>(a, Wl, acc, f32); break;
+               case 3: eco_batch<3>(a, Wl, acc, f32); break;
+               default: eco_batch<4>(a, Wl, acc, f32); break;
             }
          }
       }

@@ -1,11 +1,9 @@
 // Plans of the recurrences.
 //
-// ClassPlan: horizontal (Head-Gordon-Pople) recurrence layers and
-// cartesian -> spherical sizes of one class (la lb|lc ld).  HRR2 moves b
-// onto a, HRR1 moves d onto c, the cartesian direction is the first non-zero
-// one (x, y, z), as in reference src/plan.cpp:56-146 (rec_add).  Instead of
-// a list of 19-int ops the kernels walk fixed level loops over blocks whose
-// offsets are computed here.
+// ClassPlan: the (e0|f0) blocks of one class (la lb|lc ld) and the FLOPs of
+// the reference chain for it: VRR, horizontal recurrence (HRR1 moves d onto
+// c, HRR2 b onto a, as in reference src/plan.cpp:56-146, rec_add) and
+// cartesian -> spherical transform.
 //
 // TypePlan: the union of the (e0|f0) blocks that the classes of one quartet
 // type read, the Hermite sizes of the McMurchie-Davidson path that produces
@@ -78,49 +76,22 @@ ClassPlan make_plan(int la, int lb, int lc, int ld)
    p.LA = la + lb;
    p.LC = lc + ld;
    p.L = p.LA + p.LC;
-   p.Nc = nco(la) * nco(lb) * nco(lc) * nco(ld);
    p.Ns = nsph(la) * nsph(lb) * nsph(lc) * nsph(ld);
 
    // (e0|f0) blocks that feed the HRR, e outer, f inner
-   int off = 0;
    for (int e = la; e <= p.LA; e++)
-      for (int f = lc; f <= p.LC; f++) {
-         p.cpoff[e][f] = off;
-         off += nco(e) * nco(f);
-      }
-   p.ncp = off;
-
-   // HRR layers
-   int cap = std::max(p.ncp, p.Nc);
-   for (int dd = 0; dd <= ld; dd++) {
-      off = 0;
-      for (int e = la; e <= p.LA; e++)
-         for (int c = lc; c <= p.LC - dd; c++) {
-            p.koff[dd][e][c] = off;
-            off += nco(e) * nco(c) * nco(dd);
-         }
-      p.ksize[dd] = off;
-      cap = std::max(cap, off);
-   }
-   const int ncd = nco(lc) * nco(ld);
-   for (int bb = 0; bb <= lb; bb++) {
-      off = 0;
-      for (int a = la; a <= p.LA - bb; a++) {
-         p.boff[bb][a] = off;
-         off += nco(a) * nco(bb) * ncd;
-      }
-      p.bsize[bb] = off;
-      cap = std::max(cap, off);
-   }
-   p.ycap = cap;
-   p.hrr_ws = 3 * cap + p.Nc;
+      for (int f = lc; f <= p.LC; f++) p.ncp += nco(e) * nco(f);
 
    p.fm_flops = 52 + 211 * (p.L + 1);
    p.vrr_flops = ref_vrr_flops(la, lb, lc, ld);
-   int hf = 0;
-   for (int dd = 1; dd <= ld; dd++) hf += 2 * p.ksize[dd];
-   for (int bb = 1; bb <= lb; bb++) hf += 2 * p.bsize[bb];
-   p.hrr_flops = hf;
+   // 2 per element of the HRR layers: ket layer dd of the blocks (e,c), then
+   // bra layer bb of the blocks a
+   const int ncd = nco(lc) * nco(ld);
+   for (int dd = 1; dd <= ld; dd++)
+      for (int e = la; e <= p.LA; e++)
+         for (int c = lc; c <= p.LC - dd; c++) p.hrr_flops += 2 * nco(e) * nco(c) * nco(dd);
+   for (int bb = 1; bb <= lb; bb++)
+      for (int a = la; a <= p.LA - bb; a++) p.hrr_flops += 2 * nco(a) * nco(bb) * ncd;
    {
       int dims[4] = {nco(la), nco(lb), nco(lc), nco(ld)};
       const int ls[4] = {la, lb, lc, ld};
