@@ -9,29 +9,20 @@ KTOL_ABS, KTOL_REL = 1e-10, 1e-11   # the parity bar
 
 
 def test_noalloc_reports_slots_without_an_entry(capfd):
-    import torch
-
     from libgint_amd import driver as D, load
+    from test_zz_no_alloc import Hip, _noalloc, _planned
 
     lib = load()
-    s = D.System(n_water=1, box_A=6.0, image_shells=1, np_max=3, seed=2)
-    st = s.record()
-    P = s.P()
-    h, table = D.setup_handle(lib, "libgint_", s, P=P)
-    lib.libgint_amd_plan_begin(h)
-    st.replay(table, h)
-    lib.libgint_amd_plan_end(h)
-    dP = torch.from_numpy(P).cuda()
+    hip = Hip()
+    s, st, P, h = _planned(lib, D, dict(n_water=1, box_A=6.0, image_shells=1, np_max=3, seed=2))
     K = []
     for debug in (0, 1):
-        dK = torch.zeros_like(dP)
-        torch.cuda.synchronize()
         lib.libgint_amd_set_debug(h, debug)
-        assert lib.libgint_amd_plan_execute_noalloc(h, dP.data_ptr(), None, dK.data_ptr(), None, s.P_size) == 0
-        lib.libgint_amd_synchronize(h)
-        K.append(dK.cpu().numpy())
+        rc, k = _noalloc(lib, hip, s, h, P)
+        assert rc == 0
+        K.append(k)
         said = capfd.readouterr().err
-        print("debug", debug, "max|K|", np.max(np.abs(K[-1])), said)
+        print("debug", debug, "max|K|", np.max(np.abs(k)), said)
         assert ("beyond the fix-up list" in said) == (debug == 1)
     lib.libgint_amd_destroy_handle(h)
     assert np.max(np.abs(K[0])) > 0
