@@ -457,10 +457,15 @@ void make_sq_plan(const TypePlan &tp, const EcoPlan &ep, int grp, int nspin, boo
 // k_sq<4>'s items of at most this much LDS (bytes, without the coefficients)
 // are launched apart: a launch takes the LDS of its largest item (48 KB of an
 // (ff|ff) class), three times the mean.  64 molecules in f shells: 20.1 ->
-// 17.0 ms.  Not so the other kernels, whose items come to 17 KB at most: apart
-// they read a set quartet's blocks twice, 47.5 -> 53.2 ms with s to f shells.
+// 17.0 ms.  Not so the other kernels, whose items come to 16.3 KB at most (20.3
+// with two spins): apart they read a set quartet's blocks twice, 47.5 -> 53.2
+// ms with s to f shells.
 constexpr int SQ_SMALL_LDS = 18 * 1024;
-constexpr size_t SQ_TYPE_LDS = 13 * 1024 + 256;   // twelve wavefronts per CU, what k_sq<1..3>'s registers allow
+// Types of at most this much LDS with the coefficients are launched apart in
+// k_sq<1..3>: twelve wavefronts per CU, what the registers of k_sq<1> and <2>
+// allow.  k_sq<3>'s allow eight; a line of its own there (20 KB) is no
+// different, K-builds with f shells 51.4 for 51.5 ms, s to f 94.0 for 94.0.
+constexpr size_t SQ_TYPE_LDS = 13 * 1024 + 256;
 constexpr int SQ_GROUPS = 3;   // register groups of k_sq's items
 constexpr int SQ_KERNELS = 4;  // k_sq<1..4>: s and p shells; and d; and f with a transform no larger than (dd|'s; any
 int launch_eco(const BatchDev *batch, const RunDev &run, uint32_t nrow, const EcoArgs &e, void *stream);

@@ -409,7 +409,16 @@ class Engine {
    double *d_P_[2] = {nullptr, nullptr};
    double *d_K_[2] = {nullptr, nullptr};
 
-   // primitive quartets per row from which a type's contraction runs on the matrix cores
+   // Primitive quartets per row of a type from which k_eco contracts it.  The
+   // line was put where all types of the K-builds with spdf centres gain and
+   // is no crossover: that lies by the contractions.  K-build ms with k_eco
+   // and with k_sq's own contraction, mean primitive quartets per row:
+   //   s to f shells of 4 to 1 contractions  9: 2.8 / 2.3   28: 3.0 / 5.6
+   //                                         105: 2.6 / 8.7   1059: 22.6 / 156
+   //   O 3s2p1d, H 2s1p                      21: 0.66 / 0.46   129: 0.56 / 0.44
+   //                                         205: 1.5 / 1.1
+   //   O 4s3p2d1f, H 3s2p1d                  25: 1.6 / 1.4   102: 1.2 / 1.0
+   //                                         544: 10.2 / 9.2
    static constexpr double ECO_MIN_PRM = 96.0;
 
    // mixed precision (plans): set quartets whose calibrated bound times

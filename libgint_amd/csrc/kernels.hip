@@ -317,9 +317,8 @@ static FmLayout fm_layout(const TypePlan &tp, bool fix)
 // types, for LDS) and four results per lane in the transform brought 5.0
 // million quartets in 27 cells from 53.7 to 19.5 ms, 6.1 million with s to f
 // shells in 125 cells from 81 to 24.4, a cluster of 1.1 million from 9.8 to
-// 2.9.  What bounds it now is latency: a wavefront waits 70% of its time,
-// mostly for LDS in the recursion and the transform (two fifths and a third
-// of it), and the vector units are busy a quarter.
+// 2.9.  What bounds it now is latency: a wavefront waits in 59 to 64% of its
+// cycles, and the vector units are busy 14 (NACC 8) to 40% (NACC 1).
 //
 // At most 168 VGPRs (3 wavefronts per SIMD): with 128 more values go to
 // scratch in the loops, 23.2 instead of 19.5 ms.

@@ -26,6 +26,11 @@
 // columns, so the items are ordered by the first column they read and an
 // XCD takes runs of them: items that read the same columns run together,
 // through one L2.
+//
+// Bound: memory.  64 molecules and 8 spdf centres (every 16th set quartet):
+// 5.9 TB/s of reads (requests of 128 bytes, as a copy makes them) at 23.8
+// TFLOP/s, 30% of the matrix cores' rate; a large copy reaches 5.4 TB/s.
+// With 195 k of the 37 M set quartets 3.7 TB/s.
 #include <hip/hip_runtime.h>
 
 #include "device.hpp"

@@ -31,12 +31,13 @@
 //   - the item's set-up: all of its loads that do not wait for each other at
 //     once, instead of a load after another per shell (28 k -> 12 k cycles)
 //   - the items of a set quartet on one XCD, so that its blocks come from one
-//     L2 (xcd_run: 72 -> 29 GB from memory, 58 -> 46 ms; runs of 16 items 50,
-//     of 512 49; of k_sq<4>'s large items 16 are better, 27.5 for 28.4 ms)
+//     L2 (xcd_run: 172 -> 57 GB from memory and 42.8 -> 32.2 ms; at 46 ms
+//     runs of 16 items took 50, of 512 49; of k_sq<4>'s large items 16 are
+//     better, 27.5 for 28.4 ms)
 //   - tiles of at most 42 rows x 32 columns: whole matrix-core tiles of 16
-//     columns, and LDS (17 KB at most) for eight wavefronts per CU or more
-//     (38 x 38: 45.7, 30 x 38: 44.0, 35 x 32: 42.1, but 34 for 29.6 ms in f
-//     shells)
+//     columns, and LDS (16 KB at most with one spin, 20 with two, and the
+//     coefficients) for eight wavefronts per CU or more (38 x 38: 45.7,
+//     30 x 38: 44.0, 35 x 32: 42.1, but 34 for 29.6 ms in f shells)
 //   - in the contraction four independent matrix-core chains, with the next
 //     loads in flight (f shells: 58 -> 53 ms) and weights taken per column
 //     from the coefficients, not from a table of the window
@@ -46,8 +47,9 @@
 //   - matrix-core tiles of 4 rows for tiles of at most 8 units (39 -> 34 ms)
 //   - the contraction's loads at a uniform base plus 32 bits per lane instead
 //     of 64-bit addresses (K-build with s to f shells 96.5 -> 95.7 ms)
-// Bound: latency and instruction issue, at two wavefronts per SIMD (waits in
-// 41% of the wave cycles, VALU busy 34%; HBM 1 TB/s).
+// Bound: latency and instruction issue, at 2.4 wavefronts per SIMD (k_sq<3>
+// 1.9, k_sq<4> 1.2): waits in 44 to 49% of the wave cycles, VALU busy 21 to
+// 42%, matrix cores 6 to 27%; 0.5 to 2.5 TB/s from memory.
 #pragma once
 #include <hip/hip_runtime.h>
 
