@@ -148,7 +148,7 @@ def main():
     ap.add_argument("--roof-only", action="store_true",
                     help="only the roofline's serialised sample run (for kernel-trace and counter profiles)")
     ap.add_argument("--no-progress", dest="progress", action="store_false",
-                    help="no per-quartet-type progress lines (and no host wait per type) in the steps")
+                    help="no progress line (and host wait) per launch set in the steps")
     a = ap.parse_args()
     if a.gpus != 1:
         print(json.dumps({"error": "this build measures one GPU; multi-GPU runs are not part of it",
@@ -218,8 +218,8 @@ def main():
         lib.libgint_amd_plan_info(h, info)
         log(f"set-level ingestion {t_ing:.1f}s, resident plan {info[0] / 2**30:.2f} GiB, {info[1]} quartet types, "
             f"{info[2]} chunks")
-        # debug bit 2: the engine waits for each quartet type's work and reports
-        # it (progress of long K-builds; one host wait per type, ~40 per step)
+        # debug bit 2: the engine waits for each launch set's work and reports
+        # it (progress of long K-builds; one host wait per set, 89 per step)
         lib.libgint_amd_set_debug(h, 4 if a.progress else 0)
 
         def step(PP=P, out=K):
