@@ -1234,7 +1234,7 @@ void Engine::ensure_work(const LaunchPlan &lp)
       synchronize();
       if (d_fix_) HIPCHECK(hipFree(d_fix_));
       HIPCHECK(hipMalloc((void **)&d_fix_, sizeof(uint32_t) * (FIX_HEAD + FIX_WORDS * lp.n_fix)));
-      HIPCHECK(hipMemset(d_fix_, 0, sizeof(uint32_t) * FIX_HEAD));
+      if (launch_zero_u32(d_fix_, FIX_HEAD, stream_)) fatal("counter reset launch", 0);   // in order with the kernels
       fix_cap_ = lp.n_fix;
    }
    if (lp.fix_doubles > fix_ws_cap_) {
